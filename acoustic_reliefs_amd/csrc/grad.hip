@@ -22,272 +22,274 @@
 
 namespace arh {
 
-constexpr int kGT = 128;  // threads per workgroup (A and C: one touched element each; B: a quad of lanes each)
-// Rhs per lane and pass. A quad of lanes shares one touched element: the lanes split the quadrature points
-// of its derivatives and sum them with lane swaps, then each lane accumulates every fourth rhs, so a pass
-// covers 4 kRQ right-hand sides and evaluates each derivative once (37 plane waves: 2 passes; 5 per lane keeps
-// the kernels at 2 waves per SIMD, which measured faster than one pass at 1 wave).
-#ifndef ARH_GRAD_RQ
-#define ARH_GRAD_RQ 5
-#endif
-constexpr int kRQ = ARH_GRAD_RQ;
+// Restructured over the right-hand sides too: the sums over rhs and over elements commute, so
+//   B_(i,c) = Re sum_e ( dM_ie/dp_i G(i,e) + dM_ei/dq_(i,c) G(e,i) ),  G(i,e) = sum_rhs lam_i x_e,
+//   A_(i,c) = Re sum_l dQ_li/dq_(i,c) W(i,l),                          W(i,l) = sum_rhs x_i vf_l,
+// and a derivative is evaluated once per pair whatever the number of right-hand sides. G and W are GEMMs: a
+// wavefront forms a 16 x 16 tile of pairs with v_mfma_f64_16x16x4_f64 and consumes it from the accumulators,
+// so they are never stored.
+//
+// Per pair, with ir = 1 / r and the quadrature sums over a triangle's six points (weights w, beta the corner's
+// barycentric coordinate): s = -(d . n) does not depend on the point (q stays in the triangle's plane, so
+// d . n = (p - a) . n), and neither does beta_c n_y - d . dn_c, the y derivative of d . n for a moving corner
+// (it is linear in q). With D_c = (p - a) . dn_c it equals n_y - D_a for corner a and -D_b, -D_c for the others:
+//   dM_ie/dp_i     = (s sum w F' d_y ir - n_y sum w F) / 6
+//   dM_ei/dq_(i,c) = (-s sum w beta_c F' d_y ir + (n_y [c = a] - D_c) sum w F) / 2.
+//
+// Bound by FP64 VALU issue: about 68 FP64 operations per quadrature point, 12 points per pair, against 4 MFMAs per
+// two right-hand sides for 256 pairs. Reciprocal distances come from one v_rsq_f64 and one cubic correction step
+// (below 1 ulp) instead of a square root and five divisions. The loop over a lane's four pairs stays rolled: unrolled
+// it needs 249 registers, 2 wavefronts per SIMD instead of 3, and 3-5 % more time; 4 wavefronts spill (+14 %).
+// N = 9,828 with 8,190 touched elements, 8e7 pairs: 3.1 ms for one right-hand side and 4.6 ms for 37, where
+// accumulating every right-hand side's sums per lane took 10.3 ms and 24.6 ms (two passes, each with its own
+// derivatives); 1297 listeners, one right-hand side: 0.24 ms from 2.6 ms.
+constexpr int kGW = 4;           // wavefronts per workgroup; they take every kGW-th 16-column tile of the split
+constexpr int kGT = 64 * kGW;
+constexpr int kGSlots = 2048;    // workgroups aimed for (8 per compute unit): the column range is split to reach it
 
-__device__ __forceinline__ void FdF(double k, double r, double2 &F, double2 &dF) {
-    double sn, cs;
-    trig_sincos(k * r, &sn, &cs);
-    const double r2 = r * r, r3 = r2 * r, r4 = r2 * r2;
-    const double kr = k * r;
-    const double inv4pi = 1.0 / (4.0 * kPi);
-    F = make_double2((-cs - kr * sn) / r3 * inv4pi, (sn - kr * cs) / r3 * inv4pi);
-    const double A = -k * k / r2 + 3.0 / r4, B = 3.0 * k / r3;
-    dF = make_double2((cs * A + sn * B) * inv4pi, (cs * B - sn * A) * inv4pi);
+typedef double V4d __attribute__((ext_vector_type(4)));
+
+// 1 / sqrt(x): with e = 1 - x y^2 of the hardware's y (about 2^-24), y (1 + e / 2 + 3 e^2 / 8) leaves O(e^3).
+__device__ __forceinline__ double rsqrt_f64(double x) {
+    const double y = __builtin_amdgcn_rsq(x);
+    const double e = fma(-x * y, y, 1.0);
+    return fma(y * e, fma(0.375, e, 0.5), y);
 }
 
-// The value of another lane of the quad (DPP quad permutation CTRL; every lane of the quad is active).
+// Kernel factors at distance vector d without the 1 / (4 pi): F = e^{-ikr} (-1 - ikr) / r^3 and
+// H = d_y / r e^{-ikr} (-k^2 / r^2 + 3 (1 + ikr) / r^4).
+__device__ __forceinline__ void FdF(double k, double dx, double dy, double dz, double2 &F, double2 &H) {
+    const double r2 = fma(dx, dx, fma(dy, dy, dz * dz));
+    const double ir = rsqrt_f64(r2);
+    const double kr = k * (r2 * ir);
+    double sn, cs;
+    trig_sincos(kr, &sn, &cs);
+    const double ir2 = ir * ir, ir3 = ir2 * ir;
+    F = make_double2(fma(-kr, sn, -cs) * ir3, fma(-kr, cs, sn) * ir3);
+    const double g = dy * ir * ir2;
+    const double A = fma(3.0, ir2, -k * k) * g, B = 3.0 * k * ir * g;
+    H = make_double2(fma(cs, A, sn * B), fma(cs, B, -sn * A));
+}
+
+// Rows of a pair tile: the touched elements' derived geometry, in LDS (wavefront lanes of one row read the same
+// address, rows are an odd number of doubles apart).
+struct GradRow {
+    double q[6][3];         // quadrature points
+    double ax, ay, az, nx, ny, nz, gx, gy, gz;
+    double cx, cz, bx, bz;  // c - a and b - a (dn of the corners)
+    double pad[2];
+};
+static_assert(sizeof(GradRow) % 16 == 8, "odd number of doubles");
+
+// Right-hand-side values element by element for the pair GEMMs: row e holds (re, im) of the R values of one vector
+// set, zero-padded to K = 4 ceil(R / 2) reals.
+__global__ void k_grad_pack(int N, int R, int K, const double2 *__restrict__ x, double *__restrict__ out) {
+    const int64_t q = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
+    const int h = K / 2;
+    if (q >= (int64_t)N * h) return;
+    const int e = (int)(q / h), j = (int)(q % h);
+    reinterpret_cast<double2 *>(out)[q] = j < R ? x[(int64_t)j * N + e] : make_double2(0.0, 0.0);
+}
+
+// Tile of sum_k of the complex products a_i b_e over the packed rows: re and im parts, v_mfma_f64_16x16x4 (A[i][k]
+// in lane i + 16 k, B[k][e] in lane e + 16 k, D[i][e] in lane e + 16 (i % 4), element i / 4). Reals alternate
+// (re, im): re = sum +-a[k] b[k], im = sum a[k ^ 1] b[k].
+__device__ __forceinline__ void pair_gemm(const double *__restrict__ a, const double *__restrict__ b, int K, int kk,
+                                          V4d &re, V4d &im) {
+    const double sg = (kk & 1) ? -1.0 : 1.0;
+#pragma unroll 2
+    for (int k = 0; k < K; k += 4) {
+        const double a0 = a[k + kk] * sg, a1 = a[k + (kk ^ 1)], bk = b[k + kk];
+        re = __builtin_amdgcn_mfma_f64_16x16x4f64(a0, bk, re, 0, 0, 0);
+        im = __builtin_amdgcn_mfma_f64_16x16x4f64(a1, bk, im, 0, 0, 0);
+    }
+}
+
+// Sum of v over the 16 lanes of a row (DPP row rotations by 8, 4, 2, 1), the same in every lane.
 template <int CTRL>
-__device__ __forceinline__ double quad_swap(double x) {
+__device__ __forceinline__ double row_ror(double x) {
     const int lo = __builtin_amdgcn_mov_dpp(__double2loint(x), CTRL, 0xF, 0xF, false);
     const int hi = __builtin_amdgcn_mov_dpp(__double2hiint(x), CTRL, 0xF, 0xF, false);
     return __hiloint2double(hi, lo);
 }
-
-// Sum of v over the 4 lanes of a quad: (l0 + l1) + (l2 + l3), the same bits in every lane.
-__device__ __forceinline__ double quad_sum(double v) {
-    v += quad_swap<0xB1>(v);  // quad_perm [1, 0, 3, 2]
-    v += quad_swap<0x4E>(v);  // quad_perm [2, 3, 0, 1]
+__device__ __forceinline__ double row16_sum(double v) {
+    v += row_ror<0x128>(v);
+    v += row_ror<0x124>(v);
+    v += row_ror<0x122>(v);
+    v += row_ror<0x121>(v);
     return v;
 }
 
-// One lane's share of the two derivatives of pair (collocation i, element e): quadrature points
-// g = q4, q4 + 4, q4 + 8 of the list {dM_ie/dp_i: rule points 0..5 on triangle e, collocation centroid i;
-// dM_ei/dq_(i,c): rule points 0..5 on triangle i, collocation centroid e}. Both kinds share the distance
-// and kernel factors; each point's weight goes to its own kind only (the other is multiplied by 0).
-__device__ __forceinline__ void dM_share(double k, const Tri &ti, const Tri &te, int q4, double2 &dp, double2 dq[3]) {
-    const double bcx = ti.bx - ti.cx, bcz = ti.bz - ti.cz;  // dn of triangle i's corners (x and z only)
-    const double dnx[3] = {bcz, ti.cz, -ti.bz};
-    const double dnz[3] = {-bcx, -ti.cx, ti.bx};
-    dp = make_double2(0.0, 0.0);
+// Partial sums over a range of columns for 16 touched elements. Columns are elements (LISTEN false: B) or
+// listeners (LISTEN true: A); grid (row tiles, column splits); out[(split * T + t) * 3 + c]. xi, li: packed x and
+// lambda by element; pc: the columns' packed values that multiply x_i (lambda by element, or vf by listener).
+template <bool LISTEN>
+__global__ __launch_bounds__(kGT, 3) void k_grad_pairs(const Tri *__restrict__ tri, const double *__restrict__ L, int ncol,
+                                                    int T, const int *__restrict__ touched, double k, int K,
+                                                    const double *__restrict__ xp, const double *__restrict__ lp,
+                                                    const double *__restrict__ pc, int nsplit,
+                                                    double *__restrict__ out) {
+    __shared__ GradRow rows[16];
+    __shared__ double red[kGW][16][3];
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    const int i16 = lane & 15, kk = lane >> 4;
+    const int t0 = (int)blockIdx.x * 16, sp = blockIdx.y;
+    if (threadIdx.x < 16) {
+        const Tri t = tri[touched[min(t0 + (int)threadIdx.x, T - 1)]];  // surplus rows repeat the last, unused
+        GradRow &r = rows[threadIdx.x];
 #pragma unroll
-    for (int c = 0; c < 3; c++) dq[c] = make_double2(0.0, 0.0);
-#pragma unroll
-    for (int m = 0; m < 3; m++) {
-        const int g = q4 + 4 * m;
-        const bool isq = g >= 6;
-        double w, xi, eta;
-        quad_point(isq ? g - 6 : g, w, xi, eta);
-        const Tri &t = isq ? ti : te;                // integration triangle
-        const double px = isq ? te.gx : ti.gx, py = isq ? te.gy : ti.gy, pz = isq ? te.gz : ti.gz;
-        const double dx = px - (t.ax + xi * t.bx + eta * t.cx);
-        const double dy = py - (t.ay + xi * t.by + eta * t.cy);
-        const double dz = pz - (t.az + xi * t.bz + eta * t.cz);
-        const double r = sqrt(dx * dx + dy * dy + dz * dz);
-        const double sn_ = -(dx * t.nx + dy * t.ny + dz * t.nz);
-        double2 F, dF;
-        FdF(k, r, F, dF);
-        const double a = dy * sn_ / r;
-        const double wp = isq ? 0.0 : w, wq = isq ? w : 0.0;
-        dp.x += wp * (dF.x * a - F.x * t.ny);
-        dp.y += wp * (dF.y * a - F.y * t.ny);
-        const double beta[3] = {1.0 - xi - eta, xi, eta};
-#pragma unroll
-        for (int c = 0; c < 3; c++) {
-            const double f1 = -beta[c] * a;
-            const double f2 = beta[c] * t.ny - (dx * dnx[c] + dz * dnz[c]);
-            dq[c].x += wq * (dF.x * f1 + F.x * f2);
-            dq[c].y += wq * (dF.y * f1 + F.y * f2);
+        for (int g = 0; g < 6; g++) {
+            double wt, xi, eta;
+            quad_point(g, wt, xi, eta);
+            r.q[g][0] = t.ax + xi * t.bx + eta * t.cx;
+            r.q[g][1] = t.ay + xi * t.by + eta * t.cy;
+            r.q[g][2] = t.az + xi * t.bz + eta * t.cz;
         }
+        r.ax = t.ax, r.ay = t.ay, r.az = t.az, r.nx = t.nx, r.ny = t.ny, r.nz = t.nz;
+        r.gx = t.gx, r.gy = t.gy, r.gz = t.gz;
+        r.bx = t.bx, r.bz = t.bz, r.cx = t.cx, r.cz = t.cz;
     }
-    dp = make_double2(quad_sum(dp.x) * (0.5 / 3.0), quad_sum(dp.y) * (0.5 / 3.0));
-#pragma unroll
-    for (int c = 0; c < 3; c++) dq[c] = make_double2(quad_sum(dq[c].x) * 0.5, quad_sum(dq[c].y) * 0.5);
-}
-
-// Element-major copy of x and lambda: xl[(e * R + j) * 2] = x_j[e], xl[(e * R + j) * 2 + 1] = lambda_j[e], so the
-// rhs values a quad reads for one element share a few cache lines.
-__global__ void k_grad_pack(int N, int R, const double2 *__restrict__ x, const double2 *__restrict__ lam,
-                            double2 *__restrict__ xl) {
-    const int64_t q = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-    if (q >= (int64_t)N * R) return;
-    const int e = (int)(q / R), j = (int)(q % R);
-    xl[2 * q] = x[(int64_t)j * N + e];
-    xl[2 * q + 1] = lam[(int64_t)j * N + e];
-}
-
-// B partials: grid.x over touched elements (a quad of lanes each), grid.y splits the element loop; adds
-// to partB[(split * T + t) * 3 + c] (one pass over rhs j0..j0 + 4 kRQ - 1; passes accumulate).
-__global__ __launch_bounds__(kGT) void k_grad_B(const Tri *__restrict__ tri, int N, int T, const int *__restrict__ touched,
-                                                double k, int R, int j0, const double2 *__restrict__ x,
-                                                const double2 *__restrict__ lam, const double2 *__restrict__ xl,
-                                                int esplit, double *__restrict__ partB) {
-    const int t = (int)((blockIdx.x * kGT + threadIdx.x) >> 2), q4 = threadIdx.x & 3;
-    const int sp = blockIdx.y;
-    if (t >= T) return;  // the whole quad leaves together
-    const int i = touched[t];
-    const Tri ti = tri[i];
-    const int len = (N + esplit - 1) / esplit;
-    const int e0 = sp * len, e1 = min(N, e0 + len);
-    double2 s1[kRQ], s2[kRQ][3];
-#pragma unroll
-    for (int m = 0; m < kRQ; m++) {
-        s1[m] = make_double2(0.0, 0.0);
-        for (int c = 0; c < 3; c++) s2[m][c] = make_double2(0.0, 0.0);
-    }
-    for (int e = e0; e < e1; e++) {
-        const Tri te = tri[e];
-        double2 dp, dq[3];
-        dM_share(k, ti, te, q4, dp, dq);  // dM_ie/dp_i (collocation i moves), dM_ei/dq_(i,c) (corner c moves)
-#pragma unroll
-        for (int m = 0; m < kRQ; m++) {
-            const int j = j0 + q4 + 4 * m;
-            if (j < R) {
-                const double2 xe = xl[((int64_t)e * R + j) * 2];
-                const double2 le = xl[((int64_t)e * R + j) * 2 + 1];
-                cfma(s1[m], xe, dp);
-#pragma unroll
-                for (int c = 0; c < 3; c++) cfma(s2[m][c], le, dq[c]);
-            }
+    const int64_t ei = touched[min(t0 + i16, T - 1)];  // the row whose packed values this lane feeds
+    const double *xa = xp + ei * K, *la = LISTEN ? nullptr : lp + ei * K;
+    __syncthreads();
+    double acc[3] = {0.0, 0.0, 0.0};  // lane i16 = v holds row 4 v + kk
+    const int ntile = (ncol + 15) >> 4;
+    const int c0 = (int)((int64_t)ntile * sp / nsplit), c1 = (int)((int64_t)ntile * (sp + 1) / nsplit);
+    for (int ct = c0 + w; ct < c1; ct += kGW) {
+        const int e = min(ct * 16 + i16, ncol - 1);
+        const bool on = ct * 16 + i16 < ncol;  // surplus columns repeat the last, not added
+        V4d gr = {0, 0, 0, 0}, gi = {0, 0, 0, 0}, hr = {0, 0, 0, 0}, hi = {0, 0, 0, 0};
+        pair_gemm(xa, pc + (int64_t)e * K, K, kk, hr, hi);
+        Tri te{};
+        double px, py, pz;  // the column's collocation point
+        if constexpr (LISTEN) {
+            px = L[3 * e], py = L[3 * e + 1], pz = L[3 * e + 2];
+        } else {
+            pair_gemm(la, xp + (int64_t)e * K, K, kk, gr, gi);
+            te = tri[e];
+            px = te.gx, py = te.gy, pz = te.gz;
         }
-    }
-    double out[3] = {0.0, 0.0, 0.0};
+#pragma unroll 1
+        for (int v = 0; v < 4; v++) {
+            const GradRow &r = rows[v * 4 + kk];
+            double d = 0.0;
+            if constexpr (!LISTEN) {
+                // dM_ie/dp_i: rule points on the column's triangle, collocation at the row's centroid
+                double2 SF[2], SH[2];
 #pragma unroll
-    for (int m = 0; m < kRQ; m++) {
-        const int j = j0 + q4 + 4 * m;
-        if (j < R) {
-            const double2 li = lam[(int64_t)j * N + i];
-            const double2 xi = x[(int64_t)j * N + i];
-            const double a = cmul(s1[m], li).x;
+                for (int h = 0; h < 2; h++) {
+                    SF[h] = SH[h] = make_double2(0.0, 0.0);
 #pragma unroll
-            for (int c = 0; c < 3; c++) out[c] += a + cmul(s2[m][c], xi).x;
-        }
-    }
-#pragma unroll
-    for (int c = 0; c < 3; c++) out[c] = quad_sum(out[c]);
-    if (q4 == 0)
-#pragma unroll
-        for (int c = 0; c < 3; c++) partB[((int64_t)sp * T + t) * 3 + c] += out[c];
-}
-
-// dM(p, tri)/dq_c for corner c = 0, 1, 2 of the integration triangle moving in y (sum over the rule, times
-// 1/2): lane q4 of the quad takes rule points q4 and q4 + 4 (< 6), and the quad sums the shares.
-__device__ __forceinline__ void dM_dq3_quad(double k, double px, double py, double pz, const Tri &t, int q4,
-                                            double2 out[3]) {
-    const double bcx = t.bx - t.cx, bcz = t.bz - t.cz;
-    const double dnx[3] = {bcz, t.cz, -t.bz};
-    const double dnz[3] = {-bcx, -t.cx, t.bx};
-#pragma unroll
-    for (int c = 0; c < 3; c++) out[c] = make_double2(0.0, 0.0);
-#pragma unroll
-    for (int m = 0; m < 2; m++) {
-        const int g = q4 + 4 * m;
-        double w, xi, eta;
-        quad_point(g < 6 ? g : 0, w, xi, eta);
-        if (g >= 6) w = 0.0;  // lanes 2 and 3 have one point
-        const double dx = px - (t.ax + xi * t.bx + eta * t.cx);
-        const double dy = py - (t.ay + xi * t.by + eta * t.cy);
-        const double dz = pz - (t.az + xi * t.bz + eta * t.cz);
-        const double r = sqrt(dx * dx + dy * dy + dz * dz);
-        const double sn_ = -(dx * t.nx + dy * t.ny + dz * t.nz);
-        double2 F, dF;
-        FdF(k, r, F, dF);
-        const double beta[3] = {1.0 - xi - eta, xi, eta};
-        const double a = dy * sn_ / r;
-#pragma unroll
-        for (int c = 0; c < 3; c++) {
-            const double f1 = -beta[c] * a;
-            const double f2 = beta[c] * t.ny - (dx * dnx[c] + dz * dnz[c]);
-            out[c].x += w * (dF.x * f1 + F.x * f2);
-            out[c].y += w * (dF.y * f1 + F.y * f2);
-        }
-    }
-#pragma unroll
-    for (int c = 0; c < 3; c++) out[c] = make_double2(quad_sum(out[c].x) * 0.5, quad_sum(out[c].y) * 0.5);
-}
-
-// A and C per touched element, a quad of lanes each (listeners: LL is small). The lanes split each
-// listener derivative's rule points, then lane q4 accumulates rhs j = q4, q4 + 4, ... (passes of 4 kRQ),
-// so a derivative is evaluated once per pass rather than once per rhs.
-__global__ __launch_bounds__(kGT) void k_grad_AC(const Tri *__restrict__ tri, int N, int T,
-                                                 const int *__restrict__ touched, double k, int R,
-                                                 const double2 *__restrict__ x, const double2 *__restrict__ lam,
-                                                 const double2 *__restrict__ vf, const double *__restrict__ L, int LL,
-                                                 int src_kind, const double *__restrict__ src,
-                                                 double *__restrict__ cA, double *__restrict__ cC) {
-    const int t = (int)((blockIdx.x * kGT + threadIdx.x) >> 2), q4 = threadIdx.x & 3;
-    if (t >= T) return;  // the whole quad leaves together
-    const int i = touched[t];
-    const Tri ti = tri[i];
-    double a[3] = {0.0, 0.0, 0.0}, cc = 0.0;
-    for (int j0 = 0; j0 < R; j0 += 4 * kRQ) {
-        double2 sa[kRQ][3];
-#pragma unroll
-        for (int m = 0; m < kRQ; m++)
-#pragma unroll
-            for (int c = 0; c < 3; c++) sa[m][c] = make_double2(0.0, 0.0);
-        for (int l = 0; l < LL; l++) {
-            double2 dq[3];
-            dM_dq3_quad(k, L[3 * l], L[3 * l + 1], L[3 * l + 2], ti, q4, dq);
-#pragma unroll
-            for (int m = 0; m < kRQ; m++) {
-                const int j = j0 + q4 + 4 * m;
-                if (j < R) {
-                    const double2 v = vf[(int64_t)j * LL + l];
-#pragma unroll
-                    for (int c = 0; c < 3; c++) cfma(sa[m][c], v, dq[c]);
+                    for (int g = 3 * h; g < 3 * h + 3; g++) {
+                        double wt, xi, eta;
+                        quad_point(g, wt, xi, eta);
+                        const double dx = r.gx - (te.ax + xi * te.bx + eta * te.cx);
+                        const double dy = r.gy - (te.ay + xi * te.by + eta * te.cy);
+                        const double dz = r.gz - (te.az + xi * te.bz + eta * te.cz);
+                        double2 F, H;
+                        FdF(k, dx, dy, dz, F, H);
+                        SF[h] = cadd(SF[h], F);
+                        SH[h] = cadd(SH[h], H);
+                    }
                 }
+                const double s = -((r.gx - te.ax) * te.nx + (r.gy - te.ay) * te.ny + (r.gz - te.az) * te.nz);
+                const double fa = ARH_QW_A * (kInv8Pi / 3.0), fb = ARH_QW_B * (kInv8Pi / 3.0);
+                const double dpx = s * (fa * SH[0].x + fb * SH[1].x) - te.ny * (fa * SF[0].x + fb * SF[1].x);
+                const double dpy = s * (fa * SH[0].y + fb * SH[1].y) - te.ny * (fa * SF[0].y + fb * SF[1].y);
+                d = dpx * gr[v] - dpy * gi[v];
             }
-        }
+            // dM_ei/dq_(i,c): rule points on the row's triangle, collocation at the column's point
+            double2 S0 = make_double2(0.0, 0.0), T0 = S0, T1 = S0, T2 = S0;
 #pragma unroll
-        for (int m = 0; m < kRQ; m++) {
-            const int j = j0 + q4 + 4 * m;
-            if (j >= R) continue;
-            const double2 xi = x[(int64_t)j * N + i];
-#pragma unroll
-            for (int c = 0; c < 3; c++) a[c] += cmul(sa[m][c], xi).x;
-            // db_i / dh
-            double2 db;
-            const double sx = src[3 * j], sy = src[3 * j + 1], sz = src[3 * j + 2];
-            if (src_kind == ARH_RHS_POINT) {
-                const double dx = ti.gx - sx, dy = ti.gy - sy, dz = ti.gz - sz;
-                const double r = sqrt(dx * dx + dy * dy + dz * dz);
-                double sn, cs;
-                trig_sincos(k * r, &sn, &cs);
-                // e^{-ikr}(-1 - ikr) / (4 pi r^2) * d_y / (3 r)
-                const double f = dy / (3.0 * r) / (4.0 * kPi * r * r);
-                db = make_double2((-cs - k * r * sn) * f, (sn - k * r * cs) * f);
-            } else {
-                double sn, cs;
-                trig_sincos(k * (sx * ti.gx + sy * ti.gy + sz * ti.gz), &sn, &cs);
-                // (i f) e^{-i k d.c} with f = -k d_y / 3
-                const double f = -k * sy / 3.0;
-                db = make_double2(f * sn, f * cs);
+            for (int g = 0; g < 6; g++) {
+                double wt, xi, eta;
+                quad_point(g, wt, xi, eta);
+                double2 F, H;
+                FdF(k, px - r.q[g][0], py - r.q[g][1], pz - r.q[g][2], F, H);
+                const double w0 = wt * kInv8Pi;
+                S0.x = fma(w0, F.x, S0.x), S0.y = fma(w0, F.y, S0.y);
+                T0.x = fma(w0 * (1.0 - xi - eta), H.x, T0.x), T0.y = fma(w0 * (1.0 - xi - eta), H.y, T0.y);
+                T1.x = fma(w0 * xi, H.x, T1.x), T1.y = fma(w0 * xi, H.y, T1.y);
+                T2.x = fma(w0 * eta, H.x, T2.x), T2.y = fma(w0 * eta, H.y, T2.y);
             }
-            cc -= cmul(db, lam[(int64_t)j * N + i]).x;
+            const double ux = px - r.ax, uy = py - r.ay, uz = pz - r.az;
+            const double s = ux * r.nx + uy * r.ny + uz * r.nz;  // -s of the formulas above
+            // D_c = (p - a) . dn_c with dn_a = e_y x (b - c), dn_b = e_y x (c - a), dn_c = (b - a) x e_y
+            const double E0 = r.ny - (ux * (r.bz - r.cz) - uz * (r.bx - r.cx));
+            const double E1 = uz * r.cx - ux * r.cz, E2 = ux * r.bz - uz * r.bx;
+            const double h_r = hr[v], h_i = hi[v];
+            double o0 = (s * T0.x + E0 * S0.x) * h_r - (s * T0.y + E0 * S0.y) * h_i;
+            double o1 = (s * T1.x + E1 * S0.x) * h_r - (s * T1.y + E1 * S0.y) * h_i;
+            double o2 = (s * T2.x + E2 * S0.x) * h_r - (s * T2.y + E2 * S0.y) * h_i;
+            o0 += d, o1 += d, o2 += d;
+            o0 = row16_sum(on ? o0 : 0.0), o1 = row16_sum(on ? o1 : 0.0), o2 = row16_sum(on ? o2 : 0.0);
+            if (i16 == v) acc[0] += o0, acc[1] += o1, acc[2] += o2;
         }
     }
+    if (i16 < 4)
 #pragma unroll
-    for (int c = 0; c < 3; c++) a[c] = quad_sum(a[c]);
-    cc = quad_sum(cc);
-    if (q4 == 0)
-#pragma unroll
-        for (int c = 0; c < 3; c++) cA[t * 3 + c] = a[c], cC[t * 3 + c] = cc;
+        for (int c = 0; c < 3; c++) red[w][i16 * 4 + kk][c] = acc[c];
+    __syncthreads();
+    if (threadIdx.x < 48) {
+        const int r = (int)threadIdx.x / 3, c = (int)threadIdx.x % 3;
+        if (t0 + r < T) {
+            double a = red[0][r][c];
+            for (int q = 1; q < kGW; q++) a += red[q][r][c];
+            out[((int64_t)sp * T + t0 + r) * 3 + c] = a;
+        }
+    }
 }
 
-// gradient_h: sum over (touched element, corner) in list order; B summed over the splits first. With G, the
-// terms are not stored but added: G_h = G_h + ((A_h - B_h) + C_h), the order of the host sum A - B + C.
-__global__ void k_grad_scatter(int HH, int T, int esplit, const int *__restrict__ hptr, const int *__restrict__ hlist,
-                               const double *__restrict__ cA, const double *__restrict__ partB,
-                               const double *__restrict__ cC, double *__restrict__ A, double *__restrict__ B,
-                               double *__restrict__ C, double *__restrict__ G) {
+// C per touched element (one thread each): -sum_rhs Re( lam_i db_i / dp_i ).
+__global__ __launch_bounds__(64) void k_grad_C(const Tri *__restrict__ tri, int N, int T,
+                                               const int *__restrict__ touched, double k, int R,
+                                               const double2 *__restrict__ lam, int src_kind,
+                                               const double *__restrict__ src, double *__restrict__ cC) {
+    const int t = blockIdx.x * 64 + threadIdx.x;
+    if (t >= T) return;
+    const int i = touched[t];
+    const Tri ti = tri[i];
+    double cc = 0.0;
+    for (int j = 0; j < R; j++) {
+        double2 db;
+        const double sx = src[3 * j], sy = src[3 * j + 1], sz = src[3 * j + 2];
+        double sn, cs;
+        if (src_kind == ARH_RHS_POINT) {
+            const double dx = ti.gx - sx, dy = ti.gy - sy, dz = ti.gz - sz;
+            const double r = sqrt(dx * dx + dy * dy + dz * dz);
+            trig_sincos(k * r, &sn, &cs);
+            // e^{-ikr}(-1 - ikr) / (4 pi r^2) * d_y / (3 r)
+            const double f = dy / (3.0 * r) / (4.0 * kPi * r * r);
+            db = make_double2((-cs - k * r * sn) * f, (sn - k * r * cs) * f);
+        } else {
+            trig_sincos(k * (sx * ti.gx + sy * ti.gy + sz * ti.gz), &sn, &cs);
+            // (i f) e^{-i k d.c} with f = -k d_y / 3
+            const double f = -k * sy / 3.0;
+            db = make_double2(f * sn, f * cs);
+        }
+        cc -= cmul(db, lam[(int64_t)j * N + i]).x;
+    }
+    cC[t] = cc;
+}
+
+// gradient_h: sum over (touched element, corner) in list order; A and B summed over their splits first. With G,
+// the terms are not stored but added: G_h = G_h + ((A_h - B_h) + C_h), the order of the host sum A - B + C.
+__global__ void k_grad_scatter(int HH, int T, int asplit, int bsplit, const int *__restrict__ hptr,
+                               const int *__restrict__ hlist, const double *__restrict__ partA,
+                               const double *__restrict__ partB, const double *__restrict__ cC,
+                               double *__restrict__ A, double *__restrict__ B, double *__restrict__ C,
+                               double *__restrict__ G) {
     const int h = blockIdx.x * blockDim.x + threadIdx.x;
     if (h >= HH) return;
     double a = 0.0, b = 0.0, c = 0.0;
     for (int e = hptr[h]; e < hptr[h + 1]; e++) {
         const int tc = hlist[e];  // t * 3 + corner
-        a += cA[tc];
-        double bb = 0.0;
-        for (int sp = 0; sp < esplit; sp++) bb += partB[(int64_t)sp * T * 3 + tc];
+        double aa = 0.0, bb = 0.0;
+        for (int sp = 0; sp < asplit; sp++) aa += partA[(int64_t)sp * T * 3 + tc];
+        for (int sp = 0; sp < bsplit; sp++) bb += partB[(int64_t)sp * T * 3 + tc];
+        a += aa;
         b += bb;
-        c += cC[tc];
+        c += cC[tc / 3];
     }
     if (G)
         G[h] = G[h] + ((a - b) + c);
@@ -332,27 +334,39 @@ void launch_shape_grad(arh_geom *g, double k, const double *L_dev, int LL, const
         ARH_HIP(hipStreamSynchronize(s));
         return;
     }
-    const int gxb = (4 * T + kGT - 1) / kGT;  // a quad of lanes per touched element
-    const int esplit = std::max(1, std::min(std::max(1, N / 64), (2048 + gxb - 1) / gxb));
-    DBuf d_touched, d_hptr, d_hlist, cA, cC, pB;
+    const int gx = (T + 15) / 16;
+    // column splits: enough workgroups to fill the chip, at least one 16-column tile per wavefront of each
+    auto splits = [&](int ncol) {
+        const int most = std::max(1, (ncol + 16 * kGW - 1) / (16 * kGW));
+        return std::max(1, std::min(most, (kGSlots + gx - 1) / gx));
+    };
+    const int bsplit = splits(N), asplit = splits(LL);
+    const int K = 4 * ((nrhs + 1) / 2);
+    DBuf d_touched, d_hptr, d_hlist, pA, pB, cC, xp, lp, vp;
     upload(d_touched, touched, s);
     upload(d_hptr, hptr, s);
     upload(d_hlist, hlist, s);
-    cA.alloc(sizeof(double) * 3 * T);
-    cC.alloc(sizeof(double) * 3 * T);
-    pB.alloc(sizeof(double) * 3 * (size_t)T * esplit);
-    DBuf xl;
-    xl.alloc(sizeof(double2) * 2 * (size_t)N * nrhs);
-    hipLaunchKernelGGL(k_grad_pack, dim3((unsigned)(((int64_t)N * nrhs + 255) / 256)), dim3(256), 0, s, N, nrhs, x, lam,
-                       xl.as<double2>());
-    ARH_HIP(hipMemsetAsync(pB.p, 0, sizeof(double) * 3 * (size_t)T * esplit, s));
-    for (int j0 = 0; j0 < nrhs; j0 += 4 * kRQ)
-        hipLaunchKernelGGL(k_grad_B, dim3(gxb, esplit), dim3(kGT), 0, s, g->tri.as<Tri>(), N, T, d_touched.as<int>(), k,
-                           nrhs, j0, x, lam, xl.as<double2>(), esplit, pB.as<double>());
-    hipLaunchKernelGGL(k_grad_AC, dim3(gxb), dim3(kGT), 0, s, g->tri.as<Tri>(), N, T, d_touched.as<int>(), k, nrhs, x,
-                       lam, vf, L_dev, LL, src_kind, src_dev, cA.as<double>(), cC.as<double>());
-    hipLaunchKernelGGL(k_grad_scatter, dim3((HH + 255) / 256), dim3(256), 0, s, HH, T, esplit, d_hptr.as<int>(),
-                       d_hlist.as<int>(), cA.as<double>(), pB.as<double>(), cC.as<double>(), A, B, C, G);
+    pA.alloc(sizeof(double) * 3 * (size_t)T * asplit);
+    pB.alloc(sizeof(double) * 3 * (size_t)T * bsplit);
+    cC.alloc(sizeof(double) * T);
+    auto pack = [&](DBuf &out, int n, const double2 *v) {
+        out.alloc(sizeof(double) * (size_t)n * K);
+        hipLaunchKernelGGL(k_grad_pack, dim3((unsigned)(((int64_t)n * (K / 2) + 255) / 256)), dim3(256), 0, s, n, nrhs,
+                           K, v, out.as<double>());
+    };
+    pack(xp, N, x);
+    pack(lp, N, lam);
+    pack(vp, LL, vf);
+    hipLaunchKernelGGL(k_grad_pairs<false>, dim3(gx, bsplit), dim3(kGT), 0, s, g->tri.as<Tri>(),
+                       (const double *)nullptr, N, T, d_touched.as<int>(), k, K, xp.as<double>(), lp.as<double>(),
+                       lp.as<double>(), bsplit, pB.as<double>());
+    hipLaunchKernelGGL(k_grad_pairs<true>, dim3(gx, asplit), dim3(kGT), 0, s, g->tri.as<Tri>(), L_dev, LL, T,
+                       d_touched.as<int>(), k, K, xp.as<double>(), (const double *)nullptr, vp.as<double>(), asplit,
+                       pA.as<double>());
+    hipLaunchKernelGGL(k_grad_C, dim3((T + 63) / 64), dim3(64), 0, s, g->tri.as<Tri>(), N, T, d_touched.as<int>(), k,
+                       nrhs, lam, src_kind, src_dev, cC.as<double>());
+    hipLaunchKernelGGL(k_grad_scatter, dim3((HH + 255) / 256), dim3(256), 0, s, HH, T, asplit, bsplit, d_hptr.as<int>(),
+                       d_hlist.as<int>(), pA.as<double>(), pB.as<double>(), cC.as<double>(), A, B, C, G);
     ARH_HIP(hipGetLastError());
     ARH_HIP(hipStreamSynchronize(s));
 }

@@ -15,6 +15,7 @@
 // Every operation is an explicit fma or a plain product, so the host and device builds round alike.
 #pragma once
 #include <cmath>
+#include <cstring>
 
 #if defined(__HIPCC__)
 #define ARH_HD __host__ __device__
@@ -27,11 +28,34 @@ namespace arh {
 constexpr double kTrigMax = 1.0e9;  // largest |x| the reduction is accurate for
 constexpr double kTrigMaxK = 1.0e6;  // wavenumber limit the entry points enforce (k r <= kTrigMax up to 1 km)
 
+// The low 32 bits of a double.
+ARH_HD inline int trig_low_word(double t) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    return __double2loint(t);
+#else
+    long long b;
+    std::memcpy(&b, &t, sizeof(b));
+    return (int)(unsigned)b;
+#endif
+}
+
 ARH_HD inline void trig_sincos(double x, double *s, double *c) {
     // pi/2 = P1 + P2 + P3 (+ 5.6e-50), each the double nearest to what is left
     const double kTwoOverPi = 0.6366197723675814;
     const double P1 = 1.5707963267948966, P2 = 6.123233995736766e-17, P3 = -1.4973849048591698e-33;
-    const double n = rint(x * kTwoOverPi);
+    // n = x * 2 / pi rounded to the nearest integer, by adding 1.5 * 2^52: the sum's last mantissa bit is then
+    // worth 1, so the addition rounds (ties to even) and its low bits are n modulo 2^32 in two's complement. Valid
+    // for |n| < 2^51. The product is rounded first (no fused multiply-add), so n is that of rint(x * 2 / pi).
+    const double kMagic = 6755399441055744.0;
+    double t;
+    {
+#if defined(__clang__)
+#pragma clang fp contract(off)
+#endif
+        const double p = x * kTwoOverPi;
+        t = p + kMagic;
+    }
+    const double n = t - kMagic;
     double r = fma(-n, P1, x);
     r = fma(-n, P2, r);
     r = fma(-n, P3, r);
@@ -58,7 +82,7 @@ ARH_HD inline void trig_sincos(double x, double *s, double *c) {
     pc = fma(pc, r2, -0.5);                    // 1/2!
     const double cr = fma(pc, r2, 1.0);
     // quadrant: x = r + q pi/2 (mod 2 pi)
-    const int q = (int)((long long)n & 3);
+    const int q = trig_low_word(t) & 3;
     const double a = (q & 1) ? cr : sr;  // |sin x|'s source
     const double b = (q & 1) ? sr : cr;  // |cos x|'s source
     *s = (q & 2) ? -a : a;
