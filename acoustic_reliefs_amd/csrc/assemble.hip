@@ -1,14 +1,15 @@
 // H-matrix assembly on gfx950: dense near-field panels and batched partially pivoted ACA.
 #include <algorithm>
 #include <numeric>
+#include <type_traits>
 
 #include "arh_internal.h"
 #include "device_common.h"
 
 namespace arh {
 
-constexpr int kAcaThreads = 256;
-constexpr int kAcaWaves = kAcaThreads / ARH_WAVE;
+constexpr int kAcaWaves = 4;      // wavefronts of an ACA workgroup
+constexpr int kAcaThreads = kAcaWaves * ARH_WAVE;
 constexpr int kMaxRankLds = 128;  // max ACA rank kept in LDS coefficient arrays
 #ifndef ARH_ACA_BIGDIM
 #define ARH_ACA_BIGDIM 512
@@ -38,21 +39,291 @@ __global__ __launch_bounds__(256) void k_dense(const DenseTask *__restrict__ tas
     out[panel_off[t.leaf] + (int64_t)c * m + i] = v;
 }
 
-// ------------------------------------------------------------------ ACA cooperation groups
+// ------------------------------------------------------------------ wavefront reductions without LDS
+// DPP steps towards lane 63 (row_shr 1, 2, 4, 8, then row_bcast 15 and 31); lanes without a source keep `old`.
+template <int CTRL>
+__device__ __forceinline__ double dpp_f64(double old, double x) {
+    const int lo = __builtin_amdgcn_update_dpp(__double2loint(old), __double2loint(x), CTRL, 0xF, 0xF, false);
+    const int hi = __builtin_amdgcn_update_dpp(__double2hiint(old), __double2hiint(x), CTRL, 0xF, 0xF, false);
+    return __hiloint2double(hi, lo);
+}
+// A lane's value as a wavefront-uniform one (lane uniform).
+__device__ __forceinline__ double lane_f64(double x, int lane) {
+    const int lo = __builtin_amdgcn_readlane(__double2loint(x), lane);
+    const int hi = __builtin_amdgcn_readlane(__double2hiint(x), lane);
+    return __hiloint2double(hi, lo);
+}
+__device__ __forceinline__ double wsum63(double v) {  // the sum, in lane 63
+    v += dpp_f64<0x111>(0.0, v);
+    v += dpp_f64<0x112>(0.0, v);
+    v += dpp_f64<0x114>(0.0, v);
+    v += dpp_f64<0x118>(0.0, v);
+    v += dpp_f64<0x142>(0.0, v);
+    v += dpp_f64<0x143>(0.0, v);
+    return v;
+}
+__device__ __forceinline__ double wsum(double v) { return lane_f64(wsum63(v), 63); }
+__device__ __forceinline__ double wmax(double v) {
+    v = fmax(v, dpp_f64<0x111>(v, v));
+    v = fmax(v, dpp_f64<0x112>(v, v));
+    v = fmax(v, dpp_f64<0x114>(v, v));
+    v = fmax(v, dpp_f64<0x118>(v, v));
+    v = fmax(v, dpp_f64<0x142>(v, v));
+    v = fmax(v, dpp_f64<0x143>(v, v));
+    return lane_f64(v, 63);
+}
+__device__ __forceinline__ int wmin_i(int v) {
+    v = min(v, __builtin_amdgcn_update_dpp(v, v, 0x111, 0xF, 0xF, false));
+    v = min(v, __builtin_amdgcn_update_dpp(v, v, 0x112, 0xF, 0xF, false));
+    v = min(v, __builtin_amdgcn_update_dpp(v, v, 0x114, 0xF, 0xF, false));
+    v = min(v, __builtin_amdgcn_update_dpp(v, v, 0x118, 0xF, 0xF, false));
+    v = min(v, __builtin_amdgcn_update_dpp(v, v, 0x142, 0xF, 0xF, false));
+    v = min(v, __builtin_amdgcn_update_dpp(v, v, 0x143, 0xF, 0xF, false));
+    return __builtin_amdgcn_readlane(v, 63);
+}
+
+// Sums over the wavefront of eight complex values per lane, halving what each lane carries: after exchanging
+// halves (permlane32_swap) and rows (permlane16_swap) row r (lanes 16 r ..) holds values 2 r and 2 r + 1 and sums
+// them over its 16 lanes. Returns |value 2 r| in x and |value 2 r + 1| in y, the same in every lane of the row.
+__device__ __forceinline__ void swap32(double &a, double &b) {
+    const auto lo = __builtin_amdgcn_permlane32_swap(__double2loint(a), __double2loint(b), false, false);
+    const auto hi = __builtin_amdgcn_permlane32_swap(__double2hiint(a), __double2hiint(b), false, false);
+    a = __hiloint2double((int)hi[0], (int)lo[0]), b = __hiloint2double((int)hi[1], (int)lo[1]);
+}
+__device__ __forceinline__ void swap16(double &a, double &b) {
+    const auto lo = __builtin_amdgcn_permlane16_swap(__double2loint(a), __double2loint(b), false, false);
+    const auto hi = __builtin_amdgcn_permlane16_swap(__double2hiint(a), __double2hiint(b), false, false);
+    a = __hiloint2double((int)hi[0], (int)lo[0]), b = __hiloint2double((int)hi[1], (int)lo[1]);
+}
+template <int CTRL>
+__device__ __forceinline__ double row_step(double v) {
+    const int lo = __builtin_amdgcn_mov_dpp(__double2loint(v), CTRL, 0xF, 0xF, false);
+    const int hi = __builtin_amdgcn_mov_dpp(__double2hiint(v), CTRL, 0xF, 0xF, false);
+    return v + __hiloint2double(hi, lo);
+}
+__device__ __forceinline__ double row_sum(double v) {  // row_ror 8, 4, 2, 1
+    return row_step<0x121>(row_step<0x122>(row_step<0x124>(row_step<0x128>(v))));
+}
+__device__ __forceinline__ void wsum8(const double2 *s, double2 &a, double2 &b) {
+    double y[8];
+#pragma unroll
+    for (int t = 0; t < 4; t++) {
+        double p = s[t].x, q = s[t + 4].x;
+        swap32(p, q);
+        y[2 * t] = p + q;
+        p = s[t].y, q = s[t + 4].y;
+        swap32(p, q);
+        y[2 * t + 1] = p + q;
+    }
+#pragma unroll
+    for (int t = 0; t < 4; t++) {
+        swap16(y[t], y[t + 4]);
+        y[t] += y[t + 4];
+    }
+    a = make_double2(row_sum(y[0]), row_sum(y[1]));
+    b = make_double2(row_sum(y[2]), row_sum(y[3]));
+}
+
+// ------------------------------------------------------------------ ACA
+// compute_ACA_block (aca.cpp:38-82): start at row 0; residual row, first-max pivot column,
+// normalised row (unnormalised if the pivot is 0), residual column, non-conjugated norm
+// estimate, stop when sqrt(|u|^2|v|^2 / err) <= eps discarding the current cross, next row =
+// first max of |u| over unused rows; rank limit min(max_rank, m-1, n-1).
+// Crosses whose u or v is exactly zero add nothing to any later quantity, so they are counted
+// (rank_ref) but not stored (rank).
+//
+// Crosses follow one another, so a block is a serial chain of entry evaluations (about 590 VALU operations for
+// 64 entries), updates by the stored crosses, reductions and dot products. Blocks of up to 64 x 64 (four in five)
+// are one wavefront each with a row and a column per lane in registers; larger ones loop over their rows and
+// columns, as one wavefront or, from m + n >= kAcaBigDim, a workgroup. Loads of the stored crosses go out in batches
+// ahead of their use (the first before the entry is evaluated), and reductions run on DPP: through ds_bpermute the
+// dot products alone, 24 steps per stored cross, were half of a cross's time.
+// 0.6 m relief, 16,058 blocks: 1.95 ms at 4000 Hz and 1.2 ms at 1000 Hz (3.95 and 1.9 ms with the bpermute
+// reductions and unbatched loads), the factors bit for bit the same. What is left is VALU issue of mid-sized
+// blocks (3 wavefronts per SIMD) with a tail of the largest chains; 2 or 4 wavefronts per SIMD (4: spills) and 6,
+// 8 or 12 wavefronts per workgroup measured the same or slower: 2.75-3.2 ms per FP64 assembly at 4000 Hz against 2.75.
+
+// |v|^2 of the pivot searches. On symmetric meshes two entries can tie exactly, and this rounding decides between
+// them: it is part of the result, so the fused form is written out.
+__device__ __forceinline__ double pivot_norm(double2 v) { return fma(v.x, v.x, v.y * v.y); }
+
+// Factors of the rule's point (w, xi, eta) in bem_entry: its contribution is f (tr, ti).
+struct EntryPoint {
+    double f, tr, ti;
+};
+__device__ __forceinline__ EntryPoint entry_point(double k, double px, double py, double pz, const Tri &t, double w,
+                                                  double xi, double eta) {
+    const double qx = t.ax + xi * t.bx + eta * t.cx;
+    const double qy = t.ay + xi * t.by + eta * t.cy;
+    const double qz = t.az + xi * t.bz + eta * t.cz;
+    const double dx = px - qx, dy = py - qy, dz = pz - qz;
+    const double r2 = dx * dx + dy * dy + dz * dz;
+    const double r = sqrt(r2);
+    const double s = -(dx * t.nx + dy * t.ny + dz * t.nz);
+    const double kr = k * r;
+    double sn, cs;
+    trig_sincos(kr, &sn, &cs);
+    return EntryPoint{w * s / (r2 * r), -cs - kr * sn, sn - kr * cs};
+}
+
+// bem_entry of up to 64 rows or columns, one per lane, bit for bit, with the six points in three pairs shared out
+// when lanes are left over: `share` lanes per entry (3 for up to 21 entries, 2 for up to 32, else 1), lane e + s
+// 64 / share (s < share) works on entry e, lane e < 64 / share adds the pairs up in order.
+__device__ __forceinline__ double2 entry_shared(double k, double px, double py, double pz, const Tri &t, int share,
+                                                int lane) {
+    const int width = share == 3 ? 21 : share == 2 ? 32 : 64;
+    const int s = share == 1 ? 0 : lane / width;
+    double re = 0.0, im = 0.0;
+    const int rounds = 4 - share;
+#pragma unroll 1
+    for (int z = 0; z < rounds; z++) {
+        const int b = z == 0 ? s : share == 1 ? z : 2;  // (lane 63 of three shares repeats a pair, unused)
+        const bool b1 = b == 1, b2 = b >= 2;
+        const EntryPoint A = entry_point(k, px, py, pz, t, b2 ? ARH_QW_B : ARH_QW_A,
+                                         b1 ? ARH_Q_2 : b2 ? ARH_Q_3 : ARH_Q_1, b1 ? ARH_Q_1 : b2 ? ARH_Q_3 : ARH_Q_2);
+        const EntryPoint C = entry_point(k, px, py, pz, t, b1 || b2 ? ARH_QW_B : ARH_QW_A,
+                                         b1 ? ARH_Q_3 : b2 ? ARH_Q_4 : ARH_Q_1, b1 ? ARH_Q_4 : b2 ? ARH_Q_3 : ARH_Q_1);
+        re = fma(A.f, A.tr, re), im = fma(A.f, A.ti, im);
+        re = fma(C.f, C.tr, re), im = fma(C.f, C.ti, im);
+        for (int o = 1; z == 0 && o < share; o++) {
+            const int src = lane + o * width;
+            double f = __shfl(A.f, src, ARH_WAVE);
+            re = fma(f, __shfl(A.tr, src, ARH_WAVE), re), im = fma(f, __shfl(A.ti, src, ARH_WAVE), im);
+            f = __shfl(C.f, src, ARH_WAVE);
+            re = fma(f, __shfl(C.tr, src, ARH_WAVE), re), im = fma(f, __shfl(C.ti, src, ARH_WAVE), im);
+        }
+    }
+    return make_double2(re * kInv8Pi, im * kInv8Pi);
+}
+
+// v - sum_p a_p b_p over the stored crosses p < sr in order: b_p = own[p * stride], a_p = coef(p) (uniform).
+// Batches of kAcaBatch loads, two in flight; `first` was loaded by load_batch(.., 0) before.
+constexpr int kAcaBatch = 8;
+struct AcaBatch {
+    double2 b[kAcaBatch];
+};
+__device__ __forceinline__ void load_batch(AcaBatch &B, const double2 *__restrict__ own, int64_t stride, int p0,
+                                           int sr) {
+    const int last = max(sr - 1, 0);  // row 0 always exists; surplus loads repeat the last cross, unused
+#pragma unroll
+    for (int t = 0; t < kAcaBatch; t++) B.b[t] = own[min(p0 + t, last) * stride];
+}
+template <class Coef>
+__device__ __forceinline__ void use_batch(double2 &v, const AcaBatch &B, int p0, int sr, Coef &&coef) {
+#pragma unroll
+    for (int t = 0; t < kAcaBatch; t++)
+        if (p0 + t < sr) {
+            const double2 up = coef(p0 + t), vp = B.b[t];
+            v.x -= up.x * vp.x - up.y * vp.y;
+            v.y -= up.x * vp.y + up.y * vp.x;
+        }
+}
+template <class Coef>
+__device__ __forceinline__ void residual(double2 &v, AcaBatch &first, const double2 *__restrict__ own, int64_t stride,
+                                         int sr, Coef &&coef) {
+    AcaBatch next;
+    for (int p0 = 0; p0 < sr; p0 += 2 * kAcaBatch) {
+        load_batch(next, own, stride, p0 + kAcaBatch, sr);
+        use_batch(v, first, p0, sr, coef);
+        if (p0 + kAcaBatch >= sr) break;
+        load_batch(first, own, stride, p0 + 2 * kAcaBatch, sr);
+        use_batch(v, next, p0 + kAcaBatch, sr, coef);
+    }
+}
+
+// A block of at most 64 x 64, one wavefront: lane q holds row q and column q of the current cross.
+__device__ __forceinline__ void aca_small(LRBlock *__restrict__ blocks, int bid, const LRBlock &B, int lane,
+                                          const Tri *__restrict__ tri, double k, double eps, double2 *__restrict__ U,
+                                          double2 *__restrict__ V) {
+    const int m = B.re - B.rs, n = B.ce - B.cs, lim = B.lim;
+    const int q = min(lane, m - 1), c = min(lane, n - 1);
+    const bool rowon = lane < m, colon = lane < n;
+    // lanes that share an entry hold its row or column too
+    auto share_of = [](int e) { return e <= 21 ? 3 : e <= 32 ? 2 : 1; };
+    auto entry_of = [&](int e) { return min(e <= 21 ? lane % 21 : e <= 32 ? lane % 32 : lane, e - 1); };
+    const int mshare = share_of(m), nshare = share_of(n);
+    const Tri tc = tri[B.cs + entry_of(n)];
+    const Tri &tq = tri[B.rs + entry_of(m)];
+    const double gx = tq.gx, gy = tq.gy, gz = tq.gz;
+    bool used = lane == 0;
+    int i = 0, it = 0, sr = 0;
+    double err = 0.0;
+    // coefficient p of the current cross is in lane p (lim <= 63 here)
+    auto coef_in = [&](const double2 &cf) {
+        return [&cf](int p) { return make_double2(lane_f64(cf.x, p), lane_f64(cf.y, p)); };
+    };
+    while (it < lim) {
+        AcaBatch b;
+        load_batch(b, V + c, n, 0, sr);
+        double2 cf = U[(int64_t)min(lane, max(sr - 1, 0)) * m + i];
+        double2 v = entry_shared(k, lane_f64(gx, i), lane_f64(gy, i), lane_f64(gz, i), tc, nshare, lane);
+        residual(v, b, V + c, n, sr, coef_in(cf));
+        // first maximum of |v|^2 (NaN never wins; column 0 if nothing does)
+        double a = pivot_norm(v);
+        a = colon && a == a ? a : -1.0;
+        double best = wmax(a);
+        const int j = best < 0.0 ? 0 : __builtin_ctzll(__ballot(a == best));
+        load_batch(b, U + q, m, 0, sr);
+        cf = V[(int64_t)min(lane, max(sr - 1, 0)) * n + j];
+        const double2 piv = make_double2(lane_f64(v.x, j), lane_f64(v.y, j));
+        if (piv.x != 0.0 || piv.y != 0.0) v = cdiv(v, piv);
+        if (colon) V[(int64_t)sr * n + lane] = v;
+        double2 u = entry_shared(k, gx, gy, gz, tri[B.cs + j], mshare, lane);
+        residual(u, b, U + q, m, sr, coef_in(cf));
+        if (rowon) U[(int64_t)sr * m + lane] = u;
+        a = pivot_norm(u);
+        const double un = wsum(rowon ? a : 0.0), vn = wsum(colon ? cnorm2(v) : 0.0);
+        a = rowon && !used && a == a ? a : -1.0;
+        best = wmax(a);
+        const int ni = best < 0.0 ? 0 : __builtin_ctzll(__ballot(a == best));
+        // |u_p^T u| and |v v_p^T| for the stored crosses p < sr (aca.cpp:64-69), eight at a time
+        double dots = 0.0;
+        const double2 uz = rowon ? u : make_double2(0.0, 0.0), vz = colon ? v : make_double2(0.0, 0.0);
+        for (int p0 = 0; p0 < sr; p0 += kAcaBatch) {
+            AcaBatch bu, bv;
+            load_batch(bu, U + q, m, p0, sr);
+            load_batch(bv, V + c, n, p0, sr);
+#pragma unroll
+            for (int t = 0; t < kAcaBatch; t++) bu.b[t] = cmul(uz, bu.b[t]), bv.b[t] = cmul(vz, bv.b[t]);
+            double2 su, su1, sv, sv1;
+            wsum8(bu.b, su, su1);
+            wsum8(bv.b, sv, sv1);
+            const int p = p0 + 2 * (lane >> 4);  // surplus crosses (repeats) and lanes are not added
+            if ((lane & 15) == 0 && p < sr) dots += sqrt(cnorm2(su)) * sqrt(cnorm2(sv));
+            if ((lane & 15) == 1 && p + 1 < sr) dots += sqrt(cnorm2(su1)) * sqrt(cnorm2(sv1));
+        }
+        dots = wsum(dots);
+        err += un * vn + 2.0 * dots;
+        if (sqrt(un * vn / err) <= eps) break;
+        if (un * vn > 0.0) sr++;
+        i = ni;
+        used = used || lane == i;
+        it++;
+        __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");  // the new cross is read by other lanes
+        __builtin_amdgcn_wave_barrier();
+    }
+    if (lane == 0) blocks[bid].rank = sr, blocks[bid].rank_ref = it;
+}
+
 struct AcaShared {
     double2 coef[kMaxRankLds];
-    double du[kMaxRankLds], dv[kMaxRankLds];
-    double rv[kAcaWaves];
+    double2 piv;
+    double rv[4][kAcaWaves];
     int ri[kAcaWaves];
 };
+struct AcaSharedGroup : AcaShared {
+    double2 dd[kAcaWaves][kMaxRankLds][2];  // kMaxRankLds is a multiple of the batch
+};
 
-// The threads working on one ACA block: the whole 256-thread workgroup (WAVE false) or a single
-// wavefront (WAVE true, no workgroup barrier: a wavefront's memory operations complete in order,
-// so a fence at wavefront scope, which also stops compiler reordering, is its barrier).
+// The threads working on one larger block: the whole workgroup (WAVE false) or a single wavefront (WAVE true, no
+// workgroup barrier: a wavefront's memory operations complete in order, so a fence at wavefront scope, which
+// also stops compiler reordering, is its barrier).
 template <bool WAVE>
 struct AcaGroup {
-    int tid, nthr, w, nw, lane;
-    AcaShared &sh;
+    int tid, w, lane;
+    std::conditional_t<WAVE, AcaShared, AcaSharedGroup> &sh;
+    static constexpr int nthr = WAVE ? ARH_WAVE : kAcaThreads;
+    static constexpr int nw = WAVE ? 1 : kAcaWaves;
     __device__ __forceinline__ void sync() const {
         if (WAVE) {
             __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
@@ -61,60 +332,47 @@ struct AcaGroup {
             __syncthreads();
         }
     }
-    // fixed-order sums: all threads get the same bits
-    __device__ __forceinline__ double sum(double v) const {
-        v = wave_sum(v);
+    // fixed-order sum, the same bits in every thread; slot: one of the shared arrays (a later sum with the same
+    // slot needs a sync in between)
+    __device__ __forceinline__ double sum(double v, int slot) const {
+        v = wsum(v);
         if (WAVE) return v;
-        sync();
-        if (lane == 0) sh.rv[w] = v;
-        sync();
-        double s = sh.rv[0];
+        if (lane == 0) sh.rv[slot][w] = v;
+        __syncthreads();
+        double s = sh.rv[slot][0];
 #pragma unroll
-        for (int q = 1; q < kAcaWaves; q++) s += sh.rv[q];
+        for (int q = 1; q < kAcaWaves; q++) s += sh.rv[slot][q];
         return s;
     }
     // (value, index) max with ties to the lower index
-    __device__ __forceinline__ void argmax(double &v, int &i) const {
-        wave_argmax(v, i);
+    __device__ __forceinline__ void argmax(double &v, int &i, int slot) const {
+        const double b = wmax(v);
+        i = wmin_i(v == b ? i : 0x7fffffff);
+        v = b;
         if (WAVE) return;
-        sync();
-        if (lane == 0) sh.rv[w] = v, sh.ri[w] = i;
-        sync();
-        double bv = sh.rv[0];
-        int bi = sh.ri[0];
+        if (lane == 0) sh.rv[slot][w] = v, sh.ri[w] = i;
+        __syncthreads();
+        v = sh.rv[slot][0];
+        i = sh.ri[0];
 #pragma unroll
         for (int q = 1; q < kAcaWaves; q++)
-            if (sh.rv[q] > bv || (sh.rv[q] == bv && sh.ri[q] < bi)) bv = sh.rv[q], bi = sh.ri[q];
-        v = bv;
-        i = bi;
+            if (sh.rv[slot][q] > v || (sh.rv[slot][q] == v && sh.ri[q] < i)) v = sh.rv[slot][q], i = sh.ri[q];
     }
 };
 
-// ------------------------------------------------------------------ ACA of one block
-// compute_ACA_block (aca.cpp:38-82): start at row 0; residual row, first-max pivot column,
-// normalised row (unnormalised if the pivot is 0), residual column, non-conjugated norm
-// estimate, stop when sqrt(|u|^2|v|^2 / err) <= eps discarding the current cross, next row =
-// first max of |u| over unused rows; rank limit min(max_rank, m-1, n-1).
-// Crosses whose u or v is exactly zero add nothing to any later quantity, so they are counted
-// (rank_ref) but not stored (rank).
 template <bool WAVE>
 __device__ __forceinline__ void aca_block(const AcaGroup<WAVE> &G, LRBlock *__restrict__ blocks, int bid,
-                                          const Tri *__restrict__ tri, double k, double eps, double2 *__restrict__ Us,
-                                          double2 *__restrict__ Vs, unsigned char *__restrict__ flags) {
-    AcaShared &sh = G.sh;
-    const LRBlock B = blocks[bid];
+                                          const LRBlock &B, const Tri *__restrict__ tri, double k, double eps,
+                                          double2 *__restrict__ U, double2 *__restrict__ V,
+                                          unsigned char *__restrict__ used) {
+    auto &sh = G.sh;
     const int rs = B.rs, cs = B.cs, m = B.re - B.rs, n = B.ce - B.cs, lim = B.lim;
-    const int tid = G.tid, nthr = G.nthr, lane = G.lane;
-    if (lim <= 0) {
-        if (tid == 0) blocks[bid].rank = 0, blocks[bid].rank_ref = 0;
-        return;
-    }
-    double2 *U = Us + B.us_off;
-    double2 *V = Vs + B.vs_off;
-    unsigned char *used = flags + B.flag_off;
+    const int tid = G.tid, lane = G.lane;
+    constexpr int nthr = AcaGroup<WAVE>::nthr;
     for (int q = tid; q < m; q += nthr) used[q] = (q == 0) ? 1 : 0;
     int i = 0, it = 0, sr = 0;
     double err = 0.0;
+    const auto coef = [&](int p) { return sh.coef[p]; };
     G.sync();
     while (it < lim) {
         // coefficients U(i, p), p < sr
@@ -124,77 +382,100 @@ __device__ __forceinline__ void aca_block(const AcaGroup<WAVE> &G, LRBlock *__re
         const Tri ti = tri[rs + i];
         double2 *vrow = V + (int64_t)sr * n;
         double best = -1.0;
+        double2 bv = make_double2(0.0, 0.0);
         int bi = 0x7fffffff;
         for (int c = tid; c < n; c += nthr) {
+            AcaBatch b;
+            load_batch(b, V + c, n, 0, sr);
             double2 v = bem_entry(k, ti.gx, ti.gy, ti.gz, tri[cs + c]);
-            for (int p = 0; p < sr; p++) {
-                double2 vp = V[(int64_t)p * n + c];
-                double2 up = sh.coef[p];
-                v.x -= up.x * vp.x - up.y * vp.y;
-                v.y -= up.x * vp.y + up.y * vp.x;
-            }
+            residual(v, b, V + c, n, sr, coef);
             vrow[c] = v;
-            double a = cnorm2(v);
-            if (a > best) best = a, bi = c;
+            const double a = pivot_norm(v);
+            if (a > best) best = a, bi = c, bv = v;
+            if (c == 0 && best < 0.0) bv = v;  // the pivot when no entry wins (all NaN)
         }
-        G.argmax(best, bi);
+        const int mine = bi;
+        G.argmax(best, bi, 0);
         const int j = (best < 0.0) ? 0 : bi;
+        if (best < 0.0 ? tid == 0 : mine == j) sh.piv = bv;
+        // the coefficients of the column: every use of the row's is over (argmax has synchronised, or in order)
+        for (int p = tid; p < sr; p += nthr) sh.coef[p] = V[(int64_t)p * n + j];
         G.sync();
-        const double2 piv = vrow[j];
-        // every thread holds the pivot before its owner normalises it in place
-        G.sync();
+        const double2 piv = sh.piv;
         const bool nz = (piv.x != 0.0 || piv.y != 0.0);
         double vn = 0.0;
         for (int c = tid; c < n; c += nthr) {
             double2 v = vrow[c];
-            if (nz) v = cdiv(v, piv);
-            vrow[c] = v;
+            if (nz) v = cdiv(v, piv), vrow[c] = v;
             vn += cnorm2(v);
         }
-        vn = G.sum(vn);
-        for (int p = tid; p < sr; p += nthr) sh.coef[p] = V[(int64_t)p * n + j];
-        G.sync();
         // residual column into U column `sr`, with the masked first-max search for the next row
         const Tri tj = tri[cs + j];
         double2 *ucol = U + (int64_t)sr * m;
         double un = 0.0, bu = -1.0;
         int bq = 0x7fffffff;
         for (int q = tid; q < m; q += nthr) {
-            const Tri tq = tri[rs + q];
+            AcaBatch b;
+            load_batch(b, U + q, m, 0, sr);
+            const Tri &tq = tri[rs + q];
             double2 u = bem_entry(k, tq.gx, tq.gy, tq.gz, tj);
-            for (int p = 0; p < sr; p++) {
-                double2 up = U[(int64_t)p * m + q];
-                double2 vp = sh.coef[p];
-                u.x -= up.x * vp.x - up.y * vp.y;
-                u.y -= up.x * vp.y + up.y * vp.x;
-            }
+            residual(u, b, U + q, m, sr, coef);
             ucol[q] = u;
-            double a = cnorm2(u);
+            const double a = pivot_norm(u);
             un += a;
             if (!used[q] && a > bu) bu = a, bq = q;
         }
-        un = G.sum(un);
-        G.argmax(bu, bq);
-        G.sync();
-        // |u_p^T u| and |v v_p^T| for stored crosses p < sr (aca.cpp:64-69): wave w takes p = w mod nw
-        for (int p = G.w; p < sr; p += G.nw) {
-            double2 su = make_double2(0.0, 0.0), sv = make_double2(0.0, 0.0);
-            const double2 *up = U + (int64_t)p * m;
-            const double2 *vp = V + (int64_t)p * n;
-            for (int q = lane; q < m; q += ARH_WAVE) cfma(su, ucol[q], up[q]);
-            for (int c = lane; c < n; c += ARH_WAVE) cfma(sv, vrow[c], vp[c]);
-            su = wave_sum2(su);
-            sv = wave_sum2(sv);
-            if (lane == 0) sh.du[p] = cabs_(su), sh.dv[p] = cabs_(sv);
-        }
-        G.sync();
+        vn = G.sum(vn, 1);
+        un = G.sum(un, 2);
+        G.argmax(bu, bq, 3);
+        G.sync();  // the new cross is written (a wavefront alone has passed no barrier since)
+        // |u_p^T u| and |v v_p^T| for stored crosses p < sr (aca.cpp:64-69), eight at a time: every thread takes its
+        // own rows and columns, wavefront sums through wsum8, wavefronts added in order
         double dots = 0.0;
-        for (int p = 0; p < sr; p++) dots += sh.du[p] * sh.dv[p];
+        for (int p0 = 0; p0 < sr; p0 += kAcaBatch) {
+            double2 su[kAcaBatch], sv[kAcaBatch];
+#pragma unroll
+            for (int t = 0; t < kAcaBatch; t++) su[t] = sv[t] = make_double2(0.0, 0.0);
+            for (int q = tid; q < m; q += nthr) {
+                AcaBatch b;
+                load_batch(b, U + q, m, p0, sr);
+                const double2 uq = ucol[q];
+#pragma unroll
+                for (int t = 0; t < kAcaBatch; t++) cfma(su[t], uq, b.b[t]);
+            }
+            for (int c = tid; c < n; c += nthr) {
+                AcaBatch b;
+                load_batch(b, V + c, n, p0, sr);
+                const double2 vc = vrow[c];
+#pragma unroll
+                for (int t = 0; t < kAcaBatch; t++) cfma(sv[t], vc, b.b[t]);
+            }
+            double2 a[4];
+            wsum8(su, a[0], a[1]);
+            wsum8(sv, a[2], a[3]);
+            const int p = p0 + 2 * (lane >> 4);  // surplus crosses (repeats) are not added
+            if constexpr (WAVE) {
+                if ((lane & 15) == 0 && p < sr) dots += sqrt(cnorm2(a[0])) * sqrt(cnorm2(a[2]));
+                if ((lane & 15) == 1 && p + 1 < sr) dots += sqrt(cnorm2(a[1])) * sqrt(cnorm2(a[3]));
+            } else if ((lane & 15) == 0) {
+                sh.dd[G.w][p][0] = a[0], sh.dd[G.w][p][1] = a[2];
+                sh.dd[G.w][p + 1][0] = a[1], sh.dd[G.w][p + 1][1] = a[3];
+            }
+        }
+        if constexpr (!WAVE) {
+            __syncthreads();
+            for (int p = lane; p < sr; p += ARH_WAVE) {
+                double2 su = sh.dd[0][p][0], sv = sh.dd[0][p][1];
+#pragma unroll
+                for (int q = 1; q < kAcaWaves; q++) su = cadd(su, sh.dd[q][p][0]), sv = cadd(sv, sh.dd[q][p][1]);
+                dots += sqrt(cnorm2(su)) * sqrt(cnorm2(sv));
+            }
+        }
+        dots = wsum(dots);
         err += un * vn + 2.0 * dots;
         if (sqrt(un * vn / err) <= eps) break;
         if (un * vn > 0.0) sr++;
         i = (bu < 0.0) ? 0 : bq;
-        G.sync();
         if (tid == 0) used[i] = 1;
         it++;
         G.sync();
@@ -202,24 +483,39 @@ __device__ __forceinline__ void aca_block(const AcaGroup<WAVE> &G, LRBlock *__re
     if (tid == 0) blocks[bid].rank = sr, blocks[bid].rank_ref = it;
 }
 
-// Workgroups [0, nbig) each take one big block (order[0..nbig)); the others take four small
+// Workgroups [0, nbig) each take one big block (order[0..nbig)); the others take kAcaWaves smaller
 // blocks, one per wavefront.
-__global__ __launch_bounds__(kAcaThreads) void k_aca(LRBlock *__restrict__ blocks, const int *__restrict__ order,
+__global__ __launch_bounds__(kAcaThreads, 3) void k_aca(LRBlock *__restrict__ blocks, const int *__restrict__ order,
                                                      int nbig, int na, const Tri *__restrict__ tri, double k,
                                                      double eps, double2 *__restrict__ Us, double2 *__restrict__ Vs,
                                                      unsigned char *__restrict__ flags) {
-    __shared__ AcaShared sh[kAcaWaves];
+    __shared__ union Shared {
+        AcaSharedGroup group;
+        AcaShared wave[kAcaWaves];
+        __device__ Shared() {}
+    } sh;
     const int lane = threadIdx.x % ARH_WAVE;
     const int w = __builtin_amdgcn_readfirstlane((int)(threadIdx.x / ARH_WAVE));
-    if ((int)blockIdx.x < nbig) {
-        const AcaGroup<false> G{(int)threadIdx.x, kAcaThreads, w, kAcaWaves, lane, sh[0]};
-        aca_block<false>(G, blocks, order[blockIdx.x], tri, k, eps, Us, Vs, flags);
+    const bool big = (int)blockIdx.x < nbig;
+    const int u = big ? (int)blockIdx.x : nbig + ((int)blockIdx.x - nbig) * kAcaWaves + w;
+    if (u >= na) return;
+    const int bid = order[u];
+    const LRBlock B = blocks[bid];
+    if (B.lim <= 0) {  // a single row or column, or max_rank 0
+        if (lane == 0 && (!big || w == 0)) blocks[bid].rank = 0, blocks[bid].rank_ref = 0;
         return;
     }
-    const int u = nbig + ((int)blockIdx.x - nbig) * kAcaWaves + w;
-    if (u >= na) return;
-    const AcaGroup<true> G{lane, ARH_WAVE, 0, 1, lane, sh[w]};
-    aca_block<true>(G, blocks, order[u], tri, k, eps, Us, Vs, flags);
+    double2 *U = Us + B.us_off, *V = Vs + B.vs_off;
+    unsigned char *used = flags + B.flag_off;
+    if (big) {
+        const AcaGroup<false> G{(int)threadIdx.x, w, lane, sh.group};
+        aca_block<false>(G, blocks, bid, B, tri, k, eps, U, V, used);
+    } else if (B.re - B.rs <= ARH_WAVE && B.ce - B.cs <= ARH_WAVE) {
+        aca_small(blocks, bid, B, lane, tri, k, eps, U, V);
+    } else {
+        const AcaGroup<true> G{lane, 0, lane, sh.wave[w]};
+        aca_block<true>(G, blocks, bid, B, tri, k, eps, U, V, used);
+    }
 }
 
 // ------------------------------------------------------------------ compaction
