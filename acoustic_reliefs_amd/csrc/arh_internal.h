@@ -359,7 +359,8 @@ void hmat_apply(arh_hmat *h, int transpose, int precision, int nrhs, const doubl
                 const int *cols = nullptr, int ncols = 0, const int *gate = nullptr);
 // matvec_mfma.hip
 void hmat_apply_mfma(arh_hmat *h, int transpose, int fp64, int nrhs, const double2 *x, double2 *y, hipStream_t s,
-                     const int *cols = nullptr, int ncols = 0, const int *gate = nullptr);
+                     const int *cols = nullptr, int ncols = 0, const int *gate = nullptr, bool packed = false);
+void *mfma_packed_rows(arh_hmat *h, int transpose, int fp64, int nc, int *rp);
 void mfma_prepare(arh_hmat *h, int transpose, int fp64);
 // matvec64.hip
 void hmat_apply64(arh_hmat *h, int nrhs, const double2 *x, double2 *y, hipStream_t s);

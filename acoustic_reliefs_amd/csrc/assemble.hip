@@ -39,30 +39,7 @@ __global__ __launch_bounds__(256) void k_dense(const DenseTask *__restrict__ tas
     out[panel_off[t.leaf] + (int64_t)c * m + i] = v;
 }
 
-// ------------------------------------------------------------------ wavefront reductions without LDS
-// DPP steps towards lane 63 (row_shr 1, 2, 4, 8, then row_bcast 15 and 31); lanes without a source keep `old`.
-template <int CTRL>
-__device__ __forceinline__ double dpp_f64(double old, double x) {
-    const int lo = __builtin_amdgcn_update_dpp(__double2loint(old), __double2loint(x), CTRL, 0xF, 0xF, false);
-    const int hi = __builtin_amdgcn_update_dpp(__double2hiint(old), __double2hiint(x), CTRL, 0xF, 0xF, false);
-    return __hiloint2double(hi, lo);
-}
-// A lane's value as a wavefront-uniform one (lane uniform).
-__device__ __forceinline__ double lane_f64(double x, int lane) {
-    const int lo = __builtin_amdgcn_readlane(__double2loint(x), lane);
-    const int hi = __builtin_amdgcn_readlane(__double2hiint(x), lane);
-    return __hiloint2double(hi, lo);
-}
-__device__ __forceinline__ double wsum63(double v) {  // the sum, in lane 63
-    v += dpp_f64<0x111>(0.0, v);
-    v += dpp_f64<0x112>(0.0, v);
-    v += dpp_f64<0x114>(0.0, v);
-    v += dpp_f64<0x118>(0.0, v);
-    v += dpp_f64<0x142>(0.0, v);
-    v += dpp_f64<0x143>(0.0, v);
-    return v;
-}
-__device__ __forceinline__ double wsum(double v) { return lane_f64(wsum63(v), 63); }
+// ------------------------------------------------------------------ wavefront maxima
 __device__ __forceinline__ double wmax(double v) {
     v = fmax(v, dpp_f64<0x111>(v, v));
     v = fmax(v, dpp_f64<0x112>(v, v));
@@ -85,25 +62,6 @@ __device__ __forceinline__ int wmin_i(int v) {
 // Sums over the wavefront of eight complex values per lane, halving what each lane carries: after exchanging
 // halves (permlane32_swap) and rows (permlane16_swap) row r (lanes 16 r ..) holds values 2 r and 2 r + 1 and sums
 // them over its 16 lanes. Returns |value 2 r| in x and |value 2 r + 1| in y, the same in every lane of the row.
-__device__ __forceinline__ void swap32(double &a, double &b) {
-    const auto lo = __builtin_amdgcn_permlane32_swap(__double2loint(a), __double2loint(b), false, false);
-    const auto hi = __builtin_amdgcn_permlane32_swap(__double2hiint(a), __double2hiint(b), false, false);
-    a = __hiloint2double((int)hi[0], (int)lo[0]), b = __hiloint2double((int)hi[1], (int)lo[1]);
-}
-__device__ __forceinline__ void swap16(double &a, double &b) {
-    const auto lo = __builtin_amdgcn_permlane16_swap(__double2loint(a), __double2loint(b), false, false);
-    const auto hi = __builtin_amdgcn_permlane16_swap(__double2hiint(a), __double2hiint(b), false, false);
-    a = __hiloint2double((int)hi[0], (int)lo[0]), b = __hiloint2double((int)hi[1], (int)lo[1]);
-}
-template <int CTRL>
-__device__ __forceinline__ double row_step(double v) {
-    const int lo = __builtin_amdgcn_mov_dpp(__double2loint(v), CTRL, 0xF, 0xF, false);
-    const int hi = __builtin_amdgcn_mov_dpp(__double2hiint(v), CTRL, 0xF, 0xF, false);
-    return v + __hiloint2double(hi, lo);
-}
-__device__ __forceinline__ double row_sum(double v) {  // row_ror 8, 4, 2, 1
-    return row_step<0x121>(row_step<0x122>(row_step<0x124>(row_step<0x128>(v))));
-}
 __device__ __forceinline__ void wsum8(const double2 *s, double2 &a, double2 &b) {
     double y[8];
 #pragma unroll

@@ -97,20 +97,62 @@ __device__ __forceinline__ double2 cdiv(double2 a, double2 b) {
 __device__ __forceinline__ double cnorm2(double2 a) { return a.x * a.x + a.y * a.y; }
 __device__ __forceinline__ double cabs_(double2 a) { return hypot(a.x, a.y); }
 
-// ---------------------------------------------------------------- wavefront reductions (64 lanes)
+// ---------------------------------------------------------------- wavefront reductions (64 lanes, all active)
+// Exchange of wavefront halves and of 16-lane rows: a takes b's lower half (even rows) into its upper half (odd rows),
+// b the other way round.
+__device__ __forceinline__ void swap32(double &a, double &b) {
+    const auto lo = __builtin_amdgcn_permlane32_swap(__double2loint(a), __double2loint(b), false, false);
+    const auto hi = __builtin_amdgcn_permlane32_swap(__double2hiint(a), __double2hiint(b), false, false);
+    a = __hiloint2double((int)hi[0], (int)lo[0]), b = __hiloint2double((int)hi[1], (int)lo[1]);
+}
+__device__ __forceinline__ void swap16(double &a, double &b) {
+    const auto lo = __builtin_amdgcn_permlane16_swap(__double2loint(a), __double2loint(b), false, false);
+    const auto hi = __builtin_amdgcn_permlane16_swap(__double2hiint(a), __double2hiint(b), false, false);
+    a = __hiloint2double((int)hi[0], (int)lo[0]), b = __hiloint2double((int)hi[1], (int)lo[1]);
+}
+template <int CTRL>
+__device__ __forceinline__ double row_step(double v) {
+    const int lo = __builtin_amdgcn_mov_dpp(__double2loint(v), CTRL, 0xF, 0xF, false);
+    const int hi = __builtin_amdgcn_mov_dpp(__double2hiint(v), CTRL, 0xF, 0xF, false);
+    return v + __hiloint2double(hi, lo);
+}
+__device__ __forceinline__ double row_sum(double v) {  // over a row of 16 lanes: row_ror 8, 4, 2, 1
+    return row_step<0x121>(row_step<0x122>(row_step<0x124>(row_step<0x128>(v))));
+}
+// The sum of v over the wavefront, in every lane: lanes 32 apart first, then 16, 8, 4, 2, 1 apart. (Rotating a row by 4
+// after the step by 8 meets the same value as exchanging lanes 4 apart, and so on.)
 __device__ __forceinline__ double wave_sum(double v) {
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
+    double a = v, b = v;
+    swap32(a, b);
+    a = b = a + b;
+    swap16(a, b);
+    return row_sum(a + b);
+}
+__device__ __forceinline__ double2 wave_sum2(double2 v) { return make_double2(wave_sum(v.x), wave_sum(v.y)); }
+// ---------------------------------------------------------------- wavefront reductions on DPP (no LDS)
+// Steps towards lane 63 (row_shr 1, 2, 4, 8, then row_bcast 15 and 31); lanes without a source keep `old`.
+template <int CTRL>
+__device__ __forceinline__ double dpp_f64(double old, double x) {
+    const int lo = __builtin_amdgcn_update_dpp(__double2loint(old), __double2loint(x), CTRL, 0xF, 0xF, false);
+    const int hi = __builtin_amdgcn_update_dpp(__double2hiint(old), __double2hiint(x), CTRL, 0xF, 0xF, false);
+    return __hiloint2double(hi, lo);
+}
+// A lane's value as a wavefront-uniform one (lane uniform).
+__device__ __forceinline__ double lane_f64(double x, int lane) {
+    const int lo = __builtin_amdgcn_readlane(__double2loint(x), lane);
+    const int hi = __builtin_amdgcn_readlane(__double2hiint(x), lane);
+    return __hiloint2double(hi, lo);
+}
+__device__ __forceinline__ double wsum63(double v) {  // the sum, in lane 63
+    v += dpp_f64<0x111>(0.0, v);
+    v += dpp_f64<0x112>(0.0, v);
+    v += dpp_f64<0x114>(0.0, v);
+    v += dpp_f64<0x118>(0.0, v);
+    v += dpp_f64<0x142>(0.0, v);
+    v += dpp_f64<0x143>(0.0, v);
     return v;
 }
-__device__ __forceinline__ double2 wave_sum2(double2 v) {
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) {
-        v.x += __shfl_xor(v.x, o, 64);
-        v.y += __shfl_xor(v.y, o, 64);
-    }
-    return v;
-}
+__device__ __forceinline__ double wsum(double v) { return lane_f64(wsum63(v), 63); }
 // (value, index) max with ties to the lower index; value -1 = empty.
 __device__ __forceinline__ void wave_argmax(double &v, int &i) {
 #pragma unroll

@@ -105,21 +105,6 @@ __device__ __forceinline__ void pair_gemm(const double *__restrict__ a, const do
     }
 }
 
-// Sum of v over the 16 lanes of a row (DPP row rotations by 8, 4, 2, 1), the same in every lane.
-template <int CTRL>
-__device__ __forceinline__ double row_ror(double x) {
-    const int lo = __builtin_amdgcn_mov_dpp(__double2loint(x), CTRL, 0xF, 0xF, false);
-    const int hi = __builtin_amdgcn_mov_dpp(__double2hiint(x), CTRL, 0xF, 0xF, false);
-    return __hiloint2double(hi, lo);
-}
-__device__ __forceinline__ double row16_sum(double v) {
-    v += row_ror<0x128>(v);
-    v += row_ror<0x124>(v);
-    v += row_ror<0x122>(v);
-    v += row_ror<0x121>(v);
-    return v;
-}
-
 // Partial sums over a range of columns for 16 touched elements. Columns are elements (LISTEN false: B) or
 // listeners (LISTEN true: A); grid (row tiles, column splits); out[(split * T + t) * 3 + c]. xi, li: packed x and
 // lambda by element; pc: the columns' packed values that multiply x_i (lambda by element, or vf by listener).
@@ -222,7 +207,7 @@ __global__ __launch_bounds__(kGT, 3) void k_grad_pairs(const Tri *__restrict__ t
             double o1 = (s * T1.x + E1 * S0.x) * h_r - (s * T1.y + E1 * S0.y) * h_i;
             double o2 = (s * T2.x + E2 * S0.x) * h_r - (s * T2.y + E2 * S0.y) * h_i;
             o0 += d, o1 += d, o2 += d;
-            o0 = row16_sum(on ? o0 : 0.0), o1 = row16_sum(on ? o1 : 0.0), o2 = row16_sum(on ? o2 : 0.0);
+            o0 = row_sum(on ? o0 : 0.0), o1 = row_sum(on ? o1 : 0.0), o2 = row_sum(on ? o2 : 0.0);
             if (i16 == v) acc[0] += o0, acc[1] += o1, acc[2] += o2;
         }
     }

@@ -914,7 +914,7 @@ inline int part_rows(int maxrt) { return maxrt > 4 ? kMaxLeaf : kPartRows; }
 
 template <class T, int NT>
 static void launch_nt(arh_hmat *h, MfmaLayout &M, int R, const double2 *x, double2 *y, const int *cols, int j0,
-                      const int *gate, hipStream_t s, int maxrt) {
+                      const int *gate, hipStream_t s, int maxrt, bool packed) {
     typedef typename Mfma<T>::T2 T2;
     constexpr int pi = sizeof(T) == 8 ? 1 : 0;
     arh_geom *g = h->g;
@@ -925,8 +925,9 @@ static void launch_nt(arh_hmat *h, MfmaLayout &M, int R, const double2 *x, doubl
     const int prow = part_rows(maxrt);
     if (M.nslots) M.part[pi].alloc(sizeof(T) * (size_t)M.nslots * prow * 2 * RP);
     T2 *xt = M.xt[pi].as<T2>();
-    hipLaunchKernelGGL(k_pack_xf<T>, dim3((unsigned)std::min<int64_t>(2048, ((int64_t)N * RP + 255) / 256)), dim3(256),
-                       0, s, x, N, R, RP, xt, cols, j0, gate);
+    if (!packed)
+        hipLaunchKernelGGL(k_pack_xf<T>, dim3((unsigned)std::min<int64_t>(2048, ((int64_t)N * RP + 255) / 256)),
+                           dim3(256), 0, s, x, N, R, RP, xt, cols, j0, gate);
     auto timed = [&](int kind, double bytes, double flops, auto &&launch) {
         if (!pf.on) {
             launch();
@@ -985,39 +986,65 @@ static void launch_nt(arh_hmat *h, MfmaLayout &M, int R, const double2 *x, doubl
 
 int mfma_max_leaf() { return kMaxLeaf; }
 
+// Right-hand sides per pass of a geometry's leaves.
+template <class T>
+static int pass_width(const arh_geom *g) {
+    const int maxrt = (g->max_leaf + 15) / 16;
+    return maxrt > 4 ? 8 * max_nt_xtall<T>() : maxrt > 2 ? 8 * max_nt_tall<T>() : kMaxRC;
+}
+
 // y = (M - I/2) x, or its transpose, on the MFMA layout of one precision, right-hand sides in passes
 // of up to kMaxRC. With a column list (device array of ncols indices into the nrhs columns of x
 // and y), only those columns are computed; the others of y are left untouched. A non-null gate
-// skips every pass when *gate is 0.
+// skips every pass when *gate is 0. packed: the caller has filled the packed rows (mfma_packed_rows).
 template <class T>
 static void apply_t(arh_hmat *h, MfmaLayout &M, int R, const double2 *x, double2 *y, hipStream_t s, const int *cols,
-                    int ncols, const int *gate) {
+                    int ncols, const int *gate, bool packed) {
     arh_geom *g = h->g;
     const int maxrt = (g->max_leaf + 15) / 16;
     const int nc = cols ? ncols : R;
     ARH_CHECK(nc >= 0 && nc <= R, ARH_EINVAL, "column list longer than the number of right-hand sides");
-    const int maxrc = maxrt > 4 ? 8 * max_nt_xtall<T>() : maxrt > 2 ? 8 * max_nt_tall<T>() : kMaxRC;
+    const int maxrc = pass_width<T>(g);
     for (int j0 = 0; j0 < nc; j0 += maxrc) {
         const int Rc = std::min(maxrc, nc - j0);
         switch ((Rc + 7) / 8) {
-        case 1: launch_nt<T, 1>(h, M, Rc, x, y, cols, j0, gate, s, maxrt); break;
-        case 2: launch_nt<T, 2>(h, M, Rc, x, y, cols, j0, gate, s, maxrt); break;
-        case 3: launch_nt<T, 3>(h, M, Rc, x, y, cols, j0, gate, s, maxrt); break;
-        case 4: launch_nt<T, 4>(h, M, Rc, x, y, cols, j0, gate, s, maxrt); break;
-        default: launch_nt<T, 5>(h, M, Rc, x, y, cols, j0, gate, s, maxrt); break;
+        case 1: launch_nt<T, 1>(h, M, Rc, x, y, cols, j0, gate, s, maxrt, packed); break;
+        case 2: launch_nt<T, 2>(h, M, Rc, x, y, cols, j0, gate, s, maxrt, packed); break;
+        case 3: launch_nt<T, 3>(h, M, Rc, x, y, cols, j0, gate, s, maxrt, packed); break;
+        case 4: launch_nt<T, 4>(h, M, Rc, x, y, cols, j0, gate, s, maxrt, packed); break;
+        default: launch_nt<T, 5>(h, M, Rc, x, y, cols, j0, gate, s, maxrt, packed); break;
         }
     }
 }
 
+// Where the packed rows of a product with nc right-hand sides go (N rows of *rp complex values of the operator's
+// precision, columns nc .. *rp - 1 zero), for a caller that fills them itself; nullptr if the product takes more
+// than one pass, each of which packs its own rows.
+template <class T>
+static void *packed_rows_t(arh_hmat *h, MfmaLayout &M, int nc, int *rp) {
+    typedef typename Mfma<T>::T2 T2;
+    if (nc < 1 || nc > pass_width<T>(h->g)) return nullptr;
+    *rp = 8 * ((nc + 7) / 8);
+    DBuf &xt = M.xt[sizeof(T) == 8 ? 1 : 0];
+    xt.alloc(sizeof(T2) * (size_t)(h->g->N + h->t_total) * *rp);
+    return xt.p;
+}
+
+void *mfma_packed_rows(arh_hmat *h, int transpose, int fp64, int nc, int *rp) {
+    const int tr = transpose ? 1 : 0;
+    mfma_prepare(h, tr, fp64 ? 1 : 0);
+    return fp64 ? packed_rows_t<double>(h, h->mf[tr], nc, rp) : packed_rows_t<float>(h, h->mf[tr], nc, rp);
+}
+
 void hmat_apply_mfma(arh_hmat *h, int transpose, int fp64, int R, const double2 *x, double2 *y, hipStream_t s,
-                     const int *cols, int ncols, const int *gate) {
+                     const int *cols, int ncols, const int *gate, bool packed) {
     ARH_CHECK(h->g->max_leaf <= mfma_max_leaf(), ARH_EINVAL, "MFMA product supports leaves of at most 128 elements");
     const int tr = transpose ? 1 : 0;
     mfma_prepare(h, tr, fp64 ? 1 : 0);
     if (fp64)
-        apply_t<double>(h, h->mf[tr], R, x, y, s, cols, ncols, gate);
+        apply_t<double>(h, h->mf[tr], R, x, y, s, cols, ncols, gate, packed);
     else
-        apply_t<float>(h, h->mf[tr], R, x, y, s, cols, ncols, gate);
+        apply_t<float>(h, h->mf[tr], R, x, y, s, cols, ncols, gate, packed);
 }
 
 }  // namespace arh

@@ -10,8 +10,8 @@
 //     alpha = rho / (r0^H v); s = r - alpha v; t = A s
 //     w = t^H s / ||t||^2 (0 if ||t|| = 0); x += alpha p + w s; r = s - w t; i++
 // The reductions are two-stage with a fixed split, so every rhs gets the same bits whatever
-// the batch. The loop control (convergence, maxit, breakdown restarts) runs on the device in
-// k_finish, so the host launches K iterations between synchronisations, K chosen from the
+// the batch. The loop control (convergence, maxit, breakdown restarts) runs on the device at
+// the end of an iteration (finish_rhs), so the host launches K iterations between synchronisations, K chosen from the
 // observed convergence rate; a right-hand side that meets a restart pauses until the host
 // restarts it at the next synchronisation, which leaves its arithmetic unchanged.
 #include <algorithm>
@@ -57,7 +57,7 @@ struct RhsState {
     double2 alpha, w;
     double r0sq, rhs_sq, rn, tol2;  // tol2 = tol^2 ||b||^2
     int active;    // iterating
-    int restart;   // restart pending (set at init, or by k_finish on breakdown: then paused)
+    int restart;   // restart pending (set at init, or by finish_rhs on breakdown: then paused)
     int it;        // iterations counted toward maxit (reset at the first restart)
     int iters;     // iterations done
     int nrestart;  // restarts done
@@ -77,12 +77,13 @@ constexpr int kInnerBudget = 256;      // mixed refinement: iterations an inner 
 #endif
 constexpr int kMaxK = ARH_SOLVER_MAXK;  // iterations per host synchronisation, at most
 constexpr int kMaxNB = 128;   // blocks per rhs of a reduction
+constexpr int kLoads = 8, kXrLoads = 4;  // elements of a thread loaded together by the reductions
 
+// v summed over the block, in thread 0
 __device__ __forceinline__ void block_reduce4(double v[4], double *sh) {
     const int lane = threadIdx.x % ARH_WAVE, w = threadIdx.x / ARH_WAVE;
 #pragma unroll
     for (int k = 0; k < 4; k++) v[k] = wave_sum(v[k]);
-    __syncthreads();
     if (lane == 0)
 #pragma unroll
         for (int k = 0; k < 4; k++) sh[w * 4 + k] = v[k];
@@ -95,12 +96,35 @@ __device__ __forceinline__ void block_reduce4(double v[4], double *sh) {
         }
 }
 
-// fixed-order sum of NB partial quadruples
-__device__ __forceinline__ void sum_parts(const double *part, int NB, double out[4]) {
-    out[0] = out[1] = out[2] = out[3] = 0.0;
-    for (int b = 0; b < NB; b++)
+// Sums of the first K components of NB (<= 128) partial quadruples in order, by a wavefront: lane b loads partials b
+// and b + 64 (one load latency instead of NB), then they are added up one by one.
+template <int K>
+__device__ __forceinline__ void sum_parts(const double *part, int NB, double out[K]) {
+    const int lane = threadIdx.x % ARH_WAVE;
+    double v[K], u[K];
 #pragma unroll
-        for (int k = 0; k < 4; k++) out[k] += part[b * 4 + k];
+    for (int k = 0; k < K; k++) v[k] = part[min(lane, NB - 1) * 4 + k];
+    if (NB > ARH_WAVE)
+#pragma unroll
+        for (int k = 0; k < K; k++) u[k] = part[min(lane + ARH_WAVE, NB - 1) * 4 + k];
+#pragma unroll
+    for (int k = 0; k < K; k++) out[k] = 0.0;
+    for (int b = 0; b < min(NB, ARH_WAVE); b++)
+#pragma unroll
+        for (int k = 0; k < K; k++) out[k] += lane_f64(v[k], b);
+    for (int b = ARH_WAVE; b < NB; b++)
+#pragma unroll
+        for (int k = 0; k < K; k++) out[k] += lane_f64(u[k], b - ARH_WAVE);
+}
+
+// Complex products of the vector updates with their rounding written out. BiCGSTAB amplifies a last-bit change to
+// the size of its tolerance within a hundred iterations, so the fused forms are part of the solver's results: the
+// imaginary part rounds a.x b.y (cmul_xy) or a.y b.x (cmul_yx) before the fused multiply-add of the other.
+__device__ __forceinline__ double2 cmul_xy(double2 a, double2 b) {
+    return make_double2(fma(a.x, b.x, -(a.y * b.y)), fma(a.y, b.x, a.x * b.y));
+}
+__device__ __forceinline__ double2 cmul_yx(double2 a, double2 b) {
+    return make_double2(fma(a.x, b.x, -(a.y * b.y)), fma(a.x, b.y, a.y * b.x));
 }
 
 struct Chunk {
@@ -122,13 +146,25 @@ __global__ __launch_bounds__(kVT) void k_dot(const RhsState *__restrict__ S, int
     const Chunk ch = chunk_of(N, NB);
     const int64_t o = (int64_t)j * N;
     double v[4] = {0, 0, 0, 0};
-    for (int i = ch.lo + threadIdx.x; i < ch.hi; i += kVT) {
-        double2 ai = a[o + i], bi = b[o + i];
-        v[0] += ai.x * bi.x + ai.y * bi.y;
-        v[1] += ai.x * bi.y - ai.y * bi.x;
-        if (c) {
-            double2 ci = c[o + i];
-            v[2] += ci.x * ci.x + ci.y * ci.y;
+    // the elements of a thread in order, kLoads of them in flight (surplus loads repeat the chunk's last)
+    for (int i0 = ch.lo + threadIdx.x; i0 < ch.hi; i0 += kLoads * kVT) {
+        double2 av[kLoads], bv[kLoads], cv[kLoads];
+#pragma unroll
+        for (int q = 0; q < kLoads; q++) {
+            const int64_t e = o + min(i0 + q * kVT, ch.hi - 1);
+            av[q] = a[e], bv[q] = b[e];
+            if (c) cv[q] = c[e];
+        }
+#pragma unroll
+        for (int q = 0; q < kLoads; q++) {
+            if (i0 + q * kVT >= ch.hi) break;
+            const double2 ai = av[q], bi = bv[q];
+            v[0] += ai.x * bi.x + ai.y * bi.y;
+            v[1] += ai.x * bi.y - ai.y * bi.x;
+            if (c) {
+                const double2 ci = cv[q];
+                v[2] += ci.x * ci.x + ci.y * ci.y;
+            }
         }
     }
     block_reduce4(v, sh);
@@ -136,36 +172,179 @@ __global__ __launch_bounds__(kVT) void k_dot(const RhsState *__restrict__ S, int
         for (int k = 0; k < 4; k++) part[((int64_t)j * NB + blockIdx.x) * 4 + k] = v[k];
 }
 
-// p = r + beta (p - w v), beta = (rho_new / rho)(alpha / w)
-__global__ __launch_bounds__(kVT) void k_p_update(const RhsState *__restrict__ S, int N, int NB,
-                                                  const double2 *__restrict__ r, double2 *__restrict__ p,
-                                                  const double2 *__restrict__ v) {
-    const int j = blockIdx.y;
-    const RhsState st = S[j];
-    if (!st.active) return;
-    const double2 beta = cmul(cdiv(st.rho_new, st.rho), cdiv(st.alpha, st.w));
-    const Chunk ch = chunk_of(N, NB);
-    const int64_t o = (int64_t)j * N;
-    for (int i = ch.lo + threadIdx.x; i < ch.hi; i += kVT) {
-        double2 pi = p[o + i], vi = v[o + i], ri = r[o + i];
-        double2 q = csub(pi, cmul(st.w, vi));
-        p[o + i] = cadd(ri, cmul(beta, q));
+// The end of an iteration for one rhs, by a wavefront: alpha, w, rho committed; rho_new = r0^H r, rn = |r|^2; then
+// Eigen's loop control: stop when ||r||^2 <= tol2 or it == maxit, pause for a restart when |r0^H r| < eps^2 ||r0||^2.
+__device__ __forceinline__ void finish_rhs(RhsState &st, int j, int NB, const double *__restrict__ part_r0v,
+                                           const double *__restrict__ part_ts, const double *__restrict__ part_rr) {
+    const double eps2 = 4.930380657631324e-32;  // (2^-52)^2, Eigen's NumTraits<double>::epsilon() squared
+    double d[2], e[3], f[3];
+    const int64_t o = (int64_t)j * NB * 4;
+    sum_parts<2>(part_r0v + o, NB, d);
+    sum_parts<3>(part_ts + o, NB, e);
+    sum_parts<3>(part_rr + o, NB, f);
+    st.alpha = cdiv(st.rho_new, make_double2(d[0], d[1]));
+    st.w = e[2] > 0.0 ? make_double2(e[0] / e[2], e[1] / e[2]) : make_double2(0.0, 0.0);
+    st.rho = st.rho_new;
+    st.rho_new = make_double2(f[0], f[1]);
+    st.rn = f[2];
+    st.it++;
+    st.iters++;
+    if (!(st.rn > st.tol2 && st.it < st.maxit)) {
+        st.active = 0;
+    } else if (hypot(st.rho_new.x, st.rho_new.y) < eps2 * st.r0sq) {
+        st.active = 0;
+        st.restart = 1;
     }
 }
 
-// s = r - alpha v, alpha = rho_new / (r0^H v) from the partials
-__global__ __launch_bounds__(kVT) void k_s_update(const RhsState *__restrict__ S, int N, int NB,
-                                                  const double *__restrict__ part_r0v, const double2 *__restrict__ r,
-                                                  const double2 *__restrict__ v, double2 *__restrict__ s) {
-    const int j = blockIdx.y;
-    const RhsState st = S[j];
-    if (!st.active) return;
-    double d[4];
-    sum_parts(part_r0v + (int64_t)j * NB * 4, NB, d);
-    const double2 alpha = cdiv(st.rho_new, make_double2(d[0], d[1]));
-    const Chunk ch = chunk_of(N, NB);
-    const int64_t o = (int64_t)j * N;
-    for (int i = ch.lo + threadIdx.x; i < ch.hi; i += kVT) s[o + i] = csub(r[o + i], cmul(alpha, v[o + i]));
+// States of all rhs after finish_rhs (their new values to out; history of ||r|| / ||b|| on request), a wavefront per rhs:
+// wavefront q of nq. gate[0] (zero before) receives the number of right-hand sides still active.
+__device__ __forceinline__ void finish_all(const RhsState *__restrict__ S, RhsState *__restrict__ out, int R, int NB,
+                                           const double *__restrict__ part_r0v, const double *__restrict__ part_ts,
+                                           const double *__restrict__ part_rr, double *__restrict__ hist, int hist_cap,
+                                           int *__restrict__ gate, int q, int nq) {
+    const int lane = threadIdx.x % ARH_WAVE;
+    for (int j = q; j < R; j += nq) {
+        RhsState st = S[j];
+        if (st.active) {
+            finish_rhs(st, j, NB, part_r0v, part_ts, part_rr);
+            if (lane == 0) {
+                if (hist && st.iters < hist_cap) hist[(int64_t)j * hist_cap + st.iters] = sqrt(st.rn / st.rhs_sq);
+                if (st.active) atomicAdd(gate, 1);
+            }
+        }
+        if (lane == 0) out[j] = st;
+    }
+}
+
+// The end of a batch's last iteration (one wavefront per workgroup).
+__global__ __launch_bounds__(ARH_WAVE) void k_finish(const RhsState *__restrict__ S, RhsState *__restrict__ out, int R,
+                                                     int NB, const double *__restrict__ part_r0v,
+                                                     const double *__restrict__ part_ts,
+                                                     const double *__restrict__ part_rr, double *__restrict__ hist,
+                                                     int hist_cap, int *__restrict__ gate) {
+    finish_all(S, out, R, NB, part_r0v, part_ts, part_rr, hist, hist_cap, gate, blockIdx.x, gridDim.x);
+}
+
+// The vector updates before a product also write the product's packed rows (row i: RP complex values, listed column c
+// at c, zero up to RP), through LDS: a workgroup takes up_rows of the rows and kUpCols of the columns, a wavefront each
+// (every wavefront forms its rhs's scalars, some 400 operations; N = 9,828, p update: 37 right-hand sides FP32 10.4,
+// 7.4, 8.2 us at 64, 128, 192 rows, one FP64 6.0, 6.8, 8.0 us. The end of the previous iteration and the packing
+// were launches of their own: 16.4 us for 37, 15 us for one). T2: complex type of the operator's precision; xf == nullptr leaves the
+// packing to the product.
+constexpr int kUpCols = 16;
+template <class T2>
+constexpr int up_rows() {
+    return sizeof(T2) == 8 ? 128 : 64;
+}
+__device__ __forceinline__ float2 to_packed(double2 v, float2) { return make_float2((float)v.x, (float)v.y); }
+__device__ __forceinline__ double2 to_packed(double2 v, double2) { return v; }
+template <class T2>
+__device__ __forceinline__ void write_packed(const T2 (*tile)[kUpCols + 1], int bx, int N, int nc, int RP,
+                                             T2 *__restrict__ xf) {
+    __syncthreads();
+    const int r0 = bx * up_rows<T2>(), rows = min(up_rows<T2>(), N - r0);
+    const int c0 = (int)blockIdx.y * kUpCols;
+    const int c = threadIdx.x % kUpCols;
+    if (c0 + c >= RP) return;
+    for (int r = threadIdx.x / kUpCols; r < rows; r += blockDim.x / kUpCols) {
+        T2 v{};
+        if (c0 + c < nc) v = tile[r][c];
+        xf[(int64_t)(r0 + r) * RP + c0 + c] = v;
+    }
+}
+
+// p = r + beta (p - w v), beta = (rho_new / rho)(alpha / w), for the listed right-hand sides. finish: the states are
+// those before the end of the previous iteration; every workgroup derives the new ones from the partials, and the
+// workgroups with x = 0 do nothing but write them to out (the others read S, which nothing writes).
+template <class T2>
+__global__ __launch_bounds__(ARH_WAVE * kUpCols) void k_p_update(const RhsState *__restrict__ S, RhsState *__restrict__ out, int R,
+                                                   int finish, int N, int NB, const int *__restrict__ cols, int nc,
+                                                   const double *__restrict__ part_r0v,
+                                                   const double *__restrict__ part_ts,
+                                                   const double *__restrict__ part_rr, const double2 *__restrict__ r,
+                                                   double2 *__restrict__ p, const double2 *__restrict__ v,
+                                                   double *__restrict__ hist, int hist_cap, int *__restrict__ gate,
+                                                   T2 *__restrict__ xf, int RP) {
+    constexpr int Q = up_rows<T2>() / ARH_WAVE;  // rows per lane
+    __shared__ T2 tile[up_rows<T2>()][kUpCols + 1];
+    const int lane = threadIdx.x % ARH_WAVE, w = threadIdx.x / ARH_WAVE, nw = blockDim.x / ARH_WAVE;
+    if (finish && blockIdx.x == 0) {
+        finish_all(S, out, R, NB, part_r0v, part_ts, part_rr, hist, hist_cap, gate, (int)blockIdx.y * nw + w,
+                   (int)gridDim.y * nw);
+        return;
+    }
+    const int bx = (int)blockIdx.x - (finish ? 1 : 0);
+    const int i0 = bx * up_rows<T2>() + lane;
+    const int c0 = (int)blockIdx.y * kUpCols;
+    for (int c = w; c < kUpCols && c0 + c < nc; c += nw) {
+        const int j = cols[c0 + c];
+        RhsState st = S[j];
+        const int64_t o = (int64_t)j * N;
+        double2 q[Q], vi[Q], ri[Q];
+#pragma unroll
+        for (int t = 0; t < Q; t++) {
+            const int64_t e = o + min(i0 + t * ARH_WAVE, N - 1);
+            q[t] = p[e], vi[t] = v[e], ri[t] = r[e];
+        }
+        if (st.active) {
+            if (finish) finish_rhs(st, j, NB, part_r0v, part_ts, part_rr);
+            if (st.active) {
+                const double2 beta = cmul_xy(cdiv(st.rho_new, st.rho), cdiv(st.alpha, st.w));
+#pragma unroll
+                for (int t = 0; t < Q; t++) {
+                    q[t] = cadd(ri[t], cmul_yx(beta, csub(q[t], cmul_xy(st.w, vi[t]))));
+                    if (i0 + t * ARH_WAVE < N) p[o + i0 + t * ARH_WAVE] = q[t];
+                }
+            }
+        }
+        if (xf)
+#pragma unroll
+            for (int t = 0; t < Q; t++) tile[t * ARH_WAVE + lane][c] = to_packed(q[t], T2{});
+    }
+    if (xf) write_packed<T2>(tile, bx, N, nc, RP, xf);
+}
+
+// s = r - alpha v, alpha = rho_new / (r0^H v) from the partials, for the listed right-hand sides
+template <class T2>
+__global__ __launch_bounds__(ARH_WAVE * kUpCols) void k_s_update(const RhsState *__restrict__ S, int N, int NB,
+                                                   const int *__restrict__ cols, int nc,
+                                                   const double *__restrict__ part_r0v, const double2 *__restrict__ r,
+                                                   const double2 *__restrict__ v, double2 *__restrict__ s,
+                                                   T2 *__restrict__ xf, int RP) {
+    constexpr int Q = up_rows<T2>() / ARH_WAVE;  // rows per lane
+    __shared__ T2 tile[up_rows<T2>()][kUpCols + 1];
+    const int lane = threadIdx.x % ARH_WAVE, w = threadIdx.x / ARH_WAVE, nw = blockDim.x / ARH_WAVE;
+    const int i0 = (int)blockIdx.x * up_rows<T2>() + lane;
+    const int c0 = (int)blockIdx.y * kUpCols;
+    for (int c = w; c < kUpCols && c0 + c < nc; c += nw) {
+        const int j = cols[c0 + c];
+        const int64_t o = (int64_t)j * N;
+        double2 q[Q];
+        if (S[j].active) {
+            double2 vi[Q];
+#pragma unroll
+            for (int t = 0; t < Q; t++) {
+                const int64_t e = o + min(i0 + t * ARH_WAVE, N - 1);
+                q[t] = r[e], vi[t] = v[e];
+            }
+            double d[2];
+            sum_parts<2>(part_r0v + (int64_t)j * NB * 4, NB, d);
+            const double2 alpha = cdiv(S[j].rho_new, make_double2(d[0], d[1]));
+#pragma unroll
+            for (int t = 0; t < Q; t++) {
+                q[t] = csub(q[t], cmul_xy(alpha, vi[t]));
+                if (i0 + t * ARH_WAVE < N) s[o + i0 + t * ARH_WAVE] = q[t];
+            }
+        } else {  // a paused rhs keeps its vectors: the product recomputes the same t
+#pragma unroll
+            for (int t = 0; t < Q; t++) q[t] = s[o + min(i0 + t * ARH_WAVE, N - 1)];
+        }
+        if (xf)
+#pragma unroll
+            for (int t = 0; t < Q; t++) tile[t * ARH_WAVE + lane][c] = to_packed(q[t], T2{});
+    }
+    if (xf) write_packed<T2>(tile, (int)blockIdx.x, N, nc, RP, xf);
 }
 
 // x += alpha p + w s; r = s - w t; partials of r0^H r and |r|^2
@@ -179,79 +358,41 @@ __global__ __launch_bounds__(kVT) void k_xr_update(const RhsState *__restrict__ 
     const int j = blockIdx.y;
     const RhsState st = S[j];
     if (!st.active) return;
-    double d[4], e[4];
-    sum_parts(part_r0v + (int64_t)j * NB * 4, NB, d);
-    sum_parts(part_ts + (int64_t)j * NB * 4, NB, e);
+    double d[2], e[3];
+    sum_parts<2>(part_r0v + (int64_t)j * NB * 4, NB, d);
+    sum_parts<3>(part_ts + (int64_t)j * NB * 4, NB, e);
     const double2 alpha = cdiv(st.rho_new, make_double2(d[0], d[1]));
     const double tt = e[2];
     const double2 w = tt > 0.0 ? make_double2(e[0] / tt, e[1] / tt) : make_double2(0.0, 0.0);
     const Chunk ch = chunk_of(N, NB);
     const int64_t o = (int64_t)j * N;
     double v[4] = {0, 0, 0, 0};
-    for (int i = ch.lo + threadIdx.x; i < ch.hi; i += kVT) {
-        double2 si = s[o + i], ti = t[o + i];
-        double2 xi = x[o + i];
-        xi = cadd(xi, cadd(cmul(alpha, p[o + i]), cmul(w, si)));
-        x[o + i] = xi;
-        double2 ri = csub(si, cmul(w, ti));
-        r[o + i] = ri;
-        double2 qi = r0[o + i];
-        v[0] += qi.x * ri.x + qi.y * ri.y;
-        v[1] += qi.x * ri.y - qi.y * ri.x;
-        v[2] += ri.x * ri.x + ri.y * ri.y;
+    for (int i0 = ch.lo + threadIdx.x; i0 < ch.hi; i0 += kXrLoads * kVT) {
+        double2 sv[kXrLoads], tv[kXrLoads], xv[kXrLoads], pv[kXrLoads], qv[kXrLoads];
+#pragma unroll
+        for (int q = 0; q < kXrLoads; q++) {
+            const int64_t e = o + min(i0 + q * kVT, ch.hi - 1);
+            sv[q] = s[e], tv[q] = t[e], xv[q] = x[e], pv[q] = p[e], qv[q] = r0[e];
+        }
+#pragma unroll
+        for (int q = 0; q < kXrLoads; q++) {
+            const int i = i0 + q * kVT;
+            if (i >= ch.hi) break;
+            const double2 si = sv[q], ti = tv[q];
+            double2 xi = xv[q];
+            xi = cadd(xi, cadd(cmul_xy(alpha, pv[q]), cmul_xy(w, si)));
+            x[o + i] = xi;
+            double2 ri = csub(si, cmul_xy(w, ti));
+            r[o + i] = ri;
+            double2 qi = qv[q];
+            v[0] += qi.x * ri.x + qi.y * ri.y;
+            v[1] += qi.x * ri.y - qi.y * ri.x;
+            v[2] += ri.x * ri.x + ri.y * ri.y;
+        }
     }
     block_reduce4(v, sh);
     if (threadIdx.x == 0)
         for (int k = 0; k < 4; k++) part_rr[((int64_t)j * NB + blockIdx.x) * 4 + k] = v[k];
-}
-
-// end of an iteration: commit alpha, w, rho; rho_new = r0^H r, rn = |r|^2; then Eigen's loop
-// control for the next iteration: stop when ||r||^2 <= tol2 or it == maxit, pause for a restart
-// when |r0^H r| < eps^2 ||r0||^2. Optional history of ||r|| / ||b||. One workgroup; gate[0]
-// receives the number of right-hand sides still active.
-__global__ __launch_bounds__(256) void k_finish(RhsState *__restrict__ S, int R, int NB,
-                                                const double *__restrict__ part_r0v,
-                                                const double *__restrict__ part_ts, const double *__restrict__ part_rr,
-                                                double *__restrict__ hist, int hist_cap, int *__restrict__ gate,
-                                                int *__restrict__ gate_hist) {
-    __shared__ int cnt[256 / ARH_WAVE];
-    const double eps2 = 4.930380657631324e-32;  // (2^-52)^2, Eigen's NumTraits<double>::epsilon() squared
-    int nact = 0;
-    for (int j = threadIdx.x; j < R; j += blockDim.x) {
-        RhsState st = S[j];
-        if (!st.active) continue;
-        double d[4], e[4], f[4];
-        sum_parts(part_r0v + (int64_t)j * NB * 4, NB, d);
-        sum_parts(part_ts + (int64_t)j * NB * 4, NB, e);
-        sum_parts(part_rr + (int64_t)j * NB * 4, NB, f);
-        st.alpha = cdiv(st.rho_new, make_double2(d[0], d[1]));
-        st.w = e[2] > 0.0 ? make_double2(e[0] / e[2], e[1] / e[2]) : make_double2(0.0, 0.0);
-        st.rho = st.rho_new;
-        st.rho_new = make_double2(f[0], f[1]);
-        st.rn = f[2];
-        st.it++;
-        st.iters++;
-        if (hist && st.iters < hist_cap) hist[(int64_t)j * hist_cap + st.iters] = sqrt(st.rn / st.rhs_sq);
-        if (!(st.rn > st.tol2 && st.it < st.maxit)) {
-            st.active = 0;
-        } else if (hypot(st.rho_new.x, st.rho_new.y) < eps2 * st.r0sq) {
-            st.active = 0;
-            st.restart = 1;
-        } else {
-            nact++;
-        }
-        S[j] = st;
-    }
-    // integer count: the same whatever the order of the additions
-    for (int off = ARH_WAVE / 2; off > 0; off >>= 1) nact += __shfl_xor(nact, off, ARH_WAVE);
-    if (threadIdx.x % ARH_WAVE == 0) cnt[threadIdx.x / ARH_WAVE] = nact;
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        int c = 0;
-        for (int k = 0; k < (int)blockDim.x / ARH_WAVE; k++) c += cnt[k];
-        gate[0] = c;
-        gate_hist[0] = c;
-    }
 }
 
 // (re)start of rhs j: r = b - Ax (Ax given, or zero), r0 = r, partials of |r|^2 (and b^2 on init)
@@ -281,13 +422,14 @@ __global__ __launch_bounds__(kVT) void k_restart(const RhsState *__restrict__ S,
 // full restart: rho = r0sq = |r|^2; fresh: also alpha = w = rho_old = 1, rhs_sq, and the caller
 // zeroes p, v (the host decides activity after a fresh start); a breakdown restart resumes the
 // iteration (active again) and resets the iteration count on the first restart (Eigen)
-__global__ void k_restart_finish(RhsState *__restrict__ S, int R, int NB, const double *__restrict__ part,
-                                 int fresh) {
-    const int j = blockIdx.x * blockDim.x + threadIdx.x;
-    if (j >= R || !S[j].restart) return;
+// (a wavefront per rhs)
+__global__ __launch_bounds__(ARH_WAVE) void k_restart_finish(RhsState *__restrict__ S, int NB,
+                                                             const double *__restrict__ part, int fresh) {
+    const int j = blockIdx.x;
+    if (!S[j].restart) return;
     RhsState st = S[j];
-    double f[4];
-    sum_parts(part + (int64_t)j * NB * 4, NB, f);
+    double f[2];
+    sum_parts<2>(part + (int64_t)j * NB * 4, NB, f);
     st.r0sq = f[0];
     st.rho_new = make_double2(f[0], 0.0);
     st.rn = f[0];
@@ -301,7 +443,7 @@ __global__ void k_restart_finish(RhsState *__restrict__ S, int R, int NB, const 
         st.active = 1;
     }
     st.restart = 0;
-    S[j] = st;
+    if (threadIdx.x == 0) S[j] = st;
 }
 
 // masked zeroing of columns (p, v on fresh starts; x on init)
@@ -353,18 +495,18 @@ struct Work {
     DBuf buf, hbuf;
     double2 *r, *r0, *p, *v, *s, *t, *Ax;
     double *part;
-    RhsState *S;
+    RhsState *S, *S2;  // states, and the other copy an iteration writes
     int *mask;
-    int *ctl;  // [0]: gate (active count), [1..]: column list
-    int *ghist;  // active count after each iteration of a batch
+    int *ctl;  // [0]: active count at a batch's start, [1..R]: column list
+    int *ghist;  // after the list: active count after each iteration of a batch (the gate of the next one)
     void init(int64_t N, int R, int NB) {
         const int64_t vec = N * R;
         const size_t vb = sizeof(double2) * vec;
         const size_t pb = sizeof(double) * 4 * (size_t)R * NB;
         // every piece starts on a 256-byte boundary: the total is the sum of the rounded sizes
         auto rnd = [](size_t n) { return (n + 255) / 256 * 256; };
-        const size_t total = 7 * rnd(vb) + rnd(4 * pb) + rnd(sizeof(RhsState) * R) + rnd(sizeof(int) * R) +
-                             rnd(sizeof(int) * (R + 1)) + rnd(sizeof(int) * kMaxK);
+        const size_t total = 7 * rnd(vb) + rnd(4 * pb) + 2 * rnd(sizeof(RhsState) * R) + rnd(sizeof(int) * R) +
+                             rnd(sizeof(int) * (R + 1 + kMaxK));
         buf.alloc(total);
         char *c = buf.as<char>();
         char *const end = c + total;
@@ -378,9 +520,10 @@ struct Work {
         s = (double2 *)take(vb), t = (double2 *)take(vb), Ax = (double2 *)take(vb);
         part = (double *)take(4 * pb);
         S = (RhsState *)take(sizeof(RhsState) * R);
+        S2 = (RhsState *)take(sizeof(RhsState) * R);
         mask = (int *)take(sizeof(int) * R);
-        ctl = (int *)take(sizeof(int) * (R + 1));
-        ghist = (int *)take(sizeof(int) * kMaxK);
+        ctl = (int *)take(sizeof(int) * (R + 1 + kMaxK));
+        ghist = ctl + R + 1;
     }
 };
 
@@ -406,7 +549,6 @@ static void bicgstab(arh_hmat *h, int transpose, int prec, int R, const double2 
     hipStream_t s = ctx->stream;
     const int N = h->g->N;
     const dim3 gv(NB, R), bv(kVT);
-    const int pblk = (R + 63) / 64;
     const int zblk = std::max(1, std::min(1024, (N + 255) / 256));
     double *P1 = W.part, *P2 = W.part + 4 * (size_t)R * NB, *P3 = W.part + 8 * (size_t)R * NB;
     const bool hist_on = record_hist && st && st->hist && st->hist_len && o.hist_cap > 0;
@@ -426,7 +568,7 @@ static void bicgstab(arh_hmat *h, int transpose, int prec, int R, const double2 
     hipLaunchKernelGGL(k_zero_cols, dim3(zblk, R), dim3(256), 0, s, W.S, N, W.p, 1);
     hipLaunchKernelGGL(k_zero_cols, dim3(zblk, R), dim3(256), 0, s, W.S, N, W.v, 1);
     hipLaunchKernelGGL(k_restart, gv, bv, 0, s, W.S, N, NB, b, (const double2 *)nullptr, W.r, W.r0, P1);
-    hipLaunchKernelGGL(k_restart_finish, dim3(pblk), dim3(64), 0, s, W.S, R, NB, P1, 1);
+    hipLaunchKernelGGL(k_restart_finish, dim3(R), dim3(ARH_WAVE), 0, s, W.S, NB, P1, 1);
     ARH_HIP(hipGetLastError());
     ARH_HIP(hipMemcpyAsync(hs.data(), W.S, sizeof(RhsState) * R, hipMemcpyDeviceToHost, s));
     ARH_HIP(hipStreamSynchronize(s));
@@ -456,33 +598,63 @@ static void bicgstab(arh_hmat *h, int transpose, int prec, int R, const double2 
     int K = 2;
     // separate host buffers for the two lists: a list is rewritten only after the stream has been
     // synchronised since its last copy
-    std::vector<int> ctl(R + 1), ctl_rs(R + 1);
+    std::vector<int> ctl(R + 1 + kMaxK, 0), ctl_rs(R + 1);
     std::vector<double> best(err);
     std::vector<int> best_it(R, 0);
+    RhsState *S = W.S, *So = W.S2;  // current states, and where the next iteration's go
+    const bool fp64 = prec != ARH_MIXED, fused = h->g->max_leaf <= mfma_max_leaf();
     while (nact > 0) {
         int nc = 0;
         for (int j = 0; j < R; j++)
             if (hs[j].active) ctl[1 + nc++] = j;
         ctl[0] = nc;
-        ARH_HIP(hipMemcpyAsync(W.ctl, ctl.data(), sizeof(int) * (nc + 1), hipMemcpyHostToDevice, s));
-        const int *cols = W.ctl + 1, *gate = W.ctl;
+        ARH_HIP(hipMemcpyAsync(W.ctl, ctl.data(), sizeof(int) * ctl.size(), hipMemcpyHostToDevice, s));
+        const int *cols = W.ctl + 1;
+        // the updates write the product's packed rows where one pass takes every active rhs
+        int rp = 0;
+        void *xf = fused ? mfma_packed_rows(h, transpose, fp64 ? 1 : 0, nc, &rp) : nullptr;
+        // a wavefront per listed rhs, and enough of them for the workgroups that write all states
+        const dim3 bu(ARH_WAVE * std::min(kUpCols, std::max(nc, (R + 3) / 4)));
+        const unsigned guy = (unsigned)((std::max(nc, rp) + kUpCols - 1) / kUpCols);
+        const int ur = xf && !fp64 ? up_rows<float2>() : up_rows<double2>();
+        const unsigned gu = (unsigned)((N + ur - 1) / ur);
+        auto apply = [&](const double2 *in, double2 *out, const int *gate) {
+            if (xf)
+                hmat_apply_mfma(h, transpose, fp64 ? 1 : 0, R, in, out, s, cols, nc, gate, true);
+            else
+                hmat_apply(h, transpose, prec, R, in, out, s, cols, nc, gate);
+        };
         for (int k = 0; k < K; k++) {
             ctx->prof.cur_slot = k;
-            hipLaunchKernelGGL(k_p_update, gv, bv, 0, s, W.S, N, NB, W.r, W.p, W.v);
-            hmat_apply(h, transpose, prec, R, W.p, W.v, s, cols, nc, gate);
-            hipLaunchKernelGGL(k_dot, gv, bv, 0, s, W.S, N, NB, W.r0, W.v, (const double2 *)nullptr, P1);
-            hipLaunchKernelGGL(k_s_update, gv, bv, 0, s, W.S, N, NB, P1, W.r, W.v, W.s);
-            hmat_apply(h, transpose, prec, R, W.s, W.t, s, cols, nc, gate);
-            hipLaunchKernelGGL(k_dot, gv, bv, 0, s, W.S, N, NB, W.t, W.s, W.t, P2);
-            hipLaunchKernelGGL(k_xr_update, gv, bv, 0, s, W.S, N, NB, P1, P2, W.p, W.s, W.t, W.r0, x, W.r, P3);
-            hipLaunchKernelGGL(k_finish, dim3(1), dim3(256), 0, s, W.S, R, NB, P1, P2, P3, hist_dev, cap, W.ctl,
-                               W.ghist + k);
-            ARH_HIP(hipGetLastError());
+            const int fin = k > 0 ? 1 : 0;  // the end of the previous iteration
+            int *gate = fin ? W.ghist + k - 1 : W.ctl;  // active right-hand sides
+            if (xf && !fp64)
+                hipLaunchKernelGGL(k_p_update<float2>, dim3(gu + fin, guy), bu, 0, s, S, So, R, fin, N, NB, cols, nc, P1, P2,
+                                   P3, W.r, W.p, W.v, hist_dev, cap, gate, (float2 *)xf, rp);
+            else
+                hipLaunchKernelGGL(k_p_update<double2>, dim3(gu + fin, guy), bu, 0, s, S, So, R, fin, N, NB, cols, nc, P1,
+                                   P2, P3, W.r, W.p, W.v, hist_dev, cap, gate, (double2 *)xf, rp);
+            if (fin) std::swap(S, So);
+            apply(W.p, W.v, gate);
+            hipLaunchKernelGGL(k_dot, gv, bv, 0, s, S, N, NB, W.r0, W.v, (const double2 *)nullptr, P1);
+            if (xf && !fp64)
+                hipLaunchKernelGGL(k_s_update<float2>, dim3(gu, guy), bu, 0, s, S, N, NB, cols, nc, P1, W.r, W.v, W.s,
+                                   (float2 *)xf, rp);
+            else
+                hipLaunchKernelGGL(k_s_update<double2>, dim3(gu, guy), bu, 0, s, S, N, NB, cols, nc, P1, W.r, W.v, W.s,
+                                   (double2 *)xf, rp);
+            apply(W.s, W.t, gate);
+            hipLaunchKernelGGL(k_dot, gv, bv, 0, s, S, N, NB, W.t, W.s, W.t, P2);
+            hipLaunchKernelGGL(k_xr_update, gv, bv, 0, s, S, N, NB, P1, P2, W.p, W.s, W.t, W.r0, x, W.r, P3);
         }
+        hipLaunchKernelGGL(k_finish, dim3(R), dim3(ARH_WAVE), 0, s, S, So, R, NB, P1, P2, P3, hist_dev, cap,
+                           W.ghist + K - 1);
+        std::swap(S, So);
+        ARH_HIP(hipGetLastError());
         ctx->prof.cur_slot = -1;
         int gh[kMaxK];
         ARH_HIP(hipMemcpyAsync(gh, W.ghist, sizeof(int) * K, hipMemcpyDeviceToHost, s));
-        ARH_HIP(hipMemcpyAsync(hs.data(), W.S, sizeof(RhsState) * R, hipMemcpyDeviceToHost, s));
+        ARH_HIP(hipMemcpyAsync(hs.data(), S, sizeof(RhsState) * R, hipMemcpyDeviceToHost, s));
         ARH_HIP(hipStreamSynchronize(s));
         if (ctx->prof.on) {
             // iteration k's products ran iff some rhs was active after iteration k - 1
@@ -510,7 +682,7 @@ static void bicgstab(arh_hmat *h, int transpose, int prec, int R, const double2 
                     changed = true;
                 }
             }
-            if (changed) ARH_HIP(hipMemcpyAsync(W.S, hs.data(), sizeof(RhsState) * R, hipMemcpyHostToDevice, s));
+            if (changed) ARH_HIP(hipMemcpyAsync(S, hs.data(), sizeof(RhsState) * R, hipMemcpyHostToDevice, s));
         }
         // breakdown restarts: r = b - A x, r0 = r for the paused right-hand sides
         int nrs = 0;
@@ -521,8 +693,8 @@ static void bicgstab(arh_hmat *h, int transpose, int prec, int R, const double2 
             ARH_HIP(hipMemcpyAsync(W.ctl, ctl_rs.data(), sizeof(int) * (nrs + 1), hipMemcpyHostToDevice, s));
             hmat_apply(h, transpose, prec, R, x, W.Ax, s, W.ctl + 1, nrs, W.ctl);
             if (st) st->matvecs++;
-            hipLaunchKernelGGL(k_restart, gv, bv, 0, s, W.S, N, NB, b, W.Ax, W.r, W.r0, P1);
-            hipLaunchKernelGGL(k_restart_finish, dim3(pblk), dim3(64), 0, s, W.S, R, NB, P1, 0);
+            hipLaunchKernelGGL(k_restart, gv, bv, 0, s, S, N, NB, b, W.Ax, W.r, W.r0, P1);
+            hipLaunchKernelGGL(k_restart_finish, dim3(R), dim3(ARH_WAVE), 0, s, S, NB, P1, 0);
             ARH_HIP(hipGetLastError());
             for (int j = 0; j < R; j++)
                 if (hs[j].restart) {
