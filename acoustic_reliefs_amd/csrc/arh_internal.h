@@ -223,7 +223,7 @@ struct RowTask {
 
 // One orientation (forward or transposed) of the MFMA product: operator copies in their own layout
 // ([0] FP32, [1] FP64, each built on first use or at assembly), the packed rhs + intermediates
-// buffer ([x; t] rows of RP complex), split leaves' partial tiles, and the shared work lists:
+// buffer ([x; t] rows), split leaves' partial tiles, and the shared work lists:
 // stacks, phase-1 units (stack, 32-row tile; stacks with many columns first, one workgroup each),
 // per-leaf panels and their source rows, row tasks, split leaves (leaf, first partial slot, task
 // count), layout builder maps.
@@ -360,7 +360,7 @@ void hmat_apply(arh_hmat *h, int transpose, int precision, int nrhs, const doubl
 // matvec_mfma.hip
 void hmat_apply_mfma(arh_hmat *h, int transpose, int fp64, int nrhs, const double2 *x, double2 *y, hipStream_t s,
                      const int *cols = nullptr, int ncols = 0, const int *gate = nullptr, bool packed = false);
-void *mfma_packed_rows(arh_hmat *h, int transpose, int fp64, int nc, int *rp);
+void *mfma_packed_rows(arh_hmat *h, int transpose, int fp64, int nc, int *rw);
 void mfma_prepare(arh_hmat *h, int transpose, int fp64);
 // matvec64.hip
 void hmat_apply64(arh_hmat *h, int nrhs, const double2 *x, double2 *y, hipStream_t s);

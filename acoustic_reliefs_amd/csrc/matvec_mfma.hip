@@ -17,7 +17,8 @@
 //  * fused row-leaf panels: per row leaf, its dense columns followed by the U columns of every
 //    low-rank block covering it (zero-padded to a multiple of 4 columns), with one source row per
 //    column into the packed [x; t] buffer, so phase 2 (y = D x + U t) is one uniform column sweep.
-// The rhs block and the intermediates share one row-major buffer xt (row i: RP complex values).
+// The rhs block and the intermediates share one row-major buffer xt (row i: row_width(R) complex
+// values).
 //
 // Work is cut into "groups" of 4 consecutive columns. Each wavefront loads the next stage of groups
 // (A entries + xt rows) before multiplying the current one, which hides the memory latency
@@ -98,6 +99,10 @@ constexpr int row_depth() {
 // so the register budget, not the workgroup size, sets how many fit a compute unit.
 constexpr int kLrWaves = ARH_MV_WAVES;    // V-stack units (big stacks: the whole workgroup)
 constexpr int kRowWaves = ARH_MV_RWAVES;  // row tasks
+// Small V-stack units per workgroup: one wavefront per SIMD, the other wavefronts leave at once. Units differ in length,
+// and eight to a workgroup kept its registers until the longest was done: FP32 37 rhs 62.5 -> 61 us (58 -> 53.5 us
+// at 1000 Hz, transposed 65 -> 61), FP64 one rhs 48 -> 42 us; 2, 3, 5 and 6 units are slower than 4.
+constexpr int kLrSmall = 4;
 constexpr bool kChunked = ARH_MV_CHUNKED;  // a workgroup's waves take contiguous group ranges (else strided)
 constexpr bool kXcdOrder = ARH_MV_XCD;     // row tasks ordered for the per-die L2s
 constexpr int kXcds = 8;                   // dies (XCDs) of an MI355X, each with its own L2
@@ -116,14 +121,14 @@ __device__ __forceinline__ int64_t col_of(const int *cols, int j0, int j) { retu
 // A pass is skipped when the gate (the solver's count of active right-hand sides) is 0.
 __device__ __forceinline__ bool gated(const int *gate) { return gate && *gate == 0; }
 
-// xt[i * RP + j] = x[col j][i] for j < R, 0 for R <= j < RP (rows i < N)
+// xt[i * RW + j] = x[col j][i] for j < R, 0 for R <= j < RW (rows i < N)
 template <class T>
-__global__ void k_pack_xf(const double2 *__restrict__ x, int N, int R, int RP, typename Mfma<T>::T2 *__restrict__ xf,
+__global__ void k_pack_xf(const double2 *__restrict__ x, int N, int R, int RW, typename Mfma<T>::T2 *__restrict__ xf,
                           const int *__restrict__ cols, int j0, const int *__restrict__ gate) {
     if (gated(gate)) return;
-    const int64_t total = (int64_t)N * RP;
+    const int64_t total = (int64_t)N * RW;
     for (int64_t e = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; e < total; e += (int64_t)gridDim.x * blockDim.x) {
-        const int i = (int)(e / RP), j = (int)(e % RP);
+        const int i = (int)(e / RW), j = (int)(e % RW);
         double2 d = make_double2(0.0, 0.0);
         if (j < R) d = x[col_of(cols, j0, j) * N + i];
         xf[e] = Mfma<T>::make(d.x, d.y);
@@ -194,6 +199,19 @@ __device__ __forceinline__ void grp_load(Grp<T, NT, NRT> &g, T okf, const typena
     for (int rt = 0; rt < NRT; rt++) g.a[rt] = acol[min(rt * 16 + i16, amax)];
 #pragma unroll
     for (int nt = 0; nt < NT; nt++) g.xb[nt] = brow[nt * 16];
+}
+
+// Packed rows hold row_width(R) complex values: R up to kNarrow, so that one right-hand side does not move eight values a
+// row through the caches (FP64, one rhs, 2000 Hz: V stacks 42 -> 37 us, rows 60 -> 55 us), else R rounded up to whole
+// tiles (rows of 37 values are not aligned: stacks 60 -> 62.5 us, 0.9 m relief 444 -> 477 us).
+constexpr int kNarrow = 4;
+__host__ __device__ constexpr int row_width(int R) { return R <= kNarrow ? R : (R + 7) / 8 * 8; }
+
+// Column of a packed row that a lane reads for its tiles: lanes past the last rhs of a narrow row read that one again
+// (their outputs are dropped).
+template <bool NARROW>
+__device__ __forceinline__ int lane_col(int i16, int R) {
+    return NARROW ? 2 * min(i16 >> 1, R - 1) + (i16 & 1) : i16;
 }
 
 // Component kk (0..3) of v as bit selects (lane-dependent kk: no branches, no exec-mask changes).
@@ -324,10 +342,9 @@ __device__ __forceinline__ void reduce_waves(Acc<T, NT, NRT> &acc, T *red, int w
     }
 }
 
-// Write a wave's result tile as rows of 2 RP values: tile[row * 2 RP + n] (row < rows).
+// Write a wave's result tile as rows of W <= 16 NT values: tile[row * W + n] (row < rows, n < W).
 template <class T, int NT, int NRT>
-__device__ __forceinline__ void store_tile(const Acc<T, NT, NRT> &acc, T *tile, int rows, int lane) {
-    constexpr int W = 16 * NT;
+__device__ __forceinline__ void store_tile(const Acc<T, NT, NRT> &acc, T *tile, int rows, int W, int lane) {
     const int i16 = lane & 15, kk = lane >> 4;
 #pragma unroll
     for (int rt = 0; rt < NRT; rt++)
@@ -336,7 +353,7 @@ __device__ __forceinline__ void store_tile(const Acc<T, NT, NRT> &acc, T *tile, 
 #pragma unroll
             for (int v = 0; v < 4; v++) {
                 const int row = rt * 16 + Mfma<T>::row(kk, v);
-                if (row < rows) tile[row * W + nt * 16 + i16] = acc[rt][nt][v];
+                if (row < rows && nt * 16 + i16 < W) tile[row * W + nt * 16 + i16] = acc[rt][nt][v];
             }
 }
 
@@ -344,16 +361,17 @@ __device__ __forceinline__ void store_tile(const Acc<T, NT, NRT> &acc, T *tile, 
 // A unit is (stack, 32 stacked rows). Units [0, nbig) belong to stacks with at least kBigCols
 // columns: the whole workgroup takes the unit and reduces in LDS. The rest are taken one per
 // wavefront. The results go to xt rows t_row + p.
-template <class T, int NT, int NRT>
+template <class T, int NT, bool NARROW, int NRT>
 __device__ __forceinline__ void lr_run(const VStack &S, int base, const typename Mfma<T>::T2 *__restrict__ V,
-                                       typename Mfma<T>::T2 *__restrict__ xt, T *red, bool big, int w, int lane) {
+                                       typename Mfma<T>::T2 *__restrict__ xt, int R, T *red, bool big, int w,
+                                       int lane) {
     typedef typename Mfma<T>::T2 T2;
-    constexpr int RP = 8 * NT;
     const int r = S.rtot, n = S.n;
     const int i16 = lane & 15, kk = lane >> 4, s = i16 & 1;
     const int amax = min(32, r - base) - 1;
     const T2 *A0 = V + S.v_off + base;
-    const T *B0 = reinterpret_cast<const T *>(xt) + (int64_t)S.cs * 2 * RP + i16;
+    const int RW = NARROW ? R : 8 * NT;
+    const T *B0 = reinterpret_cast<const T *>(xt) + (int64_t)S.cs * 2 * RW + lane_col<NARROW>(i16, R);
     Acc<T, NT, NRT> acc;
     zero_acc<T, NT, NRT>(acc);
     const int ngr = (n + 3) >> 2;
@@ -364,21 +382,21 @@ __device__ __forceinline__ void lr_run(const VStack &S, int base, const typename
             const int c = q * 4 + kk;
             const bool ok = c < n;
             const int cc = ok ? c : q * 4;
-            grp_load<T, NT, NRT>(g, ok ? T(1) : T(0), A0 + (int64_t)cc * r, amax, i16, B0 + (int64_t)cc * 2 * RP);
+            grp_load<T, NT, NRT>(g, ok ? T(1) : T(0), A0 + (int64_t)cc * r, amax, i16, B0 + (int64_t)cc * 2 * RW);
         });
     if (big) {
         reduce_waves<kLrWaves, T, NT, NRT>(acc, red, w, lane);
         if (w != 0) return;
     }
-    T *out = reinterpret_cast<T *>(xt + (S.t_row + base) * RP);
-    store_tile<T, NT, NRT>(acc, out, r - base, lane);
+    T *out = reinterpret_cast<T *>(xt + (S.t_row + base) * RW);
+    store_tile<T, NT, NRT>(acc, out, r - base, 2 * RW, lane);
 }
 
-template <class T, int NT>
+template <class T, int NT, bool NARROW = false>
 __global__ __launch_bounds__(64 * kLrWaves) void k_lr_mfma(const VStack *__restrict__ stacks,
                                                          const int2 *__restrict__ units, int nbig, int nunits,
                                                          const typename Mfma<T>::T2 *__restrict__ V,
-                                                         typename Mfma<T>::T2 *__restrict__ xt,
+                                                         typename Mfma<T>::T2 *__restrict__ xt, int R,
                                                          const int *__restrict__ gate) {
     __shared__ Lds<T, NT, kLrWaves> red;
     if (gated(gate)) return;
@@ -387,12 +405,13 @@ __global__ __launch_bounds__(64 * kLrWaves) void k_lr_mfma(const VStack *__restr
     const int u = big ? (int)blockIdx.x : nbig + ((int)blockIdx.x - nbig) * kLrWaves + w;
     if (u >= nunits) return;  // small units only: big workgroups always have a unit
     const int2 un = units[u];
+    if (un.x < 0) return;  // padding
     const VStack S = stacks[un.x];
     const int base = un.y * 32;
     if (S.rtot - base > 16)
-        lr_run<T, NT, 2>(S, base, V, xt, red.v, big, w, lane);
+        lr_run<T, NT, NARROW, 2>(S, base, V, xt, R, red.v, big, w, lane);
     else
-        lr_run<T, NT, 1>(S, base, V, xt, red.v, big, w, lane);
+        lr_run<T, NT, NARROW, 1>(S, base, V, xt, R, red.v, big, w, lane);
 }
 
 // ---------------------------------------------------------------- phase 2: row-leaf tasks
@@ -400,7 +419,7 @@ __global__ __launch_bounds__(64 * kLrWaves) void k_lr_mfma(const VStack *__restr
 // of the groups (wave_share) and the partial tiles are summed in a fixed order in LDS. A leaf with
 // a single task writes y = -x/2 + acc itself; the tasks of a split leaf write partial tiles that
 // k_rows_sum adds in task order. Output goes through LDS so that y rows are written contiguously.
-template <class T, int NT, int NRT>
+template <class T, int NT, bool NARROW, int NRT>
 __device__ __forceinline__ void rows_run(const RowTask &T_, int rs, int m, const LeafPanel &L,
                                          const int *__restrict__ psrc,
                                          const typename Mfma<T>::T2 *__restrict__ panel,
@@ -413,6 +432,8 @@ __device__ __forceinline__ void rows_run(const RowTask &T_, int rs, int m, const
     Acc<T, NT, NRT> acc;
     zero_acc<T, NT, NRT>(acc);
     const T2 *A0 = panel + L.off + (int64_t)kk * m;
+    const int RW = NARROW ? R : RP;
+    const int bcol = lane_col<NARROW>(i16, R);
     const int4 *src4 = reinterpret_cast<const int4 *>(psrc + L.col0) + T_.g0;
     const int3 sh = wave_share<kRowWaves>(T_.g1 - T_.g0, w);
     ring_run<T, NT, NRT, false, row_depth<T>(), int4>(
@@ -420,11 +441,11 @@ __device__ __forceinline__ void rows_run(const RowTask &T_, int rs, int m, const
         [&](int q, const int4 &sr, Grp<T, NT, NRT> &g) {
             const int row = pick4(sr, kk);
             grp_load<T, NT, NRT>(g, T(1), A0 + (int64_t)(T_.g0 + q) * 4 * m, m - 1, i16,
-                                 reinterpret_cast<const T *>(xt) + (int64_t)row * 2 * RP + i16);
+                                 reinterpret_cast<const T *>(xt) + (int64_t)row * 2 * RW + bcol);
         });
     reduce_waves<kRowWaves, T, NT, NRT>(acc, red, w, lane);
     __syncthreads();  // every wave has read the reduction buffer before it is reused for staging
-    if (w == 0) store_tile<T, NT, NRT>(acc, red, m, lane);
+    if (w == 0) store_tile<T, NT, NRT>(acc, red, m, 2 * RP, lane);
     __syncthreads();
     if (T_.slot >= 0) {
         T *dst = part + (int64_t)T_.slot * prow * (2 * RP);
@@ -438,7 +459,7 @@ __device__ __forceinline__ void rows_run(const RowTask &T_, int rs, int m, const
     }
 }
 
-template <class T, int NT, int MAXRT>
+template <class T, int NT, int MAXRT, bool NARROW = false>
 __global__ __launch_bounds__(64 * kRowWaves) void k_rows_mfma(
     const RowTask *__restrict__ tasks, const int *__restrict__ leaf_start, const LeafPanel *__restrict__ lpanel,
     const int *__restrict__ psrc, const typename Mfma<T>::T2 *__restrict__ panel,
@@ -454,21 +475,21 @@ __global__ __launch_bounds__(64 * kRowWaves) void k_rows_mfma(
     const LeafPanel L = lpanel[T_.leaf];
     const int nrt = (m + 15) >> 4;
     if (nrt <= 1)
-        rows_run<T, NT, 1>(T_, rs, m, L, psrc, panel, xt, x, N, R, y, cols, j0, part, prow, red.v, w, lane);
+        rows_run<T, NT, NARROW, 1>(T_, rs, m, L, psrc, panel, xt, x, N, R, y, cols, j0, part, prow, red.v, w, lane);
     else if (nrt == 2 || MAXRT == 2)
-        rows_run<T, NT, 2>(T_, rs, m, L, psrc, panel, xt, x, N, R, y, cols, j0, part, prow, red.v, w, lane);
+        rows_run<T, NT, NARROW, 2>(T_, rs, m, L, psrc, panel, xt, x, N, R, y, cols, j0, part, prow, red.v, w, lane);
     else if constexpr (MAXRT == 4) {
         if (nrt == 3)
-            rows_run<T, NT, 3>(T_, rs, m, L, psrc, panel, xt, x, N, R, y, cols, j0, part, prow, red.v, w, lane);
+            rows_run<T, NT, NARROW, 3>(T_, rs, m, L, psrc, panel, xt, x, N, R, y, cols, j0, part, prow, red.v, w, lane);
         else
-            rows_run<T, NT, 4>(T_, rs, m, L, psrc, panel, xt, x, N, R, y, cols, j0, part, prow, red.v, w, lane);
+            rows_run<T, NT, NARROW, 4>(T_, rs, m, L, psrc, panel, xt, x, N, R, y, cols, j0, part, prow, red.v, w, lane);
     } else if constexpr (MAXRT == 8) {
         if (nrt <= 4)
-            rows_run<T, NT, 4>(T_, rs, m, L, psrc, panel, xt, x, N, R, y, cols, j0, part, prow, red.v, w, lane);
+            rows_run<T, NT, NARROW, 4>(T_, rs, m, L, psrc, panel, xt, x, N, R, y, cols, j0, part, prow, red.v, w, lane);
         else if (nrt <= 6)
-            rows_run<T, NT, 6>(T_, rs, m, L, psrc, panel, xt, x, N, R, y, cols, j0, part, prow, red.v, w, lane);
+            rows_run<T, NT, NARROW, 6>(T_, rs, m, L, psrc, panel, xt, x, N, R, y, cols, j0, part, prow, red.v, w, lane);
         else
-            rows_run<T, NT, 8>(T_, rs, m, L, psrc, panel, xt, x, N, R, y, cols, j0, part, prow, red.v, w, lane);
+            rows_run<T, NT, NARROW, 8>(T_, rs, m, L, psrc, panel, xt, x, N, R, y, cols, j0, part, prow, red.v, w, lane);
     }
 }
 
@@ -769,7 +790,9 @@ static void build_lists(arh_hmat *h, int tr) {
     std::sort(small.begin(), small.end(), by_cols);
     M.p1big = (int)big.size();
     M.p1units = big;
-    M.p1units.insert(M.p1units.end(), small.begin(), small.end());
+    for (size_t q = 0; q < small.size();)
+        for (int w = 0; w < kLrWaves; w++)
+            M.p1units.push_back(w < kLrSmall && q < small.size() ? small[q++] : int2{-1, 0});
     // fused panels: column counts here, the column lists on the device (k_panel_cols)
     M.lpanel.assign(g->nleaf, LeafPanel{0, 0, 0});
     int64_t poff = 0, ncols = 0;
@@ -921,13 +944,14 @@ static void launch_nt(arh_hmat *h, MfmaLayout &M, int R, const double2 *x, doubl
     Profiler &pf = g->ctx->prof;
     const int N = g->N;
     constexpr int RP = 8 * NT;
-    M.xt[pi].alloc(sizeof(T2) * (size_t)(N + h->t_total) * RP);
+    const int RW = row_width(R);
+    M.xt[pi].alloc(sizeof(T2) * (size_t)(N + h->t_total) * RW);
     const int prow = part_rows(maxrt);
     if (M.nslots) M.part[pi].alloc(sizeof(T) * (size_t)M.nslots * prow * 2 * RP);
     T2 *xt = M.xt[pi].as<T2>();
     if (!packed)
-        hipLaunchKernelGGL(k_pack_xf<T>, dim3((unsigned)std::min<int64_t>(2048, ((int64_t)N * RP + 255) / 256)),
-                           dim3(256), 0, s, x, N, R, RP, xt, cols, j0, gate);
+        hipLaunchKernelGGL(k_pack_xf<T>, dim3((unsigned)std::min<int64_t>(2048, ((int64_t)N * RW + 255) / 256)),
+                           dim3(256), 0, s, x, N, R, RW, xt, cols, j0, gate);
     auto timed = [&](int kind, double bytes, double flops, auto &&launch) {
         if (!pf.on) {
             launch();
@@ -945,13 +969,19 @@ static void launch_nt(arh_hmat *h, MfmaLayout &M, int R, const double2 *x, doubl
     // leaves and re-reads are not algorithmic.
     const double eb = 2.0 * sizeof(T);
     const int nu = (int)M.p1units.size(), nb = M.p1big;
+    const bool narrow = R <= kNarrow;
     // phase-1 entries: V (forward) or U (transposed); both total sum_b r_b (m_b or n_b)
     const int64_t e1 = M.vs_total;
     if (nu)
         timed(pi ? PROF_LR64 : PROF_LR32, eb * e1 + eb * R * (N + h->t_total), 8.0 * R * e1, [&] {
-            hipLaunchKernelGGL((k_lr_mfma<T, NT>), dim3(nb + (nu - nb + kLrWaves - 1) / kLrWaves),
-                               dim3(64 * kLrWaves), 0, s, M.d_stacks.as<VStack>(), M.d_p1units.as<int2>(), nb, nu,
-                               M.vs[pi].as<T2>(), xt, gate);
+            auto launch_lr = [&](auto kern) {
+                hipLaunchKernelGGL(kern, dim3(nb + (nu - nb + kLrWaves - 1) / kLrWaves), dim3(64 * kLrWaves), 0, s,
+                                   M.d_stacks.as<VStack>(), M.d_p1units.as<int2>(), nb, nu, M.vs[pi].as<T2>(), xt, R,
+                                   gate);
+            };
+            if constexpr (NT == 1)
+                if (narrow) return launch_lr(k_lr_mfma<T, 1, true>);
+            launch_lr(k_lr_mfma<T, NT>);
         });
     const int64_t ent = g->dense_entries + (h->u_total + h->v_total - e1);
     T *part = M.nslots ? M.part[pi].as<T>() : nullptr;
@@ -964,6 +994,11 @@ static void launch_nt(arh_hmat *h, MfmaLayout &M, int R, const double2 *x, doubl
                                g->d_leaf_start.as<int>(), M.d_lpanel.as<LeafPanel>(), M.d_psrc.as<int>(),
                                M.panel[pi].as<T2>(), (const T2 *)xt, xd, N, R, yd, cols, j0, gate, part, prow);
         };
+        if constexpr (NT == 1)
+            if (narrow)
+                return launch_rows(maxrt <= 2   ? k_rows_mfma<T, 1, 2, true>
+                                   : maxrt <= 4 ? k_rows_mfma<T, 1, 4, true>
+                                                : k_rows_mfma<T, 1, 8, true>);
         if (maxrt <= 2) {
             launch_rows(k_rows_mfma<T, NT, 2>);
         } else if (maxrt <= 4) {
@@ -1017,23 +1052,23 @@ static void apply_t(arh_hmat *h, MfmaLayout &M, int R, const double2 *x, double2
     }
 }
 
-// Where the packed rows of a product with nc right-hand sides go (N rows of *rp complex values of the operator's
-// precision, columns nc .. *rp - 1 zero), for a caller that fills them itself; nullptr if the product takes more
+// Where the packed rows of a product with nc right-hand sides go (N rows of *rw complex values of the operator's
+// precision, columns nc .. *rw - 1 zero), for a caller that fills them itself; nullptr if the product takes more
 // than one pass, each of which packs its own rows.
 template <class T>
-static void *packed_rows_t(arh_hmat *h, MfmaLayout &M, int nc, int *rp) {
+static void *packed_rows_t(arh_hmat *h, MfmaLayout &M, int nc, int *rw) {
     typedef typename Mfma<T>::T2 T2;
     if (nc < 1 || nc > pass_width<T>(h->g)) return nullptr;
-    *rp = 8 * ((nc + 7) / 8);
+    *rw = row_width(nc);
     DBuf &xt = M.xt[sizeof(T) == 8 ? 1 : 0];
-    xt.alloc(sizeof(T2) * (size_t)(h->g->N + h->t_total) * *rp);
+    xt.alloc(sizeof(T2) * (size_t)(h->g->N + h->t_total) * *rw);
     return xt.p;
 }
 
-void *mfma_packed_rows(arh_hmat *h, int transpose, int fp64, int nc, int *rp) {
+void *mfma_packed_rows(arh_hmat *h, int transpose, int fp64, int nc, int *rw) {
     const int tr = transpose ? 1 : 0;
     mfma_prepare(h, tr, fp64 ? 1 : 0);
-    return fp64 ? packed_rows_t<double>(h, h->mf[tr], nc, rp) : packed_rows_t<float>(h, h->mf[tr], nc, rp);
+    return fp64 ? packed_rows_t<double>(h, h->mf[tr], nc, rw) : packed_rows_t<float>(h, h->mf[tr], nc, rw);
 }
 
 void hmat_apply_mfma(arh_hmat *h, int transpose, int fp64, int R, const double2 *x, double2 *y, hipStream_t s,

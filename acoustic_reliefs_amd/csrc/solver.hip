@@ -226,8 +226,8 @@ __global__ __launch_bounds__(ARH_WAVE) void k_finish(const RhsState *__restrict_
     finish_all(S, out, R, NB, part_r0v, part_ts, part_rr, hist, hist_cap, gate, blockIdx.x, gridDim.x);
 }
 
-// The vector updates before a product also write the product's packed rows (row i: RP complex values, listed column c
-// at c, zero up to RP), through LDS: a workgroup takes up_rows of the rows and kUpCols of the columns, a wavefront each
+// The vector updates before a product also write the product's packed rows (row i: rw complex values, listed column c
+// at c, zero from nc on), through LDS: a workgroup takes up_rows of the rows and kUpCols of the columns, a wavefront each
 // (every wavefront forms its rhs's scalars, some 400 operations; N = 9,828, p update: 37 right-hand sides FP32 10.4,
 // 7.4, 8.2 us at 64, 128, 192 rows, one FP64 6.0, 6.8, 8.0 us. The end of the previous iteration and the packing
 // were launches of their own: 16.4 us for 37, 15 us for one). T2: complex type of the operator's precision; xf == nullptr leaves the
@@ -240,17 +240,17 @@ constexpr int up_rows() {
 __device__ __forceinline__ float2 to_packed(double2 v, float2) { return make_float2((float)v.x, (float)v.y); }
 __device__ __forceinline__ double2 to_packed(double2 v, double2) { return v; }
 template <class T2>
-__device__ __forceinline__ void write_packed(const T2 (*tile)[kUpCols + 1], int bx, int N, int nc, int RP,
+__device__ __forceinline__ void write_packed(const T2 (*tile)[kUpCols + 1], int bx, int N, int nc, int rw,
                                              T2 *__restrict__ xf) {
     __syncthreads();
     const int r0 = bx * up_rows<T2>(), rows = min(up_rows<T2>(), N - r0);
     const int c0 = (int)blockIdx.y * kUpCols;
     const int c = threadIdx.x % kUpCols;
-    if (c0 + c >= RP) return;
+    if (c0 + c >= rw) return;
     for (int r = threadIdx.x / kUpCols; r < rows; r += blockDim.x / kUpCols) {
         T2 v{};
         if (c0 + c < nc) v = tile[r][c];
-        xf[(int64_t)(r0 + r) * RP + c0 + c] = v;
+        xf[(int64_t)(r0 + r) * rw + c0 + c] = v;
     }
 }
 
@@ -265,7 +265,7 @@ __global__ __launch_bounds__(ARH_WAVE * kUpCols) void k_p_update(const RhsState 
                                                    const double *__restrict__ part_rr, const double2 *__restrict__ r,
                                                    double2 *__restrict__ p, const double2 *__restrict__ v,
                                                    double *__restrict__ hist, int hist_cap, int *__restrict__ gate,
-                                                   T2 *__restrict__ xf, int RP) {
+                                                   T2 *__restrict__ xf, int rw) {
     constexpr int Q = up_rows<T2>() / ARH_WAVE;  // rows per lane
     __shared__ T2 tile[up_rows<T2>()][kUpCols + 1];
     const int lane = threadIdx.x % ARH_WAVE, w = threadIdx.x / ARH_WAVE, nw = blockDim.x / ARH_WAVE;
@@ -302,7 +302,7 @@ __global__ __launch_bounds__(ARH_WAVE * kUpCols) void k_p_update(const RhsState 
 #pragma unroll
             for (int t = 0; t < Q; t++) tile[t * ARH_WAVE + lane][c] = to_packed(q[t], T2{});
     }
-    if (xf) write_packed<T2>(tile, bx, N, nc, RP, xf);
+    if (xf) write_packed<T2>(tile, bx, N, nc, rw, xf);
 }
 
 // s = r - alpha v, alpha = rho_new / (r0^H v) from the partials, for the listed right-hand sides
@@ -311,7 +311,7 @@ __global__ __launch_bounds__(ARH_WAVE * kUpCols) void k_s_update(const RhsState 
                                                    const int *__restrict__ cols, int nc,
                                                    const double *__restrict__ part_r0v, const double2 *__restrict__ r,
                                                    const double2 *__restrict__ v, double2 *__restrict__ s,
-                                                   T2 *__restrict__ xf, int RP) {
+                                                   T2 *__restrict__ xf, int rw) {
     constexpr int Q = up_rows<T2>() / ARH_WAVE;  // rows per lane
     __shared__ T2 tile[up_rows<T2>()][kUpCols + 1];
     const int lane = threadIdx.x % ARH_WAVE, w = threadIdx.x / ARH_WAVE, nw = blockDim.x / ARH_WAVE;
@@ -344,7 +344,7 @@ __global__ __launch_bounds__(ARH_WAVE * kUpCols) void k_s_update(const RhsState 
 #pragma unroll
             for (int t = 0; t < Q; t++) tile[t * ARH_WAVE + lane][c] = to_packed(q[t], T2{});
     }
-    if (xf) write_packed<T2>(tile, (int)blockIdx.x, N, nc, RP, xf);
+    if (xf) write_packed<T2>(tile, (int)blockIdx.x, N, nc, rw, xf);
 }
 
 // x += alpha p + w s; r = s - w t; partials of r0^H r and |r|^2
@@ -611,11 +611,11 @@ static void bicgstab(arh_hmat *h, int transpose, int prec, int R, const double2 
         ARH_HIP(hipMemcpyAsync(W.ctl, ctl.data(), sizeof(int) * ctl.size(), hipMemcpyHostToDevice, s));
         const int *cols = W.ctl + 1;
         // the updates write the product's packed rows where one pass takes every active rhs
-        int rp = 0;
-        void *xf = fused ? mfma_packed_rows(h, transpose, fp64 ? 1 : 0, nc, &rp) : nullptr;
+        int rw = 0;
+        void *xf = fused ? mfma_packed_rows(h, transpose, fp64 ? 1 : 0, nc, &rw) : nullptr;
         // a wavefront per listed rhs, and enough of them for the workgroups that write all states
         const dim3 bu(ARH_WAVE * std::min(kUpCols, std::max(nc, (R + 3) / 4)));
-        const unsigned guy = (unsigned)((std::max(nc, rp) + kUpCols - 1) / kUpCols);
+        const unsigned guy = (unsigned)((std::max(nc, rw) + kUpCols - 1) / kUpCols);
         const int ur = xf && !fp64 ? up_rows<float2>() : up_rows<double2>();
         const unsigned gu = (unsigned)((N + ur - 1) / ur);
         auto apply = [&](const double2 *in, double2 *out, const int *gate) {
@@ -630,19 +630,19 @@ static void bicgstab(arh_hmat *h, int transpose, int prec, int R, const double2 
             int *gate = fin ? W.ghist + k - 1 : W.ctl;  // active right-hand sides
             if (xf && !fp64)
                 hipLaunchKernelGGL(k_p_update<float2>, dim3(gu + fin, guy), bu, 0, s, S, So, R, fin, N, NB, cols, nc, P1, P2,
-                                   P3, W.r, W.p, W.v, hist_dev, cap, gate, (float2 *)xf, rp);
+                                   P3, W.r, W.p, W.v, hist_dev, cap, gate, (float2 *)xf, rw);
             else
                 hipLaunchKernelGGL(k_p_update<double2>, dim3(gu + fin, guy), bu, 0, s, S, So, R, fin, N, NB, cols, nc, P1,
-                                   P2, P3, W.r, W.p, W.v, hist_dev, cap, gate, (double2 *)xf, rp);
+                                   P2, P3, W.r, W.p, W.v, hist_dev, cap, gate, (double2 *)xf, rw);
             if (fin) std::swap(S, So);
             apply(W.p, W.v, gate);
             hipLaunchKernelGGL(k_dot, gv, bv, 0, s, S, N, NB, W.r0, W.v, (const double2 *)nullptr, P1);
             if (xf && !fp64)
                 hipLaunchKernelGGL(k_s_update<float2>, dim3(gu, guy), bu, 0, s, S, N, NB, cols, nc, P1, W.r, W.v, W.s,
-                                   (float2 *)xf, rp);
+                                   (float2 *)xf, rw);
             else
                 hipLaunchKernelGGL(k_s_update<double2>, dim3(gu, guy), bu, 0, s, S, N, NB, cols, nc, P1, W.r, W.v, W.s,
-                                   (double2 *)xf, rp);
+                                   (double2 *)xf, rw);
             apply(W.s, W.t, gate);
             hipLaunchKernelGGL(k_dot, gv, bv, 0, s, S, N, NB, W.t, W.s, W.t, P2);
             hipLaunchKernelGGL(k_xr_update, gv, bv, 0, s, S, N, NB, P1, P2, W.p, W.s, W.t, W.r0, x, W.r, P3);
