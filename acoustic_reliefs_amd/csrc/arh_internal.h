@@ -47,6 +47,33 @@ void dev_free(void *p, size_t n, hipStream_t s, int device);
 size_t dev_trim(int device);    // frees every cached block of the device; returns the bytes
 size_t dev_cached(int device);  // bytes held in the cache
 
+// Pinned host blocks, cached per device (pool.cpp); dev_trim frees the cached ones too.
+void *host_alloc(size_t &n, int dev);
+void host_free(void *p, size_t n, int dev);
+
+// Owning pinned host block for work on stream s: kernels read and write it directly, the host after a
+// synchronisation. It goes back when nothing on the stream can use it any more.
+struct HostBuf {
+    void *p = nullptr;
+    size_t bytes = 0;
+    hipStream_t s = nullptr;
+    int dev = 0;
+    HostBuf(size_t n, hipStream_t stream) : bytes(n), s(stream) {
+        ARH_HIP(hipGetDevice(&dev));
+        p = host_alloc(bytes, dev);
+    }
+    template <class T>
+    T *as() const {
+        return reinterpret_cast<T *>(p);
+    }
+    HostBuf(const HostBuf &) = delete;
+    HostBuf &operator=(const HostBuf &) = delete;
+    ~HostBuf() {
+        (void)hipStreamSynchronize(s);
+        host_free(p, bytes, dev);
+    }
+};
+
 // Owning device buffer, from the device memory cache; it belongs to the stream it was allocated
 // for (the calling context's).
 struct DBuf {
@@ -167,9 +194,6 @@ struct arh_ctx_s {
     // reduction / scalar scratch reused by the solver
     arh::DBuf red;      // partial sums
     arh::DBuf scal;     // per-rhs scalars
-    arh::DBuf hostpin;  // pinned host staging
-    size_t hostpin_bytes = 0;
-    void *pinned(size_t bytes);
 };
 
 // FP64 product work unit: up to 64 consecutive columns of one row leaf's column list, taken from

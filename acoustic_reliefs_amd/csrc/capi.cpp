@@ -45,17 +45,6 @@ static void set_device(arh_ctx *ctx) {
     tl_stream = ctx->stream;
 }
 
-void *arh_ctx_s::pinned(size_t bytes) {
-    if (bytes > hostpin_bytes) {
-        if (hostpin.p) (void)hipHostFree(hostpin.p), hostpin.p = nullptr;
-        void *p = nullptr;
-        ARH_HIP(hipHostMalloc(&p, bytes, hipHostMallocDefault));
-        hostpin.p = p;
-        hostpin_bytes = bytes;
-    }
-    return hostpin.p;
-}
-
 extern "C" {
 
 int arh_ctx_create(int device, arh_ctx **out) {
@@ -81,7 +70,6 @@ static void ctx_release(arh_ctx *ctx) {
     if (--ctx->refs > 0) return;
     (void)hipSetDevice(ctx->device);
     (void)hipStreamSynchronize(ctx->stream);
-    if (ctx->hostpin.p) (void)hipHostFree(ctx->hostpin.p), ctx->hostpin.p = nullptr;
     ctx->red.reset();
     ctx->scal.reset();
     if (tl_stream == ctx->stream || tl_stream == ctx->own) tl_stream = nullptr;

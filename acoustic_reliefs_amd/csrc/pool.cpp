@@ -5,6 +5,9 @@
 // Stream safety: a block remembers the stream of its last owner and an event recorded there when it
 // was freed; a new owner on another stream waits on that event (hipStreamWaitEvent) before its first
 // use, an owner on the same stream needs nothing (the stream runs in order).
+//
+// Pinned host blocks (HostBuf) are kept the same way, up to kHostCached bytes per device: pinning takes
+// some hundred microseconds, a solve's control blocks a few kilobytes.
 #include <cstdlib>
 #include <map>
 #include <mutex>
@@ -28,8 +31,11 @@ struct DevPool {
     std::mutex mu;
     std::multimap<size_t, Block> free;
     size_t cached = 0;
+    std::multimap<size_t, void *> host;  // pinned host blocks, no stream uses them
+    size_t host_cached = 0;
 };
 
+constexpr size_t kHostCached = size_t(32) << 20;
 constexpr int kMaxDevices = 64;
 constexpr size_t kSmall = size_t(1) << 20;  // below: power-of-two classes; above: 2 MiB granules
 constexpr size_t kGranule = size_t(2) << 20;
@@ -145,15 +151,55 @@ void dev_free(void *p, size_t n, hipStream_t s, int dev) {
     P.cached += n;
 }
 
+void *host_alloc(size_t &n, int dev) {
+    n = round_size(n);
+    if (enabled() && dev >= 0 && dev < kMaxDevices) {
+        DevPool &P = pool(dev);
+        std::lock_guard<std::mutex> lk(P.mu);
+        auto it = P.host.lower_bound(n);
+        if (it != P.host.end() && it->first <= 2 * n) {
+            void *p = it->second;
+            n = it->first;
+            P.host_cached -= n;
+            P.host.erase(it);
+            return p;
+        }
+    }
+    void *p = nullptr;
+    hipError_t e = hipHostMalloc(&p, n, hipHostMallocDefault);
+    if (e != hipSuccess) {
+        (void)hipGetLastError();
+        throw Error(ARH_ENOMEM, "hipHostMalloc(" + std::to_string(n) + " B): " + hipGetErrorString(e));
+    }
+    return p;
+}
+
+void host_free(void *p, size_t n, int dev) {
+    if (enabled() && dev >= 0 && dev < kMaxDevices) {
+        DevPool &P = pool(dev);
+        std::lock_guard<std::mutex> lk(P.mu);
+        if (P.host_cached + n <= kHostCached) {
+            P.host.emplace(n, p);
+            P.host_cached += n;
+            return;
+        }
+    }
+    (void)hipHostFree(p);
+}
+
 size_t dev_trim(int dev) {
     if (dev < 0 || dev >= kMaxDevices) return 0;
     DevPool &P = pool(dev);
     std::multimap<size_t, Block> blocks;
+    std::multimap<size_t, void *> host;
     {
         std::lock_guard<std::mutex> lk(P.mu);
         blocks.swap(P.free);
+        host.swap(P.host);
         P.cached = 0;
+        P.host_cached = 0;
     }
+    for (auto &kv : host) (void)hipHostFree(kv.second);
     size_t freed = 0;
     for (auto &kv : blocks) {
         freed += kv.second.bytes;

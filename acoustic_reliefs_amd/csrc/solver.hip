@@ -55,14 +55,15 @@ struct RhsState {
     double2 rho;      // rho of the previous iteration (Eigen's rho_old at the next step)
     double2 rho_new;  // r0^H r for the coming iteration
     double2 alpha, w;
-    double r0sq, rhs_sq, rn, tol2;  // tol2 = tol^2 ||b||^2
+    double r0sq, rhs_sq, rn, tol2;  // tol2 = tol^2 ||b||^2 (tol until the start)
     int active;    // iterating
     int restart;   // restart pending (set at init, or by finish_rhs on breakdown: then paused)
     int it;        // iterations counted toward maxit (reset at the first restart)
     int iters;     // iterations done
     int nrestart;  // restarts done
     int maxit;
-    int pad[2];
+    int pad;
+    double rn0;  // |b|^2 at the start, when x = 0
 };
 
 constexpr int kVT = 256;      // threads per block of vector kernels
@@ -202,7 +203,7 @@ __device__ __forceinline__ void finish_rhs(RhsState &st, int j, int NB, const do
 __device__ __forceinline__ void finish_all(const RhsState *__restrict__ S, RhsState *__restrict__ out, int R, int NB,
                                            const double *__restrict__ part_r0v, const double *__restrict__ part_ts,
                                            const double *__restrict__ part_rr, double *__restrict__ hist, int hist_cap,
-                                           int *__restrict__ gate, int q, int nq) {
+                                           int *__restrict__ gate, int q, int nq, RhsState *__restrict__ host) {
     const int lane = threadIdx.x % ARH_WAVE;
     for (int j = q; j < R; j += nq) {
         RhsState st = S[j];
@@ -213,17 +214,22 @@ __device__ __forceinline__ void finish_all(const RhsState *__restrict__ S, RhsSt
                 if (st.active) atomicAdd(gate, 1);
             }
         }
-        if (lane == 0) out[j] = st;
+        if (lane == 0) {
+            out[j] = st;
+            if (host) host[j] = st;
+        }
     }
 }
 
-// The end of a batch's last iteration (one wavefront per workgroup).
+// The end of a batch's last iteration (one wavefront per workgroup); host: the host's copy of the states, in pinned
+// memory.
 __global__ __launch_bounds__(ARH_WAVE) void k_finish(const RhsState *__restrict__ S, RhsState *__restrict__ out, int R,
                                                      int NB, const double *__restrict__ part_r0v,
                                                      const double *__restrict__ part_ts,
                                                      const double *__restrict__ part_rr, double *__restrict__ hist,
-                                                     int hist_cap, int *__restrict__ gate) {
-    finish_all(S, out, R, NB, part_r0v, part_ts, part_rr, hist, hist_cap, gate, blockIdx.x, gridDim.x);
+                                                     int hist_cap, int *__restrict__ gate,
+                                                     RhsState *__restrict__ host) {
+    finish_all(S, out, R, NB, part_r0v, part_ts, part_rr, hist, hist_cap, gate, blockIdx.x, gridDim.x, host);
 }
 
 // The vector updates before a product also write the product's packed rows (row i: rw complex values, listed column c
@@ -271,7 +277,7 @@ __global__ __launch_bounds__(ARH_WAVE * kUpCols) void k_p_update(const RhsState 
     const int lane = threadIdx.x % ARH_WAVE, w = threadIdx.x / ARH_WAVE, nw = blockDim.x / ARH_WAVE;
     if (finish && blockIdx.x == 0) {
         finish_all(S, out, R, NB, part_r0v, part_ts, part_rr, hist, hist_cap, gate, (int)blockIdx.y * nw + w,
-                   (int)gridDim.y * nw);
+                   (int)gridDim.y * nw, nullptr);
         return;
     }
     const int bx = (int)blockIdx.x - (finish ? 1 : 0);
@@ -395,11 +401,24 @@ __global__ __launch_bounds__(kVT) void k_xr_update(const RhsState *__restrict__ 
         for (int k = 0; k < 4; k++) part_rr[((int64_t)j * NB + blockIdx.x) * 4 + k] = v[k];
 }
 
-// (re)start of rhs j: r = b - Ax (Ax given, or zero), r0 = r, partials of |r|^2 (and b^2 on init)
+// Host lists to the device: two arrays of ints from pinned memory, which the host rewrites only after a
+// synchronisation. (A small hipMemcpyAsync each way cost 25 to 45 us of an idle GPU at every synchronisation.)
+__global__ __launch_bounds__(256) void k_load(int *__restrict__ d0, const int *__restrict__ s0, int n0,
+                                              int *__restrict__ d1, const int *__restrict__ s1, int n1) {
+    const int e = blockIdx.x * 256 + threadIdx.x;
+    if (e < n0)
+        d0[e] = s0[e];
+    else if (e - n0 < n1)
+        d1[e - n0] = s1[e - n0];
+}
+
+// (re)start of rhs j: r = b - Ax, r0 = r, partials of |r|^2 and b^2. A fresh start (Ax null) is from x = 0: it zeroes
+// x, p and v too (launches of their own otherwise).
 __global__ __launch_bounds__(kVT) void k_restart(const RhsState *__restrict__ S, int N, int NB,
                                                  const double2 *__restrict__ b, const double2 *__restrict__ Ax,
                                                  double2 *__restrict__ r, double2 *__restrict__ r0,
-                                                 double *__restrict__ part) {
+                                                 double2 *__restrict__ x, double2 *__restrict__ p,
+                                                 double2 *__restrict__ v_, double *__restrict__ part) {
     __shared__ double sh[4 * kVT / ARH_WAVE];
     const int j = blockIdx.y;
     if (!S[j].restart) return;
@@ -411,6 +430,7 @@ __global__ __launch_bounds__(kVT) void k_restart(const RhsState *__restrict__ S,
         double2 ri = Ax ? csub(bi, Ax[o + i]) : bi;
         r[o + i] = ri;
         r0[o + i] = ri;
+        if (!Ax) x[o + i] = p[o + i] = v_[o + i] = make_double2(0.0, 0.0);
         v[0] += ri.x * ri.x + ri.y * ri.y;
         v[1] += bi.x * bi.x + bi.y * bi.y;
     }
@@ -419,12 +439,14 @@ __global__ __launch_bounds__(kVT) void k_restart(const RhsState *__restrict__ S,
         for (int k = 0; k < 4; k++) part[((int64_t)j * NB + blockIdx.x) * 4 + k] = v[k];
 }
 
-// full restart: rho = r0sq = |r|^2; fresh: also alpha = w = rho_old = 1, rhs_sq, and the caller
-// zeroes p, v (the host decides activity after a fresh start); a breakdown restart resumes the
-// iteration (active again) and resets the iteration count on the first restart (Eigen)
+// full restart: rho = r0sq = |r|^2; fresh: also alpha = w = rho_old = 1, rhs_sq, the stopping bound, and
+// whether the rhs iterates at all (a zero right-hand side does not, nor one that meets its tolerance already), counted in
+// count; a breakdown restart resumes the iteration (active again) and resets the iteration count on the
+// first restart (Eigen)
 // (a wavefront per rhs)
 __global__ __launch_bounds__(ARH_WAVE) void k_restart_finish(RhsState *__restrict__ S, int NB,
-                                                             const double *__restrict__ part, int fresh) {
+                                                             const double *__restrict__ part, int fresh,
+                                                             int *__restrict__ count) {
     const int j = blockIdx.x;
     if (!S[j].restart) return;
     RhsState st = S[j];
@@ -438,21 +460,16 @@ __global__ __launch_bounds__(ARH_WAVE) void k_restart_finish(RhsState *__restric
         st.rho = make_double2(1.0, 0.0);
         st.alpha = make_double2(1.0, 0.0);
         st.w = make_double2(1.0, 0.0);
+        st.rn0 = f[0];
+        st.tol2 = st.tol2 * st.tol2 * st.rhs_sq;
+        st.active = st.rhs_sq != 0.0 && st.rn > st.tol2 && st.maxit > 0 ? 1 : 0;
+        if (threadIdx.x == 0 && st.active) atomicAdd(count, 1);
     } else {
         if (st.nrestart++ == 0) st.it = 0;
         st.active = 1;
     }
     st.restart = 0;
     if (threadIdx.x == 0) S[j] = st;
-}
-
-// masked zeroing of columns (p, v on fresh starts; x on init)
-__global__ void k_zero_cols(const RhsState *__restrict__ S, int N, double2 *__restrict__ a, int use_restart_mask) {
-    const int j = blockIdx.y;
-    if (use_restart_mask && !S[j].restart) return;
-    const int64_t o = (int64_t)j * N;
-    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < N; i += gridDim.x * blockDim.x)
-        a[o + i] = make_double2(0.0, 0.0);
 }
 
 // x += f d (refinement; f = -1 reverts a correction), masked per column
@@ -499,13 +516,25 @@ struct Work {
     int *mask;
     int *ctl;  // [0]: active count at a batch's start, [1..R]: column list
     int *ghist;  // after the list: active count after each iteration of a batch (the gate of the next one)
-    void init(int64_t N, int R, int NB) {
+    // pinned host block: states as the device last wrote them, states and lists on their way to the device, the
+    // partials of the true residual
+    HostBuf host;
+    RhsState *hs, *hs_up;
+    int *h_ctl, *h_rs, *h_mask;
+    double *h_part;
+    static size_t host_bytes(int R, int NB) {
+        return 2 * sizeof(RhsState) * R + sizeof(double) * 4 * (size_t)R * NB + sizeof(int) * (3 * (size_t)R + 2 + kMaxK);
+    }
+    Work(int64_t N, int R, int NB, hipStream_t stream) : host(host_bytes(R, NB), stream) {
+        hs = host.as<RhsState>(), hs_up = hs + R;
+        h_part = (double *)(hs_up + R);
+        h_ctl = (int *)(h_part + 4 * (size_t)R * NB), h_rs = h_ctl + R + 1 + kMaxK, h_mask = h_rs + R + 1;
         const int64_t vec = N * R;
         const size_t vb = sizeof(double2) * vec;
         const size_t pb = sizeof(double) * 4 * (size_t)R * NB;
         // every piece starts on a 256-byte boundary: the total is the sum of the rounded sizes
         auto rnd = [](size_t n) { return (n + 255) / 256 * 256; };
-        const size_t total = 7 * rnd(vb) + rnd(4 * pb) + 2 * rnd(sizeof(RhsState) * R) + rnd(sizeof(int) * R) +
+        const size_t total = 7 * rnd(vb) + rnd(3 * pb) + 2 * rnd(sizeof(RhsState) * R) + rnd(sizeof(int) * R) +
                              rnd(sizeof(int) * (R + 1 + kMaxK));
         buf.alloc(total);
         char *c = buf.as<char>();
@@ -518,12 +547,28 @@ struct Work {
         };
         r = (double2 *)take(vb), r0 = (double2 *)take(vb), p = (double2 *)take(vb), v = (double2 *)take(vb);
         s = (double2 *)take(vb), t = (double2 *)take(vb), Ax = (double2 *)take(vb);
-        part = (double *)take(4 * pb);
+        part = (double *)take(3 * pb);
         S = (RhsState *)take(sizeof(RhsState) * R);
         S2 = (RhsState *)take(sizeof(RhsState) * R);
         mask = (int *)take(sizeof(int) * R);
         ctl = (int *)take(sizeof(int) * (R + 1 + kMaxK));
         ghist = ctl + R + 1;
+    }
+    // int arrays from the pinned block to the device
+    void load(void *d0, const void *s0, size_t b0, void *d1 = nullptr, const void *s1 = nullptr, size_t b1 = 0) const {
+        const int n0 = (int)(b0 / sizeof(int)), n1 = (int)(b1 / sizeof(int));
+        hipLaunchKernelGGL(k_load, dim3((n0 + n1 + 255) / 256), dim3(256), 0, host.s, (int *)d0, (const int *)s0, n0,
+                           (int *)d1, (const int *)s1, n1);
+        ARH_HIP(hipGetLastError());
+    }
+    // x += f d for the masked right-hand sides (a true residual, which synchronises, follows every call: the mask of
+    // the previous one has been read)
+    void axpy(const std::vector<int> &m, int N, double2 *x, const double2 *d, double f) {
+        std::copy(m.begin(), m.end(), h_mask);
+        load(mask, h_mask, sizeof(int) * m.size());
+        hipLaunchKernelGGL(k_axpy_cols, dim3(std::max(1, std::min(1024, (N + 255) / 256)), (unsigned)m.size()), dim3(256),
+                           0, host.s, mask, N, x, d, f);
+        ARH_HIP(hipGetLastError());
     }
 };
 
@@ -549,7 +594,6 @@ static void bicgstab(arh_hmat *h, int transpose, int prec, int R, const double2 
     hipStream_t s = ctx->stream;
     const int N = h->g->N;
     const dim3 gv(NB, R), bv(kVT);
-    const int zblk = std::max(1, std::min(1024, (N + 255) / 256));
     double *P1 = W.part, *P2 = W.part + 4 * (size_t)R * NB, *P3 = W.part + 8 * (size_t)R * NB;
     const bool hist_on = record_hist && st && st->hist && st->hist_len && o.hist_cap > 0;
     const int cap = hist_on ? o.hist_cap : 0;
@@ -558,57 +602,49 @@ static void bicgstab(arh_hmat *h, int transpose, int prec, int R, const double2 
         W.hbuf.alloc(sizeof(double) * (size_t)R * cap);
         hist_dev = W.hbuf.as<double>();
     }
-    std::vector<RhsState> hs(R);
+    RhsState *hs = W.hs;
+    int *ctl = W.h_ctl, *ctl_rs = W.h_rs;
+    int nlist = 0;
     for (int j = 0; j < R; j++) {
-        std::memset(&hs[j], 0, sizeof(RhsState));
-        hs[j].restart = want[j] ? 1 : 0;
+        RhsState st;
+        std::memset(&st, 0, sizeof(RhsState));
+        st.restart = want[j] ? 1 : 0;
+        st.tol2 = tolj[j];
+        st.maxit = maxit;
+        W.hs_up[j] = st;
+        if (want[j]) ctl[1 + nlist++] = j;
     }
-    ARH_HIP(hipMemcpyAsync(W.S, hs.data(), sizeof(RhsState) * R, hipMemcpyHostToDevice, s));
-    hipLaunchKernelGGL(k_zero_cols, dim3(zblk, R), dim3(256), 0, s, W.S, N, x, 1);
-    hipLaunchKernelGGL(k_zero_cols, dim3(zblk, R), dim3(256), 0, s, W.S, N, W.p, 1);
-    hipLaunchKernelGGL(k_zero_cols, dim3(zblk, R), dim3(256), 0, s, W.S, N, W.v, 1);
-    hipLaunchKernelGGL(k_restart, gv, bv, 0, s, W.S, N, NB, b, (const double2 *)nullptr, W.r, W.r0, P1);
-    hipLaunchKernelGGL(k_restart_finish, dim3(R), dim3(ARH_WAVE), 0, s, W.S, NB, P1, 1);
-    ARH_HIP(hipGetLastError());
-    ARH_HIP(hipMemcpyAsync(hs.data(), W.S, sizeof(RhsState) * R, hipMemcpyDeviceToHost, s));
-    ARH_HIP(hipStreamSynchronize(s));
     iters.assign(R, 0);
     err.assign(R, 0.0);
+    if (nlist == 0) return;
+    // the first batch follows the start at once: its list is every wanted rhs, and the device says which of them
+    // iterate (in ctl[0], the batch's gate)
+    ctl[0] = 0;
+    std::fill(ctl + R + 1, ctl + R + 1 + kMaxK, 0);
+    W.load(W.S, W.hs_up, sizeof(RhsState) * R, W.ctl, ctl, sizeof(int) * (R + 1 + kMaxK));
+    hipLaunchKernelGGL(k_restart, gv, bv, 0, s, W.S, N, NB, b, (const double2 *)nullptr, W.r, W.r0, x, W.p, W.v, P1);
+    hipLaunchKernelGGL(k_restart_finish, dim3(R), dim3(ARH_WAVE), 0, s, W.S, NB, P1, 1, W.ctl);
+    ARH_HIP(hipGetLastError());
     std::vector<double> hist0(R, 0.0);
-    int nact = 0;
-    for (int j = 0; j < R; j++) {
-        hs[j].active = 0;
-        if (!want[j]) continue;
-        if (hs[j].rhs_sq == 0.0) {  // Eigen: x = 0, done
-            err[j] = 0.0;
-            continue;
-        }
-        hs[j].tol2 = tolj[j] * tolj[j] * hs[j].rhs_sq;
-        hs[j].maxit = maxit;
-        hist0[j] = std::sqrt(hs[j].rn / hs[j].rhs_sq);
-        if (hs[j].rn > hs[j].tol2 && maxit > 0) hs[j].active = 1, nact++;
-        err[j] = std::sqrt(hs[j].rn / hs[j].rhs_sq);
-    }
-    ARH_HIP(hipMemcpyAsync(W.S, hs.data(), sizeof(RhsState) * R, hipMemcpyHostToDevice, s));
     // K from the observed convergence: iterations until the fastest active rhs is predicted to
     // reach its tolerance (so that few iterations run past convergence), 1..kMaxK
     std::vector<double> e_prev(R, 0.0);
     std::vector<int> i_prev(R, 0);
-    for (int j = 0; j < R; j++) e_prev[j] = err[j];
     int K = 2;
-    // separate host buffers for the two lists: a list is rewritten only after the stream has been
-    // synchronised since its last copy
-    std::vector<int> ctl(R + 1 + kMaxK, 0), ctl_rs(R + 1);
-    std::vector<double> best(err);
+    std::vector<double> best;
     std::vector<int> best_it(R, 0);
     RhsState *S = W.S, *So = W.S2;  // current states, and where the next iteration's go
     const bool fp64 = prec != ARH_MIXED, fused = h->g->max_leaf <= mfma_max_leaf();
-    while (nact > 0) {
-        int nc = 0;
-        for (int j = 0; j < R; j++)
-            if (hs[j].active) ctl[1 + nc++] = j;
-        ctl[0] = nc;
-        ARH_HIP(hipMemcpyAsync(W.ctl, ctl.data(), sizeof(int) * ctl.size(), hipMemcpyHostToDevice, s));
+    bool first = true;
+    for (int nact = nlist; nact > 0;) {
+        int nc = nlist;
+        if (!first) {
+            nc = 0;
+            for (int j = 0; j < R; j++)
+                if (hs[j].active) ctl[1 + nc++] = j;
+            ctl[0] = nc;
+            W.load(W.ctl, ctl, sizeof(int) * (R + 1 + kMaxK));
+        }
         const int *cols = W.ctl + 1;
         // the updates write the product's packed rows where one pass takes every active rhs
         int rw = 0;
@@ -648,21 +684,32 @@ static void bicgstab(arh_hmat *h, int transpose, int prec, int R, const double2 
             hipLaunchKernelGGL(k_xr_update, gv, bv, 0, s, S, N, NB, P1, P2, W.p, W.s, W.t, W.r0, x, W.r, P3);
         }
         hipLaunchKernelGGL(k_finish, dim3(R), dim3(ARH_WAVE), 0, s, S, So, R, NB, P1, P2, P3, hist_dev, cap,
-                           W.ghist + K - 1);
+                           W.ghist + K - 1, hs);
         std::swap(S, So);
         ARH_HIP(hipGetLastError());
         ctx->prof.cur_slot = -1;
         int gh[kMaxK];
-        ARH_HIP(hipMemcpyAsync(gh, W.ghist, sizeof(int) * K, hipMemcpyDeviceToHost, s));
-        ARH_HIP(hipMemcpyAsync(hs.data(), S, sizeof(RhsState) * R, hipMemcpyDeviceToHost, s));
+        if (ctx->prof.on) ARH_HIP(hipMemcpyAsync(gh, W.ghist, sizeof(int) * K, hipMemcpyDeviceToHost, s));
         ARH_HIP(hipStreamSynchronize(s));
+        bool none = false;  // the device found no rhs to iterate at the start
+        if (first) {
+            none = true;
+            for (int j = 0; j < R; j++) {
+                if (!want[j] || hs[j].rhs_sq == 0.0) continue;  // Eigen: x = 0, done
+                hist0[j] = err[j] = e_prev[j] = std::sqrt(hs[j].rn0 / hs[j].rhs_sq);
+                if (hs[j].iters > 0) none = false;
+            }
+            best = err;
+            first = false;
+        }
         if (ctx->prof.on) {
             // iteration k's products ran iff some rhs was active after iteration k - 1
-            ctx->prof.slot_ok.assign(K, 1);
+            ctx->prof.slot_ok.assign(K, none ? 0 : 1);
             for (int k = 1; k < K; k++) ctx->prof.slot_ok[k] = gh[k - 1] > 0;
             ctx->prof.flush(false);
             ctx->prof.slot_ok.clear();
         }
+        if (none) break;
         // stalled inner solves stop here (nothing has run on the device since the state was read)
         if (stall_window > 0 || budget > 0) {
             bool changed = false;
@@ -682,7 +729,10 @@ static void bicgstab(arh_hmat *h, int transpose, int prec, int R, const double2 
                     changed = true;
                 }
             }
-            if (changed) ARH_HIP(hipMemcpyAsync(S, hs.data(), sizeof(RhsState) * R, hipMemcpyHostToDevice, s));
+            if (changed) {  // from a copy: hs changes below before the device reads it
+                std::copy(hs, hs + R, W.hs_up);
+                W.load(S, W.hs_up, sizeof(RhsState) * R);
+            }
         }
         // breakdown restarts: r = b - A x, r0 = r for the paused right-hand sides
         int nrs = 0;
@@ -690,11 +740,11 @@ static void bicgstab(arh_hmat *h, int transpose, int prec, int R, const double2 
             if (hs[j].restart) ctl_rs[1 + nrs++] = j;
         if (nrs) {
             ctl_rs[0] = nrs;
-            ARH_HIP(hipMemcpyAsync(W.ctl, ctl_rs.data(), sizeof(int) * (nrs + 1), hipMemcpyHostToDevice, s));
+            W.load(W.ctl, ctl_rs, sizeof(int) * (nrs + 1));
             hmat_apply(h, transpose, prec, R, x, W.Ax, s, W.ctl + 1, nrs, W.ctl);
             if (st) st->matvecs++;
-            hipLaunchKernelGGL(k_restart, gv, bv, 0, s, S, N, NB, b, W.Ax, W.r, W.r0, P1);
-            hipLaunchKernelGGL(k_restart_finish, dim3(R), dim3(ARH_WAVE), 0, s, S, NB, P1, 0);
+            hipLaunchKernelGGL(k_restart, gv, bv, 0, s, S, N, NB, b, W.Ax, W.r, W.r0, x, W.p, W.v, P1);
+            hipLaunchKernelGGL(k_restart_finish, dim3(R), dim3(ARH_WAVE), 0, s, S, NB, P1, 0, (int *)nullptr);
             ARH_HIP(hipGetLastError());
             for (int j = 0; j < R; j++)
                 if (hs[j].restart) {
@@ -745,11 +795,10 @@ static void true_residual(arh_hmat *h, int transpose, int R, const double2 *b, c
     const int N = h->g->N;
     hmat_apply(h, transpose, ARH_FP64, R, x, W.Ax, s);
     if (st) st->matvecs++;
-    hipLaunchKernelGGL(k_resid, dim3(NB, R), dim3(kVT), 0, s, N, NB, b, W.Ax, r, W.part);
+    hipLaunchKernelGGL(k_resid, dim3(NB, R), dim3(kVT), 0, s, N, NB, b, W.Ax, r, W.h_part);
     ARH_HIP(hipGetLastError());
-    std::vector<double> part(4 * (size_t)R * NB);
-    ARH_HIP(hipMemcpyAsync(part.data(), W.part, sizeof(double) * part.size(), hipMemcpyDeviceToHost, s));
     ARH_HIP(hipStreamSynchronize(s));
+    const double *part = W.h_part;
     res.assign(R, 0.0);
     for (int j = 0; j < R; j++) {
         double rr = 0, bb = 0;
@@ -769,8 +818,7 @@ void solve(arh_hmat *h, int transpose, int R, const double2 *b, double2 *x, cons
     ARH_CHECK(R >= 1, ARH_EINVAL, "nrhs must be >= 1");
     ARH_CHECK(tol >= 0.0, ARH_EINVAL, "tol must be >= 0");
     const auto t0 = std::chrono::steady_clock::now();
-    Work W;
-    W.init(N, R, NB);
+    Work W(N, R, NB, s);
     if (st) {
         st->iters = st->matvecs = st->refinements = st->restarts = 0;
         st->max_err = st->max_true_res = 0.0;
@@ -807,10 +855,7 @@ void solve(arh_hmat *h, int transpose, int R, const double2 *b, double2 *x, cons
             bicgstab(h, transpose, ARH_FP64, R, rb.as<double2>(), dx.as<double2>(), redo, ctol, left, o, st, iters,
                      err, W, NB, false);
             left -= *std::max_element(iters.begin(), iters.end());
-            ARH_HIP(hipMemcpyAsync(W.mask, redo.data(), sizeof(int) * R, hipMemcpyHostToDevice, s));
-            hipLaunchKernelGGL(k_axpy_cols, dim3(std::max(1, std::min(1024, (N + 255) / 256)), R), dim3(256), 0, s,
-                               W.mask, N, x, dx.as<double2>(), 1.0);
-            ARH_HIP(hipGetLastError());
+            W.axpy(redo, N, x, dx.as<double2>(), 1.0);
             for (int j = 0; j < R; j++) iters_tot[j] += redo[j] ? iters[j] : 0;
             true_residual(h, transpose, R, b, x, nullptr, W, NB, tres, st);
             sweeps++;
@@ -826,11 +871,9 @@ void solve(arh_hmat *h, int transpose, int R, const double2 *b, double2 *x, cons
         DBuf rb, dx;
         rb.alloc(sizeof(double2) * (size_t)N * R);
         dx.alloc(sizeof(double2) * (size_t)N * R);
-        ARH_HIP(hipMemcpyAsync(rb.p, b, sizeof(double2) * (size_t)N * R, hipMemcpyDeviceToDevice, s));
         ARH_HIP(hipMemsetAsync(x, 0, sizeof(double2) * (size_t)N * R, s));
         std::vector<double> bnorm_rel(R, 1.0);  // ||r|| / ||b|| of the current residual
         std::vector<int> redo(R, 1), fp64(R, 0);
-        const dim3 ga(std::max(1, std::min(1024, (N + 255) / 256)), R);
         const int stall = std::max(200, std::min(maxit, 400));
         for (int sweep = 0; sweep < 10; sweep++) {
             // per-rhs inner tolerance relative to its current residual, aiming at half the target (not
@@ -841,12 +884,10 @@ void solve(arh_hmat *h, int transpose, int R, const double2 *b, double2 *x, cons
             std::vector<double> itol(R);
             for (int j = 0; j < R; j++)
                 itol[j] = std::min(0.5, std::max(kInnerFloor, kInnerFrac * tol / std::max(bnorm_rel[j], 1e-300)));
-            bicgstab(h, transpose, ARH_MIXED, R, rb.as<double2>(), dx.as<double2>(), redo, itol, maxit, o, st, iters,
+            bicgstab(h, transpose, ARH_MIXED, R, sweep == 0 ? b : rb.as<double2>(), dx.as<double2>(), redo, itol, maxit, o, st, iters,
                      err, W, NB, sweep == 0, stall, kInnerBudget);
             for (int j = 0; j < R; j++) iters_tot[j] += redo[j] ? iters[j] : 0;
-            ARH_HIP(hipMemcpyAsync(W.mask, redo.data(), sizeof(int) * R, hipMemcpyHostToDevice, s));
-            hipLaunchKernelGGL(k_axpy_cols, ga, dim3(256), 0, s, W.mask, N, x, dx.as<double2>(), 1.0);
-            ARH_HIP(hipGetLastError());
+            W.axpy(redo, N, x, dx.as<double2>(), 1.0);
             true_residual(h, transpose, R, b, x, rb.as<double2>(), W, NB, tres, st);
             if (st) st->refinements++;
             trace_sweep("fp32", sweep, redo, iters, tres);
@@ -865,9 +906,7 @@ void solve(arh_hmat *h, int transpose, int R, const double2 *b, double2 *x, cons
                 nre += redo[j];
             }
             if (nundo) {  // revert corrections that made the residual worse
-                ARH_HIP(hipMemcpyAsync(W.mask, undo.data(), sizeof(int) * R, hipMemcpyHostToDevice, s));
-                hipLaunchKernelGGL(k_axpy_cols, ga, dim3(256), 0, s, W.mask, N, x, dx.as<double2>(), -1.0);
-                ARH_HIP(hipGetLastError());
+                W.axpy(undo, N, x, dx.as<double2>(), -1.0);
                 true_residual(h, transpose, R, b, x, rb.as<double2>(), W, NB, tres, st);
                 for (int j = 0; j < R; j++) bnorm_rel[j] = tres[j];
             }
@@ -889,9 +928,7 @@ void solve(arh_hmat *h, int transpose, int R, const double2 *b, double2 *x, cons
                      err, W, NB, false);
             for (int j = 0; j < R; j++) iters_tot[j] += f64[j] ? iters[j] : 0;
             left -= *std::max_element(iters.begin(), iters.end());
-            ARH_HIP(hipMemcpyAsync(W.mask, f64.data(), sizeof(int) * R, hipMemcpyHostToDevice, s));
-            hipLaunchKernelGGL(k_axpy_cols, ga, dim3(256), 0, s, W.mask, N, x, dx.as<double2>(), 1.0);
-            ARH_HIP(hipGetLastError());
+            W.axpy(f64, N, x, dx.as<double2>(), 1.0);
             true_residual(h, transpose, R, b, x, rb.as<double2>(), W, NB, tres, st);
             if (st) st->refinements++;
             trace_sweep("fp64 correction", sweep, f64, iters, tres);
