@@ -3,13 +3,20 @@
 // its transpose V^T (U^T x) (adjoint.cpp:101-102, 177-178).
 //
 // Unlike the block ACA (one workgroup per block), this is a single large block, so every stage of a
-// cross is a grid-wide kernel: residual row (N entries) with block-partial first-max; pivot, row
-// normalisation and residual column (LL entries, masked first-max) in one launch; the non-conjugated dot
-// products with the stored crosses (chunk partials over a 2-D grid); and a one-workgroup finish that
-// applies the stopping rule. A residual row or column block takes 64 entries (one per lane) and splits the sum
-// over the stored crosses between its kQS wavefronts, so the grid grows with the rank as well as with
-// N or LL. All reductions are two-stage with a fixed order. The loop control lives on the device (a `done` flag every kernel
-// checks), so the host launches a few crosses at a time and synchronises once per batch.
+// cross is a grid-wide kernel, two launches per cross c:
+//   k_qa_row: the next row from the column maxima of cross c - 1; residual row c (N entries) with block-partial
+//     first-max; in further workgroups the non-conjugated dot products of cross c - 1 with the stored crosses (chunk
+//     partials);
+//   k_qa_normcol: pivot, row normalisation and residual column c (LL entries, masked first-max); in one further
+//     workgroup the stopping rule for cross c - 1.
+// So cross c is begun before the rule has seen cross c - 1; if that one stops, c is left behind unused. A launch takes
+// 4 to 7 us whatever it holds (serial chains: maxima, entry, stored crosses, sums) and the gap to the next
+// one 5, so the count of launches is what the time goes with: with the dots and the rule as launches of their own
+// a cross of the 1297 x 9828 matrix (rank 195) took 28 us, now 17.6.
+// A residual row or column block takes 64 entries (one per lane), the sum over the stored crosses split between kQS
+// wavefronts and the entry formed by another one, so the grid grows with the rank as well as with
+// N or LL. All reductions are two-stage with a fixed order. The loop control lives on the device (a `done` flag every
+// kernel checks); the host launches a few crosses at a time and reads the state of one such batch while the next one runs.
 //
 // Semantics kept from aca.cpp:84-134: start at row 0 (used = {0}); V row = v / v_j with no zero-pivot
 // guard (aca.cpp:104); error estimate with |u|^2 |v|^2 + 2 sum |u_p^T u| |v v_p^T|; stop when
@@ -22,34 +29,24 @@
 
 namespace arh {
 
-constexpr int kQT = 256;  // threads per block
-constexpr int kQS = 8;    // wavefronts of a residual row / column block (slices of the stored crosses)
+constexpr int kQT = 256;  // threads per block of the products, per half block of the dots
+constexpr int kQS = 8;    // slices of the stored crosses in a residual row / column block, a wavefront each
+constexpr int kQB = (kQS + 1) * ARH_WAVE;  // its threads: one more wavefront for the entries
+constexpr int kQBatch = 8;  // crosses launched together
 
+// State after the stopping rule has seen crosses < it (it crosses kept), in two copies: k_qa_normcol of cross c
+// reads copy (c + 1) & 1 and writes copy c & 1.
 struct QAcaState {
     double err;
-    int i, it, done, lim;
+    int it, done, lim, pad;
 };
 
-// block first-max of (value, index); ties to the lower index; value -1 = none
-__device__ __forceinline__ void block_argmax_q(double &v, int &idx, double *sv, int *si) {
-    wave_argmax(v, idx);
-    const int w = threadIdx.x / ARH_WAVE, lane = threadIdx.x % ARH_WAVE;
-    __syncthreads();
-    if (lane == 0) sv[w] = v, si[w] = idx;
-    __syncthreads();
-    double bv = sv[0];
-    int bi = si[0];
-    for (int q = 1; q < kQT / ARH_WAVE; q++)
-        if (sv[q] > bv || (sv[q] == bv && si[q] < bi)) bv = sv[q], bi = si[q];
-    v = bv;
-    idx = bi;
-}
-
+// sum over the block's first kQT threads; every thread of the block calls it
 __device__ __forceinline__ double block_sum_q(double v, double *sv) {
     v = wave_sum(v);
     const int w = threadIdx.x / ARH_WAVE, lane = threadIdx.x % ARH_WAVE;
     __syncthreads();
-    if (lane == 0) sv[w] = v;
+    if (lane == 0 && w < kQT / ARH_WAVE) sv[w] = v;
     __syncthreads();
     double s = sv[0];
     for (int q = 1; q < kQT / ARH_WAVE; q++) s += sv[q];
@@ -62,7 +59,7 @@ __device__ __forceinline__ double2 cross_slice(int it, int w, const double2 *__r
                                                const double2 *__restrict__ shared, int64_t sstride) {
     const int chunk = (it + kQS - 1) / kQS, p0 = w * chunk, p1 = min(it, p0 + chunk);
     double2 acc = make_double2(0.0, 0.0);
-#pragma unroll 4
+#pragma unroll 8
     for (int p = p0; p < p1; p++) {
         const double2 a = shared[p * sstride], b = own[p * ostride];
         acc.x += a.x * b.x - a.y * b.y;
@@ -71,41 +68,92 @@ __device__ __forceinline__ double2 cross_slice(int it, int w, const double2 *__r
     return acc;
 }
 
-// entry - (slice 0 + ... ): wave 0 subtracts the kQS slice sums in wave order (the other waves leave
-// theirs in red and return false)
-__device__ __forceinline__ bool combine_slices(double2 &v, const double2 &mine, double2 (*red)[ARH_WAVE], int w,
-                                               int lane) {
-    if (w > 0) red[w - 1][lane] = mine;
+// entry - (slice 0 + ... ): the last wave subtracts the kQS slice sums in order (the others leave theirs in red and
+// return false)
+__device__ __forceinline__ bool combine_slices(double2 &v, double2 (*red)[ARH_WAVE], int w, int lane) {
+    if (w < kQS) red[w][lane] = v;
     __syncthreads();
-    if (w != 0) return false;
-    v.x -= mine.x;
-    v.y -= mine.y;
+    if (w < kQS) return false;
 #pragma unroll
-    for (int q = 0; q < kQS - 1; q++) v.x -= red[q][lane].x, v.y -= red[q][lane].y;
+    for (int q = 0; q < kQS; q++) v.x -= red[q][lane].x, v.y -= red[q][lane].y;
     return true;
 }
 
-// residual row i into V row `it` (unnormalised) + block partial first-max of |v|^2 (64 columns a block)
-__global__ __launch_bounds__(kQS * ARH_WAVE) void k_qa_row(const QAcaState *__restrict__ S,
-                                                          const double *__restrict__ L, const Tri *__restrict__ tri,
-                                                          double k, int LL, int N, const double2 *__restrict__ U,
-                                                          double2 *__restrict__ V, double *__restrict__ pmax) {
-    __shared__ double2 red[kQS - 1][ARH_WAVE];
-    const QAcaState st = *S;
-    if (st.done) return;
-    const int i = st.i, it = st.it;
+constexpr int kQC = 8 * kQT;  // entries of a dot product chunk
+
+// Workgroups [0, nbr): residual row i of cross c into V row c (unnormalised) + block partial first-max of |v|^2 (64
+// columns a block). The row is 0 for c = 0, else the first maximum over the column blocks' partials of cross c - 1 (ties to
+// the lower index; 0 if every row is used), which the first workgroup marks as used.
+// The others: chunk partials of the non-conjugated products u^T u_p and v v_p^T of cross c - 1 with the stored
+// crosses p < c - 1 (aca.cpp:64-69 / :114-116), two (p, chunk) pairs per workgroup: chunks [0, ncu) over U's LL rows
+// and [ncu, ncu + ncv) over V's N columns; pu[p * ncu + chunk], pv[p * ncv + chunk].
+__global__ __launch_bounds__(kQB) void k_qa_row(const QAcaState *__restrict__ S, int c, const double *__restrict__ L,
+                                                const Tri *__restrict__ tri, double k, int LL, int N,
+                                                const double2 *__restrict__ U, double2 *__restrict__ V,
+                                                unsigned char *__restrict__ used, const double *__restrict__ pcol,
+                                                int nbc, int nbr, double *__restrict__ pmax, int ncu, int ncv,
+                                                double2 *__restrict__ pu, double2 *__restrict__ pv) {
+    __shared__ double2 red[kQS][ARH_WAVE];
+    __shared__ double sv[kQB / ARH_WAVE];
+    __shared__ int si;
+    if (S->done) return;
     const int w = __builtin_amdgcn_readfirstlane((int)(threadIdx.x / ARH_WAVE)), lane = threadIdx.x % ARH_WAVE;
-    const int c = blockIdx.x * ARH_WAVE + lane, cc = min(c, N - 1);  // loads clamped, stores guarded
-    double2 v = make_double2(0.0, 0.0);
-    if (w == 0) v = bem_entry(k, L[3 * i], L[3 * i + 1], L[3 * i + 2], tri[cc]);
-    const double2 mine = cross_slice(it, w, V + cc, N, U + i, LL);
-    if (!combine_slices(v, mine, red, w, lane)) return;
+    if ((int)blockIdx.x >= nbr) {
+        const int half = w / (kQT / ARH_WAVE);  // the last wave takes no part
+        const int e = 2 * ((int)blockIdx.x - nbr) + half, p = e / (ncu + ncv), h = e - p * (ncu + ncv);
+        const bool on = half < 2 && p < c - 1, isu = h < ncu;
+        double2 acc = make_double2(0.0, 0.0);
+        if (on) {
+            const int n = isu ? LL : N, c0 = (isu ? h : h - ncu) * kQC, c1 = min(n, c0 + kQC);
+            const double2 *a = isu ? U + (int64_t)(c - 1) * LL : V + (int64_t)(c - 1) * N;
+            const double2 *b = isu ? U + (int64_t)p * LL : V + (int64_t)p * N;
+            for (int q = c0 + (int)threadIdx.x % kQT; q < c1; q += kQT) cfma(acc, a[q], b[q]);
+        }
+        acc.x = wave_sum(acc.x);
+        acc.y = wave_sum(acc.y);
+        if (lane == 0) red[0][w] = acc;
+        __syncthreads();
+        if (on && threadIdx.x % kQT == 0) {
+            const int w0 = half * (kQT / ARH_WAVE);
+            double2 s = red[0][w0];
+            for (int q = 1; q < kQT / ARH_WAVE; q++) s.x += red[0][w0 + q].x, s.y += red[0][w0 + q].y;
+            if (isu)
+                pu[(int64_t)p * ncu + h] = s;
+            else
+                pv[(int64_t)p * ncv + (h - ncu)] = s;
+        }
+        return;
+    }
+    int i = 0;
+    if (c > 0) {
+        if (w == 0) {
+            double bv = -1.0;
+            int bi = 0x7fffffff;
+            for (int b = lane; b < nbc; b += ARH_WAVE) {
+                const double v = pcol[3 * b + 1];
+                const int l = (int)pcol[3 * b + 2];
+                if (v > bv || (v == bv && l < bi)) bv = v, bi = l;
+            }
+            wave_argmax(bv, bi);
+            if (lane == 0) si = bv < 0.0 ? 0 : bi;
+        }
+        __syncthreads();
+        i = __builtin_amdgcn_readfirstlane(si);
+        if (blockIdx.x == 0 && threadIdx.x == 0) used[i] = 1;
+    }
+    const int col = blockIdx.x * ARH_WAVE + lane, cc = min(col, N - 1);  // loads clamped, stores guarded
+    double2 v;
+    if (w == kQS)
+        v = bem_entry(k, L[3 * i], L[3 * i + 1], L[3 * i + 2], tri[cc]);
+    else
+        v = cross_slice(c, w, V + cc, N, U + i, LL);
+    if (!combine_slices(v, red, w, lane)) return;
     double best = -1.0;
     int bi = 0x7fffffff;
-    if (c < N) {
-        V[(int64_t)it * N + c] = v;
+    if (col < N) {
+        V[(int64_t)c * N + col] = v;
         const double a = cnorm2(v);
-        best = a == a ? a : -1.0, bi = c;  // NaN never wins
+        best = a == a ? a : -1.0, bi = col;  // NaN never wins
     }
     wave_argmax(best, bi);
     // the partial carries v at the block's first maximum, so the pivot value is known without reading the
@@ -119,24 +167,70 @@ __global__ __launch_bounds__(kQS * ARH_WAVE) void k_qa_row(const QAcaState *__re
     }
 }
 
-// One launch after the residual row, workgroups [0, nbn) normalising V row `it` (512 columns each, block
-// partials of |v|^2) and [nbn, nbn + nbc) forming the residual column j (64 rows each). Every workgroup
+// Stopping rule for cross c - 1 (a whole workgroup; fixed-order reductions): error estimate with its norms and dot
+// products, the new state to out and, for the last launch of a batch, to the host's pinned copy.
+__device__ __forceinline__ void qa_finish(const QAcaState &st0, QAcaState *__restrict__ out, QAcaState *host, int c,
+                                          double eps, const double *__restrict__ pvn, int nbn,
+                                          const double *__restrict__ pcol, int nbc, const double2 *__restrict__ pu, int ncu,
+                                          const double2 *__restrict__ pv, int ncv, double *sv) {
+    QAcaState st = st0;
+    if (c > 0 && !st0.done) {
+        const int t = threadIdx.x;
+        double vn = 0.0, un = 0.0, d = 0.0;
+        if (t < kQT) {
+            for (int b = t; b < nbn; b += kQT) vn += pvn[b];
+            for (int b = t; b < nbc; b += kQT) un += pcol[3 * b];
+            for (int p = t; p < c - 1; p += kQT) {
+                double2 su = make_double2(0.0, 0.0), sq = make_double2(0.0, 0.0);
+                for (int q = 0; q < ncu; q++) su.x += pu[(int64_t)p * ncu + q].x, su.y += pu[(int64_t)p * ncu + q].y;
+                for (int q = 0; q < ncv; q++) sq.x += pv[(int64_t)p * ncv + q].x, sq.y += pv[(int64_t)p * ncv + q].y;
+                d += cabs_(su) * cabs_(sq);
+            }
+        }
+        vn = block_sum_q(vn, sv);
+        un = block_sum_q(un, sv);
+        d = block_sum_q(d, sv);
+        st.err += un * vn + 2.0 * d;
+        if (sqrt(un * vn / st.err) <= eps) {
+            st.done = 1;  // cross c - 1 discarded: rank = c - 1
+        } else {
+            st.it = c;
+            if (st.it >= st.lim) st.done = 1;
+        }
+    }
+    if (threadIdx.x == 0) {
+        *out = st;
+        if (host) *host = st;
+    }
+}
+
+// One launch after the residual row of cross c, workgroups [0, nbn) normalising V row c (512 columns each, block
+// partials of |v|^2), [nbn, nbn + nbc) forming the residual column j (64 rows each), and a last one applying the stopping
+// rule to cross c - 1. Every workgroup of the first two kinds
 // first finds the pivot column j = the first maximum over the row blocks' partials (ties to the lower
 // index, so it is the sequential first maximum) and takes v_j from the winning partial.
-__global__ __launch_bounds__(kQS * ARH_WAVE) void k_qa_normcol(const QAcaState *__restrict__ S,
-                                                              const double *__restrict__ L,
-                                                              const Tri *__restrict__ tri, double k, int LL, int N,
-                                                              double2 *__restrict__ U, double2 *__restrict__ V,
-                                                              const unsigned char *__restrict__ used,
-                                                              const double *__restrict__ pmax, int nbr, int nbn,
-                                                              double *__restrict__ pvn, double *__restrict__ pcol) {
-    __shared__ double2 red[kQS - 1][ARH_WAVE];
-    __shared__ double sv[kQS];
+__global__ __launch_bounds__(kQB) void k_qa_normcol(const QAcaState *__restrict__ S, QAcaState *__restrict__ So,
+                                                    QAcaState *__restrict__ host, int c, double eps,
+                                                    const double *__restrict__ L, const Tri *__restrict__ tri, double k,
+                                                    int LL, int N, double2 *__restrict__ U, double2 *__restrict__ V,
+                                                    const unsigned char *__restrict__ used,
+                                                    const double *__restrict__ pmax, int nbr, int nbn, int nbc,
+                                                    double *__restrict__ pvn, double *__restrict__ pcol,
+                                                    const double *__restrict__ pvn1, const double *__restrict__ pcol1,
+                                                    const double2 *__restrict__ pu, int ncu,
+                                                    const double2 *__restrict__ pv, int ncv) {
+    __shared__ double2 red[kQS][ARH_WAVE];
+    __shared__ double sv[kQB / ARH_WAVE];
     __shared__ int sj;
     __shared__ double2 spiv;
     const QAcaState st = *S;
+    if (blockIdx.x == gridDim.x - 1) {
+        // (nbn and nbc are 0 in a launch of this workgroup alone: the partials' counts come from the sizes)
+        qa_finish(st, So, host, c, eps, pvn1, (N + kQS * ARH_WAVE - 1) / (kQS * ARH_WAVE), pcol1,
+                  (LL + ARH_WAVE - 1) / ARH_WAVE, pu, ncu, pv, ncv, sv);
+        return;
+    }
     if (st.done) return;
-    const int it = st.it;
     const int w = __builtin_amdgcn_readfirstlane((int)(threadIdx.x / ARH_WAVE)), lane = threadIdx.x % ARH_WAVE;
     if (w == 0) {
         double bv = -1.0;
@@ -153,14 +247,14 @@ __global__ __launch_bounds__(kQS * ARH_WAVE) void k_qa_normcol(const QAcaState *
         }
     }
     __syncthreads();
-    const int j = sj;
+    const int j = __builtin_amdgcn_readfirstlane(sj);
     if ((int)blockIdx.x < nbn) {
-        // V row `it` /= v_j (no zero-pivot guard, aca.cpp:104) + block partial of |v|^2
-        const int c = blockIdx.x * (kQS * ARH_WAVE) + threadIdx.x;
+        // V row c /= v_j (no zero-pivot guard, aca.cpp:104) + block partial of |v|^2 (the last wave has no columns)
+        const int col = blockIdx.x * (kQS * ARH_WAVE) + threadIdx.x;
         double a = 0.0;
-        if (c < N) {
-            const double2 v = cdiv(V[(int64_t)it * N + c], spiv);
-            V[(int64_t)it * N + c] = v;
+        if (w < kQS && col < N) {
+            const double2 v = cdiv(V[(int64_t)c * N + col], spiv);
+            V[(int64_t)c * N + col] = v;
             a = cnorm2(v);
         }
         a = wave_sum(a);
@@ -173,17 +267,19 @@ __global__ __launch_bounds__(kQS * ARH_WAVE) void k_qa_normcol(const QAcaState *
         }
         return;
     }
-    // residual column j into U column `it` + block partials of |u|^2 and of the masked first-max
+    // residual column j into U column c + block partials of |u|^2 and of the masked first-max
     const int bc = (int)blockIdx.x - nbn;
     const int l = bc * ARH_WAVE + lane, ll = min(l, LL - 1);
-    double2 u = make_double2(0.0, 0.0);
-    if (w == 0) u = bem_entry(k, L[3 * ll], L[3 * ll + 1], L[3 * ll + 2], tri[j]);
-    const double2 mine = cross_slice(it, w, U + ll, LL, V + j, N);
-    if (!combine_slices(u, mine, red, w, lane)) return;
+    double2 u;
+    if (w == kQS)
+        u = bem_entry(k, L[3 * ll], L[3 * ll + 1], L[3 * ll + 2], tri[j]);
+    else
+        u = cross_slice(c, w, U + ll, LL, V + j, N);
+    if (!combine_slices(u, red, w, lane)) return;
     double a = 0.0, best = -1.0;
     int bi = 0x7fffffff;
     if (l < LL) {
-        U[(int64_t)it * LL + l] = u;
+        U[(int64_t)c * LL + l] = u;
         a = cnorm2(u);
         if (!used[l]) best = a == a ? a : -1.0, bi = l;
     }
@@ -192,79 +288,8 @@ __global__ __launch_bounds__(kQS * ARH_WAVE) void k_qa_normcol(const QAcaState *
     if (lane == 0) pcol[3 * bc] = a, pcol[3 * bc + 1] = best, pcol[3 * bc + 2] = (double)bi;
 }
 
-// Chunk partials of the non-conjugated products u^T u_p and v v_p^T with the stored crosses p < it
-// (aca.cpp:64-69 / :114-116): block (p, c) sums chunk c of kQC entries, chunks [0, ncu) over U's
-// LL rows and [ncu, ncu + ncv) over V's N columns; pu[p * ncu + c], pv[p * ncv + c'].
-constexpr int kQC = 8 * kQT;
-__global__ __launch_bounds__(kQT) void k_qa_dots(const QAcaState *__restrict__ S, int LL, int N, int ncu, int ncv,
-                                                const double2 *__restrict__ U, const double2 *__restrict__ V,
-                                                double2 *__restrict__ pu, double2 *__restrict__ pv) {
-    __shared__ double sv[kQT / ARH_WAVE];
-    const QAcaState st = *S;
-    const int p = blockIdx.x, c = blockIdx.y;
-    if (st.done || p >= st.it) return;
-    const bool isu = c < ncu;
-    const int n = isu ? LL : N, c0 = (isu ? c : c - ncu) * kQC;
-    const double2 *a = isu ? U + (int64_t)st.it * LL : V + (int64_t)st.it * N;
-    const double2 *b = isu ? U + (int64_t)p * LL : V + (int64_t)p * N;
-    double2 acc = make_double2(0.0, 0.0);
-    const int e1 = min(n, c0 + kQC);
-    for (int e = c0 + threadIdx.x; e < e1; e += kQT) cfma(acc, a[e], b[e]);
-    acc.x = block_sum_q(acc.x, sv);
-    acc.y = block_sum_q(acc.y, sv);
-    if (threadIdx.x == 0) {
-        if (isu)
-            pu[(int64_t)p * ncu + c] = acc;
-        else
-            pv[(int64_t)p * ncv + (c - ncu)] = acc;
-    }
-}
-
-// error estimate, stopping rule, next row (one workgroup; fixed-order reductions)
-__global__ __launch_bounds__(kQT) void k_qa_finish(QAcaState *__restrict__ S, double eps,
-                                                  const double *__restrict__ pvn, int nbn,
-                                                  const double *__restrict__ pcol, int nbc,
-                                                  const double2 *__restrict__ pu, int ncu,
-                                                  const double2 *__restrict__ pv, int ncv,
-                                                  unsigned char *__restrict__ used) {
-    __shared__ double sv[kQT / ARH_WAVE];
-    __shared__ int si[kQT / ARH_WAVE];
-    const QAcaState st0 = *S;
-    if (st0.done) return;
-    double vn = 0.0, un = 0.0, d = 0.0, bv = -1.0;
-    int bi = 0x7fffffff;
-    for (int b = threadIdx.x; b < nbn; b += kQT) vn += pvn[b];
-    for (int b = threadIdx.x; b < nbc; b += kQT) {
-        un += pcol[3 * b];
-        const double v = pcol[3 * b + 1];
-        const int l = (int)pcol[3 * b + 2];
-        if (v > bv || (v == bv && l < bi)) bv = v, bi = l;
-    }
-    for (int p = threadIdx.x; p < st0.it; p += kQT) {
-        double2 su = make_double2(0.0, 0.0), sq = make_double2(0.0, 0.0);
-        for (int c = 0; c < ncu; c++) su.x += pu[(int64_t)p * ncu + c].x, su.y += pu[(int64_t)p * ncu + c].y;
-        for (int c = 0; c < ncv; c++) sq.x += pv[(int64_t)p * ncv + c].x, sq.y += pv[(int64_t)p * ncv + c].y;
-        d += cabs_(su) * cabs_(sq);
-    }
-    vn = block_sum_q(vn, sv);
-    un = block_sum_q(un, sv);
-    d = block_sum_q(d, sv);
-    block_argmax_q(bv, bi, sv, si);
-    if (threadIdx.x != 0) return;
-    QAcaState st = st0;
-    st.err += un * vn + 2.0 * d;
-    if (sqrt(un * vn / st.err) <= eps) {
-        st.done = 1;  // current cross discarded: rank = it
-    } else {
-        st.i = bv < 0.0 ? 0 : bi;
-        used[st.i] = 1;
-        st.it++;
-        if (st.it >= st.lim) st.done = 1;
-    }
-    *S = st;
-}
-
-// products: t = V x (rank x nrhs, one block per (p, j)); y = U t
+// products: t = V x (rank x nrhs, one block per (p, j)); y = U t (a thread per row: eight loads in flight keep its
+// serial sum from waiting for each: 43 -> 26 us at 1297 x 9828, rank 182)
 __global__ __launch_bounds__(kQT) void k_qa_vx(int N, int r, const double2 *__restrict__ V, const double2 *__restrict__ x,
                                               double2 *__restrict__ t) {
     __shared__ double sv[kQT / ARH_WAVE];
@@ -286,6 +311,7 @@ __global__ void k_qa_ut(int LL, int r, int nrhs, const double2 *__restrict__ U, 
     if (e >= (int64_t)LL * nrhs) return;
     const int j = (int)(e / LL), l = (int)(e % LL);
     double2 s = make_double2(0.0, 0.0);
+#pragma unroll 8
     for (int p = 0; p < r; p++) {
         const double2 a = U[(int64_t)p * LL + l], b = t[(int64_t)j * r + p];
         s.x += a.x * b.x - a.y * b.y;
@@ -316,6 +342,7 @@ __global__ void k_qa_vts(int N, int r, int nrhs, const double2 *__restrict__ V, 
     if (e >= (int64_t)N * nrhs) return;
     const int j = (int)(e / N), c = (int)(e % N);
     double2 s = make_double2(0.0, 0.0);
+#pragma unroll 8
     for (int p = 0; p < r; p++) {
         const double2 a = V[(int64_t)p * N + c], b = t[(int64_t)j * r + p];
         s.x += a.x * b.x - a.y * b.y;
@@ -336,48 +363,71 @@ void qaca_build(arh_qaca *q, const double *L_host) {
     q->nbr = (N + ARH_WAVE - 1) / ARH_WAVE;               // residual row blocks
     q->nbn = (N + kQS * ARH_WAVE - 1) / (kQS * ARH_WAVE);  // row normalisation blocks
     q->nbc = (LL + ARH_WAVE - 1) / ARH_WAVE;               // residual column blocks
-    q->part.alloc(sizeof(double) * (4 * (size_t)q->nbr + q->nbn + 3 * (size_t)q->nbc + 16));
+    // first maxima of the row blocks, then norms and first maxima of two crosses
+    const size_t np = q->nbn + 3 * (size_t)q->nbc;
+    q->part.alloc(sizeof(double) * (4 * (size_t)q->nbr + 2 * np + 16));
     const int ncu = (LL + kQC - 1) / kQC, ncv = (N + kQC - 1) / kQC;
     q->dots.alloc(sizeof(double2) * (size_t)std::max(1, lim) * (ncu + ncv));
+    q->rank = 0;
+    if (lim <= 0) {
+        ARH_HIP(hipStreamSynchronize(s));
+        return;
+    }
     std::vector<unsigned char> used(LL, 0);
     used[0] = 1;
     upload(q->used, used, s);
-    QAcaState st0{};
-    st0.i = 0, st0.it = 0, st0.done = lim <= 0 ? 1 : 0, st0.lim = lim;
-    q->st.alloc(sizeof(QAcaState));
-    ARH_HIP(hipMemcpyAsync(q->st.p, &st0, sizeof(QAcaState), hipMemcpyHostToDevice, s));
-    double *pmax = q->part.as<double>(), *pvn = pmax + 4 * q->nbr, *pcol = pvn + q->nbn;
+    HostBuf hb(4 * sizeof(QAcaState), s);
+    QAcaState *hst = hb.as<QAcaState>();  // state after batch b at b & 1; then the initial copies
+    hst[2].err = 0.0, hst[2].it = 0, hst[2].done = 0, hst[2].lim = lim, hst[2].pad = 0;
+    hst[3] = hst[2];
+    q->st.alloc(2 * sizeof(QAcaState));
+    ARH_HIP(hipMemcpyAsync(q->st.p, hst + 2, 2 * sizeof(QAcaState), hipMemcpyHostToDevice, s));
+    double *pmax = q->part.as<double>(), *par = pmax + 4 * q->nbr;
     QAcaState *S = q->st.as<QAcaState>();
     const Tri *tri = g->tri.as<Tri>();
-    const double2 *Uc = q->U.as<double2>();
-    const double2 *Vc = q->V.as<double2>();
-    double2 *pu = q->dots.as<double2>(), *pv = pu + (size_t)std::max(1, lim) * ncu;
-    int launched = 0;  // crosses launched so far (an upper bound of it on the device)
-    QAcaState hs = st0;
-    while (!hs.done) {
-        // a few crosses per synchronisation at first, more once the rank grows (launches after the
-        // stop return at once)
-        const int batch = std::min(std::max(8, std::min(32, launched / 4)), lim - launched);
-        for (int b = 0; b < batch; b++) {
-            const int itb = launched + b;  // the cross index if none of the previous ones stopped
-            hipLaunchKernelGGL(k_qa_row, dim3(q->nbr), dim3(kQS * ARH_WAVE), 0, s, S, q->L.as<double>(), tri, q->k,
-                               LL, N, Uc, q->V.as<double2>(), pmax);
-            hipLaunchKernelGGL(k_qa_normcol, dim3(q->nbn + q->nbc), dim3(kQS * ARH_WAVE), 0, s, S, q->L.as<double>(),
-                               tri, q->k, LL, N, q->U.as<double2>(), q->V.as<double2>(), q->used.as<unsigned char>(),
-                               pmax, q->nbr, q->nbn, pvn, pcol);
-            if (itb > 0)
-                hipLaunchKernelGGL(k_qa_dots, dim3(itb, ncu + ncv), dim3(kQT), 0, s, S, LL, N, ncu, ncv, Uc, Vc, pu,
-                                   pv);
-            hipLaunchKernelGGL(k_qa_finish, dim3(1), dim3(kQT), 0, s, S, q->tol, pvn, q->nbn, pcol, q->nbc, pu, ncu,
-                               pv, ncv, q->used.as<unsigned char>());
+    double2 *U = q->U.as<double2>(), *V = q->V.as<double2>();
+    double2 *pu = q->dots.as<double2>(), *pv = pu + (size_t)lim * ncu;
+    // cross c (c == lim: the stopping rule for the last cross alone)
+    auto cross = [&](int c, QAcaState *host) {
+        double *cur = par + (c & 1) * np, *prev = par + ((c + 1) & 1) * np;
+        const QAcaState *Si = S + ((c + 1) & 1);
+        const int nbr = c < lim ? q->nbr : 0, nbn = c < lim ? q->nbn : 0, nbc = c < lim ? q->nbc : 0;
+        const int nd = c > 1 ? ((c - 1) * (ncu + ncv) + 1) / 2 : 0;
+        if (nbr + nd > 0)
+            hipLaunchKernelGGL(k_qa_row, dim3(nbr + nd), dim3(kQB), 0, s, Si, c, q->L.as<double>(), tri, q->k, LL, N, U,
+                               V, q->used.as<unsigned char>(), prev + q->nbn, q->nbc, nbr, pmax, ncu, ncv, pu, pv);
+        hipLaunchKernelGGL(k_qa_normcol, dim3(nbn + nbc + 1), dim3(kQB), 0, s, Si, S + (c & 1), host, c, q->tol,
+                           q->L.as<double>(), tri, q->k, LL, N, U, V, q->used.as<unsigned char>(), pmax, nbr, nbn, nbc,
+                           cur, cur + q->nbn, prev, prev + q->nbn, pu, ncu, pv, ncv);
+    };
+    struct Events {
+        hipEvent_t e[2] = {};
+        ~Events() {
+            for (hipEvent_t v : e)
+                if (v) (void)hipEventDestroy(v);
         }
-        ARH_HIP(hipGetLastError());
-        launched += batch;
-        ARH_HIP(hipMemcpyAsync(&hs, q->st.p, sizeof(QAcaState), hipMemcpyDeviceToHost, s));
-        ARH_HIP(hipStreamSynchronize(s));
-        ARH_CHECK(hs.done || launched < lim, ARH_EINVAL, "internal: listener ACA ran past its limit");
+    } ev;
+    for (hipEvent_t &e : ev.e) ARH_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+    // batch b is launched before the state after batch b - 1 is read (launches after the stop return at once)
+    int launched = 0;  // crosses 0 .. launched - 1
+    for (int b = 0;; b++) {
+        if (launched < lim) {
+            const int end = std::min(lim, launched + kQBatch);
+            for (; launched < end; launched++)
+                cross(launched, launched + 1 == end && end < lim ? hst + (b & 1) : nullptr);
+            if (end == lim) cross(lim, hst + (b & 1));
+            ARH_HIP(hipGetLastError());
+            ARH_HIP(hipEventRecord(ev.e[b & 1], s));
+        }
+        if (b == 0) continue;
+        ARH_HIP(hipEventSynchronize(ev.e[(b - 1) & 1]));
+        const QAcaState hs = hst[(b - 1) & 1];
+        if (hs.done) {
+            q->rank = hs.it;
+            break;
+        }
+        ARH_CHECK(b <= lim, ARH_EINVAL, "internal: listener ACA ran past its limit");
     }
-    q->rank = hs.it;
 }
 
 void qaca_apply(arh_qaca *q, int transpose, int nrhs, const double2 *x, double2 *y) {
