@@ -255,14 +255,15 @@ struct MfmaLayout {
     arh::DBuf panel[2], vs[2], xt[2], part[2];
     bool built[2] = {false, false};
     bool lists = false;
-    arh::DBuf d_stacks, d_p1units, d_lpanel, d_psrc, d_rtasks, d_rsplit, d_maps, d_csrc, d_trow;
-    std::vector<VStack> stacks;
-    std::vector<int2> p1units;
-    int p1big = 0, nmaps = 0;
-    std::vector<LeafPanel> lpanel;
-    std::vector<RowTask> rtasks;
-    std::vector<int4> rsplit;
-    int nslots = 0;
+    // lists made on the host (one upload) and where they are in it; those made on the device
+    arh::DBuf d_lists, d_psrc, d_csrc, d_maps, d_trow;
+    const int *bad = nullptr;  // raised when the device's panel columns disagree with the host's counts
+    const VStack *stacks = nullptr;
+    const int2 *p1units = nullptr;
+    const LeafPanel *lpanel = nullptr;
+    const RowTask *rtasks = nullptr;
+    const int4 *rsplit = nullptr;
+    int nunits = 0, p1big = 0, nmaps = 0, ntasks = 0, nsplit = 0, nslots = 0;
     int64_t panel_total = 0, vs_total = 0;
 };
 
@@ -270,8 +271,8 @@ struct MfmaLayout {
 struct LRBlock {
     int rs, re, cs, ce;
     int lim;        // min(max_rank, m-1, n-1)
-    int rank;       // stored rank (crosses with u, v != 0); filled by the ACA
-    int rank_ref;   // rank as the reference counts it (aca.cpp:80)
+    int rank;       // stored rank (crosses with u, v != 0)
+    int pad;
     int l0;         // first row leaf
     int64_t us_off, vs_off;  // ACA scratch (U: m x lim col-major, V: lim x n row-major)
     int64_t u_off, v_off;    // packed storage (U leaf-segmented, V row-major)
@@ -310,16 +311,19 @@ struct arh_geom_s {
     // low-rank: per row leaf / per col leaf lists of blocks
     std::vector<int> lrR_ptr, lrR_blk, lrC_ptr, lrC_blk;
     arh::DBuf d_lrR_ptr, d_lrR_blk, d_lrC_ptr, d_lrC_blk;
-    // ACA scratch sized for the largest max_rank seen
-    int scratch_rank = -1;
-    arh::DBuf aca_U, aca_V, aca_flags;
+    // Low-rank blocks as the partition and max_rank fix them (-1: not made yet): descriptors with their scratch
+    // offsets, the ACA's launch order (largest work first, workgroup blocks leading), scratch totals
+    int lr_plan_rank = -1, aca_nbig = 0;
     int64_t aca_u_total = 0, aca_v_total = 0, aca_f_total = 0;
-    std::vector<int64_t> us_off, vs_off, flag_off;
-    std::vector<int> lim;
-    // ACA launch order (largest work first, workgroup blocks leading): fixed by the partition and
-    // max_rank, so it is computed once per max_rank
-    int aca_order_rank = -1, aca_nbig = 0;
+    arh::DBuf d_lr0;
     arh::DBuf d_aca_order;
+    // Low-rank blocks by column cluster [0] / row cluster [1]: clusters and members in order of first
+    // appearance (members mem[ptr[k]..ptr[k + 1])), and the clusters by decreasing size
+    struct Clusters {
+        std::vector<int> start, n, ptr, mem, by_size;
+        arh::DBuf d_ptr, d_mem;
+        bool made = false;
+    } clusters[2];
 };
 
 struct arh_hmat_s {
@@ -332,10 +336,10 @@ struct arh_hmat_s {
     arh::DBuf denseT, denseT32;  // the same panels row-major per leaf (generic transposed product, built on use)
     arh::DBuf blocks;          // LRBlock[na]
     arh::DBuf U, V, U32, V32;  // packed factors
-    std::vector<LRBlock> hblocks;
+    std::vector<int2> ranks;  // per low-rank block: stored rank, rank as the reference counts it
     int64_t u_total = 0, v_total = 0, t_total = 0;
-    std::vector<int> active_lr;  // lr blocks with rank > 0
-    arh::DBuf d_active_lr;
+    int n_active = 0;
+    arh::DBuf d_active_lr;  // lr blocks with rank > 0
     arh::DBuf tbuf;  // intermediate t / s values (t_total x nrhs c128)
     MfmaLayout mf[2];  // MFMA product: [0] forward, [1] transposed
     bool generic32 = false;  // dense32 / U32 / V32 (the non-MFMA FP32 product) built
@@ -371,8 +375,7 @@ namespace arh {
 void geom_set_heights(arh_geom *g, const double *base, const int *vid_dev, int HH, const double *h);
 void geom_build_tri(arh_geom *g);
 // assemble.hip
-void assemble_dense(arh_hmat *h);
-void assemble_aca(arh_hmat *h);
+void assemble(arh_hmat *h);
 void make_fp32_copy(arh_hmat *h);
 void make_generic_fp32(arh_hmat *h);
 // matvec.hip

@@ -190,7 +190,7 @@ __device__ __forceinline__ void residual(double2 &v, AcaBatch &first, const doub
 }
 
 // A block of at most 64 x 64, one wavefront: lane q holds row q and column q of the current cross.
-__device__ __forceinline__ void aca_small(LRBlock *__restrict__ blocks, int bid, const LRBlock &B, int lane,
+__device__ __forceinline__ void aca_small(int2 *__restrict__ ranks, int bid, const LRBlock &B, int lane,
                                           const Tri *__restrict__ tri, double k, double eps, double2 *__restrict__ U,
                                           double2 *__restrict__ V) {
     const int m = B.re - B.rs, n = B.ce - B.cs, lim = B.lim;
@@ -260,7 +260,7 @@ __device__ __forceinline__ void aca_small(LRBlock *__restrict__ blocks, int bid,
         __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");  // the new cross is read by other lanes
         __builtin_amdgcn_wave_barrier();
     }
-    if (lane == 0) blocks[bid].rank = sr, blocks[bid].rank_ref = it;
+    if (lane == 0) ranks[bid] = make_int2(sr, it);
 }
 
 struct AcaShared {
@@ -319,7 +319,7 @@ struct AcaGroup {
 };
 
 template <bool WAVE>
-__device__ __forceinline__ void aca_block(const AcaGroup<WAVE> &G, LRBlock *__restrict__ blocks, int bid,
+__device__ __forceinline__ void aca_block(const AcaGroup<WAVE> &G, int2 *__restrict__ ranks, int bid,
                                           const LRBlock &B, const Tri *__restrict__ tri, double k, double eps,
                                           double2 *__restrict__ U, double2 *__restrict__ V,
                                           unsigned char *__restrict__ used) {
@@ -438,20 +438,22 @@ __device__ __forceinline__ void aca_block(const AcaGroup<WAVE> &G, LRBlock *__re
         it++;
         G.sync();
     }
-    if (tid == 0) blocks[bid].rank = sr, blocks[bid].rank_ref = it;
+    if (tid == 0) ranks[bid] = make_int2(sr, it);
 }
 
 // Workgroups [0, nbig) each take one big block (order[0..nbig)); the others take kAcaWaves smaller
-// blocks, one per wavefront.
-__global__ __launch_bounds__(kAcaThreads, 3) void k_aca(LRBlock *__restrict__ blocks, const int *__restrict__ order,
+// blocks, one per wavefront. nan: raised by the dense blocks.
+__global__ __launch_bounds__(kAcaThreads, 3) void k_aca(const LRBlock *__restrict__ blocks, const int *__restrict__ order,
                                                      int nbig, int na, const Tri *__restrict__ tri, double k,
                                                      double eps, double2 *__restrict__ Us, double2 *__restrict__ Vs,
-                                                     unsigned char *__restrict__ flags) {
+                                                     unsigned char *__restrict__ flags, const int *__restrict__ nan,
+                                                     int2 *__restrict__ ranks) {
     __shared__ union Shared {
         AcaSharedGroup group;
         AcaShared wave[kAcaWaves];
         __device__ Shared() {}
     } sh;
+    if (*nan) return;  // the assembly fails
     const int lane = threadIdx.x % ARH_WAVE;
     const int w = __builtin_amdgcn_readfirstlane((int)(threadIdx.x / ARH_WAVE));
     const bool big = (int)blockIdx.x < nbig;
@@ -460,19 +462,81 @@ __global__ __launch_bounds__(kAcaThreads, 3) void k_aca(LRBlock *__restrict__ bl
     const int bid = order[u];
     const LRBlock B = blocks[bid];
     if (B.lim <= 0) {  // a single row or column, or max_rank 0
-        if (lane == 0 && (!big || w == 0)) blocks[bid].rank = 0, blocks[bid].rank_ref = 0;
+        if (lane == 0 && (!big || w == 0)) ranks[bid] = make_int2(0, 0);
         return;
     }
     double2 *U = Us + B.us_off, *V = Vs + B.vs_off;
     unsigned char *used = flags + B.flag_off;
     if (big) {
         const AcaGroup<false> G{(int)threadIdx.x, w, lane, sh.group};
-        aca_block<false>(G, blocks, bid, B, tri, k, eps, U, V, used);
+        aca_block<false>(G, ranks, bid, B, tri, k, eps, U, V, used);
     } else if (B.re - B.rs <= ARH_WAVE && B.ce - B.cs <= ARH_WAVE) {
-        aca_small(blocks, bid, B, lane, tri, k, eps, U, V);
+        aca_small(ranks, bid, B, lane, tri, k, eps, U, V);
     } else {
         const AcaGroup<true> G{lane, 0, lane, sh.wave[w]};
-        aca_block<true>(G, blocks, bid, B, tri, k, eps, U, V, used);
+        aca_block<true>(G, ranks, bid, B, tri, k, eps, U, V, used);
+    }
+}
+
+// ------------------------------------------------------------------ offsets
+// The blocks' descriptors with their ranks and the offsets of their factors (running sums over the blocks in order), the
+// blocks of rank > 0, and for the host, in pinned memory, ranks and totals. Workgroup b takes blocks [1024 b, 1024 b +
+// 1024) and sums up all before them by itself, so one launch does. (The host ran the sums between two 1.3 MB copies of
+// the descriptors, 0.7 ms of an idle GPU at 17,500 blocks.)
+struct LrTotals {
+    int64_t u, v, t;
+    int nact, nan;
+};
+__device__ __forceinline__ void lr_sizes(const LRBlock &B, int r, int64_t q[4]) {
+    q[0] = (int64_t)r * (B.re - B.rs), q[1] = (int64_t)r * (B.ce - B.cs), q[2] = r, q[3] = r > 0 ? 1 : 0;
+}
+__global__ __launch_bounds__(1024) void k_lr_offsets(int na, const LRBlock *__restrict__ lr0,
+                                                     const int2 *__restrict__ ranks, const int *__restrict__ nan,
+                                                     LRBlock *__restrict__ blocks, int *__restrict__ active,
+                                                     int2 *__restrict__ hranks, LrTotals *__restrict__ tot) {
+    __shared__ int64_t sh[2][1024 / ARH_WAVE][4];
+    const int lane = threadIdx.x % ARH_WAVE, w = threadIdx.x / ARH_WAVE;
+    const int a0 = (int)blockIdx.x * 1024, a = a0 + (int)threadIdx.x;
+    if (*nan) {
+        if (a == na - 1) tot->nan = 1;
+        return;
+    }
+    int64_t pre[4] = {0, 0, 0, 0}, own[4] = {0, 0, 0, 0}, q[4];
+#pragma unroll 8
+    for (int b = threadIdx.x; b < a0; b += 1024) {
+        lr_sizes(lr0[b], ranks[b].x, q);
+#pragma unroll
+        for (int k = 0; k < 4; k++) pre[k] += q[k];
+    }
+    LRBlock B{};
+    int2 r = make_int2(0, 0);
+    if (a < na) {
+        B = lr0[a], r = ranks[a];
+        lr_sizes(B, r.x, own);
+    }
+    int64_t inc[4];
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+        inc[k] = own[k];
+        for (int d = 1; d < ARH_WAVE; d <<= 1) {
+            const int64_t up = __shfl_up(inc[k], d, ARH_WAVE);
+            if (lane >= d) inc[k] += up;
+            pre[k] += __shfl_xor(pre[k], d, ARH_WAVE);
+        }
+        if (lane == ARH_WAVE - 1) sh[0][w][k] = inc[k], sh[1][w][k] = pre[k];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < 4; k++)
+        for (int v = 0; v < 1024 / ARH_WAVE; v++) inc[k] += sh[1][v][k] + (v < w ? sh[0][v][k] : 0);
+    if (a >= na) return;
+    B.rank = r.x, B.u_off = inc[0] - own[0], B.v_off = inc[1] - own[1], B.t_off = inc[2] - own[2];
+    blocks[a] = B;
+    if (r.x > 0) active[inc[3] - 1] = a;
+    hranks[a] = r;
+    if (a == na - 1) {
+        tot->u = inc[0], tot->v = inc[1], tot->t = inc[2], tot->nact = (int)inc[3];
+        tot->nan = 0;
     }
 }
 
@@ -524,9 +588,55 @@ __global__ void k_to_c64(const double2 *__restrict__ a, float2 *__restrict__ b, 
 }
 
 // ------------------------------------------------------------------ host drivers
-void assemble_dense(arh_hmat *h) {
+static void check_nan(int nan) {
+    ARH_CHECK(!nan, ARH_ENAN, "NaN in a dense near-field block (a collocation point coincides with a quadrature point)");
+}
+
+// Low-rank blocks as the partition and max_rank fix them.
+static void lr_plan(arh_geom *g, int max_rank) {
+    if (g->lr_plan_rank == max_rank) return;
+    g->lr_plan_rank = -1;
+    hipStream_t s = g->ctx->stream;
+    const int na = g->na;
+    std::vector<LRBlock> lr(na, LRBlock{});
+    int64_t uo = 0, vo = 0, fo = 0;
+    for (int a = 0; a < na; a++) {
+        LRBlock &B = lr[a];
+        B.rs = g->lowrank[4 * a], B.re = g->lowrank[4 * a + 1], B.cs = g->lowrank[4 * a + 2];
+        B.ce = g->lowrank[4 * a + 3];
+        const int m = B.re - B.rs, n = B.ce - B.cs;
+        B.lim = std::max(0, std::min(max_rank, std::min(m - 1, n - 1)));
+        B.l0 = g->leaf_of[B.rs];
+        B.us_off = uo, B.vs_off = vo, B.flag_off = fo;
+        uo += (int64_t)m * B.lim, vo += (int64_t)B.lim * n, fo += m;
+    }
+    g->aca_u_total = uo, g->aca_v_total = vo, g->aca_f_total = fo;
+    // largest work first: the ACA cost grows like lim^2 (m + n)
+    std::vector<int> order(na);
+    std::vector<double> work(na);
+    for (int a = 0; a < na; a++) {
+        const LRBlock &B = lr[a];
+        const double mn = B.re - B.rs + B.ce - B.cs;
+        order[a] = a, work[a] = (double)B.lim * B.lim * mn + mn;
+    }
+    std::stable_sort(order.begin(), order.end(), [&](int x, int y) { return work[x] > work[y]; });
+    // blocks with m + n >= kAcaBigDim get a workgroup each (they lead the order, largest first);
+    // the rest one wavefront each
+    const auto big = [&](int x) { return lr[x].re - lr[x].rs + lr[x].ce - lr[x].cs >= kAcaBigDim; };
+    const auto mid = std::stable_partition(order.begin(), order.end(), big);
+    g->aca_nbig = (int)(mid - order.begin());
+    upload(g->d_lr0, lr, s);
+    upload(g->d_aca_order, order, s);
+    ARH_HIP(hipStreamSynchronize(s));  // the host vectors are freed on return
+    g->lr_plan_rank = max_rank;
+}
+
+// Dense panels, then the ACA: one wait for the device, with the ranks (and whether a dense entry was a NaN) in pinned
+// memory, before the factors' storage can be allocated.
+void assemble(arh_hmat *h) {
     arh_geom *g = h->g;
     hipStream_t s = g->ctx->stream;
+    const int na = g->na;
     h->dense.alloc(sizeof(double2) * std::max<int64_t>(1, g->dense_entries));
     DBuf flag;
     flag.alloc(sizeof(int));
@@ -537,116 +647,55 @@ void assemble_dense(arh_hmat *h) {
                            g->d_pcol_idx.as<int>(), g->tri.as<Tri>(), h->k, h->dense.as<double2>(), flag.as<int>());
         ARH_HIP(hipGetLastError());
     }
-    int nan = 0;
-    ARH_HIP(hipMemcpyAsync(&nan, flag.p, sizeof(int), hipMemcpyDeviceToHost, s));
-    ARH_HIP(hipStreamSynchronize(s));
-    ARH_CHECK(!nan, ARH_ENAN, "NaN in a dense near-field block (a collocation point coincides with a quadrature point)");
-}
-
-static void ensure_aca_scratch(arh_geom *g, int max_rank) {
-    if (g->scratch_rank == max_rank) return;
-    const int na = g->na;
-    g->lim.assign(na, 0);
-    g->us_off.assign(na, 0);
-    g->vs_off.assign(na, 0);
-    g->flag_off.assign(na, 0);
-    int64_t uo = 0, vo = 0, fo = 0;
-    for (int a = 0; a < na; a++) {
-        int m = g->lowrank[4 * a + 1] - g->lowrank[4 * a], n = g->lowrank[4 * a + 3] - g->lowrank[4 * a + 2];
-        int lim = std::min(max_rank, std::min(m - 1, n - 1));
-        lim = std::max(lim, 0);
-        g->lim[a] = lim;
-        g->us_off[a] = uo, g->vs_off[a] = vo, g->flag_off[a] = fo;
-        uo += (int64_t)m * lim, vo += (int64_t)lim * n, fo += m;
-    }
-    g->aca_U.alloc(sizeof(double2) * std::max<int64_t>(1, uo));
-    g->aca_V.alloc(sizeof(double2) * std::max<int64_t>(1, vo));
-    g->aca_flags.alloc(std::max<int64_t>(16, fo));
-    g->aca_u_total = uo, g->aca_v_total = vo, g->aca_f_total = fo;
-    g->scratch_rank = max_rank;
-}
-
-void assemble_aca(arh_hmat *h) {
-    arh_geom *g = h->g;
-    hipStream_t s = g->ctx->stream;
-    const int na = g->na;
-    h->hblocks.assign(na, LRBlock{});
-    h->active_lr.clear();
+    h->ranks.clear();
+    h->n_active = 0;
     h->u_total = h->v_total = h->t_total = 0;
-    if (na == 0) return;
-    ARH_CHECK(h->max_rank <= kMaxRankLds, ARH_EINVAL, "max_rank above the supported 128");
-    ensure_aca_scratch(g, h->max_rank);
-    for (int a = 0; a < na; a++) {
-        LRBlock &B = h->hblocks[a];
-        B.rs = g->lowrank[4 * a], B.re = g->lowrank[4 * a + 1], B.cs = g->lowrank[4 * a + 2];
-        B.ce = g->lowrank[4 * a + 3];
-        B.lim = g->lim[a];
-        B.l0 = g->leaf_of[B.rs];
-        B.us_off = g->us_off[a], B.vs_off = g->vs_off[a], B.flag_off = g->flag_off[a];
+    if (na == 0 || h->max_rank > kMaxRankLds) {
+        int nan = 0;
+        ARH_HIP(hipMemcpyAsync(&nan, flag.p, sizeof(int), hipMemcpyDeviceToHost, s));
+        ARH_HIP(hipStreamSynchronize(s));
+        check_nan(nan);
+        ARH_CHECK(na == 0, ARH_EINVAL, "max_rank above the supported 128");
+        if (h->storage == ARH_MIXED) make_fp32_copy(h);
+        return;
     }
-    std::vector<int> order;  // kept until the synchronisation below (the upload may read it late)
-    if (g->aca_order_rank != h->max_rank) {
-        order.resize(na);
-        for (int a = 0; a < na; a++) order[a] = a;
-        // largest work first: the ACA cost grows like lim^2 (m + n)
-        std::stable_sort(order.begin(), order.end(), [&](int x, int y) {
-            const LRBlock &X = h->hblocks[x], &Y = h->hblocks[y];
-            double wx = (double)X.lim * X.lim * (X.re - X.rs + X.ce - X.cs) + (X.re - X.rs + X.ce - X.cs);
-            double wy = (double)Y.lim * Y.lim * (Y.re - Y.rs + Y.ce - Y.cs) + (Y.re - Y.rs + Y.ce - Y.cs);
-            return wx > wy;
-        });
-        // blocks with m + n >= kAcaBigDim get a workgroup each (they lead the order, largest first);
-        // the rest one wavefront each
-        std::stable_partition(order.begin(), order.end(), [&](int x) {
-            const LRBlock &X = h->hblocks[x];
-            return X.re - X.rs + X.ce - X.cs >= kAcaBigDim;
-        });
-        int nbig = 0;
-        while (nbig < na && h->hblocks[order[nbig]].re - h->hblocks[order[nbig]].rs + h->hblocks[order[nbig]].ce -
-                                    h->hblocks[order[nbig]].cs >=
-                                kAcaBigDim)
-            nbig++;
-        upload(g->d_aca_order, order, s);
-        g->aca_nbig = nbig;
-        g->aca_order_rank = h->max_rank;
-    }
+    lr_plan(g, h->max_rank);
+    // scratch from the device memory cache; it goes back there on return, so an idle geometry holds none
+    DBuf us, vs, used, ranks, active;
+    us.alloc(sizeof(double2) * std::max<int64_t>(1, g->aca_u_total));
+    vs.alloc(sizeof(double2) * std::max<int64_t>(1, g->aca_v_total));
+    used.alloc(std::max<int64_t>(16, g->aca_f_total));
+    ranks.alloc(sizeof(int2) * (size_t)na);
+    active.alloc(sizeof(int) * (size_t)na);
+    h->blocks.alloc(sizeof(LRBlock) * (size_t)na);
+    HostBuf hb(sizeof(LrTotals) + sizeof(int2) * (size_t)na, s);
+    LrTotals *tot = hb.as<LrTotals>();
+    int2 *hranks = (int2 *)(tot + 1);
     const int nbig = g->aca_nbig;
-    upload(h->blocks, h->hblocks, s);
     const int grid = nbig + (na - nbig + kAcaWaves - 1) / kAcaWaves;
-    hipLaunchKernelGGL(k_aca, dim3(grid), dim3(kAcaThreads), 0, s, h->blocks.as<LRBlock>(), g->d_aca_order.as<int>(),
-                       nbig, na, g->tri.as<Tri>(), h->k, h->aca_tol, g->aca_U.as<double2>(), g->aca_V.as<double2>(),
-                       g->aca_flags.as<unsigned char>());
+    hipLaunchKernelGGL(k_aca, dim3(grid), dim3(kAcaThreads), 0, s, g->d_lr0.as<LRBlock>(), g->d_aca_order.as<int>(), nbig,
+                       na, g->tri.as<Tri>(), h->k, h->aca_tol, us.as<double2>(), vs.as<double2>(),
+                       used.as<unsigned char>(), flag.as<int>(), ranks.as<int2>());
+    hipLaunchKernelGGL(k_lr_offsets, dim3((na + 1023) / 1024), dim3(1024), 0, s, na, g->d_lr0.as<LRBlock>(),
+                       ranks.as<int2>(), flag.as<int>(), h->blocks.as<LRBlock>(), active.as<int>(), hranks, tot);
     ARH_HIP(hipGetLastError());
-    ARH_HIP(hipMemcpyAsync(h->hblocks.data(), h->blocks.p, sizeof(LRBlock) * na, hipMemcpyDeviceToHost, s));
     ARH_HIP(hipStreamSynchronize(s));
-    int64_t uo = 0, vo = 0, to = 0;
-    for (int a = 0; a < na; a++) {
-        LRBlock &B = h->hblocks[a];
-        B.u_off = uo, B.v_off = vo, B.t_off = to;
-        uo += (int64_t)B.rank * (B.re - B.rs);
-        vo += (int64_t)B.rank * (B.ce - B.cs);
-        to += B.rank;
-        if (B.rank > 0) h->active_lr.push_back(a);
-    }
-    h->u_total = uo, h->v_total = vo, h->t_total = to;
-    upload(h->blocks, h->hblocks, s);
-    upload(h->d_active_lr, h->active_lr, s);
-    h->U.alloc(sizeof(double2) * std::max<int64_t>(1, uo));
-    h->V.alloc(sizeof(double2) * std::max<int64_t>(1, vo));
-    if (!h->active_lr.empty()) {
-        hipLaunchKernelGGL(k_pack, dim3((unsigned)h->active_lr.size(), kPackSplit), dim3(256), 0, s,
-                           h->blocks.as<LRBlock>(), h->d_active_lr.as<int>(), g->d_leaf_start.as<int>(),
-                           g->d_leaf_of.as<int>(), g->aca_U.as<double2>(), g->aca_V.as<double2>(), h->U.as<double2>(),
-                           h->V.as<double2>());
+    check_nan(tot->nan);
+    h->u_total = tot->u, h->v_total = tot->v, h->t_total = tot->t;
+    h->n_active = tot->nact;
+    h->U.alloc(sizeof(double2) * std::max<int64_t>(1, h->u_total));
+    h->V.alloc(sizeof(double2) * std::max<int64_t>(1, h->v_total));
+    h->d_active_lr.alloc(sizeof(int) * (size_t)h->n_active);
+    if (h->n_active) {
+        hipLaunchKernelGGL(k_pack, dim3((unsigned)h->n_active, kPackSplit), dim3(256), 0, s, h->blocks.as<LRBlock>(),
+                           active.as<int>(), g->d_leaf_start.as<int>(), g->d_leaf_of.as<int>(), us.as<double2>(),
+                           vs.as<double2>(), h->U.as<double2>(), h->V.as<double2>());
         ARH_HIP(hipGetLastError());
+        ARH_HIP(hipMemcpyAsync(h->d_active_lr.p, active.p, sizeof(int) * (size_t)h->n_active, hipMemcpyDeviceToDevice, s));
     }
-    ARH_HIP(hipStreamSynchronize(s));
-    // the scratch goes back to the device memory cache (the next assembly takes it from there), so an
-    // idle geometry holds no ACA scratch
-    g->aca_U.reset();
-    g->aca_V.reset();
-    g->aca_flags.reset();
-    g->scratch_rank = -1;
+    // while the factors are packed
+    h->ranks.assign(hranks, hranks + na);
+    if (h->storage == ARH_MIXED) make_fp32_copy(h);
 }
 
 // FP32 copy for the generic (non-MFMA) product: dense panels and U elementwise, V column-major
@@ -666,8 +715,8 @@ void make_generic_fp32(arh_hmat *h) {
     conv(h->dense, h->dense32, g->dense_entries);
     conv(h->U, h->U32, h->u_total);
     h->V32.alloc(sizeof(float2) * std::max<int64_t>(1, h->v_total));
-    if (!h->active_lr.empty()) {
-        hipLaunchKernelGGL(k_v_to_c64_cm, dim3((unsigned)h->active_lr.size()), dim3(256), 0, s, h->blocks.as<LRBlock>(),
+    if (h->n_active) {
+        hipLaunchKernelGGL(k_v_to_c64_cm, dim3((unsigned)h->n_active), dim3(256), 0, s, h->blocks.as<LRBlock>(),
                            h->d_active_lr.as<int>(), h->V.as<double2>(), h->V32.as<float2>());
         ARH_HIP(hipGetLastError());
     }

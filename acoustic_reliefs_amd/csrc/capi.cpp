@@ -306,7 +306,7 @@ static void fill_info(arh_hmat *h) {
     I.lowrank_entries = h->u_total + h->v_total;
     I.max_rank = 0;
     I.sum_rank = 0;
-    for (auto &B : h->hblocks) I.max_rank = std::max(I.max_rank, B.rank_ref), I.sum_rank += B.rank;
+    for (const int2 &r : h->ranks) I.max_rank = std::max(I.max_rank, r.y), I.sum_rank += r.x;
     I.bytes_fp64 = (int64_t)sizeof(double2) * (g->dense_entries + h->u_total + h->v_total);
     I.bytes_fp32 = (int64_t)(h->dense32.bytes + h->denseT32.bytes + h->U32.bytes + h->V32.bytes);
     int64_t fp64_extra = (int64_t)h->denseT.bytes;
@@ -333,9 +333,7 @@ int arh_hmat_assemble(arh_geom *g, double k, double aca_tol, int max_rank, int s
         ARH_HIP(hipEventCreate(&e0));
         ARH_HIP(hipEventCreate(&e1));
         ARH_HIP(hipEventRecord(e0, g->ctx->stream));
-        assemble_dense(h.get());
-        assemble_aca(h.get());
-        if (storage == ARH_MIXED) make_fp32_copy(h.get());
+        assemble(h.get());
         ARH_HIP(hipEventRecord(e1, g->ctx->stream));
         ARH_HIP(hipEventSynchronize(e1));
         float ms = 0;
@@ -359,7 +357,7 @@ int arh_hmat_get_info(const arh_hmat *h, arh_hmat_info *info) {
 int arh_hmat_ranks(const arh_hmat *h, int *ranks) {
     return guard(nullptr, [&] {
         ARH_CHECK(h && ranks, ARH_EINVAL, "NULL argument");
-        for (size_t a = 0; a < h->hblocks.size(); a++) ranks[a] = h->hblocks[a].rank_ref;
+        for (size_t a = 0; a < h->ranks.size(); a++) ranks[a] = h->ranks[a].y;
     });
 }
 
@@ -385,7 +383,9 @@ int arh_hmat_factors(const arh_hmat *h, int a, double *U, double *V, int *rank) 
         arh_geom *g = h->g;
         ARH_CHECK(a >= 0 && a < g->na, ARH_EINVAL, "low-rank block index out of range");
         set_device(g->ctx);
-        const LRBlock &B = h->hblocks[a];
+        LRBlock B;
+        ARH_HIP(hipMemcpyAsync(&B, h->blocks.as<LRBlock>() + a, sizeof(LRBlock), hipMemcpyDeviceToHost, g->ctx->stream));
+        ARH_HIP(hipStreamSynchronize(g->ctx->stream));
         const int m = B.re - B.rs, n = B.ce - B.cs, r = B.rank;
         *rank = r;
         if (!U || !V) return;

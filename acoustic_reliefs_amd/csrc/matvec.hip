@@ -271,7 +271,7 @@ static void apply_t(arh_hmat *h, int transpose, int R, const S *panel, const S *
     const int N = g->N;
     h->tbuf.alloc(sizeof(double2) * std::max<int64_t>(1, h->t_total * R));
     double2 *t = h->tbuf.as<double2>();
-    const int nact = (int)h->active_lr.size();
+    const int nact = h->n_active;
     const double es = (double)sizeof(S), vs = 16.0 * R;
     const int64_t lr_entries = transpose ? h->u_total : h->v_total;   // phase-1 factor
     const int64_t rw_entries = g->dense_entries + (transpose ? h->v_total : h->u_total);

@@ -166,14 +166,14 @@ static void build_units64(arh_hmat *h, hipStream_t s) {
         const int ncol = g->pcol_ptr[l + 1] - g->pcol_ptr[l];
         for (int c0 = 0; c0 < ncol; c0 += kUnitCols) h->mv_units.push_back(MvUnit{l, 0, -1, c0, std::min(kUnitCols, ncol - c0)});
         for (int e = g->lrR_ptr[l]; e < g->lrR_ptr[l + 1]; e++) {
-            const int b = g->lrR_blk[e], r = h->hblocks[b].rank;
+            const int b = g->lrR_blk[e], r = h->ranks[b].x;
             for (int c0 = 0; c0 < r; c0 += kUnitCols) h->mv_units.push_back(MvUnit{l, 1, b, c0, std::min(kUnitCols, r - c0)});
         }
         h->mv_uptr[l + 1] = (int)h->mv_units.size();
     }
     h->p1units64.clear();
-    for (int a : h->active_lr)
-        for (int q = 0; q * 4 < h->hblocks[a].rank; q++) h->p1units64.push_back(int2{a, q});
+    for (int a = 0; a < g->na; a++)
+        for (int q = 0; q * 4 < h->ranks[a].x; q++) h->p1units64.push_back(int2{a, q});
     upload(h->d_mv_units, h->mv_units, s);
     upload(h->d_mv_uptr, h->mv_uptr, s);
     upload(h->d_p1units64, h->p1units64, s);

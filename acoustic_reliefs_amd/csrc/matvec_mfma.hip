@@ -27,6 +27,8 @@
 // Lane layouts (64 lanes, 16x16x4): A[i][k] in lane i + 16 k, B[k][j] in lane j + 16 k; D[i][j] in
 // lane j + 16 (i / 4), element i % 4 for f32, lane j + 16 (i % 4), element i / 4 for f64.
 #include <algorithm>
+#include <memory>
+#include <type_traits>
 #include <unordered_map>
 
 #include "arh_internal.h"
@@ -604,7 +606,9 @@ __global__ __launch_bounds__(256) void k_fuse_panel(const int *__restrict__ leaf
                                                     const LeafPanel *__restrict__ lpanel,
                                                     const ColSrc *__restrict__ csrc, const double2 *__restrict__ dense,
                                                     const double2 *__restrict__ U, const double2 *__restrict__ V,
-                                                    typename Mfma<T>::T2 *__restrict__ panel) {
+                                                    typename Mfma<T>::T2 *__restrict__ panel,
+                                                    const int *__restrict__ bad) {
+    if (*bad) return;  // the lists are refused
     const int l = blockIdx.x;
     const int m = leaf_start[l + 1] - leaf_start[l];
     const LeafPanel L = lpanel[l];
@@ -635,8 +639,8 @@ __global__ __launch_bounds__(256) void k_fuse_panel(const int *__restrict__ leaf
 //              column-major block in its row leaf's panel, stride mr), then the V columns restricted to
 //              the leaf of each low-rank block whose column range covers it;
 // zero columns (source row 0, kind 0) up to the leaf's ncol. A list's column offsets are a wavefront
-// prefix sum of the entries' widths. bad[0] is raised when a column count disagrees with the host's
-// ncol, a source row falls outside [0, nsrc), or a low-rank block does not cover the leaf.
+// prefix sum of the entries' widths. bad[0], and hbad[0] in pinned memory, are raised when a column count disagrees
+// with the host's ncol, a source row falls outside [0, nsrc), or a low-rank block does not cover the leaf.
 __device__ __forceinline__ int wave_incl_scan(int v, int lane) {
 #pragma unroll
     for (int d = 1; d < ARH_WAVE; d <<= 1) {
@@ -652,7 +656,7 @@ __global__ __launch_bounds__(ARH_WAVE) void k_panel_cols(
     const int *__restrict__ dT_ptr, const int *__restrict__ dT_blk, const int *__restrict__ dblk_info,
     const int *__restrict__ lr_ptr, const int *__restrict__ lr_blk,
     const LRBlock *__restrict__ blocks, const int *__restrict__ t_row, int nsrc, int *__restrict__ psrc,
-    ColSrc *__restrict__ csrc, int *__restrict__ bad) {
+    ColSrc *__restrict__ csrc, int *__restrict__ bad, int *__restrict__ hbad) {
     const int l = blockIdx.x, lane = threadIdx.x;
     const int ls = leaf_start[l], m = leaf_start[l + 1] - ls;
     const LeafPanel L = lpanel[l];
@@ -716,7 +720,58 @@ __global__ __launch_bounds__(ARH_WAVE) void k_panel_cols(
         ps[c] = 0;
         cs[c] = ColSrc{0, 0, 0};
     }
-    if (!ok) atomicOr(bad, 1);
+    if (!ok) *bad = 1, *hbad = 1;  // every writer writes the same
+}
+
+// Where the stacks' members go, a wavefront per stack: the rows of a stack are its members' crosses in order, so a
+// member's first row is the sum of the ranks before it.
+__global__ __launch_bounds__(256) void k_stack_maps(int ns, const VStack *__restrict__ stacks, const int *__restrict__ ptr,
+                                                    const int *__restrict__ mem, const LRBlock *__restrict__ blocks,
+                                                    StackMap *__restrict__ maps, int *__restrict__ t_row) {
+    const int k = (int)blockIdx.x * 4 + threadIdx.x / ARH_WAVE, lane = threadIdx.x % ARH_WAVE;
+    if (k >= ns) return;
+    const VStack S = stacks[k];
+    int base = 0;
+    for (int q0 = ptr[k], q1 = ptr[k + 1]; q0 < q1; q0 += ARH_WAVE) {
+        const int q = q0 + lane, b = q < q1 ? mem[q] : 0, r = q < q1 ? blocks[b].rank : 0;
+        const int inc = wave_incl_scan(r, lane);
+        if (q < q1) {
+            const int o = base + inc - r;
+            maps[q] = StackMap{b, S.rtot, S.v_off + o};
+            t_row[b] = (int)(S.t_row + o);
+        }
+        base += __shfl(inc, ARH_WAVE - 1, ARH_WAVE);
+    }
+}
+
+// Low-rank blocks by the cluster that their stacked factor belongs to, fixed by the partition.
+static arh_geom_s::Clusters &clusters_of(arh_geom *g, int tr) {
+    arh_geom_s::Clusters &C = g->clusters[tr];
+    if (C.made) return C;
+    hipStream_t s = g->ctx->stream;
+    const int na = g->na, *lr = g->lowrank.data() + (tr ? 0 : 2);  // row or column range of block a: lr[4 a], lr[4 a + 1]
+    std::unordered_map<int64_t, int> id;
+    std::vector<int> of(na);
+    C.start.clear(), C.n.clear();
+    for (int a = 0; a < na; a++) {
+        const auto it = id.emplace(((int64_t)lr[4 * a] << 32) | (uint32_t)lr[4 * a + 1], (int)C.start.size());
+        if (it.second) C.start.push_back(lr[4 * a]), C.n.push_back(lr[4 * a + 1] - lr[4 * a]);
+        of[a] = it.first->second;
+    }
+    const int ns = (int)C.start.size();
+    C.ptr.assign(ns + 1, 0);
+    C.mem.resize(na);
+    for (int a = 0; a < na; a++) C.ptr[of[a] + 1]++;
+    for (int k = 0; k < ns; k++) C.ptr[k + 1] += C.ptr[k];
+    std::vector<int> fill(C.ptr.begin(), C.ptr.end() - 1);
+    for (int a = 0; a < na; a++) C.mem[fill[of[a]]++] = a;
+    C.by_size.resize(ns);
+    for (int k = 0; k < ns; k++) C.by_size[k] = k;
+    std::stable_sort(C.by_size.begin(), C.by_size.end(), [&](int p, int q) { return C.n[p] > C.n[q]; });
+    upload(C.d_ptr, C.ptr, s);
+    upload(C.d_mem, C.mem, s);
+    C.made = true;
+    return C;
 }
 
 // Work lists of one orientation, shared by both precisions (host + device copies).
@@ -725,83 +780,53 @@ __global__ __launch_bounds__(ARH_WAVE) void k_panel_cols(
 //  transposed: stacks of U^T by row cluster; panels of column leaves: the transposed dense blocks
 //              of the leaf, then the V columns (restricted to the leaf) of the low-rank blocks
 //              whose column range covers it.
-static void build_lists(arh_hmat *h, int tr) {
+// Returns the pinned block that the lists are uploaded from; its first int is raised by the device if the lists are not
+// to be used, which the caller asks after a synchronisation.
+static std::unique_ptr<HostBuf> build_lists(arh_hmat *h, int tr) {
     arh_geom *g = h->g;
     MfmaLayout &M = h->mf[tr];
     hipStream_t s = g->ctx->stream;
     const int N = g->N;
+    const int2 *rank = h->ranks.data();
     ARH_CHECK(g->max_leaf <= kMaxLeaf, ARH_EINVAL, "MFMA product supports leaves of at most 128 elements");
-    // stacks: active low-rank blocks grouped by their column (forward) / row (transposed) cluster,
-    // stacks in order of first appearance, members in active-block order
-    auto key = [&](const LRBlock &B) {
-        return tr ? ((int64_t)B.rs << 32) | (uint32_t)B.re : ((int64_t)B.cs << 32) | (uint32_t)B.ce;
-    };
-    const int nact = (int)h->active_lr.size();
-    std::unordered_map<int64_t, int> sid;
-    sid.reserve(2 * (size_t)nact + 1);
-    std::vector<int> bsid(nact), first;
-    for (int q = 0; q < nact; q++) {
-        auto it = sid.emplace(key(h->hblocks[h->active_lr[q]]), (int)first.size());
-        if (it.second) first.push_back(q);
-        bsid[q] = it.first->second;
-    }
-    const int ns = (int)first.size();
-    std::vector<int> mptr(ns + 1, 0), mem(nact);
-    for (int q = 0; q < nact; q++) mptr[bsid[q] + 1]++;
-    for (int k = 0; k < ns; k++) mptr[k + 1] += mptr[k];
-    {
-        std::vector<int> fill(mptr.begin(), mptr.end() - 1);
-        for (int q = 0; q < nact; q++) mem[fill[bsid[q]]++] = h->active_lr[q];
-    }
-    M.stacks.clear();
-    M.stacks.reserve(ns);
-    std::vector<StackMap> maps;
-    maps.reserve(nact);
-    std::vector<int> t_row(h->hblocks.size(), -1);
+    // stacks: the low-rank blocks grouped by their column (forward) / row (transposed) cluster
+    const arh_geom_s::Clusters &C = clusters_of(g, tr);
+    const int ns = (int)C.start.size();
+    std::vector<VStack> stacks(ns);
     int64_t voff = 0, trow = N;
+    size_t nsmall = 0, nbig = 0;
     for (int k = 0; k < ns; k++) {
-        const LRBlock &B0 = h->hblocks[mem[mptr[k]]];
-        VStack S{tr ? B0.rs : B0.cs, tr ? B0.re - B0.rs : B0.ce - B0.cs, 0, 0, voff, trow};
-        for (int q = mptr[k]; q < mptr[k + 1]; q++) S.rtot += h->hblocks[mem[q]].rank;
+        VStack S{C.start[k], C.n[k], 0, 0, voff, trow};
+        for (int q = C.ptr[k]; q < C.ptr[k + 1]; q++) S.rtot += rank[C.mem[q]].x;
         ARH_CHECK(trow + S.rtot < INT32_MAX, ARH_EINVAL, "stacked intermediates exceed the 32-bit row range");
-        int o = 0;
-        for (int q = mptr[k]; q < mptr[k + 1]; q++) {
-            const int a = mem[q];
-            maps.push_back(StackMap{a, S.rtot, voff + o});
-            t_row[a] = (int)(trow + o);
-            o += h->hblocks[a].rank;
-        }
-        M.stacks.push_back(S);
+        stacks[k] = S;
         voff += (int64_t)S.n * S.rtot;
         trow += S.rtot;
+        (S.n >= kBigCols ? nbig : nsmall) += (S.rtot + 31) / 32;
     }
     M.vs_total = voff;
     ARH_CHECK(trow - N == h->t_total, ARH_EINVAL, "stacked intermediates do not match the ranks");
     // phase-1 units: big stacks first, each list by decreasing column count
-    std::vector<int2> big, small;
-    for (int k = 0; k < (int)M.stacks.size(); k++)
-        for (int rt = 0; rt * 32 < M.stacks[k].rtot; rt++)
-            (M.stacks[k].n >= kBigCols ? big : small).push_back(int2{k, rt});
-    auto by_cols = [&](const int2 &p, const int2 &q) {
-        const int np = M.stacks[p.x].n, nq = M.stacks[q.x].n;
-        return np != nq ? np > nq : (p.x != q.x ? p.x < q.x : p.y < q.y);
-    };
-    std::sort(big.begin(), big.end(), by_cols);
-    std::sort(small.begin(), small.end(), by_cols);
-    M.p1big = (int)big.size();
-    M.p1units = big;
-    for (size_t q = 0; q < small.size();)
-        for (int w = 0; w < kLrWaves; w++)
-            M.p1units.push_back(w < kLrSmall && q < small.size() ? small[q++] : int2{-1, 0});
+    std::vector<int2> units(nbig + (nsmall + kLrSmall - 1) / kLrSmall * kLrWaves, int2{-1, 0});
+    size_t ub = 0, us = 0;
+    for (int k : C.by_size)
+        for (int rt = 0; rt * 32 < stacks[k].rtot; rt++) {
+            if (stacks[k].n >= kBigCols)
+                units[ub++] = int2{k, rt};
+            else
+                units[nbig + us / kLrSmall * kLrWaves + us % kLrSmall] = int2{k, rt}, us++;
+        }
+    M.p1big = (int)nbig;
+    M.nunits = (int)units.size();
     // fused panels: column counts here, the column lists on the device (k_panel_cols)
-    M.lpanel.assign(g->nleaf, LeafPanel{0, 0, 0});
+    std::vector<LeafPanel> lpanel(g->nleaf);
     int64_t poff = 0, ncols = 0;
     for (int l = 0; l < g->nleaf; l++) {
         const int ls = g->leaf_start[l], m = g->leaf_start[l + 1] - ls;
         int64_t nc = 0;
         if (!tr) {
             nc = g->pcol_ptr[l + 1] - g->pcol_ptr[l];
-            for (int e = g->lrR_ptr[l]; e < g->lrR_ptr[l + 1]; e++) nc += h->hblocks[g->lrR_blk[e]].rank;
+            for (int e = g->lrR_ptr[l]; e < g->lrR_ptr[l + 1]; e++) nc += rank[g->lrR_blk[e]].x;
         } else {
             for (int e = g->dT_ptr[l]; e < g->dT_ptr[l + 1]; e++) {
                 const int b = g->dT_blk[e], rl = g->dblk_leafr[b];
@@ -809,44 +834,29 @@ static void build_lists(arh_hmat *h, int tr) {
                           "dense block is not a leaf column");
                 nc += g->leaf_start[rl + 1] - g->leaf_start[rl];
             }
-            for (int e = g->lrC_ptr[l]; e < g->lrC_ptr[l + 1]; e++) nc += h->hblocks[g->lrC_blk[e]].rank;
+            for (int e = g->lrC_ptr[l]; e < g->lrC_ptr[l + 1]; e++) nc += rank[g->lrC_blk[e]].x;
         }
         nc = (nc + 3) / 4 * 4;
         ARH_CHECK(ncols + nc < INT32_MAX, ARH_EINVAL, "panel columns exceed the 32-bit range");
-        M.lpanel[l] = LeafPanel{poff, (int)ncols, (int)(nc / 4)};
+        lpanel[l] = LeafPanel{poff, (int)ncols, (int)(nc / 4)};
         ncols += nc;
         poff += nc * m;
     }
     M.panel_total = poff;
-    upload(M.d_lpanel, M.lpanel, s);
-    upload(M.d_trow, t_row, s);
-    M.d_psrc.alloc(sizeof(int) * std::max<int64_t>(1, ncols));
-    M.d_csrc.alloc(sizeof(ColSrc) * std::max<int64_t>(1, ncols));
-    DBuf bad;
-    bad.alloc(sizeof(int));
-    ARH_HIP(hipMemsetAsync(bad.p, 0, sizeof(int), s));
-    hipLaunchKernelGGL(k_panel_cols, dim3(g->nleaf), dim3(ARH_WAVE), 0, s, tr, M.d_lpanel.as<LeafPanel>(),
-                       g->d_leaf_start.as<int>(), g->d_pcol_ptr.as<int>(), g->d_panel_off.as<int64_t>(),
-                       g->d_pcol_idx.as<int>(), g->d_dT_ptr.as<int>(), g->d_dT_blk.as<int>(),
-                       g->d_dblk_info.as<int>(), tr ? g->d_lrC_ptr.as<int>() : g->d_lrR_ptr.as<int>(),
-                       tr ? g->d_lrC_blk.as<int>() : g->d_lrR_blk.as<int>(), h->blocks.as<LRBlock>(),
-                       M.d_trow.as<int>(), (int)(N + h->t_total), M.d_psrc.as<int>(), M.d_csrc.as<ColSrc>(),
-                       bad.as<int>());
-    ARH_HIP(hipGetLastError());
     // row tasks: leaves with more than tg groups are split evenly
     int64_t gt = 0;
-    for (auto &L : M.lpanel) gt += L.ngroups;
+    for (const LeafPanel &L : lpanel) gt += L.ngroups;
     int tg = (int)std::max<int64_t>(8 * kRowWaves, (gt + kTaskSlots - 1) / kTaskSlots);
     tg = (tg + kRowWaves - 1) / kRowWaves * kRowWaves;
-    M.rtasks.clear();
-    M.rsplit.clear();
+    std::vector<RowTask> rtasks;
+    std::vector<int4> rsplit;
     M.nslots = 0;
     for (int l = 0; l < g->nleaf; l++) {
-        const int n = M.lpanel[l].ngroups;
+        const int n = lpanel[l].ngroups;
         const int nt = std::max(1, (n + tg - 1) / tg);
-        if (nt > 1) M.rsplit.push_back(int4{l, M.nslots, nt, 0});
+        if (nt > 1) rsplit.push_back(int4{l, M.nslots, nt, 0});
         for (int t = 0; t < nt; t++)
-            M.rtasks.push_back(RowTask{l, (int)((int64_t)n * t / nt), (int)((int64_t)n * (t + 1) / nt),
+            rtasks.push_back(RowTask{l, (int)((int64_t)n * t / nt), (int)((int64_t)n * (t + 1) / nt),
                                        nt > 1 ? M.nslots + t : -1});
         if (nt > 1) M.nslots += nt;
     }
@@ -857,31 +867,61 @@ static void build_lists(arh_hmat *h, int tr) {
     if (kXcdOrder) {
         std::vector<std::vector<RowTask>> run(kXcds);
         int64_t acc = 0;
-        for (const RowTask &T : M.rtasks) {
+        for (const RowTask &T : rtasks) {
             const int x = (int)std::min<int64_t>(kXcds - 1, acc * kXcds / std::max<int64_t>(1, gt));
             run[x].push_back(T);
             acc += T.g1 - T.g0;
         }
         size_t len = 0;
         for (auto &r : run) len = std::max(len, r.size());
-        M.rtasks.assign(len * kXcds, RowTask{-1, 0, 0, -1});
+        rtasks.assign(len * kXcds, RowTask{-1, 0, 0, -1});
         for (int x = 0; x < kXcds; x++)
-            for (size_t i = 0; i < run[x].size(); i++) M.rtasks[i * kXcds + x] = run[x][i];
+            for (size_t i = 0; i < run[x].size(); i++) rtasks[i * kXcds + x] = run[x][i];
     } else {
-        std::stable_sort(M.rtasks.begin(), M.rtasks.end(),
+        std::stable_sort(rtasks.begin(), rtasks.end(),
                          [](const RowTask &p, const RowTask &q) { return p.g1 - p.g0 > q.g1 - q.g0; });
     }
-    upload(M.d_stacks, M.stacks, s);
-    upload(M.d_p1units, M.p1units, s);
-    upload(M.d_rtasks, M.rtasks, s);
-    upload(M.d_rsplit, M.rsplit, s);
-    upload(M.d_maps, maps, s);
-    M.nmaps = (int)maps.size();
-    int nbad = 0;
-    ARH_HIP(hipMemcpyAsync(&nbad, bad.p, sizeof(int), hipMemcpyDeviceToHost, s));
-    ARH_HIP(hipStreamSynchronize(s));  // the host vectors above are freed on return
-    ARH_CHECK(!nbad, ARH_EINVAL, "panel column lists disagree with the partition or the ranks");
-    M.lists = true;
+    M.ntasks = (int)rtasks.size();
+    M.nsplit = (int)rsplit.size();
+    // all lists in one block, one upload; in front of them the flag of the device's check
+    size_t total = 0;
+    auto room = [&](size_t bytes) {
+        const size_t o = total;
+        total += (bytes + 255) / 256 * 256;
+        return o;
+    };
+    auto bytes_of = [](const auto &v) { return v.size() * sizeof(v[0]); };
+    const size_t o_bad = room(sizeof(int)), o_st = room(bytes_of(stacks)), o_un = room(bytes_of(units)),
+                 o_lp = room(bytes_of(lpanel)), o_rt = room(bytes_of(rtasks)), o_rs = room(bytes_of(rsplit));
+    auto hb = std::make_unique<HostBuf>(total, s);
+    M.d_lists.alloc(total);
+    char *hp = hb->as<char>(), *dp = M.d_lists.as<char>();
+    auto put = [&](size_t o, const auto &v) { std::copy(v.begin(), v.end(), (std::decay_t<decltype(v[0])> *)(hp + o)); };
+    *(int *)(hp + o_bad) = 0;
+    put(o_st, stacks), put(o_un, units), put(o_lp, lpanel), put(o_rt, rtasks), put(o_rs, rsplit);
+    M.bad = (const int *)(dp + o_bad);
+    M.stacks = (const VStack *)(dp + o_st), M.p1units = (const int2 *)(dp + o_un);
+    M.lpanel = (const LeafPanel *)(dp + o_lp), M.rtasks = (const RowTask *)(dp + o_rt);
+    M.rsplit = (const int4 *)(dp + o_rs);
+    ARH_HIP(hipMemcpyAsync(dp, hp, total, hipMemcpyHostToDevice, s));
+    // the lists that follow from these on the device
+    M.nmaps = g->na;
+    M.d_maps.alloc(sizeof(StackMap) * std::max(1, M.nmaps));
+    M.d_trow.alloc(sizeof(int) * std::max(1, M.nmaps));
+    M.d_psrc.alloc(sizeof(int) * std::max<int64_t>(1, ncols));
+    M.d_csrc.alloc(sizeof(ColSrc) * std::max<int64_t>(1, ncols));
+    if (ns)
+        hipLaunchKernelGGL(k_stack_maps, dim3((ns + 3) / 4), dim3(256), 0, s, ns, M.stacks, C.d_ptr.as<int>(),
+                           C.d_mem.as<int>(), h->blocks.as<LRBlock>(), M.d_maps.as<StackMap>(), M.d_trow.as<int>());
+    hipLaunchKernelGGL(k_panel_cols, dim3(g->nleaf), dim3(ARH_WAVE), 0, s, tr, M.lpanel, g->d_leaf_start.as<int>(),
+                       g->d_pcol_ptr.as<int>(), g->d_panel_off.as<int64_t>(), g->d_pcol_idx.as<int>(),
+                       g->d_dT_ptr.as<int>(), g->d_dT_blk.as<int>(), g->d_dblk_info.as<int>(),
+                       tr ? g->d_lrC_ptr.as<int>() : g->d_lrR_ptr.as<int>(),
+                       tr ? g->d_lrC_blk.as<int>() : g->d_lrR_blk.as<int>(), h->blocks.as<LRBlock>(), M.d_trow.as<int>(),
+                       (int)(N + h->t_total), M.d_psrc.as<int>(), M.d_csrc.as<ColSrc>(), (int *)(dp + o_bad),
+                       (int *)(hp + o_bad));
+    ARH_HIP(hipGetLastError());
+    return hb;
 }
 
 // The operator copy of one orientation and precision (0: FP32, 1: FP64) in the MFMA layout.
@@ -904,21 +944,25 @@ static void build_copy(arh_hmat *h, int tr, int pi) {
                                g->d_leaf_of.as<int>(), M.vs[pi].as<T2>());
     }
     hipLaunchKernelGGL(k_fuse_panel<T>, dim3(g->nleaf, kFuseSplit), dim3(256), 0, s, g->d_leaf_start.as<int>(),
-                       M.d_lpanel.as<LeafPanel>(), M.d_csrc.as<ColSrc>(), h->dense.as<double2>(), h->U.as<double2>(),
-                       h->V.as<double2>(), M.panel[pi].as<T2>());
+                       M.lpanel, M.d_csrc.as<ColSrc>(), h->dense.as<double2>(), h->U.as<double2>(),
+                       h->V.as<double2>(), M.panel[pi].as<T2>(), M.bad);
     ARH_HIP(hipGetLastError());
-    ARH_HIP(hipStreamSynchronize(s));
-    M.built[pi] = true;
 }
 
 void mfma_prepare(arh_hmat *h, int tr, int fp64) {
     MfmaLayout &M = h->mf[tr];
-    if (!M.lists) build_lists(h, tr);
     if (M.built[fp64]) return;
+    std::unique_ptr<HostBuf> up;
+    if (!M.lists) up = build_lists(h, tr);
     if (fp64)
         build_copy<double>(h, tr, 1);
     else
         build_copy<float>(h, tr, 0);
+    if (up) {
+        ARH_HIP(hipStreamSynchronize(h->g->ctx->stream));
+        ARH_CHECK(!*up->as<int>(), ARH_EINVAL, "panel column lists disagree with the partition or the ranks");
+    }
+    M.lists = M.built[fp64] = true;
 }
 
 // Widest pass (NT output tiles) that fits the registers with 4 row tiles (leaves over 32 elements) and with
@@ -968,7 +1012,7 @@ static void launch_nt(arh_hmat *h, MfmaLayout &M, int R, const double2 *x, doubl
     // -x/2 term and the FP64 y write (16 B per rhs per element) in phase 2. Partial tiles of split
     // leaves and re-reads are not algorithmic.
     const double eb = 2.0 * sizeof(T);
-    const int nu = (int)M.p1units.size(), nb = M.p1big;
+    const int nu = M.nunits, nb = M.p1big;
     const bool narrow = R <= kNarrow;
     // phase-1 entries: V (forward) or U (transposed); both total sum_b r_b (m_b or n_b)
     const int64_t e1 = M.vs_total;
@@ -976,7 +1020,7 @@ static void launch_nt(arh_hmat *h, MfmaLayout &M, int R, const double2 *x, doubl
         timed(pi ? PROF_LR64 : PROF_LR32, eb * e1 + eb * R * (N + h->t_total), 8.0 * R * e1, [&] {
             auto launch_lr = [&](auto kern) {
                 hipLaunchKernelGGL(kern, dim3(nb + (nu - nb + kLrWaves - 1) / kLrWaves), dim3(64 * kLrWaves), 0, s,
-                                   M.d_stacks.as<VStack>(), M.d_p1units.as<int2>(), nb, nu, M.vs[pi].as<T2>(), xt, R,
+                                   M.stacks, M.p1units, nb, nu, M.vs[pi].as<T2>(), xt, R,
                                    gate);
             };
             if constexpr (NT == 1)
@@ -985,13 +1029,13 @@ static void launch_nt(arh_hmat *h, MfmaLayout &M, int R, const double2 *x, doubl
         });
     const int64_t ent = g->dense_entries + (h->u_total + h->v_total - e1);
     T *part = M.nslots ? M.part[pi].as<T>() : nullptr;
-    const int ntask = (int)M.rtasks.size(), nsp = (int)M.rsplit.size();
+    const int ntask = M.ntasks, nsp = M.nsplit;
     const double *xd = (const double *)x;
     double *yd = (double *)y;
     timed(pi ? PROF_ROWS64 : PROF_ROWS32, eb * ent + eb * R * (N + h->t_total) + 32.0 * R * N, 8.0 * R * ent, [&] {
         auto launch_rows = [&](auto kern) {
-            hipLaunchKernelGGL(kern, dim3(ntask), dim3(64 * kRowWaves), 0, s, M.d_rtasks.as<RowTask>(),
-                               g->d_leaf_start.as<int>(), M.d_lpanel.as<LeafPanel>(), M.d_psrc.as<int>(),
+            hipLaunchKernelGGL(kern, dim3(ntask), dim3(64 * kRowWaves), 0, s, M.rtasks,
+                               g->d_leaf_start.as<int>(), M.lpanel, M.d_psrc.as<int>(),
                                M.panel[pi].as<T2>(), (const T2 *)xt, xd, N, R, yd, cols, j0, gate, part, prow);
         };
         if constexpr (NT == 1)
@@ -1015,7 +1059,7 @@ static void launch_nt(arh_hmat *h, MfmaLayout &M, int R, const double2 *x, doubl
     });
     if (nsp)
         hipLaunchKernelGGL((k_rows_sum<T, NT>), dim3(nsp, (g->max_leaf + kSumRows - 1) / kSumRows), dim3(256), 0, s,
-                           M.d_rsplit.as<int4>(), g->d_leaf_start.as<int>(), part, xd, N, R, yd, cols, j0, gate, prow);
+                           M.rsplit, g->d_leaf_start.as<int>(), part, xd, N, R, yd, cols, j0, gate, prow);
     ARH_HIP(hipGetLastError());
 }
 
