@@ -80,8 +80,7 @@ class ReliefBEM:
             H = self.g.assemble(k, self.aca_tol, 100, self.storage)
             info = H.info()
             B = self.g.rhs(k, capi.ARH_RHS_PLANE, self.dirs)
-            Bn = B.numpy()
-            B.upload(-Bn)
+            self.ctx.scale(B, -1.0)  # M x - x/2 = -b
             X = self.ctx.empty((R, self.g.N))
             st = H.solve(B, X, R, tol=self.tol, true_residual=True)
             t0 = time.perf_counter()

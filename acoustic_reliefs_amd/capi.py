@@ -110,6 +110,7 @@ SIGNATURES = [
     ("arh_solve", c_int, [c_void_p, c_int, c_int, c_void_p, c_void_p, ctypes.POINTER(SolveOpts),
                           ctypes.POINTER(SolveStats)]),
     ("arh_rhs", c_int, [c_void_p, c_double, c_int, c_int, P_D, c_void_p]),
+    ("arh_scale", c_int, [c_void_p, ctypes.c_int64, c_double, c_void_p]),
     ("arh_receivers", c_int, [c_void_p, c_double, P_D, c_int, c_int, c_int, c_void_p, c_void_p]),
     ("arh_receivers_noalloc", c_int, [c_void_p, c_double, P_D, c_int, c_int, c_int, c_void_p, c_void_p]),
     ("arh_relief_create", c_int, [c_void_p, P_D, c_int, c_int, c_int, ctypes.POINTER(c_void_p)]),
@@ -261,6 +262,11 @@ class Context:
         d = DeviceArray(self, a.shape, a.dtype)
         d.upload(a)
         return d
+
+    def scale(self, a, f):
+        """a *= f on the device (complex128 DeviceArray)."""
+        assert a.dtype == np.complex128, a.dtype
+        _check(lib().arh_scale(self.h, a.nbytes // 16, float(f), c_void_p(a.ptr)), self.h)
 
     def diffusion(self, y, LL, nrhs, want_u=False, want_vf=False):
         d = np.zeros(nrhs)

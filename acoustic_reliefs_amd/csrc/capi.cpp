@@ -591,6 +591,15 @@ void arh_relief_destroy(arh_relief *r) {
     ctx_release(ctx);
 }
 
+int arh_scale(arh_ctx *ctx, int64_t n, double f, double *a) {
+    return guard(ctx, [&] {
+        ARH_CHECK(ctx && a, ARH_EINVAL, "NULL argument");
+        ARH_CHECK(n >= 0, ARH_EINVAL, "n must be >= 0");
+        set_device(ctx);
+        launch_scale(ctx->stream, (double2 *)a, n, f);
+    });
+}
+
 int arh_diffusion(arh_ctx *ctx, int LL, int nrhs, const double *y, double *d, double *u, double *vf) {
     return guard(ctx, [&] {
         ARH_CHECK(ctx && y && d, ARH_EINVAL, "NULL argument");

@@ -488,10 +488,7 @@ private:
         DevBuf b(ctx_->c, sizeof(cd) * N);
         auto x = std::make_shared<DevBuf>(ctx_->c, sizeof(cd) * N);
         check(arh_rhs(m.g, k, ARH_RHS_POINT, 1, src_.data(), b.d()), ctx_->c);
-        std::vector<cd> hb(N);
-        b.down(hb.data(), sizeof(cd) * N);
-        for (auto &v : hb) v = -v;
-        b.up(hb.data(), sizeof(cd) * N);
+        check(arh_scale(ctx_->c, N, -1.0, b.d()), ctx_->c);
         arh_solve_opts o = opts(actual);
         arh_solve_stats st{};
         int rc = arh_solve(h, 0, 1, b.d(), x->d(), &o, &st);
@@ -660,10 +657,7 @@ py::array_t<cd> sphere(const std::string &path, double freq, int LL, double lrad
         DevBuf b(ctx->c, sizeof(cd) * N), x(ctx->c, sizeof(cd) * N), yd(ctx->c, sizeof(cd) * LL);
         const double dir[3] = {1.0, 0.0, 0.0};
         check(arh_rhs(m->g, k, ARH_RHS_PLANE, 1, dir, b.d()), ctx->c);
-        std::vector<cd> hb(N);
-        b.down(hb.data(), sizeof(cd) * N);
-        for (auto &v : hb) v = -v;
-        b.up(hb.data(), sizeof(cd) * N);
+        check(arh_scale(ctx->c, N, -1.0, b.d()), ctx->c);
         arh_solve_opts o{};
         o.tol = actual ? 1e-13 : tols;
         o.true_residual = actual ? 1 : 0;

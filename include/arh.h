@@ -205,6 +205,8 @@ int arh_solve(arh_hmat *h, int transpose, int nrhs, const double *b, double *x, 
  * (kind PLANE), host arrays of 3*nrhs doubles. compute_G_r (helpers.cpp:46-50) / compute_b
  * (sphere.h:22-26). */
 int arh_rhs(arh_geom *g, double k, int kind, int nrhs, const double *vecs, double *b);
+/* a (device c128, n values) *= f, on the context's stream: the solves take -b (adjoint.cpp:95). */
+int arh_scale(arh_ctx *ctx, int64_t n, double f, double *a);
 
 /* y (device c128, nrhs x LL) = Q x with Q_lj = M(L_l, element j) computed exactly on the fly
  * (the dense listener matrix, integrate.cpp:46-57; the reference's default approximates it by
