@@ -286,6 +286,7 @@ struct arh_geom_s {
     arh_ctx *ctx = nullptr;
     int V = 0, N = 0;
     arh::DBuf P, E, tri;  // Ps (V x 3), Es (N x 3), Tri records
+    std::vector<int> hE;  // Es on the host
     // partition (host copies)
     std::vector<int> dense;    // nd x 4
     std::vector<int> lowrank;  // na x 4

@@ -239,9 +239,9 @@ int arh_geom_create(arh_ctx *ctx, const double *Ps, int V, const int *Es, int N,
         g->dense.assign(blocks, blocks + 4 * n_dense);
         g->lowrank.assign(blocks + 4 * n_dense, blocks + 4 * (n_dense + n_lowrank));
         std::vector<double> P(Ps, Ps + 3 * (size_t)V);
-        std::vector<int> E(Es, Es + 3 * (size_t)N);
+        g->hE.assign(Es, Es + 3 * (size_t)N);
         upload(g->P, P, ctx->stream);
-        upload(g->E, E, ctx->stream);
+        upload(g->E, g->hE, ctx->stream);
         geom_build_index(g.get());
         geom_build_tri(g.get());
         ARH_HIP(hipStreamSynchronize(ctx->stream));

@@ -42,10 +42,16 @@ namespace arh {
 // it needs 249 registers, 2 wavefronts per SIMD instead of 3, and 3-5 % more time; 4 wavefronts spill (+14 %).
 // N = 9,828 with 8,190 touched elements, 8e7 pairs: 3.1 ms for one right-hand side and 4.6 ms for 37, where
 // accumulating every right-hand side's sums per lane took 10.3 ms and 24.6 ms (two passes, each with its own
-// derivatives); 1297 listeners, one right-hand side: 0.24 ms from 2.6 ms.
+// derivatives); 1297 listeners, one right-hand side: 0.24 ms from 2.6 ms. With the pairs of touched elements taken
+// both ways at once (k_grad_both) the whole call goes from 3.27 to 2.15 ms and from 4.47 to 2.90 ms.
 constexpr int kGW = 4;           // wavefronts per workgroup; they take every kGW-th 16-column tile of the split
 constexpr int kGT = 64 * kGW;
 constexpr int kGSlots = 2048;    // workgroups aimed for (8 per compute unit): the column range is split to reach it
+
+// Blocks of touched elements from which their pairs are taken both ways at once: fewer leave the chip half empty (one rhs,
+// whole call, 17 blocks 371 us one way and 364 both ways, 12 blocks 283 and 327, 31 blocks 532 and 474).
+constexpr int kGMinBlocks = 20;
+constexpr int64_t kGMaxPart = int64_t(1) << 28;  // (block, touched element) partial sums: 6.4 GB
 
 typedef double V4d __attribute__((ext_vector_type(4)));
 
@@ -81,6 +87,20 @@ struct GradRow {
 };
 static_assert(sizeof(GradRow) % 16 == 8, "odd number of doubles");
 
+__device__ __forceinline__ void fill_row(GradRow &r, const Tri &t) {
+#pragma unroll
+    for (int g = 0; g < 6; g++) {
+        double wt, xi, eta;
+        quad_point(g, wt, xi, eta);
+        r.q[g][0] = t.ax + xi * t.bx + eta * t.cx;
+        r.q[g][1] = t.ay + xi * t.by + eta * t.cy;
+        r.q[g][2] = t.az + xi * t.bz + eta * t.cz;
+    }
+    r.ax = t.ax, r.ay = t.ay, r.az = t.az, r.nx = t.nx, r.ny = t.ny, r.nz = t.nz;
+    r.gx = t.gx, r.gy = t.gy, r.gz = t.gz;
+    r.bx = t.bx, r.bz = t.bz, r.cx = t.cx, r.cz = t.cz;
+}
+
 // Right-hand-side values element by element for the pair GEMMs: row e holds (re, im) of the R values of one vector
 // set, zero-padded to K = 4 ceil(R / 2) reals.
 __global__ void k_grad_pack(int N, int R, int K, const double2 *__restrict__ x, double *__restrict__ out) {
@@ -105,12 +125,12 @@ __device__ __forceinline__ void pair_gemm(const double *__restrict__ a, const do
     }
 }
 
-// Partial sums over a range of columns for 16 touched elements. Columns are elements (LISTEN false: B) or
-// listeners (LISTEN true: A); grid (row tiles, column splits); out[(split * T + t) * 3 + c]. xi, li: packed x and
+// Partial sums over a range of columns for 16 touched elements. Columns are elements (LISTEN false: B; cols: a list of
+// them, or null for all) or listeners (LISTEN true: A); grid (row tiles, column splits); out[(split * T + t) * 3 + c]. xi, li: packed x and
 // lambda by element; pc: the columns' packed values that multiply x_i (lambda by element, or vf by listener).
 template <bool LISTEN>
-__global__ __launch_bounds__(kGT, 3) void k_grad_pairs(const Tri *__restrict__ tri, const double *__restrict__ L, int ncol,
-                                                    int T, const int *__restrict__ touched, double k, int K,
+__global__ __launch_bounds__(kGT, 3) void k_grad_pairs(const Tri *__restrict__ tri, const double *__restrict__ L,
+                                                    const int *__restrict__ cols, int ncol, int T, const int *__restrict__ touched, double k, int K,
                                                     const double *__restrict__ xp, const double *__restrict__ lp,
                                                     const double *__restrict__ pc, int nsplit,
                                                     double *__restrict__ out) {
@@ -119,21 +139,8 @@ __global__ __launch_bounds__(kGT, 3) void k_grad_pairs(const Tri *__restrict__ t
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
     const int i16 = lane & 15, kk = lane >> 4;
     const int t0 = (int)blockIdx.x * 16, sp = blockIdx.y;
-    if (threadIdx.x < 16) {
-        const Tri t = tri[touched[min(t0 + (int)threadIdx.x, T - 1)]];  // surplus rows repeat the last, unused
-        GradRow &r = rows[threadIdx.x];
-#pragma unroll
-        for (int g = 0; g < 6; g++) {
-            double wt, xi, eta;
-            quad_point(g, wt, xi, eta);
-            r.q[g][0] = t.ax + xi * t.bx + eta * t.cx;
-            r.q[g][1] = t.ay + xi * t.by + eta * t.cy;
-            r.q[g][2] = t.az + xi * t.bz + eta * t.cz;
-        }
-        r.ax = t.ax, r.ay = t.ay, r.az = t.az, r.nx = t.nx, r.ny = t.ny, r.nz = t.nz;
-        r.gx = t.gx, r.gy = t.gy, r.gz = t.gz;
-        r.bx = t.bx, r.bz = t.bz, r.cx = t.cx, r.cz = t.cz;
-    }
+    if (threadIdx.x < 16)  // surplus rows repeat the last, unused
+        fill_row(rows[threadIdx.x], tri[touched[min(t0 + (int)threadIdx.x, T - 1)]]);
     const int64_t ei = touched[min(t0 + i16, T - 1)];  // the row whose packed values this lane feeds
     const double *xa = xp + ei * K, *la = LISTEN ? nullptr : lp + ei * K;
     __syncthreads();
@@ -141,7 +148,7 @@ __global__ __launch_bounds__(kGT, 3) void k_grad_pairs(const Tri *__restrict__ t
     const int ntile = (ncol + 15) >> 4;
     const int c0 = (int)((int64_t)ntile * sp / nsplit), c1 = (int)((int64_t)ntile * (sp + 1) / nsplit);
     for (int ct = c0 + w; ct < c1; ct += kGW) {
-        const int e = min(ct * 16 + i16, ncol - 1);
+        const int ec = min(ct * 16 + i16, ncol - 1), e = !LISTEN && cols ? cols[ec] : ec;
         const bool on = ct * 16 + i16 < ncol;  // surplus columns repeat the last, not added
         V4d gr = {0, 0, 0, 0}, gi = {0, 0, 0, 0}, hr = {0, 0, 0, 0}, hi = {0, 0, 0, 0};
         pair_gemm(xa, pc + (int64_t)e * K, K, kk, hr, hi);
@@ -225,6 +232,134 @@ __global__ __launch_bounds__(kGT, 3) void k_grad_pairs(const Tri *__restrict__ t
     }
 }
 
+// Pairs of touched elements, both ways at once. The distances between the collocation point of i and the rule points of e
+// serve dM_ie/dp_i (i's centroid moves, times G(i, e)) and dM_ie/dq_(e,c) (e's corners move, times the same G(i, e)), so
+// a pair {i, e} takes the twelve distances and the two products once where k_grad_pairs, for i and for e, takes them
+// twice. A workgroup takes a pair of blocks of kGB touched elements (grid: block b with the blocks b, b + 1, .. in
+// circular order, up to half of them, so each pair of blocks once), a wavefront 16 of the second block's elements as
+// columns; both blocks' geometry is in LDS. The two directions of a pair come one after the other, each with its own
+// product tile: with both tiles in registers at once the kernel spills at 3 wavefronts per SIMD (one rhs 2.4 ms, 37 3.4;
+// now 2.15 and 2.9, 159 registers; at 4 wavefronts 2.6 and 3.6). out[(o * T + t) * 3 + c]: the sum of element t with the elements of block o.
+constexpr int kGB = 64;
+static_assert(kGB == 16 * kGW, "a column tile per wavefront");
+
+// Pair of a collocation point p and a triangle, times g: the y derivative for p's centroid (o[3]) and for the
+// triangle's corners (o[0..2]).
+__device__ __forceinline__ void pair_side(double k, const GradRow &r, double px, double py, double pz, double g_r,
+                                          double g_i, double o[4]) {
+    double2 S0 = make_double2(0.0, 0.0), T0 = S0, T1 = S0, T2 = S0;
+#pragma unroll
+    for (int g = 0; g < 6; g++) {
+        double wt, xi, eta;
+        quad_point(g, wt, xi, eta);
+        double2 F, H;
+        FdF(k, px - r.q[g][0], py - r.q[g][1], pz - r.q[g][2], F, H);
+        const double w0 = wt * kInv8Pi;
+        S0.x = fma(w0, F.x, S0.x), S0.y = fma(w0, F.y, S0.y);
+        T0.x = fma(w0 * (1.0 - xi - eta), H.x, T0.x), T0.y = fma(w0 * (1.0 - xi - eta), H.y, T0.y);
+        T1.x = fma(w0 * xi, H.x, T1.x), T1.y = fma(w0 * xi, H.y, T1.y);
+        T2.x = fma(w0 * eta, H.x, T2.x), T2.y = fma(w0 * eta, H.y, T2.y);
+    }
+    const double ux = px - r.ax, uy = py - r.ay, uz = pz - r.az;
+    const double s = ux * r.nx + uy * r.ny + uz * r.nz;  // -s of the formulas above
+    const double E0 = r.ny - (ux * (r.bz - r.cz) - uz * (r.bx - r.cx));
+    const double E1 = uz * r.cx - ux * r.cz, E2 = ux * r.bz - uz * r.bx;
+    o[0] = (s * T0.x + E0 * S0.x) * g_r - (s * T0.y + E0 * S0.y) * g_i;
+    o[1] = (s * T1.x + E1 * S0.x) * g_r - (s * T1.y + E1 * S0.y) * g_i;
+    o[2] = (s * T2.x + E2 * S0.x) * g_r - (s * T2.y + E2 * S0.y) * g_i;
+    const double cr = s * (T0.x + T1.x + T2.x) + r.ny * S0.x, ci = s * (T0.y + T1.y + T2.y) + r.ny * S0.y;
+    o[3] = (ci * g_i - cr * g_r) * (1.0 / 3.0);
+}
+
+__global__ __launch_bounds__(kGT, 3) void k_grad_both(const Tri *__restrict__ tri, int T, const int *__restrict__ touched,
+                                                   double k, int K, const double *__restrict__ xp,
+                                                   const double *__restrict__ lp, double *__restrict__ out) {
+    __shared__ GradRow rows[2][kGB];
+    __shared__ double red[kGW][kGB][3];
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    const int i16 = lane & 15, kk = lane >> 4;
+    const int nb = gridDim.x, rb = blockIdx.x, cb = (rb + (int)blockIdx.y) % nb;
+    if (2 * (int)blockIdx.y == nb && 2 * rb >= nb) return;  // its partner has the pair
+    if (threadIdx.x < 2 * kGB) {  // surplus elements repeat the last, not added
+        const int b = threadIdx.x / kGB, i = threadIdx.x % kGB;
+        fill_row(rows[b][i], tri[touched[min((b ? cb : rb) * kGB + i, T - 1)]]);
+    }
+    __syncthreads();
+    const int u = cb * kGB + w * 16 + i16;
+    const bool on = u < T;
+    const int64_t e = touched[min(u, T - 1)];
+    const GradRow &ce = rows[1][w * 16 + i16];
+    double col[3] = {0.0, 0.0, 0.0};
+#pragma unroll 1
+    for (int rt = 0; rt < kGB / 16; rt++) {
+        const int t0 = rb * kGB + rt * 16;
+        const int64_t ei = touched[min(t0 + i16, T - 1)];
+        double acc[3] = {0.0, 0.0, 0.0};  // lane i16 = v holds row 4 v + kk
+#pragma unroll 1
+        for (int side = 0; side < 2; side++) {  // the column's triangle with G(i, e), then the row's with G(e, i)
+            V4d gr = {0, 0, 0, 0}, gi = {0, 0, 0, 0};
+            pair_gemm((side ? xp : lp) + ei * K, (side ? lp : xp) + e * K, K, kk, gr, gi);
+#pragma unroll 1
+            for (int v = 0; v < 4; v++) {
+                const GradRow &r = rows[0][rt * 16 + v * 4 + kk], &t = side ? r : ce, &p = side ? ce : r;
+                const bool both = on && t0 + v * 4 + kk < T;
+                double a[4];
+                pair_side(k, t, p.gx, p.gy, p.gz, gr[v], gi[v], a);
+#pragma unroll
+                for (int c = 0; c < 4; c++) a[c] = both ? a[c] : 0.0;
+                if (side) {
+#pragma unroll
+                    for (int c = 0; c < 3; c++) {
+                        const double o = row_sum(a[c]);
+                        col[c] += a[3];
+                        if (i16 == v) acc[c] += o;
+                    }
+                } else {
+                    const double o = row_sum(a[3]);
+#pragma unroll
+                    for (int c = 0; c < 3; c++) {
+                        col[c] += a[c];
+                        if (i16 == v) acc[c] += o;
+                    }
+                }
+            }
+        }
+        if (i16 < 4)
+#pragma unroll
+            for (int c = 0; c < 3; c++) red[w][rt * 16 + i16 * 4 + kk][c] = acc[c];
+    }
+    if (cb != rb) {  // a block with itself: every ordered pair has come by as row and column
+#pragma unroll
+        for (int c = 0; c < 3; c++) {
+            col[c] += __shfl_xor(col[c], 16, ARH_WAVE);
+            col[c] += __shfl_xor(col[c], 32, ARH_WAVE);
+        }
+        if (kk == 0 && on)
+#pragma unroll
+            for (int c = 0; c < 3; c++) out[((int64_t)rb * T + u) * 3 + c] = col[c];
+    }
+    __syncthreads();
+    if (threadIdx.x < 3 * kGB) {
+        const int r = (int)threadIdx.x / 3, c = (int)threadIdx.x % 3;
+        if (rb * kGB + r < T) {
+            double a = red[0][r][c];
+            for (int q = 1; q < kGW; q++) a += red[q][r][c];
+            out[((int64_t)cb * T + rb * kGB + r) * 3 + c] = a;
+        }
+    }
+}
+
+// Sums over the other blocks, in order.
+__global__ __launch_bounds__(256) void k_grad_blocks(int n3, int nb, const double *__restrict__ part,
+                                                     double *__restrict__ out) {
+    const int i = blockIdx.x * 256 + threadIdx.x;
+    if (i >= n3) return;
+    double a = 0.0;
+#pragma unroll 8
+    for (int o = 0; o < nb; o++) a += part[(int64_t)o * n3 + i];
+    out[i] = a;
+}
+
 // C per touched element (one thread each): -sum_rhs Re( lam_i db_i / dp_i ).
 __global__ __launch_bounds__(64) void k_grad_C(const Tri *__restrict__ tri, int N, int T,
                                                const int *__restrict__ touched, double k, int R,
@@ -293,24 +428,27 @@ void launch_shape_grad(arh_geom *g, double k, const double *L_dev, int LL, const
         ARH_CHECK(diff[h] >= 0 && diff[h] < V, ARH_EINVAL, "diff vertex id out of range");
         slot[diff[h]] = h;  // a repeated id keeps its last slot, as the reference's map assignment does
     }
-    std::vector<int> Eh(3 * (size_t)N);
-    ARH_HIP(hipMemcpyAsync(Eh.data(), g->E.p, sizeof(int) * 3 * N, hipMemcpyDeviceToHost, s));
-    ARH_HIP(hipStreamSynchronize(s));
-    std::vector<int> touched, tpos(N, -1);
-    std::vector<std::vector<int>> lists(HH);
-    for (int e = 0; e < N; e++)
+    const std::vector<int> &Eh = g->hE;
+    std::vector<int> touched, others, tpos(N, -1), hptr(HH + 1, 0);
+    for (int e = 0; e < N; e++) {
+        bool any = false;
         for (int c = 0; c < 3; c++) {
             const int h = slot[Eh[3 * e + c]];
-            if (h < 0) continue;
-            if (tpos[e] < 0) tpos[e] = (int)touched.size(), touched.push_back(e);
-            lists[h].push_back(tpos[e] * 3 + c);
+            if (h >= 0) any = true, hptr[h + 1]++;
         }
-    const int T = (int)touched.size();
-    std::vector<int> hptr(HH + 1, 0), hlist;
-    for (int h = 0; h < HH; h++) {
-        hlist.insert(hlist.end(), lists[h].begin(), lists[h].end());
-        hptr[h + 1] = (int)hlist.size();
+        if (any)
+            tpos[e] = (int)touched.size(), touched.push_back(e);
+        else
+            others.push_back(e);
     }
+    const int T = (int)touched.size();
+    for (int h = 0; h < HH; h++) hptr[h + 1] += hptr[h];
+    std::vector<int> hlist(hptr[HH]), fill(hptr.begin(), hptr.end() - 1);
+    for (int e : touched)
+        for (int c = 0; c < 3; c++) {
+            const int h = slot[Eh[3 * e + c]];
+            if (h >= 0) hlist[fill[h]++] = tpos[e] * 3 + c;
+        }
     if (T == 0 && G) return;  // nothing to add
     if (T == 0) {
         ARH_HIP(hipMemsetAsync(A, 0, sizeof(double) * HH, s));
@@ -325,14 +463,18 @@ void launch_shape_grad(arh_geom *g, double k, const double *L_dev, int LL, const
         const int most = std::max(1, (ncol + 16 * kGW - 1) / (16 * kGW));
         return std::max(1, std::min(most, (kGSlots + gx - 1) / gx));
     };
-    const int bsplit = splits(N), asplit = splits(LL);
+    // enough blocks of touched elements to fill the chip: their pairs both ways at once, then the other columns
+    const int nb = (T + kGB - 1) / kGB;
+    const bool both = nb >= kGMinBlocks && (int64_t)nb * T <= kGMaxPart;
+    const int ncol = both ? (int)others.size() : N;
+    const int bsplit = ncol ? splits(ncol) : 0, asplit = splits(LL), first = both ? 1 : 0;  // first: the blocks' sum
     const int K = 4 * ((nrhs + 1) / 2);
-    DBuf d_touched, d_hptr, d_hlist, pA, pB, cC, xp, lp, vp;
+    DBuf d_touched, d_others, d_hptr, d_hlist, pA, pB, pS, cC, xp, lp, vp;
     upload(d_touched, touched, s);
     upload(d_hptr, hptr, s);
     upload(d_hlist, hlist, s);
     pA.alloc(sizeof(double) * 3 * (size_t)T * asplit);
-    pB.alloc(sizeof(double) * 3 * (size_t)T * bsplit);
+    pB.alloc(sizeof(double) * 3 * (size_t)T * (first + bsplit));
     cC.alloc(sizeof(double) * T);
     auto pack = [&](DBuf &out, int n, const double2 *v) {
         out.alloc(sizeof(double) * (size_t)n * K);
@@ -342,15 +484,25 @@ void launch_shape_grad(arh_geom *g, double k, const double *L_dev, int LL, const
     pack(xp, N, x);
     pack(lp, N, lam);
     pack(vp, LL, vf);
-    hipLaunchKernelGGL(k_grad_pairs<false>, dim3(gx, bsplit), dim3(kGT), 0, s, g->tri.as<Tri>(),
-                       (const double *)nullptr, N, T, d_touched.as<int>(), k, K, xp.as<double>(), lp.as<double>(),
-                       lp.as<double>(), bsplit, pB.as<double>());
-    hipLaunchKernelGGL(k_grad_pairs<true>, dim3(gx, asplit), dim3(kGT), 0, s, g->tri.as<Tri>(), L_dev, LL, T,
-                       d_touched.as<int>(), k, K, xp.as<double>(), (const double *)nullptr, vp.as<double>(), asplit,
+    if (both) {
+        upload(d_others, others, s);
+        pS.alloc(sizeof(double) * 3 * (size_t)T * nb);
+        hipLaunchKernelGGL(k_grad_both, dim3(nb, nb / 2 + 1), dim3(kGT), 0, s, g->tri.as<Tri>(), T, d_touched.as<int>(), k,
+                           K, xp.as<double>(), lp.as<double>(), pS.as<double>());
+        hipLaunchKernelGGL(k_grad_blocks, dim3((3 * T + 255) / 256), dim3(256), 0, s, 3 * T, nb, pS.as<double>(),
+                           pB.as<double>());
+    }
+    if (bsplit)
+        hipLaunchKernelGGL(k_grad_pairs<false>, dim3(gx, bsplit), dim3(kGT), 0, s, g->tri.as<Tri>(),
+                           (const double *)nullptr, both ? d_others.as<int>() : nullptr, ncol, T, d_touched.as<int>(), k, K,
+                           xp.as<double>(), lp.as<double>(), lp.as<double>(), bsplit,
+                           pB.as<double>() + first * 3 * (size_t)T);
+    hipLaunchKernelGGL(k_grad_pairs<true>, dim3(gx, asplit), dim3(kGT), 0, s, g->tri.as<Tri>(), L_dev,
+                       (const int *)nullptr, LL, T, d_touched.as<int>(), k, K, xp.as<double>(), (const double *)nullptr, vp.as<double>(), asplit,
                        pA.as<double>());
     hipLaunchKernelGGL(k_grad_C, dim3((T + 63) / 64), dim3(64), 0, s, g->tri.as<Tri>(), N, T, d_touched.as<int>(), k,
                        nrhs, lam, src_kind, src_dev, cC.as<double>());
-    hipLaunchKernelGGL(k_grad_scatter, dim3((HH + 255) / 256), dim3(256), 0, s, HH, T, asplit, bsplit, d_hptr.as<int>(),
+    hipLaunchKernelGGL(k_grad_scatter, dim3((HH + 255) / 256), dim3(256), 0, s, HH, T, asplit, first + bsplit, d_hptr.as<int>(),
                        d_hlist.as<int>(), pA.as<double>(), pB.as<double>(), cC.as<double>(), A, B, C, G);
     ARH_HIP(hipGetLastError());
     ARH_HIP(hipStreamSynchronize(s));
