@@ -239,15 +239,16 @@ struct LeafPanel {
     int col0, ngroups;  // ngroups = ncol / 4
 };
 
-// MFMA product row task: column groups [g0, g1) of row leaf `leaf`; slot >= 0 names the task's
-// partial tile when the leaf is split over several tasks, -1 when the task writes y itself.
+// MFMA product row task: column groups [g0, g1) of row leaf `leaf`. A leaf split over ntask > 1 tasks has their
+// partial tiles from slot0 on, this task's at slot, and an arrival counter; slot is -1 when the task has the whole leaf.
 struct RowTask {
     int leaf, g0, g1, slot;
+    int slot0, ntask, count, pad;
 };
 
 // One orientation (forward or transposed) of the MFMA product: operator copies in their own layout
 // ([0] FP32, [1] FP64, each built on first use or at assembly), the packed rhs + intermediates
-// buffer ([x; t] rows), split leaves' partial tiles, and the shared work lists:
+// buffer ([x; t] rows), split leaves' partial tiles and arrival counters, and the shared work lists:
 // stacks, phase-1 units (stack, 32-row tile; stacks with many columns first, one workgroup each),
 // per-leaf panels and their source rows, row tasks, split leaves (leaf, first partial slot, task
 // count), layout builder maps.
@@ -263,6 +264,7 @@ struct MfmaLayout {
     const LeafPanel *lpanel = nullptr;
     const RowTask *rtasks = nullptr;
     const int4 *rsplit = nullptr;
+    int *count = nullptr;  // split leaves' arrivals, 0 between products
     int nunits = 0, p1big = 0, nmaps = 0, ntasks = 0, nsplit = 0, nslots = 0;
     int64_t panel_total = 0, vs_total = 0;
 };

@@ -312,7 +312,7 @@ __device__ __forceinline__ int3 wave_share(int n, int w) {
 // LDS of a reduction / output staging: W / 2 slots of NT * 256 values (one row tile each), and room for
 // PR x 16 NT values of an output tile.
 template <class T, int NT, int W, int PR = kPartRows>
-struct Lds {
+struct alignas(16) Lds {
     T v[std::max((W / 2) * NT * 256, PR * 16 * NT)];
 };
 
@@ -421,13 +421,77 @@ __global__ __launch_bounds__(64 * kLrWaves) void k_lr_mfma(const VStack *__restr
 // of the groups (wave_share) and the partial tiles are summed in a fixed order in LDS. A leaf with
 // a single task writes y = -x/2 + acc itself; the tasks of a split leaf write partial tiles that
 // k_rows_sum adds in task order. Output goes through LDS so that y rows are written contiguously.
+//
+// With narrow rows the last of a split leaf's tasks to finish adds the tiles up itself, in task order whichever task that
+// is, which saves a launch. The tiles pass between workgroups on dies with caches of their own: they are written and read
+// with agent-scope (write-through, cache-bypassing) accesses, and the arrival is counted after every wavefront's
+// stores are acknowledged, so neither side flushes or invalidates a cache. Whole product, one right-hand side: FP64 2000 Hz
+// 105.3 -> 101.6 us, FP64 leaves of 128 transposed 144.6 -> 135.2, FP32 4000 Hz 69.6 -> 67.0; four: 111.1 -> 109.6, 147.9
+// -> 148.1, 70.9 -> 68.2. From five on the tiles' round trip at the end of each task costs what the launch
+// did, and more as they grow (FP32 4000 Hz, 37: 158.6 -> 165.0), so the other kernels leave the sum to k_rows_sum.
+__device__ __forceinline__ void store_agent(uint64_t *p, uint64_t v) {
+    __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ uint64_t load_agent(const uint64_t *p) {
+    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// A split leaf's tile (in red) to its slot; true in every thread of the task that arrives last, with the leaf's sum in
+// red instead. Only the 2 R values of a row that are used pass through memory, as 64-bit words.
+constexpr int kSumBatch = 8;
+template <class T, int RP>
+__device__ __forceinline__ bool sum_tasks(const RowTask &T_, int m, int R, T *__restrict__ part, int prow,
+                                          int *__restrict__ count, T *red, int *arrived) {
+    constexpr int kVals = 8 / (int)sizeof(T), kStride = 2 * RP / kVals;  // values per word, words per row of red
+    const int rw = 2 * R / kVals, n = m * rw;                            // words per row, words
+    const int64_t slot_words = (int64_t)prow * kStride;
+    uint64_t *words = reinterpret_cast<uint64_t *>(red), *p0 = reinterpret_cast<uint64_t *>(part) + T_.slot0 * slot_words;
+    uint64_t *dst = p0 + (T_.slot - T_.slot0) * slot_words;
+    for (int e = threadIdx.x; e < n; e += blockDim.x) {
+        const int row = e / rw;
+        store_agent(dst + e, words[row * kStride + (e - row * rw)]);
+    }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // this wavefront's stores are at the point of coherence
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        const int a = __hip_atomic_fetch_add(count + T_.count, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if (a == T_.ntask - 1) __hip_atomic_store(count + T_.count, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        *arrived = a;
+    }
+    __syncthreads();
+    if (*arrived != T_.ntask - 1) return false;
+    union Word {
+        uint64_t w;
+        T v[kVals];
+    };
+    for (int e = threadIdx.x; e < n; e += blockDim.x) {
+        Word a;
+#pragma unroll
+        for (int i = 0; i < kVals; i++) a.v[i] = T(0);
+        for (int k0 = 0; k0 < T_.ntask; k0 += kSumBatch) {
+            Word v[kSumBatch];
+#pragma unroll
+            for (int b = 0; b < kSumBatch; b++) v[b].w = load_agent(p0 + min(k0 + b, T_.ntask - 1) * slot_words + e);
+#pragma unroll
+            for (int b = 0; b < kSumBatch; b++)
+#pragma unroll
+                for (int i = 0; i < kVals; i++) a.v[i] = k0 + b < T_.ntask ? a.v[i] + v[b].v[i] : a.v[i];
+        }
+        const int row = e / rw;
+        words[row * kStride + (e - row * rw)] = a.w;
+    }
+    __syncthreads();
+    return true;
+}
+
 template <class T, int NT, bool NARROW, int NRT>
 __device__ __forceinline__ void rows_run(const RowTask &T_, int rs, int m, const LeafPanel &L,
                                          const int *__restrict__ psrc,
                                          const typename Mfma<T>::T2 *__restrict__ panel,
                                          const typename Mfma<T>::T2 *__restrict__ xt, const double *__restrict__ x,
                                          int N, int R, double *__restrict__ y, const int *__restrict__ cols, int j0,
-                                         T *__restrict__ part, int prow, T *red, int w, int lane) {
+                                         T *__restrict__ part, int prow, int *__restrict__ count, T *red, int *arrived,
+                                         int w, int lane) {
     typedef typename Mfma<T>::T2 T2;
     constexpr int RP = 8 * NT;
     const int i16 = lane & 15, kk = lane >> 4, s = i16 & 1;
@@ -450,14 +514,18 @@ __device__ __forceinline__ void rows_run(const RowTask &T_, int rs, int m, const
     if (w == 0) store_tile<T, NT, NRT>(acc, red, m, 2 * RP, lane);
     __syncthreads();
     if (T_.slot >= 0) {
-        T *dst = part + (int64_t)T_.slot * prow * (2 * RP);
-        for (int e = threadIdx.x; e < m * 2 * RP; e += blockDim.x) dst[e] = red[e];
-    } else {
-        for (int e = threadIdx.x; e < 2 * m * R; e += blockDim.x) {
-            const int j = e / (2 * m), q = e - j * 2 * m, row = q >> 1, p = q & 1;
-            const int64_t idx = (col_of(cols, j0, j) * N + rs + row) * 2 + p;
-            y[idx] = -0.5 * x[idx] + (double)red[row * 2 * RP + 2 * j + p];
+        if constexpr (NARROW) {
+            if (!sum_tasks<T, RP>(T_, m, R, part, prow, count, red, arrived)) return;
+        } else {
+            T *dst = part + (int64_t)T_.slot * prow * (2 * RP);
+            for (int e = threadIdx.x; e < m * 2 * RP; e += blockDim.x) dst[e] = red[e];
+            return;
         }
+    }
+    for (int e = threadIdx.x; e < 2 * m * R; e += blockDim.x) {
+        const int j = e / (2 * m), q = e - j * 2 * m, row = q >> 1, p = q & 1;
+        const int64_t idx = (col_of(cols, j0, j) * N + rs + row) * 2 + p;
+        y[idx] = -0.5 * x[idx] + (double)red[row * 2 * RP + 2 * j + p];
     }
 }
 
@@ -466,9 +534,11 @@ __global__ __launch_bounds__(64 * kRowWaves) void k_rows_mfma(
     const RowTask *__restrict__ tasks, const int *__restrict__ leaf_start, const LeafPanel *__restrict__ lpanel,
     const int *__restrict__ psrc, const typename Mfma<T>::T2 *__restrict__ panel,
     const typename Mfma<T>::T2 *__restrict__ xt, const double *__restrict__ x, int N, int R, double *__restrict__ y,
-    const int *__restrict__ cols, int j0, const int *__restrict__ gate, T *__restrict__ part, int prow) {
+    const int *__restrict__ cols, int j0, const int *__restrict__ gate, T *__restrict__ part, int prow,
+    int *__restrict__ count) {
     constexpr int PR = MAXRT > 4 ? kMaxLeaf : kPartRows;  // output staging rows
     __shared__ Lds<T, NT, kRowWaves, PR> red;
+    __shared__ int arrived;
     if (gated(gate)) return;
     const int w = wave_id(), lane = threadIdx.x & 63;
     const RowTask T_ = tasks[blockIdx.x];
@@ -477,21 +547,28 @@ __global__ __launch_bounds__(64 * kRowWaves) void k_rows_mfma(
     const LeafPanel L = lpanel[T_.leaf];
     const int nrt = (m + 15) >> 4;
     if (nrt <= 1)
-        rows_run<T, NT, NARROW, 1>(T_, rs, m, L, psrc, panel, xt, x, N, R, y, cols, j0, part, prow, red.v, w, lane);
+        rows_run<T, NT, NARROW, 1>(T_, rs, m, L, psrc, panel, xt, x, N, R, y, cols, j0, part, prow, count, red.v, &arrived, w,
+                                     lane);
     else if (nrt == 2 || MAXRT == 2)
-        rows_run<T, NT, NARROW, 2>(T_, rs, m, L, psrc, panel, xt, x, N, R, y, cols, j0, part, prow, red.v, w, lane);
+        rows_run<T, NT, NARROW, 2>(T_, rs, m, L, psrc, panel, xt, x, N, R, y, cols, j0, part, prow, count, red.v, &arrived, w,
+                                     lane);
     else if constexpr (MAXRT == 4) {
         if (nrt == 3)
-            rows_run<T, NT, NARROW, 3>(T_, rs, m, L, psrc, panel, xt, x, N, R, y, cols, j0, part, prow, red.v, w, lane);
+            rows_run<T, NT, NARROW, 3>(T_, rs, m, L, psrc, panel, xt, x, N, R, y, cols, j0, part, prow, count, red.v, &arrived, w,
+                                     lane);
         else
-            rows_run<T, NT, NARROW, 4>(T_, rs, m, L, psrc, panel, xt, x, N, R, y, cols, j0, part, prow, red.v, w, lane);
+            rows_run<T, NT, NARROW, 4>(T_, rs, m, L, psrc, panel, xt, x, N, R, y, cols, j0, part, prow, count, red.v, &arrived, w,
+                                     lane);
     } else if constexpr (MAXRT == 8) {
         if (nrt <= 4)
-            rows_run<T, NT, NARROW, 4>(T_, rs, m, L, psrc, panel, xt, x, N, R, y, cols, j0, part, prow, red.v, w, lane);
+            rows_run<T, NT, NARROW, 4>(T_, rs, m, L, psrc, panel, xt, x, N, R, y, cols, j0, part, prow, count, red.v, &arrived, w,
+                                     lane);
         else if (nrt <= 6)
-            rows_run<T, NT, NARROW, 6>(T_, rs, m, L, psrc, panel, xt, x, N, R, y, cols, j0, part, prow, red.v, w, lane);
+            rows_run<T, NT, NARROW, 6>(T_, rs, m, L, psrc, panel, xt, x, N, R, y, cols, j0, part, prow, count, red.v, &arrived, w,
+                                     lane);
         else
-            rows_run<T, NT, NARROW, 8>(T_, rs, m, L, psrc, panel, xt, x, N, R, y, cols, j0, part, prow, red.v, w, lane);
+            rows_run<T, NT, NARROW, 8>(T_, rs, m, L, psrc, panel, xt, x, N, R, y, cols, j0, part, prow, count, red.v, &arrived, w,
+                                     lane);
     }
 }
 
@@ -501,7 +578,6 @@ __global__ __launch_bounds__(64 * kRowWaves) void k_rows_mfma(
 // about once per batch rather than once per partial; the summed rows go through LDS so that y rows are
 // written contiguously.
 constexpr int kSumRows = 8;
-constexpr int kSumBatch = 8;
 template <class T, int NT>
 __global__ __launch_bounds__(256) void k_rows_sum(const int4 *__restrict__ split, const int *__restrict__ leaf_start,
                                                   const T *__restrict__ part, const double *__restrict__ x, int N,
@@ -854,11 +930,13 @@ static std::unique_ptr<HostBuf> build_lists(arh_hmat *h, int tr) {
     for (int l = 0; l < g->nleaf; l++) {
         const int n = lpanel[l].ngroups;
         const int nt = std::max(1, (n + tg - 1) / tg);
-        if (nt > 1) rsplit.push_back(int4{l, M.nslots, nt, 0});
         for (int t = 0; t < nt; t++)
             rtasks.push_back(RowTask{l, (int)((int64_t)n * t / nt), (int)((int64_t)n * (t + 1) / nt),
-                                       nt > 1 ? M.nslots + t : -1});
-        if (nt > 1) M.nslots += nt;
+                                     nt > 1 ? M.nslots + t : -1, M.nslots, nt, (int)rsplit.size(), 0});
+        if (nt > 1) {
+            rsplit.push_back(int4{l, M.nslots, nt, 0});
+            M.nslots += nt;
+        }
     }
     // XCD-aware order: workgroups are dispatched round-robin over the kXcds dies, each with its own
     // L2, so die x gets a contiguous run of leaves (in tree order, which neighbouring leaves share
@@ -874,7 +952,7 @@ static std::unique_ptr<HostBuf> build_lists(arh_hmat *h, int tr) {
         }
         size_t len = 0;
         for (auto &r : run) len = std::max(len, r.size());
-        rtasks.assign(len * kXcds, RowTask{-1, 0, 0, -1});
+        rtasks.assign(len * kXcds, RowTask{-1, 0, 0, -1, 0, 0, 0, 0});
         for (int x = 0; x < kXcds; x++)
             for (size_t i = 0; i < run[x].size(); i++) rtasks[i * kXcds + x] = run[x][i];
     } else {
@@ -882,7 +960,6 @@ static std::unique_ptr<HostBuf> build_lists(arh_hmat *h, int tr) {
                          [](const RowTask &p, const RowTask &q) { return p.g1 - p.g0 > q.g1 - q.g0; });
     }
     M.ntasks = (int)rtasks.size();
-    M.nsplit = (int)rsplit.size();
     // all lists in one block, one upload; in front of them the flag of the device's check
     size_t total = 0;
     auto room = [&](size_t bytes) {
@@ -892,17 +969,20 @@ static std::unique_ptr<HostBuf> build_lists(arh_hmat *h, int tr) {
     };
     auto bytes_of = [](const auto &v) { return v.size() * sizeof(v[0]); };
     const size_t o_bad = room(sizeof(int)), o_st = room(bytes_of(stacks)), o_un = room(bytes_of(units)),
-                 o_lp = room(bytes_of(lpanel)), o_rt = room(bytes_of(rtasks)), o_rs = room(bytes_of(rsplit));
+                 o_lp = room(bytes_of(lpanel)), o_rt = room(bytes_of(rtasks)), o_rs = room(bytes_of(rsplit)),
+                 o_ct = room(sizeof(int) * rsplit.size());
     auto hb = std::make_unique<HostBuf>(total, s);
     M.d_lists.alloc(total);
     char *hp = hb->as<char>(), *dp = M.d_lists.as<char>();
     auto put = [&](size_t o, const auto &v) { std::copy(v.begin(), v.end(), (std::decay_t<decltype(v[0])> *)(hp + o)); };
     *(int *)(hp + o_bad) = 0;
     put(o_st, stacks), put(o_un, units), put(o_lp, lpanel), put(o_rt, rtasks), put(o_rs, rsplit);
+    std::fill((int *)(hp + o_ct), (int *)(hp + o_ct) + rsplit.size(), 0);
     M.bad = (const int *)(dp + o_bad);
     M.stacks = (const VStack *)(dp + o_st), M.p1units = (const int2 *)(dp + o_un);
     M.lpanel = (const LeafPanel *)(dp + o_lp), M.rtasks = (const RowTask *)(dp + o_rt);
-    M.rsplit = (const int4 *)(dp + o_rs);
+    M.rsplit = (const int4 *)(dp + o_rs), M.count = (int *)(dp + o_ct);
+    M.nsplit = (int)rsplit.size();
     ARH_HIP(hipMemcpyAsync(dp, hp, total, hipMemcpyHostToDevice, s));
     // the lists that follow from these on the device
     M.nmaps = g->na;
@@ -1029,14 +1109,16 @@ static void launch_nt(arh_hmat *h, MfmaLayout &M, int R, const double2 *x, doubl
         });
     const int64_t ent = g->dense_entries + (h->u_total + h->v_total - e1);
     T *part = M.nslots ? M.part[pi].as<T>() : nullptr;
-    const int ntask = M.ntasks, nsp = M.nsplit;
+    const int ntask = M.ntasks;
+
     const double *xd = (const double *)x;
     double *yd = (double *)y;
     timed(pi ? PROF_ROWS64 : PROF_ROWS32, eb * ent + eb * R * (N + h->t_total) + 32.0 * R * N, 8.0 * R * ent, [&] {
         auto launch_rows = [&](auto kern) {
             hipLaunchKernelGGL(kern, dim3(ntask), dim3(64 * kRowWaves), 0, s, M.rtasks,
                                g->d_leaf_start.as<int>(), M.lpanel, M.d_psrc.as<int>(),
-                               M.panel[pi].as<T2>(), (const T2 *)xt, xd, N, R, yd, cols, j0, gate, part, prow);
+                               M.panel[pi].as<T2>(), (const T2 *)xt, xd, N, R, yd, cols, j0, gate, part, prow,
+                               M.count);
         };
         if constexpr (NT == 1)
             if (narrow)
@@ -1057,8 +1139,8 @@ static void launch_nt(arh_hmat *h, MfmaLayout &M, int R, const double2 *x, doubl
                 ARH_CHECK(false, ARH_EINVAL, "internal: pass too wide for leaves of more than 64 elements");
         }
     });
-    if (nsp)
-        hipLaunchKernelGGL((k_rows_sum<T, NT>), dim3(nsp, (g->max_leaf + kSumRows - 1) / kSumRows), dim3(256), 0, s,
+    if (M.nsplit && !narrow)
+        hipLaunchKernelGGL((k_rows_sum<T, NT>), dim3(M.nsplit, (g->max_leaf + kSumRows - 1) / kSumRows), dim3(256), 0, s,
                            M.rsplit, g->d_leaf_start.as<int>(), part, xd, N, R, yd, cols, j0, gate, prow);
     ARH_HIP(hipGetLastError());
 }
