@@ -190,6 +190,8 @@ struct arh_ctx_s {
     int device = 0;
     hipStream_t own = nullptr;
     hipStream_t stream = nullptr;
+    hipStream_t side = nullptr;  // second stream, made on first use
+    hipStream_t aux();
     std::string err;
     // reduction / scalar scratch reused by the solver
     arh::DBuf red;      // partial sums

@@ -8,8 +8,8 @@
 
 namespace arh {
 
-constexpr int kAcaWaves = 4;      // wavefronts of an ACA workgroup
-constexpr int kAcaThreads = kAcaWaves * ARH_WAVE;
+constexpr int kAcaFew = 256;  // up to so many big blocks, one per compute unit, take 8 wavefronts each, more 4
+constexpr int kAcaWaves = 8;  // wavefronts of a big block's workgroup, at most
 constexpr int kMaxRankLds = 128;  // max ACA rank kept in LDS coefficient arrays
 #ifndef ARH_ACA_BIGDIM
 #define ARH_ACA_BIGDIM 512
@@ -97,9 +97,15 @@ __device__ __forceinline__ void wsum8(const double2 *s, double2 &a, double2 &b) 
 // ahead of their use (the first before the entry is evaluated), and reductions run on DPP: through ds_bpermute the
 // dot products alone, 24 steps per stored cross, were half of a cross's time.
 // 0.6 m relief, 16,058 blocks: 1.95 ms at 4000 Hz and 1.2 ms at 1000 Hz (3.95 and 1.9 ms with the bpermute
-// reductions and unbatched loads), the factors bit for bit the same. What is left is VALU issue of mid-sized
-// blocks (3 wavefronts per SIMD) with a tail of the largest chains; 2 or 4 wavefronts per SIMD (4: spills) and 6,
-// 8 or 12 wavefronts per workgroup measured the same or slower: 2.75-3.2 ms per FP64 assembly at 4000 Hz against 2.75.
+// reductions and unbatched loads), the factors bit for bit the same. Of that, at 4000 Hz, VALU instructions took 60 %
+// and a third of the wavefront slots stood empty: the four blocks of a workgroup held their registers until the
+// longest was done, and the largest block's chain alone took 1.94 ms, all others 1.65. So a block that a wavefront
+// takes is a workgroup of its own, and up to kAcaFew big blocks get eight wavefronts instead of four, on a stream beside
+// the others: whole FP64 assembly 2.30 -> 2.10 ms at 4000 Hz, 2.25 -> 1.99 with leaves of 64, 1.48 -> 1.44 with leaves of
+// 128 at 1000 Hz, where leaves of 32 (1.53 -> 1.51) are bound by VALU issue throughout. Eight wavefronts for every big
+// block of a larger mesh (0.9 m, 1000 Hz) take 18.2 ms instead of 16.2: there the chip is full anyway and the blocks' idle
+// wavefronts cost. A queue that persistent wavefronts pull from keeps the slots full too, but the loop around the
+// chains spills (2.42 ms at 4000 Hz). 2 or 4 wavefronts per SIMD (4: spills) measured the same or slower.
 
 // |v|^2 of the pivot searches. On symmetric meshes two entries can tie exactly, and this rounding decides between
 // them: it is part of the result, so the fused form is written out.
@@ -269,19 +275,20 @@ struct AcaShared {
     double rv[4][kAcaWaves];
     int ri[kAcaWaves];
 };
+template <int W>
 struct AcaSharedGroup : AcaShared {
-    double2 dd[kAcaWaves][kMaxRankLds][2];  // kMaxRankLds is a multiple of the batch
+    double2 dd[W][kMaxRankLds][2];  // kMaxRankLds is a multiple of the batch
 };
 
-// The threads working on one larger block: the whole workgroup (WAVE false) or a single wavefront (WAVE true, no
+// The threads working on one larger block: a workgroup of W wavefronts or a single wavefront (W = 1, no
 // workgroup barrier: a wavefront's memory operations complete in order, so a fence at wavefront scope, which
 // also stops compiler reordering, is its barrier).
-template <bool WAVE>
+template <int W>
 struct AcaGroup {
+    static constexpr bool WAVE = W == 1;
     int tid, w, lane;
-    std::conditional_t<WAVE, AcaShared, AcaSharedGroup> &sh;
-    static constexpr int nthr = WAVE ? ARH_WAVE : kAcaThreads;
-    static constexpr int nw = WAVE ? 1 : kAcaWaves;
+    std::conditional_t<WAVE, AcaShared, AcaSharedGroup<W>> &sh;
+    static constexpr int nthr = W * ARH_WAVE;
     __device__ __forceinline__ void sync() const {
         if (WAVE) {
             __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
@@ -299,7 +306,7 @@ struct AcaGroup {
         __syncthreads();
         double s = sh.rv[slot][0];
 #pragma unroll
-        for (int q = 1; q < kAcaWaves; q++) s += sh.rv[slot][q];
+        for (int q = 1; q < W; q++) s += sh.rv[slot][q];
         return s;
     }
     // (value, index) max with ties to the lower index
@@ -313,20 +320,21 @@ struct AcaGroup {
         v = sh.rv[slot][0];
         i = sh.ri[0];
 #pragma unroll
-        for (int q = 1; q < kAcaWaves; q++)
+        for (int q = 1; q < W; q++)
             if (sh.rv[slot][q] > v || (sh.rv[slot][q] == v && sh.ri[q] < i)) v = sh.rv[slot][q], i = sh.ri[q];
     }
 };
 
-template <bool WAVE>
-__device__ __forceinline__ void aca_block(const AcaGroup<WAVE> &G, int2 *__restrict__ ranks, int bid,
+template <int W>
+__device__ __forceinline__ void aca_block(const AcaGroup<W> &G, int2 *__restrict__ ranks, int bid,
                                           const LRBlock &B, const Tri *__restrict__ tri, double k, double eps,
                                           double2 *__restrict__ U, double2 *__restrict__ V,
                                           unsigned char *__restrict__ used) {
     auto &sh = G.sh;
     const int rs = B.rs, cs = B.cs, m = B.re - B.rs, n = B.ce - B.cs, lim = B.lim;
     const int tid = G.tid, lane = G.lane;
-    constexpr int nthr = AcaGroup<WAVE>::nthr;
+    constexpr bool WAVE = W == 1;
+    constexpr int nthr = AcaGroup<W>::nthr;
     for (int q = tid; q < m; q += nthr) used[q] = (q == 0) ? 1 : 0;
     int i = 0, it = 0, sr = 0;
     double err = 0.0;
@@ -425,7 +433,7 @@ __device__ __forceinline__ void aca_block(const AcaGroup<WAVE> &G, int2 *__restr
             for (int p = lane; p < sr; p += ARH_WAVE) {
                 double2 su = sh.dd[0][p][0], sv = sh.dd[0][p][1];
 #pragma unroll
-                for (int q = 1; q < kAcaWaves; q++) su = cadd(su, sh.dd[q][p][0]), sv = cadd(sv, sh.dd[q][p][1]);
+                for (int q = 1; q < W; q++) su = cadd(su, sh.dd[q][p][0]), sv = cadd(sv, sh.dd[q][p][1]);
                 dots += sqrt(cnorm2(su)) * sqrt(cnorm2(sv));
             }
         }
@@ -441,40 +449,45 @@ __device__ __forceinline__ void aca_block(const AcaGroup<WAVE> &G, int2 *__restr
     if (tid == 0) ranks[bid] = make_int2(sr, it);
 }
 
-// Workgroups [0, nbig) each take one big block (order[0..nbig)); the others take kAcaWaves smaller
-// blocks, one per wavefront. nan: raised by the dense blocks.
-__global__ __launch_bounds__(kAcaThreads, 3) void k_aca(const LRBlock *__restrict__ blocks, const int *__restrict__ order,
-                                                     int nbig, int na, const Tri *__restrict__ tri, double k,
-                                                     double eps, double2 *__restrict__ Us, double2 *__restrict__ Vs,
-                                                     unsigned char *__restrict__ flags, const int *__restrict__ nan,
-                                                     int2 *__restrict__ ranks) {
-    __shared__ union Shared {
-        AcaSharedGroup group;
-        AcaShared wave[kAcaWaves];
-        __device__ Shared() {}
-    } sh;
+// A workgroup of W wavefronts per big block (order[0..nbig)). nan: raised by the dense blocks.
+template <int W>
+__global__ __launch_bounds__(W * ARH_WAVE, 2) void k_aca_big(const LRBlock *__restrict__ blocks,
+                                                          const int *__restrict__ order, const Tri *__restrict__ tri,
+                                                          double k, double eps, double2 *__restrict__ Us,
+                                                          double2 *__restrict__ Vs, unsigned char *__restrict__ flags,
+                                                          const int *__restrict__ nan, int2 *__restrict__ ranks) {
+    __shared__ AcaSharedGroup<W> sh;
     if (*nan) return;  // the assembly fails
-    const int lane = threadIdx.x % ARH_WAVE;
-    const int w = __builtin_amdgcn_readfirstlane((int)(threadIdx.x / ARH_WAVE));
-    const bool big = (int)blockIdx.x < nbig;
-    const int u = big ? (int)blockIdx.x : nbig + ((int)blockIdx.x - nbig) * kAcaWaves + w;
-    if (u >= na) return;
-    const int bid = order[u];
+    const int bid = order[blockIdx.x];
     const LRBlock B = blocks[bid];
     if (B.lim <= 0) {  // a single row or column, or max_rank 0
-        if (lane == 0 && (!big || w == 0)) ranks[bid] = make_int2(0, 0);
+        if (threadIdx.x == 0) ranks[bid] = make_int2(0, 0);
         return;
     }
+    const int w = __builtin_amdgcn_readfirstlane((int)(threadIdx.x / ARH_WAVE));
+    const AcaGroup<W> G{(int)threadIdx.x, w, (int)(threadIdx.x % ARH_WAVE), sh};
+    aca_block<W>(G, ranks, bid, B, tri, k, eps, Us + B.us_off, Vs + B.vs_off, flags + B.flag_off);
+}
+
+// A wavefront per other block, each a workgroup of its own (so that a finished block's slot is free at once).
+__global__ __launch_bounds__(ARH_WAVE, 3) void k_aca(const LRBlock *__restrict__ blocks, const int *__restrict__ order,
+                                                  const Tri *__restrict__ tri, double k, double eps,
+                                                  double2 *__restrict__ Us, double2 *__restrict__ Vs,
+                                                  unsigned char *__restrict__ flags, const int *__restrict__ nan,
+                                                  int2 *__restrict__ ranks) {
+    __shared__ AcaShared sh;
+    if (*nan) return;
+    const int lane = threadIdx.x;
+    const int bid = order[blockIdx.x];
+    const LRBlock B = blocks[bid];
     double2 *U = Us + B.us_off, *V = Vs + B.vs_off;
-    unsigned char *used = flags + B.flag_off;
-    if (big) {
-        const AcaGroup<false> G{(int)threadIdx.x, w, lane, sh.group};
-        aca_block<false>(G, ranks, bid, B, tri, k, eps, U, V, used);
+    if (B.lim <= 0) {
+        if (lane == 0) ranks[bid] = make_int2(0, 0);
     } else if (B.re - B.rs <= ARH_WAVE && B.ce - B.cs <= ARH_WAVE) {
         aca_small(ranks, bid, B, lane, tri, k, eps, U, V);
     } else {
-        const AcaGroup<true> G{lane, 0, lane, sh.wave[w]};
-        aca_block<true>(G, ranks, bid, B, tri, k, eps, U, V, used);
+        const AcaGroup<1> G{lane, 0, lane, sh};
+        aca_block<1>(G, ranks, bid, B, tri, k, eps, U, V, flags + B.flag_off);
     }
 }
 
@@ -631,6 +644,31 @@ static void lr_plan(arh_geom *g, int max_rank) {
     g->lr_plan_rank = max_rank;
 }
 
+// Work on a second stream beside a stream's own, between everything before and everything after on that one. Left
+// without join (an error on the way), it waits for the second stream, whose kernels use the first one's buffers.
+struct Fork {
+    hipStream_t main, side;
+    bool joined = false;
+    Fork(hipStream_t m, hipStream_t s) : main(m), side(s) {
+        if (side != main) order(main, side);
+    }
+    void join() {
+        if (side != main) order(side, main);
+        joined = true;
+    }
+    ~Fork() {
+        if (!joined && side != main) (void)hipStreamSynchronize(side);
+    }
+    static void order(hipStream_t from, hipStream_t to) {
+        hipEvent_t e;
+        ARH_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+        hipError_t r = hipEventRecord(e, from);
+        if (r == hipSuccess) r = hipStreamWaitEvent(to, e, 0);
+        (void)hipEventDestroy(e);
+        ARH_HIP(r);
+    }
+};
+
 // Dense panels, then the ACA: one wait for the device, with the ranks (and whether a dense entry was a NaN) in pinned
 // memory, before the factors' storage can be allocated.
 void assemble(arh_hmat *h) {
@@ -672,10 +710,25 @@ void assemble(arh_hmat *h) {
     LrTotals *tot = hb.as<LrTotals>();
     int2 *hranks = (int2 *)(tot + 1);
     const int nbig = g->aca_nbig;
-    const int grid = nbig + (na - nbig + kAcaWaves - 1) / kAcaWaves;
-    hipLaunchKernelGGL(k_aca, dim3(grid), dim3(kAcaThreads), 0, s, g->d_lr0.as<LRBlock>(), g->d_aca_order.as<int>(), nbig,
-                       na, g->tri.as<Tri>(), h->k, h->aca_tol, us.as<double2>(), vs.as<double2>(),
-                       used.as<unsigned char>(), flag.as<int>(), ranks.as<int2>());
+    {
+        // the big blocks go first, on the context's stream; the others beside them on the auxiliary one
+        Fork fork(s, nbig && na > nbig ? g->ctx->aux() : s);
+        auto big = [&](auto kern, int waves) {
+            hipLaunchKernelGGL(kern, dim3(nbig), dim3(waves * ARH_WAVE), 0, s, g->d_lr0.as<LRBlock>(),
+                               g->d_aca_order.as<int>(), g->tri.as<Tri>(), h->k, h->aca_tol, us.as<double2>(),
+                               vs.as<double2>(), used.as<unsigned char>(), flag.as<int>(), ranks.as<int2>());
+        };
+        if (nbig > kAcaFew)
+            big(k_aca_big<4>, 4);
+        else if (nbig)
+            big(k_aca_big<8>, 8);
+        if (na > nbig)
+            hipLaunchKernelGGL(k_aca, dim3(na - nbig), dim3(ARH_WAVE), 0, fork.side, g->d_lr0.as<LRBlock>(),
+                               g->d_aca_order.as<int>() + nbig, g->tri.as<Tri>(), h->k, h->aca_tol, us.as<double2>(),
+                               vs.as<double2>(), used.as<unsigned char>(), flag.as<int>(), ranks.as<int2>());
+        ARH_HIP(hipGetLastError());
+        fork.join();
+    }
     hipLaunchKernelGGL(k_lr_offsets, dim3((na + 1023) / 1024), dim3(1024), 0, s, na, g->d_lr0.as<LRBlock>(),
                        ranks.as<int2>(), flag.as<int>(), h->blocks.as<LRBlock>(), active.as<int>(), hranks, tot);
     ARH_HIP(hipGetLastError());

@@ -45,6 +45,11 @@ static void set_device(arh_ctx *ctx) {
     tl_stream = ctx->stream;
 }
 
+hipStream_t arh_ctx_s::aux() {
+    if (!side) ARH_HIP(hipStreamCreateWithFlags(&side, hipStreamNonBlocking));
+    return side;
+}
+
 extern "C" {
 
 int arh_ctx_create(int device, arh_ctx **out) {
@@ -73,6 +78,7 @@ static void ctx_release(arh_ctx *ctx) {
     ctx->red.reset();
     ctx->scal.reset();
     if (tl_stream == ctx->stream || tl_stream == ctx->own) tl_stream = nullptr;
+    if (ctx->side) (void)hipStreamDestroy(ctx->side);
     if (ctx->own) (void)hipStreamDestroy(ctx->own);
     delete ctx;
 }
