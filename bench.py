@@ -255,8 +255,9 @@ def kernel_counts(g, capi, ctx, top, f=4000.0, R=37):
     """Algorithmic work of the FP64-VALU kernels on the f Hz operator: the ACA kernel (entry evaluations of the
     crosses it computes: rank + 1 crosses per block, the last one discarded, or the rank when the limit
     min(100, m - 1, n - 1) stops it) and the dense-leaf kernel, then one shape-gradient call with R right-hand
-    sides (12 derivative points per (touched element, element) pair and pass, plus 8 flops per complex
-    multiply-add of the R right-hand sides). Run under rocprofv3 --kernel-trace for the kernel durations."""
+    sides (12 derivative points per pair of a touched element with another one, touched or not, taken both ways at
+    once, plus 8 flops per complex multiply-add of the products of the R right-hand sides, two per ordered pair with a
+    touched first). Run under rocprofv3 --kernel-trace for the kernel durations."""
     k = 2 * np.pi * f / C0
     h = g.assemble(k, 1e-4, 100, capi.ARH_FP64)
     ranks = h.ranks()
@@ -278,13 +279,14 @@ def kernel_counts(g, capi, ctx, top, f=4000.0, R=37):
     dirs = -np.column_stack([np.cos(np.linspace(0, np.pi, R)), np.sin(np.linspace(0, np.pi, R)), np.zeros(R)])
     g.shape_grad(k, L, top, R, X, LAM, VF, capi.ARH_RHS_PLANE, dirs)
     ctx.synchronize()
-    passes = -(-R // 20)
-    pairs = int(touched) * g.N
+    T, others = int(touched), g.N - int(touched)
+    both, one_way = T * (T + 1) // 2, T * others
     return {"frequency": f, "N": g.N, "aca_entries": aca_entries, "aca_points": 6 * aca_entries,
             "aca_flops": 6 * aca_entries * FLOPS_PER_ENTRY_POINT, "dense_entries": dense_entries,
-            "dense_flops": 6 * dense_entries * FLOPS_PER_ENTRY_POINT, "grad_touched": int(touched),
-            "grad_pairs_per_pass": pairs, "grad_passes": passes,
-            "grad_B_flops": passes * pairs * 12 * FLOPS_PER_DERIV_POINT + pairs * 4 * 8 * R,
+            "dense_flops": 6 * dense_entries * FLOPS_PER_ENTRY_POINT, "grad_touched": T,
+            "grad_pairs_both_ways": both, "grad_pairs_one_way": one_way,
+            "grad_both_flops": both * (12 * FLOPS_PER_DERIV_POINT + 2 * 8 * R),
+            "grad_pairs_flops": one_way * (12 * FLOPS_PER_DERIV_POINT + 2 * 8 * R),
             "flops_per_entry_point": FLOPS_PER_ENTRY_POINT, "flops_per_deriv_point": FLOPS_PER_DERIV_POINT}
 
 
