@@ -389,24 +389,27 @@ int arh_hmat_factors(const arh_hmat *h, int a, double *U, double *V, int *rank) 
         arh_geom *g = h->g;
         ARH_CHECK(a >= 0 && a < g->na, ARH_EINVAL, "low-rank block index out of range");
         set_device(g->ctx);
-        LRBlock B;
-        ARH_HIP(hipMemcpyAsync(&B, h->blocks.as<LRBlock>() + a, sizeof(LRBlock), hipMemcpyDeviceToHost, g->ctx->stream));
-        ARH_HIP(hipStreamSynchronize(g->ctx->stream));
-        const int m = B.re - B.rs, n = B.ce - B.cs, r = B.rank;
+        const int *q = &g->lowrank[4 * a];
+        const int m = q[1] - q[0], n = q[3] - q[2], r = h->ranks[a].x;
         *rank = r;
         if (!U || !V) return;
+        int64_t u_off = 0, v_off = 0;  // the factors follow one another in block order
+        for (int b = 0; b < a; b++) {
+            const int *p = &g->lowrank[4 * b];
+            u_off += (int64_t)h->ranks[b].x * (p[1] - p[0]), v_off += (int64_t)h->ranks[b].x * (p[3] - p[2]);
+        }
         std::vector<double2> seg((size_t)m * r);
         if (r > 0) {
-            ARH_HIP(hipMemcpyAsync(seg.data(), h->U.as<double2>() + B.u_off, sizeof(double2) * seg.size(),
+            ARH_HIP(hipMemcpyAsync(seg.data(), h->U.as<double2>() + u_off, sizeof(double2) * seg.size(),
                                    hipMemcpyDeviceToHost, g->ctx->stream));
-            ARH_HIP(hipMemcpyAsync(V, h->V.as<double2>() + B.v_off, sizeof(double2) * (size_t)r * n,
+            ARH_HIP(hipMemcpyAsync(V, h->V.as<double2>() + v_off, sizeof(double2) * (size_t)r * n,
                                    hipMemcpyDeviceToHost, g->ctx->stream));
         }
         ARH_HIP(hipStreamSynchronize(g->ctx->stream));
         // leaf-segmented -> plain m x r column-major
         double2 *Uo = (double2 *)U;
-        for (int l = B.l0; l < g->nleaf && g->leaf_start[l] < B.re; l++) {
-            const int ls = g->leaf_start[l] - B.rs, ms = g->leaf_start[l + 1] - g->leaf_start[l];
+        for (int l = g->leaf_of[q[0]]; l < g->nleaf && g->leaf_start[l] < q[1]; l++) {
+            const int ls = g->leaf_start[l] - q[0], ms = g->leaf_start[l + 1] - g->leaf_start[l];
             for (int p = 0; p < r; p++)
                 for (int i = 0; i < ms; i++) Uo[(size_t)p * m + ls + i] = seg[(size_t)ls * r + (size_t)p * ms + i];
         }

@@ -51,7 +51,7 @@ constexpr int kGSlots = 2048;    // workgroups aimed for (8 per compute unit): t
 // Blocks of touched elements from which their pairs are taken both ways at once: fewer leave the chip half empty (one rhs,
 // whole call, 17 blocks 371 us one way and 364 both ways, 12 blocks 283 and 327, 31 blocks 532 and 474).
 constexpr int kGMinBlocks = 20;
-constexpr int64_t kGMaxPart = int64_t(1) << 28;  // (block, touched element) partial sums: 6.4 GB
+constexpr int64_t kGMaxPart = int64_t(1) << 26;  // their (block, element) partial sums at most: 1.6 GB, 65,536 elements
 
 typedef double V4d __attribute__((ext_vector_type(4)));
 
