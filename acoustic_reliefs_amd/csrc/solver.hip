@@ -237,8 +237,10 @@ __global__ __launch_bounds__(ARH_WAVE) void k_finish(const RhsState *__restrict_
 // (every wavefront forms its rhs's scalars, some 400 operations; N = 9,828, p update: 37 right-hand sides FP32 10.4,
 // 7.4, 8.2 us at 64, 128, 192 rows, one FP64 6.0, 6.8, 8.0 us. The end of the previous iteration and the packing
 // were launches of their own: 16.4 us for 37, 15 us for one). T2: complex type of the operator's precision; xf == nullptr leaves the
-// packing to the product.
-constexpr int kUpCols = 16;
+// packing to the product. Four columns per workgroup: beside other streams' products a workgroup of sixteen wavefronts
+// waits for as many free slots on one compute unit (13 bands served, p and s updates 103 and 64 us instead of 9 and 6
+// alone); alone the two are equal, served bands 223.5 -> 221 ms, the sphere's band 1.13 -> 1.11 ms.
+constexpr int kUpCols = 4;
 template <class T2>
 constexpr int up_rows() {
     return sizeof(T2) == 8 ? 128 : 64;

@@ -1,4 +1,4 @@
-"""The solver's fused vector updates at the edges of their tiles: right-hand sides around the 16 columns of a workgroup
+"""The solver's fused vector updates at the edges of their tiles: right-hand sides around multiples of the four columns of a workgroup
 and the 40 of a product pass, sizes that do not fill the last rows, both precisions, columns that stop at
 different iterations. A batch gives every right-hand side the bits it gets alone (the updates of one right-hand side
 see nothing of the others), and the true residual meets the tolerance."""
