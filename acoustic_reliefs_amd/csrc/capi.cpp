@@ -4,6 +4,7 @@
 #include <cmath>
 #include <cstring>
 #include <memory>
+#include <mutex>
 #include <vector>
 
 #include "arh_internal.h"
@@ -46,6 +47,8 @@ static void set_device(arh_ctx *ctx) {
 }
 
 hipStream_t arh_ctx_s::aux() {
+    static std::mutex mu;
+    std::lock_guard<std::mutex> lk(mu);
     if (!side) ARH_HIP(hipStreamCreateWithFlags(&side, hipStreamNonBlocking));
     return side;
 }
