@@ -51,7 +51,11 @@ constexpr int kGSlots = 2048;    // workgroups aimed for (8 per compute unit): t
 // Blocks of touched elements from which their pairs are taken both ways at once: fewer leave the chip half empty (one rhs,
 // whole call, 17 blocks 371 us one way and 364 both ways, 12 blocks 283 and 327, 31 blocks 532 and 474).
 constexpr int kGMinBlocks = 20;
-constexpr int64_t kGMaxPart = int64_t(1) << 26;  // their (block, element) partial sums at most: 1.6 GB, 65,536 elements
+// Room for their partial sums at a time, 48 bytes per touched element and offset (k_grad_both): all of them up to 13,000
+// touched elements, else strips of offsets one after the other. 0.9 m relief (51,834 touched, 406 offsets, whole call):
+// one rhs 56.2 ms, 37 82.1 ms in 16 strips; 55.9 and 81.2 ms at once, which takes 1.0 GB. Strips of 128 and 256 MB measured
+// the same.
+constexpr int64_t kGPartBytes = int64_t(64) << 20;
 
 typedef double V4d __attribute__((ext_vector_type(4)));
 
@@ -235,11 +239,13 @@ __global__ __launch_bounds__(kGT, 3) void k_grad_pairs(const Tri *__restrict__ t
 // Pairs of touched elements, both ways at once. The distances between the collocation point of i and the rule points of e
 // serve dM_ie/dp_i (i's centroid moves, times G(i, e)) and dM_ie/dq_(e,c) (e's corners move, times the same G(i, e)), so
 // a pair {i, e} takes the twelve distances and the two products once where k_grad_pairs, for i and for e, takes them
-// twice. A workgroup takes a pair of blocks of kGB touched elements (grid: block b with the blocks b, b + 1, .. in
-// circular order, up to half of them, so each pair of blocks once), a wavefront 16 of the second block's elements as
+// twice. A workgroup takes a pair of blocks of kGB touched elements (grid: block b with block b + d in circular order, the
+// offsets d up to half of the blocks, so each pair of blocks once), a wavefront 16 of the second block's elements as
 // columns; both blocks' geometry is in LDS. The two directions of a pair come one after the other, each with its own
 // product tile: with both tiles in registers at once the kernel spills at 3 wavefronts per SIMD (one rhs 2.4 ms, 37 3.4;
-// now 2.15 and 2.9, 159 registers; at 4 wavefronts 2.6 and 3.6). out[(o * T + t) * 3 + c]: the sum of element t with the elements of block o.
+// now 2.15 and 2.9, 159 registers; at 4 wavefronts 2.6 and 3.6). The offsets are those from d0 on, gridDim.y of them;
+// out[((2 (d - d0) + s) * T + t) * 3 + c]: the sum of element t, in block b, with the elements of block b + d (s = 0) or
+// b - d (s = 1).
 constexpr int kGB = 64;
 static_assert(kGB == 16 * kGW, "a column tile per wavefront");
 
@@ -273,13 +279,14 @@ __device__ __forceinline__ void pair_side(double k, const GradRow &r, double px,
 
 __global__ __launch_bounds__(kGT, 3) void k_grad_both(const Tri *__restrict__ tri, int T, const int *__restrict__ touched,
                                                    double k, int K, const double *__restrict__ xp,
-                                                   const double *__restrict__ lp, double *__restrict__ out) {
+                                                   const double *__restrict__ lp, int d0, double *__restrict__ out) {
     __shared__ GradRow rows[2][kGB];
     __shared__ double red[kGW][kGB][3];
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
     const int i16 = lane & 15, kk = lane >> 4;
-    const int nb = gridDim.x, rb = blockIdx.x, cb = (rb + (int)blockIdx.y) % nb;
-    if (2 * (int)blockIdx.y == nb && 2 * rb >= nb) return;  // its partner has the pair
+    const int nb = gridDim.x, d = d0 + (int)blockIdx.y, rb = blockIdx.x, cb = (rb + d) % nb;
+    if (2 * d == nb && 2 * rb >= nb) return;  // its partner has the pair
+    out += (int64_t)blockIdx.y * 6 * T;
     if (threadIdx.x < 2 * kGB) {  // surplus elements repeat the last, not added
         const int b = threadIdx.x / kGB, i = threadIdx.x % kGB;
         fill_row(rows[b][i], tri[touched[min((b ? cb : rb) * kGB + i, T - 1)]]);
@@ -336,7 +343,7 @@ __global__ __launch_bounds__(kGT, 3) void k_grad_both(const Tri *__restrict__ tr
         }
         if (kk == 0 && on)
 #pragma unroll
-            for (int c = 0; c < 3; c++) out[((int64_t)rb * T + u) * 3 + c] = col[c];
+            for (int c = 0; c < 3; c++) out[((int64_t)T + u) * 3 + c] = col[c];
     }
     __syncthreads();
     if (threadIdx.x < 3 * kGB) {
@@ -344,19 +351,26 @@ __global__ __launch_bounds__(kGT, 3) void k_grad_both(const Tri *__restrict__ tr
         if (rb * kGB + r < T) {
             double a = red[0][r][c];
             for (int q = 1; q < kGW; q++) a += red[q][r][c];
-            out[((int64_t)cb * T + rb * kGB + r) * 3 + c] = a;
+            out[(rb * kGB + r) * 3 + c] = a;
         }
     }
 }
 
-// Sums over the other blocks, in order.
-__global__ __launch_bounds__(256) void k_grad_blocks(int n3, int nb, const double *__restrict__ part,
+// Sums over the other blocks of a strip of offsets, in order of the offset; added to out from the second strip on. (At
+// offset 0 a block's sum with itself is in s = 0 alone; at offset nb / 2 a block's sum is in s = 0 or in s = 1.)
+__global__ __launch_bounds__(256) void k_grad_blocks(int n3, int nb, int d0, int nd, const double *__restrict__ part,
                                                      double *__restrict__ out) {
     const int i = blockIdx.x * 256 + threadIdx.x;
     if (i >= n3) return;
-    double a = 0.0;
-#pragma unroll 8
-    for (int o = 0; o < nb; o++) a += part[(int64_t)o * n3 + i];
+    const bool low = 2 * (i / (3 * kGB)) < nb;
+    double a = d0 > 0 ? out[i] : 0.0;
+#pragma unroll 4
+    for (int q = 0; q < nd; q++) {
+        const int d = d0 + q;
+        const double u = part[(int64_t)(2 * q) * n3 + i], v = part[(int64_t)(2 * q + 1) * n3 + i];
+        a += 2 * d < nb || low ? u : 0.0;
+        a += d > 0 && (2 * d < nb || !low) ? v : 0.0;
+    }
     out[i] = a;
 }
 
@@ -465,7 +479,7 @@ void launch_shape_grad(arh_geom *g, double k, const double *L_dev, int LL, const
     };
     // enough blocks of touched elements to fill the chip: their pairs both ways at once, then the other columns
     const int nb = (T + kGB - 1) / kGB;
-    const bool both = nb >= kGMinBlocks && (int64_t)nb * T <= kGMaxPart;
+    const bool both = nb >= kGMinBlocks;
     const int ncol = both ? (int)others.size() : N;
     const int bsplit = ncol ? splits(ncol) : 0, asplit = splits(LL), first = both ? 1 : 0;  // first: the blocks' sum
     const int K = 4 * ((nrhs + 1) / 2);
@@ -486,11 +500,17 @@ void launch_shape_grad(arh_geom *g, double k, const double *L_dev, int LL, const
     pack(vp, LL, vf);
     if (both) {
         upload(d_others, others, s);
-        pS.alloc(sizeof(double) * 3 * (size_t)T * nb);
-        hipLaunchKernelGGL(k_grad_both, dim3(nb, nb / 2 + 1), dim3(kGT), 0, s, g->tri.as<Tri>(), T, d_touched.as<int>(), k,
-                           K, xp.as<double>(), lp.as<double>(), pS.as<double>());
-        hipLaunchKernelGGL(k_grad_blocks, dim3((3 * T + 255) / 256), dim3(256), 0, s, 3 * T, nb, pS.as<double>(),
-                           pB.as<double>());
+        const int no = nb / 2 + 1;  // offsets, in equal strips
+        const int64_t per = 2 * 3 * (int64_t)sizeof(double) * T, most = std::max<int64_t>(1, kGPartBytes / per);
+        const int strips = (int)((no + most - 1) / most), len = (no + strips - 1) / strips;
+        pS.alloc((size_t)per * len);
+        for (int d0 = 0; d0 < no; d0 += len) {
+            const int nd = std::min(len, no - d0);
+            hipLaunchKernelGGL(k_grad_both, dim3(nb, nd), dim3(kGT), 0, s, g->tri.as<Tri>(), T, d_touched.as<int>(), k, K,
+                               xp.as<double>(), lp.as<double>(), d0, pS.as<double>());
+            hipLaunchKernelGGL(k_grad_blocks, dim3((3 * T + 255) / 256), dim3(256), 0, s, 3 * T, nb, d0, nd,
+                               pS.as<double>(), pB.as<double>());
+        }
     }
     if (bsplit)
         hipLaunchKernelGGL(k_grad_pairs<false>, dim3(gx, bsplit), dim3(kGT), 0, s, g->tri.as<Tri>(),
