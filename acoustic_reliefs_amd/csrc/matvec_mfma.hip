@@ -33,6 +33,7 @@
 
 #include "arh_internal.h"
 #include "device_common.h"
+#include "lr_units.h"
 
 namespace arh {
 
@@ -101,10 +102,6 @@ constexpr int row_depth() {
 // so the register budget, not the workgroup size, sets how many fit a compute unit.
 constexpr int kLrWaves = ARH_MV_WAVES;    // V-stack units (big stacks: the whole workgroup)
 constexpr int kRowWaves = ARH_MV_RWAVES;  // row tasks
-// Small V-stack units per workgroup: one wavefront per SIMD, the other wavefronts leave at once. Units differ in length,
-// and eight to a workgroup kept its registers until the longest was done: FP32 37 rhs 62.5 -> 61 us (58 -> 53.5 us
-// at 1000 Hz, transposed 65 -> 61), FP64 one rhs 48 -> 42 us; 2, 3, 5 and 6 units are slower than 4.
-constexpr int kLrSmall = 4;
 constexpr bool kChunked = ARH_MV_CHUNKED;  // a workgroup's waves take contiguous group ranges (else strided)
 constexpr bool kXcdOrder = ARH_MV_XCD;     // row tasks ordered for the per-die L2s
 constexpr int kXcds = 8;                   // dies (XCDs) of an MI355X, each with its own L2
@@ -883,14 +880,14 @@ static std::unique_ptr<HostBuf> build_lists(arh_hmat *h, int tr) {
     M.vs_total = voff;
     ARH_CHECK(trow - N == h->t_total, ARH_EINVAL, "stacked intermediates do not match the ranks");
     // phase-1 units: big stacks first, each list by decreasing column count
-    std::vector<int2> units(nbig + (nsmall + kLrSmall - 1) / kLrSmall * kLrWaves, int2{-1, 0});
+    std::vector<int2> units(nbig + lr_slots(nsmall, kLrWaves), int2{-1, 0});
     size_t ub = 0, us = 0;
     for (int k : C.by_size)
         for (int rt = 0; rt * 32 < stacks[k].rtot; rt++) {
             if (stacks[k].n >= kBigCols)
                 units[ub++] = int2{k, rt};
             else
-                units[nbig + us / kLrSmall * kLrWaves + us % kLrSmall] = int2{k, rt}, us++;
+                units[nbig + lr_slot(us++, kLrWaves)] = int2{k, rt};
         }
     M.p1big = (int)nbig;
     M.nunits = (int)units.size();
