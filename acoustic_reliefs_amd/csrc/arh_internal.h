@@ -4,8 +4,10 @@
 
 #include <cmath>
 #include <cstdint>
+#include <mutex>
 #include <stdexcept>
 #include <string>
+#include <utility>
 #include <vector>
 
 #include "../../include/arh.h"
@@ -342,6 +344,9 @@ struct arh_hmat_s {
     arh::DBuf blocks;          // LRBlock[na]
     arh::DBuf U, V, U32, V32;  // packed factors
     std::vector<int2> ranks;  // per low-rank block: stored rank, rank as the reference counts it
+    // per low-rank block: where its factors start in U and V; made when they are first asked for
+    mutable std::once_flag factors_once;
+    mutable std::vector<std::pair<int64_t, int64_t>> factors_at;
     int64_t u_total = 0, v_total = 0, t_total = 0;
     int n_active = 0;
     arh::DBuf d_active_lr;  // lr blocks with rank > 0

