@@ -65,16 +65,17 @@ __device__ __forceinline__ double neighbour(double v) {
     return __hiloint2double(hi, lo);
 }
 
-// acc += (entries q, one per lane) times rows `at` of the R vectors x (length len each): column n of tile nt.
+// acc += (entries q, one per lane) times rows `at` of the R vectors x (length len each): column n of tile nt. A lane
+// that is not `on` takes a zero: its entry is one too, and its row may hold an infinity.
 template <int NT>
 __device__ __forceinline__ void recv_mma(V4d (&acc)[NT], double2 q, const double2 *__restrict__ x, int64_t len, int at,
-                                         int R, int n16) {
+                                         bool on, int R, int n16) {
     const double *xd = reinterpret_cast<const double *>(x);
     const int s = n16 & 1;
 #pragma unroll
     for (int nt = 0; nt < NT; nt++) {
         const int j = min(nt * 8 + (n16 >> 1), R - 1);  // surplus columns repeat the last, not written
-        const double v = xd[(j * len + at) * 2 + s];
+        const double xv = xd[(j * len + at) * 2 + s], v = on ? xv : 0.0;
         const double w = neighbour(v);
         acc[nt] = __builtin_amdgcn_mfma_f64_16x16x4f64(q.x, v, acc[nt], 0, 0, 0);
         acc[nt] = __builtin_amdgcn_mfma_f64_16x16x4f64(q.y, s ? w : -w, acc[nt], 0, 0, 0);
@@ -115,12 +116,16 @@ __global__ __launch_bounds__(kRT) void k_recv(const Tri *__restrict__ tri, int N
     for (int nt = 0; nt < NT; nt++) acc[nt] = V4d{0, 0, 0, 0};
     const int ng = (N + 3) >> 2, sp = blockIdx.y;
     const int g0 = (int)((int64_t)ng * sp / nsplit), g1 = (int)((int64_t)ng * (sp + 1) / nsplit);
-    for (int g = g0 + w; g < g1; g += kRW) {
+    auto step = [&](int g, auto whole) {
         const int e = 4 * g + kk, ec = min(e, N - 1);
+        const bool on = whole() || e < N;
         double2 q = bem_entry(k, px, py, pz, tri[ec]);
-        if (e >= N) q = make_double2(0.0, 0.0);
-        recv_mma<NT>(acc, q, x, N, ec, R, n16);
-    }
+        if (!on) q = make_double2(0.0, 0.0);
+        recv_mma<NT>(acc, q, x, N, ec, on, R, n16);
+    };
+    int g = g0 + w;
+    for (; g < min(g1, N >> 2); g += kRW) step(g, std::true_type{});
+    if (g < g1) step(g, std::false_type{});
     recv_reduce<NT>(acc, red, w, lane);
     double *o = part + ((int64_t)sp * gridDim.x + blockIdx.x) * 16 * 16 * NT;
     for (int e = threadIdx.x; e < 16 * 16 * NT; e += kRT) o[e] = (&red[0][0][0])[e];
@@ -154,12 +159,16 @@ __global__ __launch_bounds__(kRT) void k_recv_t(const Tri *__restrict__ tri, int
 #pragma unroll
     for (int nt = 0; nt < NT; nt++) acc[nt] = V4d{0, 0, 0, 0};
     const int ng = (LL + 3) >> 2;
-    for (int g = w; g < ng; g += kRW) {
+    auto step = [&](int g, auto whole) {
         const int l = 4 * g + kk, lc = min(l, LL - 1);
+        const bool on = whole() || l < LL;
         double2 q = bem_entry(k, L[3 * lc], L[3 * lc + 1], L[3 * lc + 2], t);
-        if (l >= LL) q = make_double2(0.0, 0.0);
-        recv_mma<NT>(acc, q, x, LL, lc, R, n16);
-    }
+        if (!on) q = make_double2(0.0, 0.0);
+        recv_mma<NT>(acc, q, x, LL, lc, on, R, n16);
+    };
+    int g = w;
+    for (; g < LL >> 2; g += kRW) step(g, std::true_type{});
+    if (g < ng) step(g, std::false_type{});
     recv_reduce<NT>(acc, red, w, lane);
     const int m = min(16, N - i0);
     for (int e = threadIdx.x; e < R * 2 * m; e += kRT) {
