@@ -48,9 +48,12 @@ constexpr int kGW = 4;           // wavefronts per workgroup; they take every kG
 constexpr int kGT = 64 * kGW;
 constexpr int kGSlots = 2048;    // workgroups aimed for (8 per compute unit): the column range is split to reach it
 
-// Blocks of touched elements from which their pairs are taken both ways at once: fewer leave the chip half empty (one rhs,
-// whole call, 17 blocks 371 us one way and 364 both ways, 12 blocks 283 and 327, 31 blocks 532 and 474).
-constexpr int kGMinBlocks = 20;
+// Blocks of touched elements from which their pairs are taken both ways at once: fewer leave the chip half empty. The two
+// are equal at 26 (N = 2,618) to 40 (N = 58,724) blocks, and little apart around there. Whole call, one way and both ways:
+//   N = 2,618:  24 blocks, one rhs 424 and 432 us, 37 rhs 523 and 536 us; 28 blocks 442 and 425, 564 and 530
+//   N = 9,828:  28 blocks 866 and 881 us, 1174 and 1180 us; 36 blocks 1008 and 997, 1396 and 1349
+//   N = 58,724: 28 blocks 3.93 and 4.00 ms, 5.78 and 5.82 ms; 48 blocks 6.62 and 6.50, 9.77 and 9.62
+constexpr int kGMinBlocks = 28;
 // Room for their partial sums at a time, 48 bytes per touched element and offset (k_grad_both): all of them up to 13,000
 // touched elements, else strips of offsets one after the other. 0.9 m relief (51,834 touched, 406 offsets, whole call):
 // one rhs 56.2 ms, 37 82.1 ms in 16 strips; 55.9 and 81.2 ms at once, which takes 1.0 GB. Strips of 128 and 256 MB measured
