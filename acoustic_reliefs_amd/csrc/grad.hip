@@ -40,7 +40,7 @@ namespace arh {
 // two right-hand sides for 256 pairs. Reciprocal distances come from one v_rsq_f64 and one cubic correction step
 // (below 1 ulp) instead of a square root and five divisions. The loop over a lane's four pairs stays rolled: unrolled
 // it needs 249 registers, 2 wavefronts per SIMD instead of 3, and 3-5 % more time; 4 wavefronts spill (+14 %).
-// N = 9,828 with 8,190 touched elements, 8e7 pairs: 3.1 ms for one right-hand side and 4.6 ms for 37, where
+// N = 9,828 with 8,442 touched elements, 8e7 pairs: 3.1 ms for one right-hand side and 4.6 ms for 37, where
 // accumulating every right-hand side's sums per lane took 10.3 ms and 24.6 ms (two passes, each with its own
 // derivatives); 1297 listeners, one right-hand side: 0.24 ms from 2.6 ms. With the pairs of touched elements taken
 // both ways at once (k_grad_both) the whole call goes from 3.27 to 2.15 ms and from 4.47 to 2.90 ms.
@@ -368,21 +368,22 @@ __global__ __launch_bounds__(kGT, 3) void k_grad_both(const Tri *__restrict__ tr
     }
 }
 
-// Sums over the other blocks of a strip of offsets, in order of the offset; added to out from the second strip on. (At
-// offset 0 a block's sum with itself is in s = 0 alone; at offset nb / 2 a block's sum is in s = 0 or in s = 1.)
+// Sums over the other blocks of a strip of offsets, in order of the offset; added to out from the second strip on. At offset
+// 0 a block's sum with itself is in s = 0 alone, at offset nb / 2 a block's sum is in s = 0 for the first half of the
+// blocks and in s = 1 for the others; both lie outside the loop, whose loads go out together that way (10 us instead of
+// 25 at 8,442 touched elements).
 __global__ __launch_bounds__(256) void k_grad_blocks(int n3, int nb, int d0, int nd, const double *__restrict__ part,
                                                      double *__restrict__ out) {
     const int i = blockIdx.x * 256 + threadIdx.x;
     if (i >= n3) return;
-    const bool low = 2 * (i / (3 * kGB)) < nb;
-    double a = d0 > 0 ? out[i] : 0.0;
+    const bool half = 2 * (d0 + nd - 1) == nb;
+    double a = d0 > 0 ? out[i] : part[i];
 #pragma unroll 4
-    for (int q = 0; q < nd; q++) {
-        const int d = d0 + q;
-        const double u = part[(int64_t)(2 * q) * n3 + i], v = part[(int64_t)(2 * q + 1) * n3 + i];
-        a += 2 * d < nb || low ? u : 0.0;
-        a += d > 0 && (2 * d < nb || !low) ? v : 0.0;
+    for (int q = d0 > 0 ? 0 : 1; q < nd - (half ? 1 : 0); q++) {
+        a += part[(int64_t)(2 * q) * n3 + i];
+        a += part[(int64_t)(2 * q + 1) * n3 + i];
     }
+    if (half) a += part[(int64_t)(2 * (nd - 1) + (2 * (i / (3 * kGB)) < nb ? 0 : 1)) * n3 + i];
     out[i] = a;
 }
 
