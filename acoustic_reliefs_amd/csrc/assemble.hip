@@ -8,7 +8,12 @@
 
 namespace arh {
 
-constexpr int kAcaFew = 256;  // up to so many big blocks, one per compute unit, take 8 wavefronts each, more 4
+// Up to so many big blocks, one per compute unit, take 8 wavefronts each, more of them 4. Norms and dot products are
+// summed per wavefront, so the stopping rule's left side rounds differently in the two: a cross within a few 1e-16 of the
+// tolerance may be kept in one and not in the other, and a big block's rank then depends on how many the partition has.
+// (One grouping for both would have 4 wavefronts form 8 partial sums: twice the dot products' reductions, for the meshes
+// that are bound by VALU issue.) A geometry's own factors are the same in every assembly.
+constexpr int kAcaFew = 256;
 constexpr int kAcaWaves = 8;  // wavefronts of a big block's workgroup, at most
 constexpr int kMaxRankLds = 128;  // max ACA rank kept in LDS coefficient arrays
 #ifndef ARH_ACA_BIGDIM

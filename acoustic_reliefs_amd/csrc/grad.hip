@@ -48,16 +48,17 @@ constexpr int kGW = 4;           // wavefronts per workgroup; they take every kG
 constexpr int kGT = 64 * kGW;
 constexpr int kGSlots = 2048;    // workgroups aimed for (8 per compute unit): the column range is split to reach it
 
-// Blocks of touched elements from which their pairs are taken both ways at once: fewer leave the chip half empty. The two
-// are equal at 26 (N = 2,618) to 40 (N = 58,724) blocks, and little apart around there. Whole call, one way and both ways:
+// Blocks of touched elements from which their pairs are taken both ways at once: fewer leave the chip half empty. The
+// two are equal at 26 (N = 2,618) to 40 (N = 58,724) blocks, and little apart around there. Whole call, one way and
+// both ways:
 //   N = 2,618:  24 blocks, one rhs 424 and 432 us, 37 rhs 523 and 536 us; 28 blocks 442 and 425, 564 and 530
 //   N = 9,828:  28 blocks 866 and 881 us, 1174 and 1180 us; 36 blocks 1008 and 997, 1396 and 1349
 //   N = 58,724: 28 blocks 3.93 and 4.00 ms, 5.78 and 5.82 ms; 48 blocks 6.62 and 6.50, 9.77 and 9.62
 constexpr int kGMinBlocks = 28;
-// Room for their partial sums at a time, 48 bytes per touched element and offset (k_grad_both): all of them up to 13,000
-// touched elements, else strips of offsets one after the other. 0.9 m relief (51,834 touched, 406 offsets, whole call):
-// one rhs 56.2 ms, 37 82.1 ms in 16 strips; 55.9 and 81.2 ms at once, which takes 1.0 GB. Strips of 128 and 256 MB measured
-// the same.
+// Room for their partial sums at a time, 48 bytes per touched element and offset (k_grad_both): all of them up to
+// 13,000 touched elements, else strips of offsets one after the other. 0.9 m relief (51,834 touched, 406 offsets, whole
+// call): one rhs 56.2 ms, 37 82.1 ms in 16 strips; 55.9 and 81.2 ms at once, which takes 1.0 GB. Strips of 128 and 256
+// MB measured the same.
 constexpr int64_t kGPartBytes = int64_t(64) << 20;
 
 typedef double V4d __attribute__((ext_vector_type(4)));
@@ -70,13 +71,13 @@ __device__ __forceinline__ double rsqrt_f64(double x) {
 }
 
 // Kernel factors at distance vector d without the 1 / (4 pi): F = e^{-ikr} (-1 - ikr) / r^3 and
-// H = d_y / r e^{-ikr} (-k^2 / r^2 + 3 (1 + ikr) / r^4). FAR: r2 ir is off by up to 1.5 units in the last place, which the
-// phase k r of a far point takes over (k r reaches some thousands at listeners), so one correction step makes r as good
-// as a rounded root. The listener term against 80 bits, 50 m and 3150 Hz, 5 m and 4000 Hz: 1.28e-13 and 2.25e-14 without the
-// step, 1.11e-13 and 1.82e-14 with it; plain double precision 1.11e-13 and 1.92e-14; no time measurable (1297
-// listeners, whole call 2.08 ms).
-// Element pairs are a metre apart at most: their error comes from the near pairs and is below a rounded root's formula
-// by division either way (7.5e-15 against 9.2e-15 at 4000 Hz), and the step would cost 2.5 % of the call there.
+// H = d_y / r e^{-ikr} (-k^2 / r^2 + 3 (1 + ikr) / r^4). FAR: r2 ir is off by up to 1.5 units in the last place, which
+// the phase k r of a far point takes over (k r reaches some thousands at listeners), so one correction step makes r as
+// good as a rounded root. The listener term against 80 bits, 50 m and 3150 Hz, 5 m and 4000 Hz: 1.28e-13 and 2.25e-14
+// without the step, 1.11e-13 and 1.82e-14 with it; plain double precision 1.11e-13 and 1.92e-14; no time measurable
+// (1297 listeners, whole call 2.08 ms). Element pairs are a metre apart at most: their error comes from the near pairs
+// and is below a rounded root's formula by division either way (7.5e-15 against 9.2e-15 at 4000 Hz), and the step would
+// cost 2.5 % of the call there.
 template <bool FAR = false>
 __device__ __forceinline__ void FdF(double k, double dx, double dy, double dz, double2 &F, double2 &H) {
     const double r2 = fma(dx, dx, fma(dy, dy, dz * dz));
@@ -142,14 +143,14 @@ __device__ __forceinline__ void pair_gemm(const double *__restrict__ a, const do
 }
 
 // Partial sums over a range of columns for 16 touched elements. Columns are elements (LISTEN false: B; cols: a list of
-// them, or null for all) or listeners (LISTEN true: A); grid (row tiles, column splits); out[(split * T + t) * 3 + c]. xi, li: packed x and
-// lambda by element; pc: the columns' packed values that multiply x_i (lambda by element, or vf by listener).
+// them, or null for all) or listeners (LISTEN true: A); grid (row tiles, column splits); out[(split * T + t) * 3 + c].
+// xi, li: packed x and lambda by element; pc: the columns' packed values that multiply x_i (lambda by element, or vf by
+// listener).
 template <bool LISTEN>
-__global__ __launch_bounds__(kGT, 3) void k_grad_pairs(const Tri *__restrict__ tri, const double *__restrict__ L,
-                                                    const int *__restrict__ cols, int ncol, int T, const int *__restrict__ touched, double k, int K,
-                                                    const double *__restrict__ xp, const double *__restrict__ lp,
-                                                    const double *__restrict__ pc, int nsplit,
-                                                    double *__restrict__ out) {
+__global__ __launch_bounds__(kGT, 3) void k_grad_pairs(
+    const Tri *__restrict__ tri, const double *__restrict__ L, const int *__restrict__ cols, int ncol, int T,
+    const int *__restrict__ touched, double k, int K, const double *__restrict__ xp, const double *__restrict__ lp,
+    const double *__restrict__ pc, int nsplit, double *__restrict__ out) {
     __shared__ GradRow rows[16];
     __shared__ double red[kGW][16][3];
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
@@ -248,16 +249,16 @@ __global__ __launch_bounds__(kGT, 3) void k_grad_pairs(const Tri *__restrict__ t
     }
 }
 
-// Pairs of touched elements, both ways at once. The distances between the collocation point of i and the rule points of e
-// serve dM_ie/dp_i (i's centroid moves, times G(i, e)) and dM_ie/dq_(e,c) (e's corners move, times the same G(i, e)), so
-// a pair {i, e} takes the twelve distances and the two products once where k_grad_pairs, for i and for e, takes them
-// twice. A workgroup takes a pair of blocks of kGB touched elements (grid: block b with block b + d in circular order, the
-// offsets d up to half of the blocks, so each pair of blocks once), a wavefront 16 of the second block's elements as
-// columns; both blocks' geometry is in LDS. The two directions of a pair come one after the other, each with its own
-// product tile: with both tiles in registers at once the kernel spills at 3 wavefronts per SIMD (one rhs 2.4 ms, 37 3.4;
-// now 2.15 and 2.9, 159 registers; at 4 wavefronts 2.6 and 3.6). The offsets are those from d0 on, gridDim.y of them;
-// out[((2 (d - d0) + s) * T + t) * 3 + c]: the sum of element t, in block b, with the elements of block b + d (s = 0) or
-// b - d (s = 1).
+// Pairs of touched elements, both ways at once. The distances between the collocation point of i and the rule points of
+// e serve dM_ie/dp_i (i's centroid moves, times G(i, e)) and dM_ie/dq_(e,c) (e's corners move, times the same G(i, e)),
+// so a pair {i, e} takes the twelve distances and the two products once where k_grad_pairs, for i and for e, takes them
+// twice. A workgroup takes a pair of blocks of kGB touched elements (grid: block b with block b + d in circular order,
+// the offsets d up to half of the blocks, so each pair of blocks once), a wavefront 16 of the second block's elements
+// as columns; both blocks' geometry is in LDS. The two directions of a pair come one after the other, each with its own
+// product tile: with both tiles in registers at once the kernel spills at 3 wavefronts per SIMD (one rhs 2.4 ms, 37
+// 3.4; now 2.15 and 2.9, 159 registers; at 4 wavefronts 2.6 and 3.6). The offsets are those from d0 on, gridDim.y of
+// them; out[((2 (d - d0) + s) * T + t) * 3 + c]: the sum of element t, in block b, with the elements of block b + d (s
+// = 0) or b - d (s = 1).
 constexpr int kGB = 64;
 static_assert(kGB == 16 * kGW, "a column tile per wavefront");
 
@@ -289,9 +290,10 @@ __device__ __forceinline__ void pair_side(double k, const GradRow &r, double px,
     o[3] = (ci * g_i - cr * g_r) * (1.0 / 3.0);
 }
 
-__global__ __launch_bounds__(kGT, 3) void k_grad_both(const Tri *__restrict__ tri, int T, const int *__restrict__ touched,
-                                                   double k, int K, const double *__restrict__ xp,
-                                                   const double *__restrict__ lp, int d0, double *__restrict__ out) {
+__global__ __launch_bounds__(kGT, 3) void k_grad_both(const Tri *__restrict__ tri, int T,
+                                                      const int *__restrict__ touched, double k, int K,
+                                                      const double *__restrict__ xp, const double *__restrict__ lp,
+                                                      int d0, double *__restrict__ out) {
     __shared__ GradRow rows[2][kGB];
     __shared__ double red[kGW][kGB][3];
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
@@ -368,10 +370,10 @@ __global__ __launch_bounds__(kGT, 3) void k_grad_both(const Tri *__restrict__ tr
     }
 }
 
-// Sums over the other blocks of a strip of offsets, in order of the offset; added to out from the second strip on. At offset
-// 0 a block's sum with itself is in s = 0 alone, at offset nb / 2 a block's sum is in s = 0 for the first half of the
-// blocks and in s = 1 for the others; both lie outside the loop, whose loads go out together that way (10 us instead of
-// 25 at 8,442 touched elements).
+// Sums over the other blocks of a strip of offsets, in order of the offset; added to out from the second strip on. At
+// offset 0 a block's sum with itself is in s = 0 alone, at offset nb / 2 a block's sum is in s = 0 for the first half
+// of the blocks and in s = 1 for the others; both lie outside the loop, whose loads go out together that way (10 us
+// instead of 25 at 8,442 touched elements).
 __global__ __launch_bounds__(256) void k_grad_blocks(int n3, int nb, int d0, int nd, const double *__restrict__ part,
                                                      double *__restrict__ out) {
     const int i = blockIdx.x * 256 + threadIdx.x;
@@ -519,24 +521,25 @@ void launch_shape_grad(arh_geom *g, double k, const double *L_dev, int LL, const
         pS.alloc((size_t)per * len);
         for (int d0 = 0; d0 < no; d0 += len) {
             const int nd = std::min(len, no - d0);
-            hipLaunchKernelGGL(k_grad_both, dim3(nb, nd), dim3(kGT), 0, s, g->tri.as<Tri>(), T, d_touched.as<int>(), k, K,
-                               xp.as<double>(), lp.as<double>(), d0, pS.as<double>());
+            hipLaunchKernelGGL(k_grad_both, dim3(nb, nd), dim3(kGT), 0, s, g->tri.as<Tri>(), T, d_touched.as<int>(), k,
+                               K, xp.as<double>(), lp.as<double>(), d0, pS.as<double>());
             hipLaunchKernelGGL(k_grad_blocks, dim3((3 * T + 255) / 256), dim3(256), 0, s, 3 * T, nb, d0, nd,
                                pS.as<double>(), pB.as<double>());
         }
     }
     if (bsplit)
         hipLaunchKernelGGL(k_grad_pairs<false>, dim3(gx, bsplit), dim3(kGT), 0, s, g->tri.as<Tri>(),
-                           (const double *)nullptr, both ? d_others.as<int>() : nullptr, ncol, T, d_touched.as<int>(), k, K,
-                           xp.as<double>(), lp.as<double>(), lp.as<double>(), bsplit,
+                           (const double *)nullptr, both ? d_others.as<int>() : nullptr, ncol, T, d_touched.as<int>(),
+                           k, K, xp.as<double>(), lp.as<double>(), lp.as<double>(), bsplit,
                            pB.as<double>() + first * 3 * (size_t)T);
     hipLaunchKernelGGL(k_grad_pairs<true>, dim3(gx, asplit), dim3(kGT), 0, s, g->tri.as<Tri>(), L_dev,
-                       (const int *)nullptr, LL, T, d_touched.as<int>(), k, K, xp.as<double>(), (const double *)nullptr, vp.as<double>(), asplit,
-                       pA.as<double>());
+                       (const int *)nullptr, LL, T, d_touched.as<int>(), k, K, xp.as<double>(),
+                       (const double *)nullptr, vp.as<double>(), asplit, pA.as<double>());
     hipLaunchKernelGGL(k_grad_C, dim3((T + 63) / 64), dim3(64), 0, s, g->tri.as<Tri>(), N, T, d_touched.as<int>(), k,
                        nrhs, lam, src_kind, src_dev, cC.as<double>());
-    hipLaunchKernelGGL(k_grad_scatter, dim3((HH + 255) / 256), dim3(256), 0, s, HH, T, asplit, first + bsplit, d_hptr.as<int>(),
-                       d_hlist.as<int>(), pA.as<double>(), pB.as<double>(), cC.as<double>(), A, B, C, G);
+    hipLaunchKernelGGL(k_grad_scatter, dim3((HH + 255) / 256), dim3(256), 0, s, HH, T, asplit, first + bsplit,
+                       d_hptr.as<int>(), d_hlist.as<int>(), pA.as<double>(), pB.as<double>(), cC.as<double>(), A, B, C,
+                       G);
     ARH_HIP(hipGetLastError());
     ARH_HIP(hipStreamSynchronize(s));
 }

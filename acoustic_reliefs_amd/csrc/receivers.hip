@@ -49,7 +49,7 @@ void launch_rhs(arh_geom *g, double k, int kind, int nrhs, const double *vecs_de
 // side's result does not depend on the batch (columns are independent, the split of the sum is fixed by LL and N).
 //
 // Bound by the entries' FP64 VALU work, about 590 operations for 64 entries against 2 MFMAs per 8 right-hand sides.
-// 181 receivers, N = 9,828, 37 right-hand sides: 64 us and 61 us transposed (45 and 47 us for one); storing Q
+// 181 receivers, N = 9,828, 37 right-hand sides: 55 us and 57 us transposed (41 and 44 us for one); storing Q
 // (40 us) and multiplying by it with vector FMAs took 355 and 57 us more.
 constexpr int kRW = 4;            // wavefronts per workgroup
 constexpr int kRT = kRW * ARH_WAVE;

@@ -234,12 +234,13 @@ __global__ __launch_bounds__(ARH_WAVE) void k_finish(const RhsState *__restrict_
 
 // The vector updates before a product also write the product's packed rows (row i: rw complex values, listed column c
 // at c, zero from nc on), through LDS: a workgroup takes up_rows of the rows and kUpCols of the columns, a wavefront each
-// (every wavefront forms its rhs's scalars, some 400 operations; N = 9,828, p update: 37 right-hand sides FP32 10.4,
-// 7.4, 8.2 us at 64, 128, 192 rows, one FP64 6.0, 6.8, 8.0 us. The end of the previous iteration and the packing
-// were launches of their own: 16.4 us for 37, 15 us for one). T2: complex type of the operator's precision; xf == nullptr leaves the
-// packing to the product. Four columns per workgroup: beside other streams' products a workgroup of sixteen wavefronts
-// waits for as many free slots on one compute unit (13 bands served, p and s updates 103 and 64 us instead of 9 and 6
-// alone); alone the two are equal, served bands 223.5 -> 221 ms, the sphere's band 1.13 -> 1.11 ms.
+// (every wavefront forms its rhs's scalars, some 400 operations; N = 9,828, p update: 37 right-hand sides FP32 11.3,
+// 9.7, 9.4 us at 64, 128, 192 rows, one FP64 4.8, 5.1, 5.4 us. The end of the previous iteration and the packing
+// were launches of their own: 16.4 us for 37, 15 us for one). T2: complex type of the operator's precision; xf == nullptr
+// leaves the packing to the product. Four columns per workgroup: beside other streams' products a workgroup of sixteen
+// wavefronts waits for as many free slots on one compute unit (13 bands served, p and s updates 104 and 63 us instead of
+// the 9.7 and 6.3 they take alone, now 39 and 28); alone the two are equal, served bands 223.5 -> 221 ms, the sphere's band
+// 1.13 -> 1.11 ms.
 constexpr int kUpCols = 4;
 template <class T2>
 constexpr int up_rows() {
