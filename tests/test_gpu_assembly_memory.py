@@ -2,6 +2,8 @@
 layout's panels (24 MB) fit a freed scratch block (28 MB; the device memory cache hands out blocks of up to a quarter more
 than the request), so an assembly that starts from an empty cache leaves less there than the scratch was; with scratch
 and layout side by side it leaves all of it."""
+import gc
+
 import numpy as np
 import pytest
 
@@ -26,6 +28,7 @@ def test_layout_takes_the_scratch(ctx, capi):
     H = g.assemble(k, 1e-13, max_rank, capi.ARH_MIXED)
     assert np.array_equal(H.ranks(), lim)
     del H
+    gc.collect()  # what earlier tests left
     ctx.synchronize()
     capi.device_trim(0)
     assert capi.device_cached(0) == 0

@@ -4,6 +4,8 @@ same terms in another order and by another formula. A term is good to about 1e-1
 test_gpu_grad_pairs.py has 1e-11 for sums over 700 elements, dominated by the neighbours' near-cancelling terms, and the
 rounding of a sum grows like the root of its length): 1e-10 of the gradient's norm for 22,000. The partial sums stay within
 their strip: less than 96 MB in the device memory cache after a call that starts from an empty one."""
+import gc
+
 import numpy as np
 import pytest
 
@@ -32,6 +34,7 @@ def test_strips_against_subsets(ctx, capi, nr, grid):
     def grad(diff):
         return np.stack(g.shape_grad(k, L, diff, nr, X, Lm, VF, capi.ARH_RHS_PLANE, src))
 
+    gc.collect()  # what earlier tests left
     ctx.synchronize()
     capi.device_trim(0)
     full = grad(top)
